@@ -109,6 +109,71 @@ DevArr::~DevArr() {
     if (had) (void)hipSetDevice(cur);
 }
 
+static std::mutex scratch_mu;
+static std::map<int, std::vector<DBuf>> scratch_free;   // per device, smallest first
+
+HvScratch::HvScratch(int device_ordinal, size_t bytes) : device(device_ordinal) {
+    bytes = std::max<size_t>(bytes, 256);
+    {
+        std::lock_guard<std::mutex> lk(scratch_mu);
+        auto& f = scratch_free[device];
+        for (size_t q = 0; q < f.size(); ++q)
+            if (f[q].n >= bytes) {
+                p = f[q].p;
+                n = f[q].n;
+                f.erase(f.begin() + q);
+                return;
+            }
+    }
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        hv_scratch_release(device);   // room held by smaller buffers
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return;
+        }
+    }
+    n = bytes;
+}
+
+HvScratch::~HvScratch() {
+    if (!p) return;
+    std::vector<DBuf> drop;
+    {
+        std::lock_guard<std::mutex> lk(scratch_mu);
+        auto& f = scratch_free[device];
+        size_t at = 0;
+        while (at < f.size() && f[at].n < n) ++at;
+        f.insert(f.begin() + at, DBuf{p, n});
+        size_t total = 0;
+        for (const DBuf& b : f) total += b.n;
+        while (!f.empty() && total > HV_SCRATCH_BYTES) {   // the largest first: small calls are the frequent ones
+            total -= f.back().n;
+            drop.push_back(f.back());
+            f.pop_back();
+        }
+        while ((int)f.size() > HV_SCRATCH_KEEP) {
+            drop.push_back(f.front());
+            f.erase(f.begin());
+        }
+    }
+    for (const DBuf& b : drop) (void)hipFree(b.p);
+}
+
+void hv_scratch_release(int device_ordinal) {
+    std::vector<DBuf> drop;
+    {
+        std::lock_guard<std::mutex> lk(scratch_mu);
+        for (auto& kv : scratch_free)
+            if (kv.first == device_ordinal || device_ordinal < 0) {
+                drop.insert(drop.end(), kv.second.begin(), kv.second.end());
+                kv.second.clear();
+            }
+    }
+    for (const DBuf& b : drop) (void)hipFree(b.p);
+}
+
 double* hv_points_for_write(hv_ctx* c, size_t bytes) {
     if (c->xw && c->xw.use_count() == 1 && c->xw->n >= bytes) return (double*)c->xw->p;
     auto a = std::make_shared<DevArr>();
@@ -617,6 +682,7 @@ static std::mutex batch_mu;
 static std::map<std::pair<int, int>, hv_ctx*> batch_ctx;
 
 int hv_batch_release(int device_ordinal) {
+    hv_scratch_release(device_ordinal);
     std::lock_guard<std::mutex> lk(batch_mu);
     for (auto it = batch_ctx.begin(); it != batch_ctx.end();) {
         if (it->first.first == device_ordinal || device_ordinal < 0) {

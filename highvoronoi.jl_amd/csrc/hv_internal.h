@@ -44,6 +44,24 @@ struct DevArr {
     std::shared_ptr<DevArr> parent;
     ~DevArr();
 };
+// Device scratch of a call that owns no context (exports), for the lifetime of one object.  The
+// buffers come from a process-wide store of at most HV_SCRATCH_KEEP free buffers and
+// HV_SCRATCH_BYTES per device (each used by one call at a time; given back with
+// hv_batch_release); p is null when the device has no room.  The owner waits for its work
+// before the object goes.
+constexpr int HV_SCRATCH_KEEP = 4;
+constexpr size_t HV_SCRATCH_BYTES = (size_t)1 << 30;
+struct HvScratch {
+    int device;
+    void* p = nullptr;
+    size_t n = 0;
+    HvScratch(int device_ordinal, size_t bytes);
+    ~HvScratch();
+    HvScratch(const HvScratch&) = delete;
+    HvScratch& operator=(const HvScratch&) = delete;
+};
+void hv_scratch_release(int device_ordinal);   // frees the store's buffers (every device when negative)
+
 using ImgOrig = std::shared_ptr<const std::vector<int32_t>>;
 using ImgShift = std::shared_ptr<const std::vector<int8_t>>;
 
