@@ -207,6 +207,7 @@ hv_bind_mesh::hv_bind_mesh(hv_ctx* ctx, const hv_mesh* m)
       pnormal(ctx->pnormal), pbc(ctx->pbc), extended(ctx->extended), delta(ctx->delta), rmax(ctx->rmax),
       img_orig(ctx->img_orig), img_shift(ctx->img_shift) {
     c->tree_ok = false;
+    hv_tree_drop(c);
     c->D = m->D;
     c->N = m->N;
     c->nreal = m->nreal;
@@ -224,6 +225,7 @@ hv_bind_mesh::hv_bind_mesh(hv_ctx* ctx, const hv_mesh* m)
 
 hv_bind_mesh::~hv_bind_mesh() {
     c->tree_ok = false;   // a tree built meanwhile belongs to the mesh's generators
+    hv_tree_drop(c);
     c->D = D;
     c->N = N;
     c->nreal = nreal;
@@ -419,6 +421,9 @@ static int set_points_common(hv_ctx* c, int d, int64_t n, const double* xs, hipM
     if (n <= d) return hv_fail(c, HV_ERR_FEW_POINTS, "There are not enough points to create a Voronoi tessellation");
     if (n >= (1ll << 30)) return hv_fail(c, HV_ERR_UNSUPPORTED, "too many generators for 32-bit keys");
     (void)hipSetDevice(c->device);
+    c->tree_ok = false;   // the points may be overwritten in place
+    c->tree_xw.reset();
+    hv_tree_drop(c);
     void* p = hv_points_for_write(c, sizeof(double) * d * n);
     if (!p) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
     if (hipMemcpyAsync(p, xs, sizeof(double) * d * n, kind, c->stream) != hipSuccess)
@@ -434,7 +439,6 @@ static int set_points_common(hv_ctx* c, int d, int64_t n, const double* xs, hipM
     c->N = n;
     c->nreal = n;
     c->extended = false;
-    c->tree_ok = false;
     c->xorig.reset();
     c->img_orig.reset();
     c->img_shift.reset();
@@ -448,6 +452,7 @@ static int restore_originals(hv_ctx* c) {
     if (!c->xorig) return hv_fail(c, HV_ERR_STATE, "the originals of the periodic set are gone");
     c->xw = std::move(c->xorig);
     c->tree_ok = false;
+    hv_tree_drop(c);
     c->N = c->nreal;
     c->extended = false;
     c->img_orig.reset();
@@ -480,6 +485,7 @@ int hv_set_boundary(hv_ctx* c, int nplanes, const double* base, const double* no
         if (!(std::fabs(s - 1.0) <= 1e-12)) return hv_fail(c, HV_ERR_ARG, "boundary normals must have unit length");
     }
     c->tree_ok = false;
+    hv_tree_drop(c);
     c->P = nplanes;
     c->pbase.assign(base, base + (size_t)nplanes * D);
     c->pnormal.assign(normal, normal + (size_t)nplanes * D);
@@ -795,6 +801,7 @@ int hv_build_mesh_batch(int device_ordinal, int32_t nmesh, const int32_t* d, con
             if (c) {
                 (void)hipStreamSynchronize(c->stream);
                 c->tree_ok = false;
+                hv_tree_drop(c);
                 constexpr size_t HV_BATCH_KEEP = (size_t)24 << 30;
                 if (c->pool->total() > HV_BATCH_KEEP) {
                     auto fresh = std::make_shared<DevPool>();

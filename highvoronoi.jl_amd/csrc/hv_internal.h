@@ -110,7 +110,20 @@ struct hv_ctx {
     int tree_leaf = 0;
     DevGeo tree_g{};
     std::shared_ptr<DevArr> tree_xw;
+    // the tables the last tree build left in the pool, for the calls that search the context's
+    // points rather than mesh them (ray batches, queries, a refinement's second search): valid
+    // while base_xw and the planes are the context's (hv_tree_drop)
+    bool base_ok = false;
+    bool base_knn = false;               // the 16-NN lists too
+    unsigned base_tables = 0;            // and these scan tables (bit HV_PREC_*)
+    DevGeo base_g{};
+    std::shared_ptr<DevArr> base_xw;
 };
+
+inline void hv_tree_drop(hv_ctx* c) {
+    c->base_ok = false;
+    c->base_xw.reset();
+}
 
 struct hv_mesh {
     std::shared_ptr<DevPool> pool;   // where the vertex tables go back on free (null: freed)

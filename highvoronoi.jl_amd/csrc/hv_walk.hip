@@ -216,7 +216,7 @@ __global__ void k_tree8_level(DevGeo g, int l, int nodes_at_l, float* __restrict
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const float* b = cb + ((int64_t)cg * 8 + q) * (2 * D);
-            if (!(b[0] < 1e30f)) continue;   // empty grandchild
+            if (b[0] == 1e30f && b[D] == 1e30f) continue;   // empty grandchild
 #pragma unroll
             for (int k = 0; k < D; ++k) { lo[k] = fminf(lo[k], b[k]); hi[k] = fmaxf(hi[k], b[D + k]); }
         }
@@ -2377,7 +2377,7 @@ struct TreeOut {
     const double* dom_lo = nullptr;    // a general polytope's bounding box (null: axis planes)
     const double* dom_hi = nullptr;
     bool unbounded = false;        // no bounded domain (dom_lo / dom_hi: the generators' box)
-    bool defer_tables = false;     // leave the 16-NN lists and the scan tables to a forest-wide pass
+    bool defer_tables = false;     // leave the 16-NN lists and the scan tables to later launches
 };
 
 // Table sizes of a tree over n points in leaves of L
@@ -2398,6 +2398,28 @@ static TreeDims tree_dims(int n, int L) {
     t.ninternal = 0;
     for (int l = 0; l < t.h; ++l) { t.ninternal += pw; pw *= 8; }
     return t;
+}
+
+// the 16-NN lists of one tree
+template <int D>
+int build_knn(hv_ctx* c, const DevGeo& g, int* knn, hipStream_t st) {
+    k_knn64<D, false><<<nblk(g.n, 64), 64, 0, st>>>(g, GeoSet{}, nullptr, knn);
+    HVCK(hipGetLastError());
+    return HV_OK;
+}
+
+// the scan tables of one tree over leaves of 32 points (nothing for HV_PREC_FP64)
+template <int D>
+int build_scan_tables(hv_ctx* c, const DevGeo& g, int tables, double* lorg, hv_u32x4* pkv, float* pxf, hipStream_t st) {
+    if (tables == HV_PREC_FP64) return HV_OK;
+    k_leaf_origin<D, false><<<(g.nleaf + 7) / 8, 64, 0, st>>>(g, GeoSet{}, nullptr, lorg);
+    HVCK(hipGetLastError());
+    if (tables == HV_PREC_BF16)
+        k_point_kvec<D, false><<<nblk((int64_t)g.nleaf * 32, 256), 256, 0, st>>>(g, GeoSet{}, nullptr, lorg, pkv);
+    else
+        k_point_f32<D, false><<<nblk((int64_t)g.nleaf * 32, 256), 256, 0, st>>>(g, GeoSet{}, nullptr, lorg, pxf);
+    HVCK(hipGetLastError());
+    return HV_OK;
 }
 
 // Points -> Morton order + leaf boxes + complete binary tree of boxes + 8-ary child-box tree +
@@ -2500,29 +2522,57 @@ int build_tree_core(hv_ctx* c, int L, int tables, const TreeOut& o, Tree& T, hip
     if (tables == HV_PREC_BF16) g.pkv = (const uint32_t*)o.pkv;
     if (tables == HV_PREC_FP32) g.pxf = o.pxf;
     if (o.defer_tables) return HV_OK;
-    k_knn64<D, false><<<nblk(N, 64), 64, 0, st>>>(g, GeoSet{}, nullptr, o.knn);
-    HVCK(hipGetLastError());
-    if (tables != HV_PREC_FP64) {
-        k_leaf_origin<D, false><<<(g.nleaf + 7) / 8, 64, 0, st>>>(g, GeoSet{}, nullptr, o.lorg);
-        HVCK(hipGetLastError());
-        if (tables == HV_PREC_BF16) {
-            k_point_kvec<D, false><<<nblk((int64_t)g.nleaf * 32, 256), 256, 0, st>>>(g, GeoSet{}, nullptr, o.lorg, o.pkv);
-            HVCK(hipGetLastError());
-        } else {
-            k_point_f32<D, false><<<nblk((int64_t)g.nleaf * 32, 256), 256, 0, st>>>(g, GeoSet{}, nullptr, o.lorg, o.pxf);
-            HVCK(hipGetLastError());
-        }
-    }
-    return HV_OK;
+    int rc = build_knn<D>(c, g, o.knn, st);
+    return rc ? rc : build_scan_tables<D>(c, g, tables, o.lorg, o.pkv, o.pxf, st);
 }
+
+// What a call needs of the tree over the context's points: TREE_FRESH builds all of it, TREE_RAYS
+// (rays start from the 16-NN lists) and TREE_SEARCH (queries, point samples: boxes and points only)
+// take what an earlier call left in the pool over the same points and planes and add what is
+// missing.  The lists are the dearest part (3D N=100k: 0.84 of 1.0 ms), and a program that asks
+// a context many questions about one point set pays for its tree once.
+enum TreeUse { TREE_FRESH, TREE_RAYS, TREE_SEARCH };
 
 // The tree over the context's working set, its tables in the context's pool.
 template <int D>
-int build_tree(hv_ctx* c, int L, Tree& T, int tables = HV_PREC_FP64) {
+int build_tree(hv_ctx* c, int L, Tree& T, int tables = HV_PREC_FP64, TreeUse use = TREE_FRESH) {
     const int N = (int)c->N;
     if (!c->xw) return hv_fail(c, HV_ERR_STATE, "no points set");
     const TreeDims td = tree_dims(N, L);
     TreeOut o;
+    o.knn = pget<int>(c, "knn", use == TREE_SEARCH ? 0 : (size_t)N * HV_KNN);
+    if (tables != HV_PREC_FP64) {
+        o.lorg = pget<double>(c, "lorg", (size_t)((td.nleaf + 7) / 8) * 8);
+        if (tables == HV_PREC_BF16) o.pkv = pget<hv_u32x4>(c, "pkv", (size_t)td.nleaf * 32 * 4);
+        else o.pxf = pget<float>(c, "pxf", (size_t)td.nleaf * 32 * 8);
+        if (!o.lorg || (tables == HV_PREC_BF16 ? !o.pkv : !o.pxf))
+            return hv_fail(c, HV_ERR_DEVICE, "out of device memory (mixed-precision tables)");
+    }
+    if (!o.knn && use != TREE_SEARCH) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (tree)");
+    // the 16-NN lists and the scan tables that are wanted and not there yet
+    auto complete = [&]() -> int {
+        DevGeo& g = c->base_g;
+        if (use != TREE_SEARCH && !c->base_knn) {
+            g.knn = o.knn;
+            const int rc = build_knn<D>(c, g, o.knn, c->stream);
+            if (rc) return rc;
+            c->base_knn = true;
+        }
+        if (tables != HV_PREC_FP64 && !(c->base_tables & (1u << tables))) {
+            g.lorg = o.lorg;
+            if (tables == HV_PREC_BF16) g.pkv = (const uint32_t*)o.pkv;
+            else g.pxf = o.pxf;
+            const int rc = build_scan_tables<D>(c, g, tables, o.lorg, o.pkv, o.pxf, c->stream);
+            if (rc) return rc;
+            c->base_tables |= 1u << tables;
+        }
+        T.g = g;
+        return HV_OK;
+    };
+    if (use != TREE_FRESH && c->base_ok && c->base_xw == c->xw && c->base_g.n == N && c->base_g.L == L) return complete();
+    hv_tree_drop(c);
+    c->base_knn = false;
+    c->base_tables = 0;
     o.xin = (const double*)c->xw->p;
     o.n = N;
     o.goff = 0;
@@ -2562,30 +2612,31 @@ int build_tree(hv_ctx* c, int L, Tree& T, int tables = HV_PREC_FP64) {
     o.xs = pget<double>(c, "xs", (size_t)N * (D + 1));
     o.sidx = pget<int>(c, "sidx", N);
     o.rank_base = pget<int>(c, "rank", N);
-    o.knn = pget<int>(c, "knn", (size_t)N * HV_KNN);
     o.xf = pget<float>(c, "xf", (size_t)N * 8);
     o.blo = pget<double>(c, "blo", (size_t)td.NN * D);
     o.bhi = pget<double>(c, "bhi", (size_t)td.NN * D);
     o.cb = pget<float>(c, "cb8", (size_t)td.ninternal * 8 * 2 * D);
     o.bad = pget<int>(c, "bad", 1);
-    if (!o.pn || !o.ph || !o.xo_base || !o.xs || !o.sidx || !o.rank_base || !o.knn || !o.xf || !o.blo || !o.bhi ||
+    if (!o.pn || !o.ph || !o.xo_base || !o.xs || !o.sidx || !o.rank_base || !o.xf || !o.blo || !o.bhi ||
         !o.cb || !o.bad)
         return hv_fail(c, HV_ERR_DEVICE, "out of device memory (tree)");
-    if (tables != HV_PREC_FP64) {
-        o.lorg = pget<double>(c, "lorg", (size_t)((td.nleaf + 7) / 8) * 8);
-        if (tables == HV_PREC_BF16) o.pkv = pget<hv_u32x4>(c, "pkv", (size_t)td.nleaf * 32 * 4);
-        else o.pxf = pget<float>(c, "pxf", (size_t)td.nleaf * 32 * 8);
-        if (!o.lorg || (tables == HV_PREC_BF16 ? !o.pkv : !o.pxf))
-            return hv_fail(c, HV_ERR_DEVICE, "out of device memory (mixed-precision tables)");
-    }
     HVCK(hipMemsetAsync(o.bad, 0, sizeof(int), c->stream));
-    int rc = build_tree_core<D>(c, L, tables, o, T);
+    o.defer_tables = true;
+    int rc = build_tree_core<D>(c, L, HV_PREC_FP64, o, T);
     if (rc) return rc;
+    T.g.knn = nullptr;
+    c->base_g = T.g;
+    if (use != TREE_SEARCH || tables != HV_PREC_FP64) {
+        rc = complete();
+        if (rc) return rc;
+    }
     int hbad = 0;
     HVCK(hipMemcpyAsync(&hbad, o.bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HVCK(hipStreamSynchronize(c->stream));
     if (hbad & 1) return hv_fail(c, HV_ERR_DOMAIN, "a node does not lie in the domain given by the boundary");
     c->tree_on_plane = hbad != 0;   // the walk refuses it; the queries do not mind
+    c->base_xw = c->xw;
+    c->base_ok = true;
     return HV_OK;
 }
 
@@ -4092,6 +4143,7 @@ static int periodic_mesh(hv_ctx* c, const hv_opts* o, hv_mesh** out, int mask, c
             }
         }
         const int64_t next = (int64_t)iorig.size();
+        hv_tree_drop(c);
         double* xin = hv_points_for_write(c, sizeof(double) * D * next);
         if (!xin) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (periodic images)");
         HVCK(hipMemcpyAsync(xin, ext.data(), sizeof(double) * D * next, hipMemcpyHostToDevice, c->stream));
@@ -4113,6 +4165,7 @@ static int periodic_mesh(hv_ctx* c, const hv_opts* o, hv_mesh** out, int mask, c
         int rc = hv_walk_mesh<D>(c, o, &m, (int)n, cells);
         c->pbase = pbase;
         c->pbc = pbc;
+        hv_tree_drop(c);   // built for the widened box
         if (rc) return rc;
         if (m->nv == 0) {
             hv_mesh_free(m);
@@ -4363,76 +4416,216 @@ __global__ __launch_bounds__(256) void k_setup_rays(int n, const int* __restrict
 }
 
 
+// Queries: one wavefront per query walks the 8-ary tree depth-first, nearest children first.  Eight
+// lanes test a node's child boxes, two leaves of 32 points are measured at once, a point per lane.
+// The boxes are rounded outward and tested in FP64 with the points' own chain of operations, so a
+// box's distance (and its largest <u, x>) bounds those of its points as computed, not only in
+// exact arithmetic: what is skipped could not have changed the result.  Latency is what bounds a
+// query, and a wavefront per query gives small batches a chip's worth of them: 3D N=100k, 1 000
+// half-space queries 18.6 -> 0.09 ms against a thread per query in heap order.
+constexpr int HV_Q_WAVES = 4;    // wavefronts per workgroup, one query each
+constexpr int HV_Q_STACK = 96;   // at most 7 waiting nodes per level (at most 9 levels), 8 on top
+constexpr int HV_Q_LIST = 512;   // hits of one query sorted in LDS (k_inrange)
+
+struct HvQueryStack {
+    int node[HV_Q_STACK];      // level << 27 | node id
+    double d2[HV_Q_STACK];
+    int child[8];              // a last-level node's leaves, nearest first
+    double cd2[8];
+};
+
+// reach(lo, hi, d2): whether the box may hold a wanted point, and its distance^2; limit(): the
+// current bound on the distance^2; leaf(j): every lane with its point (-1: none)
+template <int D, typename Reach, typename Limit, typename Leaf>
+__device__ __forceinline__ void hv_query_walk(const DevGeo& g, HvQueryStack& S, Reach reach, Limit limit, Leaf leaf) {
+    const int lane = threadIdx.x & 63, c = lane & 7;
+    int sp = 1;
+    if (lane == 0) {
+        S.node[0] = 0;
+        S.d2[0] = 0.0;
+    }
+    hv_wave_sync();
+    while (sp > 0) {
+        --sp;
+        const int e = __builtin_amdgcn_readfirstlane(S.node[sp]);
+        const double nd2 = S.d2[sp];
+        if (!(nd2 <= limit())) continue;
+        const int l = e >> 27, gid = e & ((1 << 27) - 1);
+        const float* box = g.cb + ((int64_t)gid * 8 + c) * (2 * D);
+        double lo[D], hi[D], d2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            lo[k] = (double)box[k];
+            hi[k] = (double)box[D + k];
+        }
+        const bool empty = box[0] == 1e30f && box[D] == 1e30f;
+        const bool ok = lane < 8 && !empty && reach(lo, hi, d2);
+        const unsigned m = (unsigned)(__ballot(ok) & 0xffull);
+        if (m == 0u) continue;
+        const int nv = __popc(m);
+        int rk = 0;   // rank among the reached children
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const double dq = __shfl(d2, q);
+            rk += (((m >> q) & 1u) && (dq < d2 || (dq == d2 && q < c))) ? 1 : 0;
+        }
+        const int first = l == 0 ? 0 : ((1 << (3 * l)) - 1) / 7;   // first node id of the level
+        hv_wave_sync();
+        if (l + 1 == g.h) {
+            if (ok) {
+                S.child[rk] = 8 * (gid - first) + c;
+                S.cd2[rk] = d2;
+            }
+            hv_wave_sync();
+            for (int q = 0; q < nv; q += 2) {
+                if (!(S.cd2[q] <= limit())) break;
+                const int half = lane >> 5;
+                const int j = (q + half < nv) ? S.child[q + half] * 32 + (lane & 31) : g.n;
+                leaf(j < g.n ? j : -1);
+            }
+        } else {
+            if (ok) {   // the nearest on top
+                const int at = sp + nv - 1 - rk;
+                S.node[at] = ((l + 1) << 27) | (first + (1 << (3 * l)) + 8 * (gid - first) + c);
+                S.d2[at] = d2;
+            }
+            sp += nv;
+        }
+        hv_wave_sync();
+    }
+}
+
 template <int D>
-__global__ void k_nn_halfspace(DevGeo g, int nq, const double* __restrict__ q, const double* __restrict__ u,
-                               const double* __restrict__ cc, int64_t* __restrict__ idx, double* __restrict__ dist) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nq) return;
+__global__ __launch_bounds__(64 * HV_Q_WAVES) void k_nn_halfspace(DevGeo g, int nq, const double* __restrict__ q,
+                                                                  const double* __restrict__ u,
+                                                                  const double* __restrict__ cc,
+                                                                  int64_t* __restrict__ idx, double* __restrict__ dist) {
+    __shared__ HvQueryStack stk[HV_Q_WAVES];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = blockIdx.x * HV_Q_WAVES + wv;
+    if (t >= nq) return;   // no workgroup barrier below
     double p[D], uu[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) { p[k] = q[(int64_t)t * D + k]; uu[k] = u[(int64_t)t * D + k]; }
     const double c = cc[t];
-    double best = INFINITY;
+    double bound = INFINITY;   // of the whole wavefront
+    double best = INFINITY;    // of this lane's points
     int bi = -1;
-    int node = 1;
-    while (node) {
-        if (hv_box_d2<D>(g, node, p) <= best) {
-            if (node < g.P2) { node = 2 * node; continue; }
-            const int leaf = node - g.P2;
-            const int j0 = leaf * g.L, j1 = min(j0 + g.L, g.n);
-            for (int j = j0; j < j1; ++j) {
+    hv_query_walk<D>(
+        g, stk[wv],
+        [&](const double* lo, const double* hi, double& d2) {
+            double um = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const double a = fmax(fmax(lo[k] - p[k], p[k] - hi[k]), 0.0);
+                d2 = fma(a, a, d2);
+                um = fma(uu[k], uu[k] > 0.0 ? hi[k] : lo[k], um);
+            }
+            return d2 <= bound && um > c;
+        },
+        [&]() { return bound; },
+        [&](int j) {
+            bool better = false;
+            if (j >= 0) {
                 double d2 = 0.0, ux = 0.0;
 #pragma unroll
                 for (int k = 0; k < D; ++k) {
-                    const double xk = g.xs[(int64_t)(j) * (D + 1) + k];
+                    const double xk = g.xs[(int64_t)j * (D + 1) + k];
                     const double a = xk - p[k];
                     d2 = fma(a, a, d2);
                     ux = fma(uu[k], xk, ux);
                 }
-                if (!(ux > c)) continue;
-                const int gi = g.sidx[j];
-                if (d2 < best || (d2 == best && gi < bi)) { best = d2; bi = gi; }
+                if (ux > c && d2 <= bound) {   // equal distances: the smaller id
+                    const int gi = g.sidx[j];
+                    better = d2 < bound;
+                    if (d2 < best || (d2 == best && gi < bi)) { best = d2; bi = gi; }
+                }
             }
-        }
-        node = hv_next_node(node);
+            if (__ballot(better)) {
+                double b = best;
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) b = fmin(b, __shfl_xor(b, off));
+                bound = b;
+            }
+        });
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const double b = __shfl_xor(best, off);
+        const int i = __shfl_xor(bi, off);
+        if (i >= 0 && (bi < 0 || b < best || (b == best && i < bi))) { best = b; bi = i; }
     }
-    idx[t] = bi >= 0 ? (int64_t)bi + 1 : 0;
-    dist[t] = bi >= 0 ? sqrt(best) : INFINITY;
+    if (lane == 0) {
+        idx[t] = bi >= 0 ? (int64_t)bi + 1 : 0;
+        dist[t] = bi >= 0 ? sqrt(best) : INFINITY;
+    }
 }
 
+// out == null: the number of hits per query; otherwise the hits' ids into each query's rows
+// ptr[t] .. ptr[t + 1] - 1 (never past them), ascending where there are at most HV_Q_LIST
 template <int D>
-__global__ void k_inrange(DevGeo g, int nq, const double* __restrict__ q, const double* __restrict__ rad,
-                          const int64_t* __restrict__ ptr, int64_t* __restrict__ out, int64_t* __restrict__ counts) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nq) return;
+__global__ __launch_bounds__(64 * HV_Q_WAVES) void k_inrange(DevGeo g, int nq, const double* __restrict__ q,
+                                                             const double* __restrict__ rad,
+                                                             const int64_t* __restrict__ ptr, int64_t* __restrict__ out,
+                                                             int64_t* __restrict__ counts) {
+    __shared__ HvQueryStack stk[HV_Q_WAVES];
+    __shared__ int list[HV_Q_WAVES][HV_Q_LIST];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = blockIdx.x * HV_Q_WAVES + wv;
+    if (t >= nq) return;   // no workgroup barrier below
     double p[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) p[k] = q[(int64_t)t * D + k];
     const double r2 = rad[t] * rad[t];
+    int64_t* row = out ? out + ptr[t] : nullptr;
+    const int64_t room = out ? ptr[t + 1] - ptr[t] : 0;
+    const bool in_lds = room <= HV_Q_LIST;
     int64_t cnt = 0;
-    const int64_t o = out ? ptr[t] : 0;
-    int node = 1;
-    while (node) {
-        if (hv_box_d2<D>(g, node, p) <= r2) {
-            if (node < g.P2) { node = 2 * node; continue; }
-            const int leaf = node - g.P2;
-            const int j0 = leaf * g.L, j1 = min(j0 + g.L, g.n);
-            for (int j = j0; j < j1; ++j) {
+    hv_query_walk<D>(
+        g, stk[wv],
+        [&](const double* lo, const double* hi, double& d2) {
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const double a = fmax(fmax(lo[k] - p[k], p[k] - hi[k]), 0.0);
+                d2 = fma(a, a, d2);
+            }
+            return d2 <= r2;
+        },
+        [&]() { return r2; },
+        [&](int j) {
+            bool hit = false;
+            if (j >= 0) {
                 double d2 = 0.0;
 #pragma unroll
                 for (int k = 0; k < D; ++k) {
-                    const double a = g.xs[(int64_t)(j) * (D + 1) + k] - p[k];
+                    const double a = g.xs[(int64_t)j * (D + 1) + k] - p[k];
                     d2 = fma(a, a, d2);
                 }
-                if (d2 <= r2) {
-                    if (out) out[o + cnt] = (int64_t)g.sidx[j] + 1;
-                    ++cnt;
+                hit = d2 <= r2;
+            }
+            const unsigned long long m = __ballot(hit);
+            if (out && hit) {
+                const int64_t at = cnt + __popcll(m & ((1ull << lane) - 1ull));
+                if (at < room) {
+                    if (in_lds) list[wv][at] = g.sidx[j];
+                    else row[at] = (int64_t)g.sidx[j] + 1;
                 }
             }
-        }
-        node = hv_next_node(node);
+            cnt += __popcll(m);
+        });
+    if (!out) {
+        if (lane == 0) counts[t] = cnt;
+        return;
     }
-    if (counts) counts[t] = cnt;
+    if (!in_lds) return;
+    // distinct ids: each one's place is the number of smaller ones
+    hv_wave_sync();
+    const int n = (int)(cnt < room ? cnt : room);
+    for (int a = lane; a < n; a += 64) {
+        const int id = list[wv][a];
+        int at = 0;
+        for (int b = 0; b < n; ++b) at += list[wv][b] < id ? 1 : 0;
+        row[at] = (int64_t)id + 1;
+    }
 }
 
 // Interior seed vertices (the reference's descent, src/raycast.jl:45-109, without its random
@@ -4924,7 +5117,7 @@ int hv_raycast_batch_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t
         if (first >= N) return hv_fail(c, HV_ERR_ARG, "the walked edge must contain a generator");
     }
     Tree T;
-    rc = build_tree<D>(c, 32, T, precision);
+    rc = build_tree<D>(c, 32, T, precision, TREE_RAYS);
     if (rc) return rc;
     record_tree(c, T.g, precision, 32);
     DevGeo& g = T.g;
@@ -5192,7 +5385,7 @@ int hv_nn_halfspace_impl(hv_ctx* c, int64_t nq, const double* q, const double* u
                          int64_t* idx, double* dist) {
     if (nq == 0) return HV_OK;
     Tree T;
-    int rc = build_tree<D>(c, 32, T);
+    int rc = build_tree<D>(c, 32, T, HV_PREC_FP64, TREE_SEARCH);
     if (rc) return rc;
     double* dq = pget<double>(c, "q_q", (size_t)nq * D);
     double* du_ = pget<double>(c, "q_u", (size_t)nq * D);
@@ -5203,7 +5396,7 @@ int hv_nn_halfspace_impl(hv_ctx* c, int64_t nq, const double* q, const double* u
     HVCK(hipMemcpyAsync(dq, q, sizeof(double) * nq * D, hipMemcpyHostToDevice, c->stream));
     HVCK(hipMemcpyAsync(du_, u, sizeof(double) * nq * D, hipMemcpyHostToDevice, c->stream));
     HVCK(hipMemcpyAsync(dc, cc, sizeof(double) * nq, hipMemcpyHostToDevice, c->stream));
-    k_nn_halfspace<D><<<nblk(nq, 128), 128, 0, c->stream>>>(T.g, (int)nq, dq, du_, dc, di, dd);
+    k_nn_halfspace<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, dq, du_, dc, di, dd);
     HVCK(hipGetLastError());
     HVCK(hipMemcpyAsync(idx, di, sizeof(int64_t) * nq, hipMemcpyDeviceToHost, c->stream));
     HVCK(hipMemcpyAsync(dist, dd, sizeof(double) * nq, hipMemcpyDeviceToHost, c->stream));
@@ -5216,7 +5409,7 @@ int hv_inrange_impl(hv_ctx* c, int64_t nq, const double* q, const double* radius
     ptr[0] = 0;
     if (nq == 0) return HV_OK;
     Tree T;
-    int rc = build_tree<D>(c, 32, T);
+    int rc = build_tree<D>(c, 32, T, HV_PREC_FP64, TREE_SEARCH);
     if (rc) return rc;
     double* dq = pget<double>(c, "q_q", (size_t)nq * D);
     double* dr = pget<double>(c, "q_r", nq);
@@ -5226,7 +5419,7 @@ int hv_inrange_impl(hv_ctx* c, int64_t nq, const double* q, const double* radius
     HVCK(hipMemcpyAsync(dq, q, sizeof(double) * nq * D, hipMemcpyHostToDevice, c->stream));
     HVCK(hipMemcpyAsync(dr, radius, sizeof(double) * nq, hipMemcpyHostToDevice, c->stream));
     if (!idx) {
-        k_inrange<D><<<nblk(nq, 128), 128, 0, c->stream>>>(T.g, (int)nq, dq, dr, nullptr, nullptr, dcnt);
+        k_inrange<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, dq, dr, nullptr, nullptr, dcnt);
         HVCK(hipGetLastError());
         std::vector<int64_t> cnt(nq);
         HVCK(hipMemcpyAsync(cnt.data(), dcnt, sizeof(int64_t) * nq, hipMemcpyDeviceToHost, c->stream));
@@ -5238,11 +5431,12 @@ int hv_inrange_impl(hv_ctx* c, int64_t nq, const double* q, const double* radius
     int64_t* dout = pget<int64_t>(c, "q_out", std::max<int64_t>(total, 1));
     if (!dout) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
     HVCK(hipMemcpyAsync(dptr, ptr, sizeof(int64_t) * (nq + 1), hipMemcpyHostToDevice, c->stream));
-    k_inrange<D><<<nblk(nq, 128), 128, 0, c->stream>>>(T.g, (int)nq, dq, dr, dptr, dout, nullptr);
+    k_inrange<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, dq, dr, dptr, dout, nullptr);
     HVCK(hipGetLastError());
     if (total) HVCK(hipMemcpyAsync(idx, dout, sizeof(int64_t) * total, hipMemcpyDeviceToHost, c->stream));
     HVCK(hipStreamSynchronize(c->stream));
-    for (int64_t k = 0; k < nq; ++k) std::sort(idx + ptr[k], idx + ptr[k + 1]);
+    for (int64_t k = 0; k < nq; ++k)
+        if (ptr[k + 1] - ptr[k] > HV_Q_LIST) std::sort(idx + ptr[k], idx + ptr[k + 1]);
     return HV_OK;
 }
 
@@ -5278,7 +5472,7 @@ int hv_mc_points_impl(hv_ctx* c, int64_t nsamples, uint64_t seed, double slab, c
             c->pbc[2 * k] = c->pbc[2 * k + 1] = 0;
         }
     Tree T;
-    rc = build_tree<D>(c, 32, T);
+    rc = build_tree<D>(c, 32, T, HV_PREC_FP64, TREE_SEARCH);
     c->pbase = pbase;
     c->pbc = pbc;
     if (rc) return rc;
@@ -5446,7 +5640,7 @@ int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** o
     const int nold = (int)old->N;
     const int shift = (int)(c->N - old->N);
     Tree T;
-    int rc = build_tree<D>(c, 32, T);
+    int rc = build_tree<D>(c, 32, T, HV_PREC_FP64, TREE_SEARCH);   // the walk of the new cells left it
     if (rc) return rc;
     const int nv0 = (int)old->nv;
     uint8_t* keep = pget<uint8_t>(c, "rf_keep", std::max(nv0, 1));

@@ -255,6 +255,10 @@ int hv_raycast_batch_keys(hv_ctx* ctx, int precision, int64_t nrays, const int64
 int hv_raycast_batch_noalloc(hv_ctx* ctx, int precision, int64_t nrays, const int64_t* sig, const int32_t* drop,
                              const double* r, int64_t* out_sig, double* out_r, double* out_t, int32_t* out_status);
 
+/* The ray batches and the queries below search a tree over the context's points; it is built by
+ * the first of them (or by a mesh build) and kept by the context until its points or planes
+ * change or it integrates. */
+
 /* Half-space nearest neighbour (src/extended.jl:108-142 with the predicate of
  * src/raycast.jl:385-392): for query k, the generator minimising |x - q_k| among
  * those with <x, u_k> > c_k (c_k = -inf disables the filter).  idx is 1-based
