@@ -7,17 +7,23 @@
 //   * in general position every subset S of a vertex key that holds a generator is a
 //     face; faces with |S| = m have dimension k = d + 1 - m and are identified by their
 //     generator set, packed into 128 bits (21 bits per id);
-//   * pass m: emit the (S, vertex) incidences of every vertex, radix-sort by S, run heads
-//     give the faces and their vertex lists;
+//   * the (k-1)-faces of S are the faces T = S + {j}, so pass m takes the faces T of pass m + 1
+//     (the vertices before the first pass, m = d), emits the pair (S, T) for each S = T - {j},
+//     and groups the pairs by S: the groups are the faces of pass m, each with its list of T;
 //   * edges (m = d) measure |v_a - v_b|; a face of dimension k > 1 is the union of cones
-//     from one of its vertices p over its (k-1)-faces T = S + {j} that miss p:
+//     from one of its vertices p over its (k-1)-faces T that miss p:
 //     |F_S| = (1/k) sum_T h(p, aff F_T) |F_T|, h measured inside aff F_S;
-//   * a sub-face T is found from a vertex v of S that holds j: T is the subset of v's key
-//     with S's positions and j's, whose incidence (v, subset) the pass m + 1 maps to its face
-//     (one load; the map also says whether v is T's first vertex, which takes T once);
+//   * p is the smallest vertex of S, so T holds it exactly when it is T's smallest vertex too;
 //   * facets (m = 2) are the interfaces A_ik; volumes take the generator as apex.
-// 1, 16 or 64 lanes per face read its children in a fixed order: no atomics, the result does
-// not depend on scheduling.
+// A face's T are read in a fixed order: no atomics, the result does not depend on scheduling.
+//
+// Grouping is what moves the most bytes, so it sorts 32-bit keys: the face's smallest id above 15
+// bits of a hash of its ids (4 radix passes of 8 bytes per pair; the whole key in 42 .. 105
+// bits took 6 .. 14 passes of 12).  About one face in a hundred shares its 32 bits with another
+// of its cell; such runs are put in order by their full keys afterwards.  Pairs (S, T) instead of
+// (S, vertex) are fewer from the 3-faces down and need no look-up of the sub-faces.
+// 5D N=100k mixture (16.3M vertices): the integration's kernels 207 -> 77 ms (the sorts 70 -> 22,
+// the measures 74 -> 20, the look-up tables of the former 31 -> 0).
 //
 // Monte-Carlo integrator (src/mcintegrator.jl:98-204): one workgroup per cell casts ndir
 // rays from the generator (mc_raycast, :207-226) against the cell's neighbours (boundary
@@ -28,7 +34,9 @@
 #include "hv_device.h"
 #include "hv_internal.h"
 #include <hipcub/hipcub.hpp>
+#include <rocprim/rocprim.hpp>
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <numeric>
 
@@ -46,199 +54,254 @@ static T* iget(hv_ctx* c, const char* name, size_t count) {
     return (T*)c->pool->get(name, std::max<size_t>(1, count) * sizeof(T), false, c->stream);
 }
 
-constexpr uint64_t HV_F21 = 0x1FFFFFull;   // id field; all ones = empty slot
-// face incidences one pass of a chunk may hold (a chunk of cells at a time beyond)
+constexpr uint64_t HV_F21 = 0x1FFFFFull;   // id field of a face key
+// pairs one pass of a chunk may hold (a chunk of cells at a time beyond)
 constexpr int64_t HV_INC_BUDGET = 1600000000ll;
+constexpr int HV_GROUP_HASH = 15;          // hash bits of a grouping key
+constexpr uint32_t HV_NO_FACE = 0xffffffffu;
 
-__device__ __forceinline__ void hv_fkey_put(uint64_t& lo, uint64_t& hi, int s, uint64_t id) {
-    if (s < 3) lo = (lo & ~(HV_F21 << (21 * s))) | (id << (21 * s));
-    else hi = (hi & ~(HV_F21 << (21 * (s - 3)))) | (id << (21 * (s - 3)));
-}
-__device__ __forceinline__ int hv_fkey_get(uint64_t lo, uint64_t hi, int s) {
-    return (int)(s < 3 ? (lo >> (21 * s)) & HV_F21 : (hi >> (21 * (s - 3))) & HV_F21);
-}
-// (hi, lo) lexicographic: the order the two-pass radix sort leaves
-__device__ __forceinline__ bool hv_fkey_less(uint64_t ah, uint64_t al, uint64_t bh, uint64_t bl) {
-    return ah < bh || (ah == bh && al < bl);
-}
-
-// dense copy of the live vertex records
+// used ids of the mesh's keys (a first pass over the live vertices)
 template <int D>
-__global__ void k_int_gather(const int* __restrict__ ids, int nv, const int* __restrict__ key,
-                             const double* __restrict__ x, int* __restrict__ vk, double* __restrict__ vc) {
+__global__ void k_mark_used(const int* __restrict__ ids, int nv, const int* __restrict__ key, int* __restrict__ used) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)nv * (D + 1)) return;
+    const int v = (int)(t / (D + 1)), j = (int)(t - (int64_t)v * (D + 1));
+    used[key[(int64_t)ids[v] * (D + 1) + j]] = 1;
+}
+
+// word of the dense ids first .. first + count - 1 of each key (first id most significant), for
+// the vertices in the order of perm (null: their own order, and perm0 receives 0, 1, ..)
+template <int D>
+__global__ void k_vkey_word(const int* __restrict__ ids, int nv, const int* __restrict__ key, const int* __restrict__ dense,
+                            const int* __restrict__ perm, int first, int count, int bits, uint64_t* __restrict__ word,
+                            int* __restrict__ perm0) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= nv) return;
-    const int s = ids[v];
-#pragma unroll
-    for (int j = 0; j <= D; ++j) vk[(int64_t)v * (D + 1) + j] = key[(int64_t)s * (D + 1) + j];
-#pragma unroll
-    for (int k = 0; k < D; ++k) vc[(int64_t)v * D + k] = x[(int64_t)s * D + k];
+    const int* k = key + (int64_t)ids[perm ? perm[v] : v] * (D + 1);
+    uint64_t w = 0;
+    for (int j = 0; j < count; ++j) w = (w << bits) | (uint64_t)(uint32_t)dense[k[first + j]];
+    word[v] = w;
+    if (!perm) perm0[v] = v;
 }
 
-// packed key words of each vertex (21 bits per id): word 0 holds ids 0..2, word 1 ids 3..5,
-// word 2 id 6; sorting by (w0, w1, w2) gives a numbering fixed by the vertex set alone
+// the live vertices in the order of perm: keys in dense ids, coordinates
 template <int D>
-__global__ void k_vkey_words(const int* __restrict__ vk, int nv, uint64_t* __restrict__ w0, uint64_t* __restrict__ w1,
-                             uint64_t* __restrict__ w2, int* __restrict__ idx) {
+__global__ void k_int_permute(const int* __restrict__ perm, int nv, const int* __restrict__ ids, const int* __restrict__ key,
+                              const int* __restrict__ dense, const double* __restrict__ x, int* __restrict__ vk,
+                              double* __restrict__ vc) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= nv) return;
-    uint64_t a = 0, b = 0, c = 0;
+    const int64_t s = ids[perm[v]];
 #pragma unroll
-    for (int j = 0; j <= D; ++j) {
-        const uint64_t id = (uint64_t)vk[(int64_t)v * (D + 1) + j];
-        if (j < 3) a |= id << (21 * (2 - j));
-        else if (j < 6) b |= id << (21 * (5 - j));
-        else c = id;
-    }
-    w0[v] = a;
-    w1[v] = b;
-    w2[v] = c;
-    idx[v] = v;
+    for (int j = 0; j <= D; ++j) vk[(int64_t)v * (D + 1) + j] = dense[key[s * (D + 1) + j]];
+#pragma unroll
+    for (int k = 0; k < D; ++k) vc[(int64_t)v * D + k] = x[s * D + k];
 }
 
-template <int D>
-__global__ void k_int_permute(const int* __restrict__ perm, int nv, const int* __restrict__ vk, const double* __restrict__ vc,
-                              int* __restrict__ vk2, double* __restrict__ vc2) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-    const int s = perm[v];
-#pragma unroll
-    for (int j = 0; j <= D; ++j) vk2[(int64_t)v * (D + 1) + j] = vk[(int64_t)s * (D + 1) + j];
-#pragma unroll
-    for (int k = 0; k < D; ++k) vc2[(int64_t)v * D + k] = vc[(int64_t)s * D + k];
-}
-
-// k_face_emit numbers the m-subsets of a key by their position masks in increasing order: the
-// c-th mask of popcount m (those below 2^(d+1) come first, so one list serves every d)
-struct HvMaskList {
-    unsigned char m[8][36];
-    constexpr HvMaskList() : m{} {
-        int cnt[8] = {};
-        for (int mask = 0; mask < 128; ++mask) {
-            int p = 0;
-            for (int b = 0; b < 7; ++b) p += (mask >> b) & 1;
-            m[p][cnt[p]++] = (unsigned char)mask;
-        }
-    }
+// ---- faces and their lists -------------------------------------------------------------------
+// The faces of one pass: keys (ids 0 .. 2 of the sorted set in klo, 3 .. 5 in khi, 21 bits each),
+// and per face its measure, its smallest vertex (canonical order) and its number of vertices.
+struct HvFace {
+    double meas;
+    int vmin, nv;
 };
-__constant__ HvMaskList hv_mask_list = HvMaskList();
+struct HvFaces {
+    uint64_t* klo;
+    uint64_t* khi;
+    HvFace* f;
+};
+// The pairs of pass m sorted by face: pair i belongs to T = pay[i] / (m + 1) with T's id jl[i]
+// left out; face f holds the pairs start[f] .. start[f + 1] - 1 (the last one to *nvalid - 1).
+struct HvPairs {
+    const uint32_t* pay;
+    const int* jl;
+    const int* start;
+    const int* nvalid;
+    int nface;
+};
 
-// (face, vertex) incidences of pass m, one thread each (contiguous stores): incidence
-// o = v * C + c is the c-th m-subset of vertex v's key; one holding no cell of the chunk (cmask
-// over the ids; ids below N are generators) gets the all-ones key, which sorts past the end
-// (k_first_sent counts them after the sort: no same-address atomics here)
-template <int D>
-__global__ void k_face_emit(const int* __restrict__ vk, int nv, int m, int N, const uint8_t* __restrict__ cmask, int C,
-                            uint64_t* __restrict__ lo, uint64_t* __restrict__ hi, int* __restrict__ idx) {
-    const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (o < (int64_t)nv * C) {
-        const int v = (int)(o / C), c = (int)(o - (int64_t)v * C);
-        const int mask = hv_mask_list.m[m][c];
-        const int* k = vk + (int64_t)v * (D + 1);
-        uint64_t l = ~0ull, h = ~0ull;
-        int s = 0;
-        bool real = false;
+// ids of T: a vertex (M == D: its key's row) or a face of pass M + 1
+template <int D, int M>
+__device__ __forceinline__ void hv_sub_ids(const int* __restrict__ vk, const HvFaces& F1, int64_t t, int* id) {
+    if constexpr (M == D) {
 #pragma unroll
-        for (int j = 0; j <= D; ++j) {
-            if ((mask >> j) & 1) {
-                const int id = k[j];
-                real = real || (id < N && cmask[id] != 0);
-                hv_fkey_put(l, h, s, (uint64_t)id);
-                ++s;
+        for (int j = 0; j <= M; ++j) id[j] = vk[t * (D + 1) + j];
+    } else {
+        const uint64_t lo = F1.klo[t];
+        uint64_t hi = 0;
+        if constexpr (M + 1 > 3) hi = F1.khi[t];
+#pragma unroll
+        for (int j = 0; j <= M; ++j) id[j] = (int)((j < 3 ? lo >> (21 * j) : hi >> (21 * (j - 3))) & HV_F21);
+    }
+}
+// packed key of T without its p-th id, and that id
+template <int M>
+__device__ __forceinline__ int hv_face_key(const int* id, int p, uint64_t& lo, uint64_t& hi) {
+    lo = hi = 0;
+    int out = id[0];
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        const uint64_t v = (uint64_t)(uint32_t)(j < p ? id[j] : id[j + 1]);
+        if (j < 3) lo |= v << (21 * j);
+        else hi |= v << (21 * (j - 3));
+    }
+#pragma unroll
+    for (int j = 1; j <= M; ++j) out = j == p ? id[j] : out;
+    return out;
+}
+
+// hash of each dense id, from the id it stands for (the order of a face's T then does not depend
+// on which cells a mesh or a chunk holds)
+__global__ void k_id_hash(const int* __restrict__ gid, int n, uint32_t* __restrict__ hid) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) hid[i] = (uint32_t)(hv_mix64((uint64_t)gid[i] + 0x9e3779b97f4a7c15ull) >> 32);
+}
+
+// Grouping keys of the pairs (S = T - {its p-th id}, T), pair t (M + 1) + p, one thread per T: S's
+// smallest id above hb bits of the hash of its ids (a sum over the ids, so that T's M + 1 subsets
+// share it).  HV_NO_FACE, which sorts past the end, where S holds no cell of the chunk (cmask over
+// the ids below N; null: every generator): such a face may be incomplete here.
+template <int D, int M>
+__global__ __launch_bounds__(256) void k_pair_emit(const int* __restrict__ vk, HvFaces F1, int nt, int N,
+                                                   const uint8_t* __restrict__ cmask, const uint32_t* __restrict__ hid,
+                                                   int hb, uint32_t* __restrict__ key) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nt) return;
+    int id[M + 1];
+    hv_sub_ids<D, M>(vk, F1, t, id);
+    uint32_t h[M + 1], sum = 0;
+    int cells = 0, cell[M + 1];
+#pragma unroll
+    for (int j = 0; j <= M; ++j) {
+        h[j] = hid[id[j]];
+        sum += h[j];
+        cell[j] = id[j] < N && (!cmask || cmask[id[j]] != 0) ? 1 : 0;
+        cells += cell[j];
+    }
+#pragma unroll
+    for (int p = 0; p <= M; ++p) {
+        const uint32_t a = (uint32_t)(p == 0 ? id[1] : id[0]);
+        const uint32_t hs = ((sum - h[p]) * 0x9E3779B1u) >> (32 - hb);
+        key[(int64_t)t * (M + 1) + p] = cells > cell[p] ? ((a << hb) | hs) : HV_NO_FACE;
+    }
+}
+
+// Sorted pairs -> first pair of every face, the id each pair leaves out, the number of pairs of
+// real faces, and the runs of one grouping key that hold more than one face (runs: their first
+// pairs, at their first change of face)
+template <int D, int M>
+__global__ __launch_bounds__(256) void k_pair_heads(const uint32_t* __restrict__ key, const uint32_t* __restrict__ pay,
+                                                    int64_t n, const int* __restrict__ vk, HvFaces F1,
+                                                    uint8_t* __restrict__ head, int* __restrict__ jl,
+                                                    int* __restrict__ nvalid, int* __restrict__ runs,
+                                                    int* __restrict__ nrun) {
+    __shared__ uint64_t slo[257], shi[M > 3 ? 257 : 1];
+    __shared__ uint32_t sk[257];
+    __shared__ int cnt, base;
+    const int64_t i0 = (int64_t)blockIdx.x * 256, i = i0 + threadIdx.x;
+    if (threadIdx.x == 0) cnt = 0;
+    auto stage = [&](int64_t q, int at) {   // pair q's grouping key and face key
+        const uint32_t k = key[q];
+        uint64_t lo = 0, hi = 0;
+        int j = 0;
+        if (k != HV_NO_FACE) {
+            int id[M + 1];
+            const uint32_t e = pay[q], t = e / (M + 1);
+            hv_sub_ids<D, M>(vk, F1, t, id);
+            j = hv_face_key<M>(id, (int)(e - t * (M + 1)), lo, hi);
+        }
+        sk[at] = k;
+        slo[at] = lo;
+        if constexpr (M > 3) shi[at] = hi;
+        return j;
+    };
+    int j = 0;
+    if (i < n) j = stage(i, threadIdx.x + 1);
+    if (threadIdx.x == 0 && i0 > 0) stage(i0 - 1, 0);
+    __syncthreads();
+    int start = -1;
+    if (i < n) {
+        const uint32_t k = sk[threadIdx.x + 1];
+        const bool prev = i > 0, samek = prev && sk[threadIdx.x] == k;
+        auto differs = [&](int x) {   // pairs x and x + 1 of the staged ones
+            bool d = slo[x] != slo[x + 1];
+            if constexpr (M > 3) d = d || shi[x] != shi[x + 1];
+            return d;
+        };
+        const bool change = !samek || differs(threadIdx.x);
+        if (k == HV_NO_FACE) {
+            head[i] = 0;
+            if (!samek) *nvalid = (int)i;
+        } else {
+            head[i] = change ? 1 : 0;
+            jl[i] = j;
+            if (samek && change) {
+                // the run's first change of face: none between the run's first pair and here
+                int64_t q = i - 1;
+                bool earlier = false;
+                uint64_t plo = slo[threadIdx.x], phi = 0;
+                if constexpr (M > 3) phi = shi[threadIdx.x];
+                while (q > 0 && key[q - 1] == k && !earlier) {
+                    --q;
+                    uint64_t lo, hi;
+                    int id[M + 1];
+                    const uint32_t e = pay[q], t = e / (M + 1);
+                    hv_sub_ids<D, M>(vk, F1, t, id);
+                    hv_face_key<M>(id, (int)(e - t * (M + 1)), lo, hi);
+                    earlier = lo != plo || hi != phi;
+                }
+                if (!earlier) start = (int)q;
             }
         }
-        if (!real) { l = ~0ull; h = ~0ull; }
-        lo[o] = l;
-        hi[o] = h;
-        idx[o] = (int)o;
     }
+    int at = -1;
+    if (start >= 0) at = atomicAdd(&cnt, 1);
+    __syncthreads();
+    if (threadIdx.x == 0) base = cnt ? atomicAdd(nrun, cnt) : 0;
+    __syncthreads();
+    if (at >= 0) runs[base + at] = start;
 }
 
-// incidences sent past the end of a sorted pass (lo in sorted order: all ones exactly for them,
-// a real key's first id is below all ones): n minus the first such position, by bisection
-__global__ void k_first_sent(const uint64_t* __restrict__ lo, int64_t n, unsigned long long* __restrict__ nsent) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    int64_t a = 0, b = n;
-    while (a < b) {
-        const int64_t mid = (a + b) >> 1;
-        if (lo[mid] == ~0ull) b = mid;
-        else a = mid + 1;
-    }
-    *nsent = (unsigned long long)(n - a);
-}
-
-__global__ void k_gather_u64(const uint64_t* __restrict__ src, const int* __restrict__ perm, int64_t n,
-                             uint64_t* __restrict__ dst) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[perm[i]];
-}
-
-// sorted incidences -> run heads; incidence o belongs to vertex o / C
-__global__ void k_face_heads(const uint64_t* __restrict__ lo, const uint64_t* __restrict__ hi,
-                             const int* __restrict__ perm, int64_t n, int C, int* __restrict__ vid,
-                             uint8_t* __restrict__ head) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    vid[i] = perm[i] / C;
-    head[i] = (i == 0 || lo[i] != lo[i - 1] || hi[i] != hi[i - 1]) ? 1 : 0;
-}
-
-__global__ void k_iota64(int* __restrict__ a, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = (int)i;
-}
-
-// face table of a pass: key, first incidence, apex vertex
-__global__ void k_face_table(const int* __restrict__ fstart, int nface, const uint64_t* __restrict__ lo,
-                             const uint64_t* __restrict__ hi, uint64_t* __restrict__ flo, uint64_t* __restrict__ fhi) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nface) return;
-    flo[f] = lo[fstart[f]];
-    fhi[f] = hi[fstart[f]];
-}
-
-// k_face_emit numbers the m-subsets of a key by their position masks in increasing order, so
-// the subset with mask M is the rank of M among the masks of its popcount
-struct HvMaskRank {
-    unsigned char r[256];
-    constexpr HvMaskRank() : r{} {
-        int cnt[9] = {};
-        for (int mask = 0; mask < 256; ++mask) {
-            int p = 0;
-            for (int b = 0; b < 8; ++b) p += (mask >> b) & 1;
-            r[mask] = (unsigned char)cnt[p]++;
+// A run of one grouping key with several faces: its pairs sorted by face (stably: each face's T
+// stay ascending), one thread per run
+template <int D, int M>
+__global__ __launch_bounds__(64) void k_pair_fix(const uint32_t* __restrict__ key, int64_t n, const int* __restrict__ vk,
+                                                 HvFaces F1, const int* __restrict__ runs, const int* __restrict__ nrun,
+                                                 uint32_t* __restrict__ pay, uint8_t* __restrict__ head, int* __restrict__ jl) {
+    const int nr = *nrun;
+    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < nr; r += gridDim.x * blockDim.x) {
+        const int64_t b = runs[r];
+        const uint32_t k = key[b];
+        auto face = [&](uint32_t e, uint64_t& lo, uint64_t& hi) {
+            int id[M + 1];
+            const uint32_t t = e / (M + 1);
+            hv_sub_ids<D, M>(vk, F1, t, id);
+            return hv_face_key<M>(id, (int)(e - t * (M + 1)), lo, hi);
+        };
+        int64_t e = b + 1;
+        for (; e < n && key[e] == k; ++e) {
+            const uint32_t x = pay[e];
+            uint64_t xl, xh;
+            face(x, xl, xh);
+            int64_t q = e;
+            while (q > b) {
+                uint64_t yl, yh;
+                face(pay[q - 1], yl, yh);
+                if (!(yh > xh || (yh == xh && yl > xl))) break;
+                pay[q] = pay[q - 1];
+                --q;
+            }
+            pay[q] = x;
+        }
+        uint64_t pl = 0, ph = 0;
+        for (int64_t q = b; q < e; ++q) {
+            uint64_t lo, hi;
+            jl[q] = face(pay[q], lo, hi);
+            head[q] = (q == b || lo != pl || hi != ph) ? 1 : 0;
+            pl = lo;
+            ph = hi;
         }
     }
-};
-__constant__ HvMaskRank hv_mask_rank = HvMaskRank();
-
-// face of each incidence of a pass (incidence o = vertex * C + subset): f for the face's first
-// incidence (its smallest vertex), ~f for the others; the parent pass finds a sub-face
-// S + {j} of a face S from one of its vertices with one load
-__global__ void k_face_inc(const int* __restrict__ fstart, int nface, const int* __restrict__ perm,
-                           int* __restrict__ foi) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nface) return;
-    const int b = fstart[f], e = fstart[f + 1];
-    foi[perm[b]] = f;
-    for (int i = b + 1; i < e; ++i) foi[perm[i]] = ~f;
-}
-
-template <int D>
-__global__ void k_edge_len(const int* __restrict__ fstart, int nface, const int* __restrict__ vid,
-                           const double* __restrict__ vc, double* __restrict__ meas, int* __restrict__ bad) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nface) return;
-    const int b = fstart[f], e = fstart[f + 1];
-    if (e - b != 2) { atomicOr(bad, 1); meas[f] = 0.0; return; }
-    const int va = vid[b], vb = vid[b + 1];
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < D; ++k) {
-        const double t = vc[(int64_t)va * D + k] - vc[(int64_t)vb * D + k];
-        s = fma(t, t, s);
-    }
-    meas[f] = sqrt(s);
 }
 
 struct IntGeo {
@@ -261,192 +324,162 @@ __device__ __forceinline__ void hv_face_grad(const IntGeo& g, int a, int b, doub
     }
 }
 
-// Sub-face references of the incidences of a pass, written in incidence order (vertex-major:
-// a vertex's key and its row of the previous pass's incidence-to-face map are read once for
-// all its subsets, contiguously), so that the measure of a face reads one record per vertex
-// instead of the vertex's key and that row.  Entry q of incidence o (the q-th key position e
-// not in the subset, ascending): the id j = key[e] in the low word, the pass-(m + 1) map entry
-// of the subset + {e} in the high word; the ne = d + 1 - m entries of an incidence lie together
-// at p[o * ne] (faces of m >= d - 3 ids: at most four entries, in the four key arrays' space).
-struct HvRec {
-    uint64_t* p;
-    int ne;
-};
-
-template <int D>
-__global__ void k_face_rec(const int* __restrict__ vk, int64_t tot, int m, int C, int C1, const int* __restrict__ foi1,
-                           HvRec rec) {
-    const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= tot) return;
-    const int64_t v = o / C;
-    const int mask = hv_mask_list.m[m][(int)(o - v * C)];
-    const int* kv = vk + v * (D + 1);
-    int q = 0;
+// w minus its components along the R orthonormal vectors Q (two Gram-Schmidt passes); its norm
+template <int D, int R>
+__device__ __forceinline__ double hv_project(double (*Q)[D], double* w) {
 #pragma unroll
-    for (int e = 0; e <= D; ++e) {
-        if ((mask >> e) & 1) continue;
-        const int x = foi1[v * C1 + hv_mask_rank.r[mask | (1 << e)]];
-        rec.p[o * rec.ne + q] = (uint64_t)(uint32_t)kv[e] | ((uint64_t)(uint32_t)x << 32);
-        ++q;
-    }
+    for (int pass = 0; pass < 2; ++pass)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            double cdot = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) cdot = fma(w[k], Q[r][k], cdot);
+#pragma unroll
+            for (int k = 0; k < D; ++k) w[k] = fma(-cdot, Q[r][k], w[k]);
+        }
+    double nw = 0.0;
+#pragma unroll
+    for (int k = 0; k < D; ++k) nw = fma(w[k], w[k], nw);
+    return sqrt(nw);
 }
 
-// Measure of each face of pass m from the faces of pass m + 1.  L lanes per face (1, 16 or 64),
-// splitting the face's vertex list (faces of many vertices: the facets and ridges of cells in
-// 5D and up), the partial sums reduced in a fixed order.  (A dispatch holds at most 2^32
-// work-items, so the L > 1 forms walk the faces grid-stride.)
-template <int D, int L>
-__device__ __forceinline__ void hv_face_measure_one(int f, int lane, int step, const IntGeo& g, int m,
-                                                    const int* __restrict__ fstart, const int* __restrict__ vid,
-                                                    const uint64_t* __restrict__ flo, const uint64_t* __restrict__ fhi,
-                                                    int nface1, int C1, const int* __restrict__ foi1,
-                                                    const double* __restrict__ meas1,
-                                                    const int* __restrict__ vk, const double* __restrict__ vc,
-                                                    const int* __restrict__ perm, const HvRec& rec,
-                                                    double* __restrict__ meas, int* __restrict__ bad) {
-    const uint64_t lo = flo[f], hi = fhi[f];
-    int S[D + 1];
-#pragma unroll
-    for (int s = 0; s <= D; ++s) S[s] = s < m ? hv_fkey_get(lo, hi, s) : -1;
-    const int a = S[0];   // ids sorted: generators before planes, the face holds one
-    // orthonormal basis of the face's constraint normals (two Gram-Schmidt passes)
-    double Q[D][D];
-    int q = 0;
-#pragma unroll
-    for (int s = 1; s < D + 1; ++s) {
-        if (s >= m) break;
+// orthonormal basis Q (M - 1 vectors) of the constraint normals of a face with the ids S
+template <int D, int M, int S0 = 1>
+__device__ __forceinline__ bool hv_face_basis(const IntGeo& g, const int* S, double (*Q)[D]) {
+    if constexpr (S0 < M) {
         double w[D];
-        hv_face_grad<D>(g, a, S[s], w);
-        for (int pass = 0; pass < 2; ++pass)
+        hv_face_grad<D>(g, S[0], S[S0], w);
+        const double nw = hv_project<D, S0 - 1>(Q, w);
+        if (!(nw > 0.0)) return false;
 #pragma unroll
-            for (int r = 0; r < D - 1; ++r) {   // r < q, unrolled: Q stays in registers
-                if (r >= q) break;
-                double cdot = 0.0;
-#pragma unroll
-                for (int k = 0; k < D; ++k) cdot = fma(w[k], Q[r][k], cdot);
-#pragma unroll
-                for (int k = 0; k < D; ++k) w[k] = fma(-cdot, Q[r][k], w[k]);
-            }
-        double nw = 0.0;
-#pragma unroll
-        for (int k = 0; k < D; ++k) nw = fma(w[k], w[k], nw);
-        nw = sqrt(nw);
-        if (!(nw > 0.0)) {   // the same on every lane of a wavefront
-            if (lane == 0) { atomicOr(bad, 2); meas[f] = 0.0; }
-            return;
-        }
-#pragma unroll
-        for (int k = 0; k < D; ++k) Q[s - 1][k] = w[k] / nw;   // q == s - 1
-        ++q;
+        for (int k = 0; k < D; ++k) Q[S0 - 1][k] = w[k] / nw;
+        return hv_face_basis<D, M, S0 + 1>(g, S, Q);
     }
-    const int b0 = fstart[f], e0 = fstart[f + 1];
-    const int apex = vid[b0];
-    const int* kp = vk + (int64_t)apex * (D + 1);
-    double p[D], da = 0.0;
+    return true;
+}
+
+// distance within the face (basis Q, first generator a, da = |p - x_a|^2) of the point p from its
+// sub-face on the bisector or plane of j
+template <int D, int M>
+__device__ __forceinline__ double hv_face_height(const IntGeo& g, double (*Q)[D], int a, int j, const double* p, double da) {
+    double w[D];
+    hv_face_grad<D>(g, a, j, w);
+    const double nr = hv_project<D, M - 1>(Q, w);
+    if (j >= g.N) {
+        double np_ = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; ++k) np_ = fma(g.pn[(j - g.N) * D + k], p[k], np_);
+        return fabs(g.ph[j - g.N] - np_) / nr;
+    }
+    double dj = 0.0;
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-        p[k] = vc[(int64_t)apex * D + k];
-        const double t = p[k] - g.xo[(int64_t)a * D + k];
-        da = fma(t, t, da);
+        const double t = p[k] - g.xo[(int64_t)j * D + k];
+        dj = fma(t, t, dj);
     }
-    double sum = 0.0;
-    // the sub-face T = S + {j} of the face, met at one of its vertices; x: T's entry in the
-    // incidence-to-face map of pass m + 1
-    auto subface = [&](int j, int x) {
-        bool skip = false;
-#pragma unroll
-        for (int s = 0; s <= D; ++s) skip = skip || (kp[s] == j);
-        if (skip) return;   // the sub-face holds the apex (zero height)
-        const int t1 = x >= 0 ? x : ~x;
-        if (t1 >= nface1) { atomicOr(bad, 4); return; }
-        // each sub-face once: from the first of its vertices (lists ascend by vertex)
-        if (x < 0) return;
-        double w[D];
-        hv_face_grad<D>(g, a, j, w);
-        for (int pass = 0; pass < 2; ++pass)
-#pragma unroll
-            for (int r = 0; r < D - 1; ++r) {   // r < q, unrolled: Q stays in registers
-                if (r >= q) break;
-                double cdot = 0.0;
-#pragma unroll
-                for (int k = 0; k < D; ++k) cdot = fma(w[k], Q[r][k], cdot);
-#pragma unroll
-                for (int k = 0; k < D; ++k) w[k] = fma(-cdot, Q[r][k], w[k]);
-            }
-        double nr = 0.0;
-#pragma unroll
-        for (int k = 0; k < D; ++k) nr = fma(w[k], w[k], nr);
-        nr = sqrt(nr);
-        double h;
-        if (j >= g.N) {
-            double np_ = 0.0;
-#pragma unroll
-            for (int k = 0; k < D; ++k) np_ = fma(g.pn[(j - g.N) * D + k], p[k], np_);
-            h = fabs(g.ph[j - g.N] - np_) / nr;
-        } else {
-            double dj = 0.0;
-#pragma unroll
-            for (int k = 0; k < D; ++k) {
-                const double t = p[k] - g.xo[(int64_t)j * D + k];
-                dj = fma(t, t, dj);
-            }
-            h = fabs(dj - da) / (2.0 * nr);
-        }
-        sum = fma(h, meas1[t1], sum);
-    };
-    if (rec.p) {
-        for (int i = b0 + lane; i < e0; i += step) {
-            const uint64_t* ro = rec.p + (int64_t)perm[i] * rec.ne;
-#pragma unroll
-            for (int z = 0; z < 4; ++z) {
-                if (z >= rec.ne) break;
-                const uint64_t rw = ro[z];
-                subface((int)(uint32_t)rw, (int)(uint32_t)(rw >> 32));
-            }
-        }
-    } else {
-        for (int i = b0 + lane; i < e0; i += step) {
-            const int v = vid[i];
-            const int* kv = vk + (int64_t)v * (D + 1);
-            int kr[D + 1], smask = 0;
-#pragma unroll
-            for (int e = 0; e <= D; ++e) {
-                kr[e] = kv[e];
-                bool in = false;
-#pragma unroll
-                for (int s = 0; s <= D; ++s) in = in || (S[s] == kr[e]);
-                smask |= in ? 1 << e : 0;
-            }
-            for (int e = 0; e <= D; ++e)
-                if (!((smask >> e) & 1))   // j not in S: T is the subset smask + e in pass m + 1
-                    subface(kr[e], foi1[(int64_t)v * C1 + hv_mask_rank.r[smask | (1 << e)]]);
-        }
-    }
-    if constexpr (L > 1) {
-#pragma unroll
-        for (int off = L / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-        if (lane != 0) return;
-    }
-    meas[f] = sum / (double)(D + 1 - m);
+    return fabs(dj - da) / (2.0 * nr);
 }
 
-template <int D, int L>
-__global__ __launch_bounds__(128) void k_face_measure(IntGeo g, int m, int nface, const int* __restrict__ fstart, const int* __restrict__ vid,
-                               const uint64_t* __restrict__ flo, const uint64_t* __restrict__ fhi, int nface1, int C1,
-                               const int* __restrict__ foi1, const double* __restrict__ meas1,
-                               const int* __restrict__ vk, const double* __restrict__ vc,
-                               const int* __restrict__ perm, HvRec rec, double* __restrict__ meas,
+// edges: pairs of vertices
+template <int D>
+__global__ void k_edge_measure(HvPairs L, const int* __restrict__ vk, const double* __restrict__ vc, HvFaces F,
                                int* __restrict__ bad) {
-    if constexpr (L > 1) {   // one wavefront per workgroup, 64 / L faces at a time
-        for (int64_t f = (int64_t)blockIdx.x * (64 / L) + threadIdx.x / L; f < nface; f += (int64_t)gridDim.x * (64 / L))
-            hv_face_measure_one<D, L>((int)f, (int)(threadIdx.x % L), L, g, m, fstart, vid, flo, fhi, nface1, C1,
-                                      foi1, meas1, vk, vc, perm, rec, meas, bad);
-    } else {
-        const int f = blockIdx.x * blockDim.x + threadIdx.x;
-        if (f < nface)
-            hv_face_measure_one<D, 1>(f, 0, 1, g, m, fstart, vid, flo, fhi, nface1, C1, foi1, meas1, vk, vc, perm,
-                                      rec, meas, bad);
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= L.nface) return;
+    const int b = L.start[f], e = f + 1 < L.nface ? L.start[f + 1] : *L.nvalid;
+    const uint32_t x = L.pay[b];
+    const int va = (int)(x / (D + 1));
+    int id[D + 1];
+    hv_sub_ids<D, D>(vk, F, va, id);
+    uint64_t lo, hi;
+    hv_face_key<D>(id, (int)(x - (uint32_t)va * (D + 1)), lo, hi);
+    F.klo[f] = lo;
+    if constexpr (D > 3) F.khi[f] = hi;
+    if (e - b != 2) {
+        atomicOr(bad, 1);
+        F.f[f] = HvFace{0.0, va, 2};
+        return;
     }
+    const int vb = (int)(L.pay[b + 1] / (D + 1));
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        const double t = vc[(int64_t)va * D + k] - vc[(int64_t)vb * D + k];
+        s = fma(t, t, s);
+    }
+    F.f[f] = HvFace{sqrt(s), va, 2};   // pairs ascend by vertex: va is the smaller
+}
+
+// Faces of pass M < D from the faces of pass M + 1 (F1), `lanes` of a wavefront per face (W: a power
+// of two), the partial sums combined in a fixed order.  Bound by the gathers of the sub-faces and
+// the generators' coordinates; with W > 1 a face of many sub-faces is not one lane's serial chain.
+template <int D, int M, int W>
+__global__ __launch_bounds__(128) void k_face_measure(IntGeo g, HvPairs L, const int* __restrict__ vk,
+                                                      const double* __restrict__ vc, HvFaces F1, HvFaces F,
+                                                      int* __restrict__ bad) {
+    const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = (int)(gt % W);
+    // a dispatch holds at most 2^32 work-items: the faces are walked grid-stride
+    for (int64_t f = gt / W; f < L.nface; f += (int64_t)gridDim.x * blockDim.x / W) {
+        const int b = L.start[f], e = f + 1 < L.nface ? L.start[f + 1] : *L.nvalid;
+        int S[M];
+        {
+            const uint32_t x = L.pay[b], t = x / (M + 1);
+            int id[M + 1];
+            hv_sub_ids<D, M>(vk, F1, t, id);
+            const int p = (int)(x - t * (M + 1));
+            uint64_t lo, hi;
+            hv_face_key<M>(id, p, lo, hi);
+#pragma unroll
+            for (int s = 0; s < M; ++s) S[s] = s < p ? id[s] : id[s + 1];
+            if (lane == 0) {
+                F.klo[f] = lo;
+                if constexpr (M > 3) F.khi[f] = hi;
+            }
+        }
+        // the apex: the face's smallest vertex
+        int apex = INT_MAX, nvs = 0;
+        for (int i = b + lane; i < e; i += W) {
+            const HvFace& T = F1.f[L.pay[i] / (M + 1)];
+            apex = min(apex, T.vmin);
+            nvs += T.nv;
+        }
+#pragma unroll
+        for (int off = W / 2; off > 0; off >>= 1) {
+            apex = min(apex, __shfl_xor(apex, off));
+            nvs += __shfl_xor(nvs, off);
+        }
+        double Q[M > 1 ? M - 1 : 1][D];
+        double sum = 0.0;
+        if (hv_face_basis<D, M>(g, S, Q)) {
+            double p[D], da = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                p[k] = vc[(int64_t)apex * D + k];
+                const double t = p[k] - g.xo[(int64_t)S[0] * D + k];
+                da = fma(t, t, da);
+            }
+            for (int i = b + lane; i < e; i += W) {
+                const HvFace T = F1.f[L.pay[i] / (M + 1)];
+                if (T.vmin == apex) continue;   // the sub-face holds the apex: zero height
+                sum = fma(hv_face_height<D, M>(g, Q, S[0], L.jl[i], p, da), T.meas, sum);
+            }
+        } else if (lane == 0) {
+            atomicOr(bad, 2);
+        }
+#pragma unroll
+        for (int off = W / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+        constexpr int K = D + 1 - M;   // the face's dimension; a vertex of it lies in K of its T
+        if (lane == 0) F.f[f] = HvFace{sum / (double)K, apex, nvs / K};
+    }
+}
+
+// lanes per face of pass m, by the face dimension k = d + 1 - m: a polygon has 4 to 5 edges on
+// average, a 3-face about 10 polygons, faces of higher dimension tens of sub-faces
+constexpr int hv_face_lanes(int D, int M) { return D + 1 - M >= 4 ? 4 : 1; }
+
+static inline unsigned hv_face_blocks(int nface, int lanes) {
+    return (unsigned)std::min<int64_t>(std::max<int64_t>(((int64_t)nface * lanes + 127) / 128, 1), 1 << 20);
 }
 
 // ---- integrands (the reference's rule, src/polyintegrator.jl:174-353) -----------------------
@@ -457,226 +490,93 @@ __global__ __launch_bounds__(128) void k_face_measure(IntGeo g, int m, int nface
 //   I(F) = (d-1)/d J(F) + f(c_F) |F| / d,
 // and a cell, with apex at its generator x,
 //   bulk = f(x) vol / (d+1) + sum over facets F of dist(x, F) I(F) / (d+1).
-// Exact for affine f.  nf <= HV_MAXF components per point.
+// Exact for affine f.  nf <= HV_MAXF components per point.  Every vertex of a face of dimension
+// k lies in k of its sub-faces, so the centre is the mean of theirs, weighted by their vertices.
 constexpr int HV_MAXF = 8;
 
 template <int D>
-__global__ void k_face_center(const int* __restrict__ fstart, int nface, const int* __restrict__ vid,
-                              const double* __restrict__ vc, double* __restrict__ cen) {
+__global__ void k_edge_int(HvPairs L, HvFaces F, const double* __restrict__ vc, const double* __restrict__ fv, int nf,
+                           double* __restrict__ cen, double* __restrict__ J) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nface) return;
-    const int b = fstart[f], e = fstart[f + 1];
-    double acc[D];
+    if (f >= L.nface) return;
+    const int b = L.start[f], e = f + 1 < L.nface ? L.start[f + 1] : *L.nvalid;
+    const int64_t va = L.pay[b] / (D + 1), vb = e - b == 2 ? L.pay[b + 1] / (D + 1) : va;   // flagged by k_edge_measure
 #pragma unroll
-    for (int k = 0; k < D; ++k) acc[k] = 0.0;
-    for (int i = b; i < e; ++i) {
-        const int v = vid[i];
-#pragma unroll
-        for (int k = 0; k < D; ++k) acc[k] += vc[(int64_t)v * D + k];
-    }
-    const double inv = 1.0 / (double)(e - b);
-#pragma unroll
-    for (int k = 0; k < D; ++k) cen[(int64_t)f * D + k] = acc[k] * inv;
+    for (int k = 0; k < D; ++k) cen[(int64_t)f * D + k] = (vc[va * D + k] + vc[vb * D + k]) * 0.5;
+    for (int c = 0; c < nf; ++c) J[(int64_t)f * nf + c] = F.f[f].meas * 0.5 * (fv[va * nf + c] + fv[vb * nf + c]);
 }
 
-__global__ void k_edge_int(const int* __restrict__ fstart, int nface, const int* __restrict__ vid,
-                           const double* __restrict__ meas, const double* __restrict__ fv, int nf,
-                           double* __restrict__ J) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nface) return;
-    if (fstart[f + 1] - fstart[f] != 2) {   // flagged by k_edge_len; the integration fails
-        for (int c = 0; c < nf; ++c) J[(int64_t)f * nf + c] = 0.0;
-        return;
-    }
-    const int va = vid[fstart[f]], vb = vid[fstart[f] + 1];
-    for (int c = 0; c < nf; ++c)
-        J[(int64_t)f * nf + c] = meas[f] * 0.5 * (fv[(int64_t)va * nf + c] + fv[(int64_t)vb * nf + c]);
-}
-
-// J of each face of pass m from the faces of pass m + 1, apex at the face's centre (L lanes per
-// face, as k_face_measure)
-template <int D, int L>
-__device__ __forceinline__ void hv_face_int_one(int f, int lane, int step, const IntGeo& g, int m,
-                                                const int* __restrict__ fstart, const int* __restrict__ vid,
-                                                const uint64_t* __restrict__ flo, const uint64_t* __restrict__ fhi,
-                                                const double* __restrict__ cen, int nface1, int C1,
-                                                const int* __restrict__ foi1,
-                                                const double* __restrict__ J1, int nf, const int* __restrict__ vk,
-                                                const int* __restrict__ perm, const HvRec& rec,
-                                                double* __restrict__ J, int* __restrict__ bad) {
-    const uint64_t lo = flo[f], hi = fhi[f];
-    int S[D + 1];
+// centre and J of each face of pass M from those of pass M + 1 (W lanes per face, as k_face_measure)
+template <int D, int M, int W>
+__global__ __launch_bounds__(128) void k_face_int(IntGeo g, HvPairs L, const int* __restrict__ vk, HvFaces F1,
+                                                  const double* __restrict__ cen1, const double* __restrict__ J1, int nf,
+                                                  double* __restrict__ cen, double* __restrict__ J, int* __restrict__ bad) {
+    const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = (int)(gt % W);
+    for (int64_t f = gt / W; f < L.nface; f += (int64_t)gridDim.x * blockDim.x / W) {
+        const int b = L.start[f], e = f + 1 < L.nface ? L.start[f + 1] : *L.nvalid;
+        int S[M];
+        {
+            const uint32_t x = L.pay[b], t = x / (M + 1);
+            int id[M + 1];
+            hv_sub_ids<D, M>(vk, F1, t, id);
+            const int p = (int)(x - t * (M + 1));
 #pragma unroll
-    for (int s = 0; s <= D; ++s) S[s] = s < m ? hv_fkey_get(lo, hi, s) : -1;
-    const int a = S[0];
-    double Q[D][D];
-    int q = 0;
+            for (int s = 0; s < M; ++s) S[s] = s < p ? id[s] : id[s + 1];
+        }
+        double p[D], nvs = 0.0;
 #pragma unroll
-    for (int s = 1; s < D + 1; ++s) {
-        if (s >= m) break;
-        double w[D];
-        hv_face_grad<D>(g, a, S[s], w);
-        for (int pass = 0; pass < 2; ++pass)
+        for (int k = 0; k < D; ++k) p[k] = 0.0;
+        for (int i = b + lane; i < e; i += W) {
+            const int64_t t = L.pay[i] / (M + 1);
+            const double w = (double)F1.f[t].nv;
+            nvs += w;
 #pragma unroll
-            for (int r = 0; r < D - 1; ++r) {   // r < q, unrolled: Q stays in registers
-                if (r >= q) break;
-                double cdot = 0.0;
-#pragma unroll
-                for (int k = 0; k < D; ++k) cdot = fma(w[k], Q[r][k], cdot);
-#pragma unroll
-                for (int k = 0; k < D; ++k) w[k] = fma(-cdot, Q[r][k], w[k]);
-            }
-        double nw = 0.0;
-#pragma unroll
-        for (int k = 0; k < D; ++k) nw = fma(w[k], w[k], nw);
-        nw = sqrt(nw);
-        if (!(nw > 0.0)) {
-            if (lane == 0) atomicOr(bad, 2);
-            return;
+            for (int k = 0; k < D; ++k) p[k] = fma(w, cen1[t * D + k], p[k]);
         }
 #pragma unroll
-        for (int k = 0; k < D; ++k) Q[s - 1][k] = w[k] / nw;   // q == s - 1
-        ++q;
-    }
-    double p[D], da = 0.0;
+        for (int off = W / 2; off > 0; off >>= 1) {
+            nvs += __shfl_xor(nvs, off);
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-        p[k] = cen[(int64_t)f * D + k];
-        const double t = p[k] - g.xo[(int64_t)a * D + k];
-        da = fma(t, t, da);
-    }
-    double sum[HV_MAXF];
-    for (int c = 0; c < nf; ++c) sum[c] = 0.0;
-    const int b0 = fstart[f], e0 = fstart[f + 1];
-    // the sub-face T = S + {j}; x: T's entry in the incidence-to-face map of pass m + 1
-    auto subface = [&](int j, int x) {
-        const int t1 = x >= 0 ? x : ~x;
-        if (t1 >= nface1) { atomicOr(bad, 4); return; }
-        if (x < 0) return;   // each sub-face once
-        double w[D];
-        hv_face_grad<D>(g, a, j, w);
-        for (int pass = 0; pass < 2; ++pass)
-#pragma unroll
-            for (int r = 0; r < D - 1; ++r) {   // r < q, unrolled: Q stays in registers
-                if (r >= q) break;
-                double cdot = 0.0;
-#pragma unroll
-                for (int k = 0; k < D; ++k) cdot = fma(w[k], Q[r][k], cdot);
-#pragma unroll
-                for (int k = 0; k < D; ++k) w[k] = fma(-cdot, Q[r][k], w[k]);
-            }
-        double nr = 0.0;
-#pragma unroll
-        for (int k = 0; k < D; ++k) nr = fma(w[k], w[k], nr);
-        nr = sqrt(nr);
-        double h;
-        if (j >= g.N) {
-            double np_ = 0.0;
-#pragma unroll
-            for (int k = 0; k < D; ++k) np_ = fma(g.pn[(j - g.N) * D + k], p[k], np_);
-            h = fabs(g.ph[j - g.N] - np_) / nr;
-        } else {
-            double dj = 0.0;
-#pragma unroll
-            for (int k = 0; k < D; ++k) {
-                const double t = p[k] - g.xo[(int64_t)j * D + k];
-                dj = fma(t, t, dj);
-            }
-            h = fabs(dj - da) / (2.0 * nr);
+            for (int k = 0; k < D; ++k) p[k] += __shfl_xor(p[k], off);
         }
-        for (int c = 0; c < nf; ++c) sum[c] = fma(h, J1[(int64_t)t1 * nf + c], sum[c]);
-    };
-    if (rec.p) {
-        for (int i = b0 + lane; i < e0; i += step) {
-            const uint64_t* ro = rec.p + (int64_t)perm[i] * rec.ne;
+        double Q[M > 1 ? M - 1 : 1][D];
+        double da = 0.0;
 #pragma unroll
-            for (int z = 0; z < 4; ++z) {
-                if (z >= rec.ne) break;
-                const uint64_t rw = ro[z];
-                subface((int)(uint32_t)rw, (int)(uint32_t)(rw >> 32));
-            }
+        for (int k = 0; k < D; ++k) {
+            p[k] /= nvs;
+            if (lane == 0) cen[f * D + k] = p[k];
+            const double t = p[k] - g.xo[(int64_t)S[0] * D + k];
+            da = fma(t, t, da);
         }
-    } else {
-        for (int i = b0 + lane; i < e0; i += step) {
-            const int v = vid[i];
-            const int* kv = vk + (int64_t)v * (D + 1);
-            int kr[D + 1], smask = 0;
-#pragma unroll
-            for (int e = 0; e <= D; ++e) {
-                kr[e] = kv[e];
-                bool in = false;
-#pragma unroll
-                for (int s = 0; s <= D; ++s) in = in || (S[s] == kr[e]);
-                smask |= in ? 1 << e : 0;
+        double sum[HV_MAXF];
+        for (int c = 0; c < nf; ++c) sum[c] = 0.0;
+        if (hv_face_basis<D, M>(g, S, Q)) {
+            for (int i = b + lane; i < e; i += W) {
+                const double h = hv_face_height<D, M>(g, Q, S[0], L.jl[i], p, da);
+                const int64_t t = L.pay[i] / (M + 1);
+                for (int c = 0; c < nf; ++c) sum[c] = fma(h, J1[t * nf + c], sum[c]);
             }
-            for (int e = 0; e <= D; ++e)
-                if (!((smask >> e) & 1))
-                    subface(kr[e], foi1[(int64_t)v * C1 + hv_mask_rank.r[smask | (1 << e)]]);
+        } else if (lane == 0) {
+            atomicOr(bad, 2);
         }
-    }
-    if constexpr (L > 1) {
         for (int c = 0; c < nf; ++c) {
 #pragma unroll
-            for (int off = L / 2; off > 0; off >>= 1) sum[c] += __shfl_xor(sum[c], off);
+            for (int off = W / 2; off > 0; off >>= 1) sum[c] += __shfl_xor(sum[c], off);
+            if (lane == 0) J[f * nf + c] = sum[c] / (double)(D + 1 - M);
         }
-        if (lane != 0) return;
     }
-    for (int c = 0; c < nf; ++c) J[(int64_t)f * nf + c] = sum[c] / (double)(D + 1 - m);
-}
-
-template <int D, int L>
-__global__ __launch_bounds__(128) void k_face_int(IntGeo g, int m, int nface, const int* __restrict__ fstart, const int* __restrict__ vid,
-                           const uint64_t* __restrict__ flo, const uint64_t* __restrict__ fhi,
-                           const double* __restrict__ cen, int nface1, int C1, const int* __restrict__ foi1,
-                           const double* __restrict__ J1, int nf, const int* __restrict__ vk,
-                           const int* __restrict__ perm, HvRec rec, double* __restrict__ J, int* __restrict__ bad) {
-    if constexpr (L > 1) {
-        for (int64_t f = (int64_t)blockIdx.x * (64 / L) + threadIdx.x / L; f < nface; f += (int64_t)gridDim.x * (64 / L))
-            hv_face_int_one<D, L>((int)f, (int)(threadIdx.x % L), L, g, m, fstart, vid, flo, fhi, cen, nface1, C1,
-                                  foi1, J1, nf, vk, perm, rec, J, bad);
-    } else {
-        const int f = blockIdx.x * blockDim.x + threadIdx.x;
-        if (f < nface)
-            hv_face_int_one<D, 1>(f, 0, 1, g, m, fstart, vid, flo, fhi, cen, nface1, C1, foi1, J1, nf, vk, perm, rec,
-                                  J, bad);
-    }
-}
-
-// lanes per face of pass m, by the face dimension k = d + 1 - m (polygons and 3-faces hold
-// tens of vertices, 4-faces hundreds, 5-faces more).  Measured per pass at 6D N=50k periodic
-// (ms per chunk, L = 1 / 16 / 64): k = 2: 130 / 455 / 1270, k = 3: 231 / 304 / 686,
-// k = 4: 272 / 188 / 206, k = 5: 160 / 87 / 55; at 5D N=100k: k = 3: 56 / 59 / 126,
-// k = 4: 49 / 29 / 31.  A function of (d, m) only, so that every mesh and chunk sums a face's
-// cones in the same order.
-__host__ inline int hv_face_lanes(int D, int m) {
-    const int k = D + 1 - m;
-    return k >= 5 ? 64 : (k == 4 ? 16 : 1);
-}
-
-// launches k_face_measure or k_face_int (K) with L lanes per face
-template <int L, typename K, typename... A>
-static void hv_face_launch(K kern, int nface, hipStream_t s, A... args) {
-    if (L == 1) kern<<<nblk(std::max(nface, 1), 128), 128, 0, s>>>(args...);
-    else kern<<<(unsigned)std::min<int64_t>(std::max<int64_t>(((int64_t)nface * L + 63) / 64, 1), 1 << 20), 64, 0, s>>>(args...);
 }
 
 // facets: I(F) = (d-1)/d J(F) + f(c_F) |F| / d
 template <int D>
 __global__ void k_facet_int(int nface, const double* __restrict__ J, const double* __restrict__ fc,
-                            const double* __restrict__ meas, int nf, double* __restrict__ I) {
+                            const HvFace* __restrict__ face, int nf, double* __restrict__ I) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nface) return;
     for (int c = 0; c < nf; ++c)
         I[(int64_t)f * nf + c] = (double)(D - 1) / (double)D * J[(int64_t)f * nf + c] +
-                                 fc[(int64_t)f * nf + c] * meas[f] / (double)D;
-}
-
-// row t's interface integral from its facet (rows sorted with their facet numbers)
-__global__ void k_row_int(int64_t npair, const int* __restrict__ pface, const double* __restrict__ I, int nf,
-                          double* __restrict__ out) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= npair) return;
-    for (int c = 0; c < nf; ++c) out[t * nf + c] = I[(int64_t)pface[t] * nf + c];
+                                 fc[(int64_t)f * nf + c] * face[f].meas / (double)D;
 }
 
 // cells 0 .. nreal-1: f(x) vol / (d+1) + sum over rows of dist * I(row) / (d+1)
@@ -710,28 +610,24 @@ __global__ void k_cell_bulk(IntGeo g, const uint64_t* __restrict__ pkey, const i
     for (int c = 0; c < nf; ++c) bulk[(int64_t)i * nf + c] = y[c] / (double)(D + 1);
 }
 
-// facets {a, b} -> (cell, neighbour, area) rows for both sides
-// rows (cell, neighbour) of the facets: one per side that is a cell of the chunk
-__global__ void k_facet_pairs(int nface, const uint64_t* __restrict__ flo, const double* __restrict__ meas, int N,
-                              const uint8_t* __restrict__ cmask, uint64_t* __restrict__ pkey, double* __restrict__ parea,
-                              int* __restrict__ pface, unsigned long long* __restrict__ np) {
+// facets {a, b} -> rows (cell << bits | neighbour) at 2f and 2f + 1, one per side that is a cell of
+// the chunk (~0, which sorts past the end, for the other), with their areas and interface integrals
+__global__ void k_facet_rows(int nface, HvFaces F, int N, const uint8_t* __restrict__ cmask, int bits,
+                             uint64_t* __restrict__ row, double* __restrict__ area, const double* __restrict__ I, int nf,
+                             double* __restrict__ rint) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nface) return;
-    const int a = hv_fkey_get(flo[f], 0, 0), b = hv_fkey_get(flo[f], 0, 1);
-    const bool ra = a < N && cmask[a] != 0, rb = b < N && cmask[b] != 0;
-    const int n = (ra ? 1 : 0) + (rb ? 1 : 0);
-    if (!n) return;
-    unsigned long long o = atomicAdd(np, (unsigned long long)n);
-    if (ra) {
-        pkey[o] = ((uint64_t)a << 32) | (uint64_t)b;
-        parea[o] = meas[f];
-        pface[o] = f;
-        ++o;
-    }
-    if (rb) {
-        pkey[o] = ((uint64_t)b << 32) | (uint64_t)a;
-        parea[o] = meas[f];
-        pface[o] = f;
+    const uint64_t a = F.klo[f] & HV_F21, b = (F.klo[f] >> 21) & HV_F21;
+    const bool ra = a < (uint64_t)N && (!cmask || cmask[a] != 0), rb = b < (uint64_t)N && (!cmask || cmask[b] != 0);
+    row[2 * (int64_t)f] = ra ? (a << bits) | b : ~0ull;
+    row[2 * (int64_t)f + 1] = rb ? (b << bits) | a : ~0ull;
+    const double m = F.f[f].meas;
+    area[2 * (int64_t)f] = m;
+    area[2 * (int64_t)f + 1] = m;
+    for (int c = 0; c < nf; ++c) {
+        const double v = I[(int64_t)f * nf + c];
+        rint[2 * (int64_t)f * nf + c] = v;
+        rint[(2 * (int64_t)f + 1) * nf + c] = v;
     }
 }
 
@@ -743,7 +639,7 @@ __global__ void k_set_mask(const int* __restrict__ ids, int n, uint8_t* __restri
 // vertices holding a cell of the chunk
 template <int D>
 __global__ void k_vert_in_chunk(const int* __restrict__ vk, int nv, int N, const uint8_t* __restrict__ cmask,
-                                uint8_t* __restrict__ flag, int* __restrict__ iota) {
+                                uint8_t* __restrict__ flag) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= nv) return;
     bool in = false;
@@ -753,7 +649,6 @@ __global__ void k_vert_in_chunk(const int* __restrict__ vk, int nv, int N, const
         in = in || (id < N && cmask[id] != 0);
     }
     flag[v] = in ? 1 : 0;
-    iota[v] = v;
 }
 
 template <int D>
@@ -785,15 +680,24 @@ __global__ void k_int_subset(const int* __restrict__ sel, int n, const int* __re
         for (int f = 0; f < nf; ++f) fv2[(int64_t)t * nf + f] = fv[(int64_t)v * nf + f];
 }
 
-// row payloads in the sorted order of the rows
-__global__ void k_gather_rows(const int* __restrict__ perm, int64_t n, const double* __restrict__ ra,
-                              double* __restrict__ parea, const double* __restrict__ ri, double* __restrict__ rint, int nf) {
+// sorted rows (cell << bits | neighbour, dense ids) in the caller's ids (cell << 32 | neighbour; the
+// map preserves the order) with their payloads; *npair: the number of real ones
+__global__ void k_rows_out(const uint64_t* __restrict__ row, const int* __restrict__ perm, int64_t n, int bits,
+                           const int* __restrict__ gid, const double* __restrict__ ra, const double* __restrict__ ri, int nf,
+                           uint64_t* __restrict__ pkey, double* __restrict__ parea, double* __restrict__ rint,
+                           int* __restrict__ npair) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
+    const uint64_t r = row[t];
+    if (r == ~0ull) {
+        if (t == 0 || row[t - 1] != ~0ull) *npair = (int)t;
+        return;
+    }
+    if (t == n - 1) *npair = (int)n;
+    pkey[t] = ((uint64_t)gid[r >> bits] << 32) | (uint64_t)(uint32_t)gid[r & ((1ull << bits) - 1ull)];
     const int s = perm[t];
     parea[t] = ra[s];
-    if (ri)
-        for (int f = 0; f < nf; ++f) rint[t * nf + f] = ri[(int64_t)s * nf + f];
+    for (int f = 0; f < nf; ++f) rint[t * nf + f] = ri[(int64_t)s * nf + f];
 }
 
 template <int D>
@@ -982,26 +886,10 @@ __global__ void k_mc_sym(IntGeo g, const int64_t* __restrict__ ptr, const uint64
 // Face keys pack 21 bits per id.  The face passes run on a dense numbering of the ids that
 // occur in the mesh's keys (order-preserving, so sorted keys stay sorted): with periodic images
 // the working set can exceed 2^21 generators while far fewer of them touch a walked cell.
-template <int D>
-__global__ void k_mark_used(const int* __restrict__ vk, int nv, int* __restrict__ used) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-#pragma unroll
-    for (int j = 0; j <= D; ++j) used[vk[(int64_t)v * (D + 1) + j]] = 1;
-}
-
 // dense[i] (exclusive prefix sum of used) -> gid[dense] = i for the used ids
 __global__ void k_dense_inverse(const int* __restrict__ used, const int* __restrict__ dense, int n, int* __restrict__ gid) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n && used[i]) gid[dense[i]] = i;
-}
-
-template <int D>
-__global__ void k_remap_keys(int* __restrict__ vk, int nv, const int* __restrict__ dense) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-#pragma unroll
-    for (int j = 0; j <= D; ++j) vk[(int64_t)v * (D + 1) + j] = dense[vk[(int64_t)v * (D + 1) + j]];
 }
 
 // generator rows and planes of the dense numbering: dense ids below ngen are generators
@@ -1021,14 +909,6 @@ __global__ void k_dense_geo(const int* __restrict__ gid, int nused, int ngen, in
         for (int k = 0; k < D; ++k) pnd[q * D + k] = pn[p * D + k];
         phd[q] = ph[p];
     }
-}
-
-// rows (cell << 32 | neighbour) back to the caller's ids; the map preserves the order
-__global__ void k_rows_to_ids(uint64_t* __restrict__ rows, int64_t n, const int* __restrict__ gid) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const uint64_t r = rows[t];
-    rows[t] = ((uint64_t)gid[(int)(r >> 32)] << 32) | (uint64_t)(uint32_t)gid[(int)(r & 0xffffffffull)];
 }
 
 // ---- host driver -------------------------------------------------------------------------
@@ -1068,6 +948,113 @@ static int eval_integrand(hv_ctx* c, const Integrand* fi, int D, const double* d
     return HV_OK;
 }
 
+// Host state of one chunk's face passes.
+struct FacePass {
+    const int* vk = nullptr;        // the chunk's vertices, canonical order
+    const double* vc = nullptr;
+    const double* fv = nullptr;     // integrand at the vertices
+    int nv = 0;
+    const uint8_t* cmask = nullptr;
+    const uint32_t* hid = nullptr;
+    int hb = 0, zb = 0;             // hash and id bits of a grouping key
+    int nf = 0;
+    int* bad = nullptr;
+    int* cnt = nullptr;             // device counters: pairs of real faces, faces, runs to fix
+    // the faces of the last pass
+    HvFaces F{};
+    int nface = 0;
+    double *cen = nullptr, *J = nullptr;
+};
+
+// Faces of pass M and their measures from those of pass M + 1 (the vertices for M == D)
+template <int D, int M>
+static int face_pass(hv_ctx* c, const IntGeo& g, FacePass& P) {
+    const int nt = M == D ? P.nv : P.nface;
+    const int64_t tot = (int64_t)nt * (M + 1);
+    if (tot >= (1ll << 31)) return hv_fail(c, HV_ERR_CAPACITY, "too many face incidences for one pass");
+    const size_t T = (size_t)std::max<int64_t>(tot, 1);
+    uint32_t* key = iget<uint32_t>(c, "i_key", T);
+    uint32_t* key2 = iget<uint32_t>(c, "i_key2", T);
+    uint32_t* pay = iget<uint32_t>(c, "i_pay", T);
+    uint8_t* head = iget<uint8_t>(c, "i_head", T);
+    if (!key || !key2 || !pay || !head) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
+    const HvFaces F1 = P.F;
+    HVCK(hipMemsetAsync(P.cnt, 0, 4 * sizeof(int), c->stream));
+    int nface = 0;
+    HvPairs L{};
+    if (tot > 0) {
+        k_pair_emit<D, M><<<nblk(nt, 256), 256, 0, c->stream>>>(P.vk, F1, nt, g.N, P.cmask, P.hid, P.hb, key);
+        HVCK(hipGetLastError());
+        const unsigned nbits = (unsigned)(P.zb + P.hb);
+        const rocprim::counting_iterator<uint32_t> it(0u);
+        size_t tb = 0, tb2 = 0;
+        HVCK(rocprim::radix_sort_pairs(nullptr, tb, key, key2, it, pay, T, 0u, nbits, c->stream));
+        int* jl = (int*)key;   // free once sorted
+        const hipcub::CountingInputIterator<int> pos(0);
+        int* start0 = iget<int>(c, "i_start", T + 1);
+        if (!start0) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
+        HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb2, pos, head, start0, P.cnt + 1, (int)tot, c->stream));
+        void* tmp = c->pool->get("i_tmp", std::max(tb, tb2), false, c->stream);
+        if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
+        HVCK(rocprim::radix_sort_pairs(tmp, tb, key, key2, it, pay, T, 0u, nbits, c->stream));
+        // HV_NO_FACE pairs lie at the end: their first position, or all of them real
+        HVCK(hipMemsetD32Async((hipDeviceptr_t)P.cnt, (int)tot, 1, c->stream));
+        int* runs = start0;    // room for one per pair, read before the faces' starts are written
+        k_pair_heads<D, M><<<nblk(tot, 256), 256, 0, c->stream>>>(key2, pay, tot, P.vk, F1, head, jl, P.cnt, runs, P.cnt + 2);
+        HVCK(hipGetLastError());
+        k_pair_fix<D, M><<<1024, 64, 0, c->stream>>>(key2, tot, P.vk, F1, runs, P.cnt + 2, pay, head, jl);
+        HVCK(hipGetLastError());
+        HVCK(hipcub::DeviceSelect::Flagged(tmp, tb2, pos, head, start0, P.cnt + 1, (int)tot, c->stream));
+        HVCK(hipMemcpyAsync(&nface, P.cnt + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        HVCK(hipStreamSynchronize(c->stream));
+        L = HvPairs{pay, jl, start0, P.cnt, nface};
+    }
+    // tables of this pass and the one before alternate
+    const std::string sfx = (M & 1) ? "a" : "b";
+    auto nm = [&](const char* s) { return std::string(s) + sfx; };
+    const size_t nfc = (size_t)std::max(nface, 1);
+    HvFaces F;
+    F.klo = iget<uint64_t>(c, nm("i_klo").c_str(), nfc);
+    F.khi = M > 3 ? iget<uint64_t>(c, nm("i_khi").c_str(), nfc) : nullptr;
+    F.f = iget<HvFace>(c, nm("i_face").c_str(), nfc);
+    if (!F.klo || (M > 3 && !F.khi) || !F.f) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
+    double *cen = nullptr, *J = nullptr;
+    if (P.nf) {
+        cen = iget<double>(c, nm("i_cen").c_str(), nfc * D);
+        J = iget<double>(c, nm("i_J").c_str(), nfc * P.nf);
+        if (!cen || !J) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integrand)");
+    }
+    if (nface > 0) {
+        if constexpr (M == D) {
+            k_edge_measure<D><<<nblk(nface, 256), 256, 0, c->stream>>>(L, P.vk, P.vc, F, P.bad);
+            HVCK(hipGetLastError());
+            if (P.nf) k_edge_int<D><<<nblk(nface, 256), 256, 0, c->stream>>>(L, F, P.vc, P.fv, P.nf, cen, J);
+        } else {
+            constexpr int W = hv_face_lanes(D, M);
+            k_face_measure<D, M, W><<<hv_face_blocks(nface, W), 128, 0, c->stream>>>(g, L, P.vk, P.vc, F1, F, P.bad);
+            HVCK(hipGetLastError());
+            if (P.nf)
+                k_face_int<D, M, W><<<hv_face_blocks(nface, W), 128, 0, c->stream>>>(g, L, P.vk, F1, P.cen, P.J, P.nf, cen, J,
+                                                                                    P.bad);
+        }
+        HVCK(hipGetLastError());
+    }
+    P.F = F;
+    P.nface = nface;
+    P.cen = cen;
+    P.J = J;
+    if constexpr (M > 2) return face_pass<D, M - 1>(c, g, P);
+    return HV_OK;
+}
+
+// pairs of the largest pass per vertex: C(d + 1, m + 1) faces T at most, each of at least
+// (dimension of T) + 1 vertices, with m + 1 subsets
+static double pairs_bound(int D) {
+    double most = D + 1.0;
+    for (int m = 2; m < D; ++m) most = std::max(most, (double)binom(D + 1, m + 1) * (m + 1) / (double)(D - m + 1));
+    return most;
+}
+
 // faces of the tessellation, all passes; leaves the sorted (cell, neighbour) rows with areas.
 // fi (optional): also the integrals of the rows' interfaces (*rint, npair x nf) by the
 // reference's rule (see k_face_int)
@@ -1075,42 +1062,29 @@ template <int D>
 static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t*& pkey, double*& parea, int64_t& npair,
                       const Integrand* fi = nullptr, double** rint = nullptr) {
     const int nv = (int)mesh->nv;
-    int* vk = iget<int>(c, "i_vk", (size_t)nv * (D + 1));
-    double* vc = iget<double>(c, "i_vc", (size_t)nv * D);
+    const size_t nv1 = (size_t)std::max(nv, 1);
+    int* vk = iget<int>(c, "i_vk", nv1 * (D + 1));
+    double* vc = iget<double>(c, "i_vc", nv1 * D);
     int* bad = iget<int>(c, "i_bad", 1);
-    unsigned long long* cnt = iget<unsigned long long>(c, "i_cnt", 2);
+    int* cnt = iget<int>(c, "i_cnt", 4);
     if (!vk || !vc || !bad || !cnt) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
     HVCK(hipMemsetAsync(bad, 0, sizeof(int), c->stream));
+    const int* mids = (const int*)mesh->ids.p;
+    const int* mkey = (const int*)mesh->key.p;
     IntGeo g = g0;          // the face passes' geometry, in dense ids
     int* gid = nullptr;     // dense id -> the caller's id
-    int* used = nullptr;    // caller's id -> occurs in a key
     int* dense = nullptr;   // caller's id -> dense id (exclusive prefix sum of used)
+    uint32_t* hid = nullptr;
     const int nid = g0.N + g0.P;
-    int ngen = 0, nused = 0;
+    int ngen = 0, nused = 0, zb = 1;
     {
-        // the live vertices in a numbering fixed by the vertex set (not by the walk's
-        // insertion order), so that apexes and summation orders are reproducible
-        int* vk0 = iget<int>(c, "i_vk0", (size_t)nv * (D + 1));
-        double* vc0 = iget<double>(c, "i_vc0", (size_t)nv * D);
-        uint64_t* w0 = iget<uint64_t>(c, "i_w0", nv);
-        uint64_t* w1 = iget<uint64_t>(c, "i_w1", nv);
-        uint64_t* w2 = iget<uint64_t>(c, "i_w2", nv);
-        uint64_t* ws = iget<uint64_t>(c, "i_ws", nv);
-        uint64_t* wso = iget<uint64_t>(c, "i_wso", nv);
-        int* pa = iget<int>(c, "i_vpa", nv);
-        int* pb = iget<int>(c, "i_vpb", nv);
-        if (!vk0 || !vc0 || !w0 || !w1 || !w2 || !ws || !wso || !pa || !pb)
-            return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
-        k_int_gather<D><<<nblk(nv, 256), 256, 0, c->stream>>>((const int*)mesh->ids.p, nv, (const int*)mesh->key.p,
-                                                              (const double*)mesh->x.p, vk0, vc0);
-        HVCK(hipGetLastError());
         // dense ids of the generators and planes that occur in the keys
-        used = iget<int>(c, "i_used", (size_t)nid + 1);
+        int* used = iget<int>(c, "i_used", (size_t)nid + 1);
         dense = iget<int>(c, "i_dense", (size_t)nid + 1);
         if (!used || !dense) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
         HVCK(hipMemsetAsync(used, 0, sizeof(int) * ((size_t)nid + 1), c->stream));
         if (nv) {
-            k_mark_used<D><<<nblk(nv, 256), 256, 0, c->stream>>>(vk0, nv, used);
+            k_mark_used<D><<<nblk((int64_t)nv * (D + 1), 256), 256, 0, c->stream>>>(mids, nv, mkey, used);
             HVCK(hipGetLastError());
         }
         size_t tbs = 0;
@@ -1126,19 +1100,19 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
         nused = hcnt[1];
         if (nused >= (int)HV_F21)
             return hv_fail(c, HV_ERR_UNSUPPORTED, "more than 2^21 - 2 generators and planes occur in the mesh (21-bit face keys)");
+        while ((1 << zb) < nused + 1) ++zb;   // every dense id is below 2^zb - 1
         gid = iget<int>(c, "i_gid", (size_t)std::max(1, nused));
+        hid = iget<uint32_t>(c, "i_hid", (size_t)std::max(1, nused));
         double* xd = iget<double>(c, "i_xd", (size_t)std::max(1, ngen) * D);
         double* pnd = iget<double>(c, "i_pnd", (size_t)std::max(1, nused - ngen) * D);
         double* phd = iget<double>(c, "i_phd", (size_t)std::max(1, nused - ngen));
-        if (!gid || !xd || !pnd || !phd) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
+        if (!gid || !hid || !xd || !pnd || !phd) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
         k_dense_inverse<<<nblk(nid, 256), 256, 0, c->stream>>>(used, dense, nid, gid);
         HVCK(hipGetLastError());
-        if (nv) {
-            k_remap_keys<D><<<nblk(nv, 256), 256, 0, c->stream>>>(vk0, nv, dense);
-            HVCK(hipGetLastError());
-        }
         if (nused) {
             k_dense_geo<D><<<nblk(nused, 256), 256, 0, c->stream>>>(gid, nused, ngen, g0.N, g0.xo, g0.pn, g0.ph, xd, pnd, phd);
+            HVCK(hipGetLastError());
+            k_id_hash<<<nblk(nused, 256), 256, 0, c->stream>>>(gid, nused, hid);
             HVCK(hipGetLastError());
         }
         g.N = ngen;
@@ -1147,29 +1121,41 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
         g.xo = xd;
         g.pn = pnd;
         g.ph = phd;
-        k_vkey_words<D><<<nblk(nv, 256), 256, 0, c->stream>>>(vk0, nv, w0, w1, w2, pa);
-        HVCK(hipGetLastError());
-        size_t tb = 0;
-        HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, ws, wso, pa, pb, nv, 0, 64, c->stream));
-        void* tmp = c->pool->get("i_vtmp", tb, false, c->stream);
-        if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
-        // least significant word first; each later pass is stable
-        const uint64_t* words[3] = {w2, w1, w0};
-        int* src = pa;
-        int* dst = pb;
-        for (int wi = (D >= 6 ? 0 : 1); wi < 3; ++wi) {
-            k_gather_u64<<<nblk(nv, 256), 256, 0, c->stream>>>(words[wi], src, nv, ws);
+        // the live vertices in a numbering fixed by the vertex set (not by the walk's insertion
+        // order), so that apexes and summation orders are reproducible: sorted by key, packed in
+        // words of as many ids as fit, least significant word first
+        uint64_t* w0 = iget<uint64_t>(c, "i_w0", nv1);
+        uint64_t* w1 = iget<uint64_t>(c, "i_w1", nv1);
+        int* pa = iget<int>(c, "i_vpa", nv1);
+        int* pb = iget<int>(c, "i_vpb", nv1);
+        if (!w0 || !w1 || !pa || !pb) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
+        if (nv) {
+            size_t tb = 0;
+            HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, w0, w1, pa, pb, nv, 0, 64, c->stream));
+            void* tmp = c->pool->get("i_vtmp", tb, false, c->stream);
+            if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
+            const int per = 64 / zb;
+            const int* order = nullptr;
+            for (int e = D + 1; e > 0;) {
+                const int n = order ? per : ((e % per) ? e % per : per);
+                e -= n;
+                k_vkey_word<D><<<nblk(nv, 256), 256, 0, c->stream>>>(mids, nv, mkey, dense, order, e, n, zb, w0, pa);
+                HVCK(hipGetLastError());
+                int* src = order ? pb : pa;
+                int* dst = order ? pa : pb;
+                HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, w0, w1, src, dst, nv, 0, n * zb, c->stream));
+                pa = src;
+                pb = dst;
+                order = pb;
+            }
+            k_int_permute<D><<<nblk(nv, 256), 256, 0, c->stream>>>(order, nv, mids, mkey, dense, (const double*)mesh->x.p, vk, vc);
             HVCK(hipGetLastError());
-            HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, ws, wso, src, dst, nv, 0, 64, c->stream));
-            std::swap(src, dst);
         }
-        k_int_permute<D><<<nblk(nv, 256), 256, 0, c->stream>>>(src, nv, vk0, vc0, vk, vc);
-        HVCK(hipGetLastError());
     }
     const int nf = fi ? fi->nf : 0;
     double* fv = nullptr;   // f at the vertices (edge ends)
     if (fi) {
-        fv = iget<double>(c, "i_fv", (size_t)nv * nf);
+        fv = iget<double>(c, "i_fv", nv1 * nf);
         if (!fv) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integrand)");
         int rc = eval_integrand(c, fi, D, vc, nv, fv);
         if (rc) return rc;
@@ -1177,8 +1163,8 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
     // Cells to integrate (dense ids), taken a chunk at a time.  A chunk's face passes hold the
     // vertices of its cells only: a face with one of the chunk's cells has all its vertices
     // there, and so do its sub-faces.  A facet of cells in two chunks is measured in both from
-    // the same vertex list in the same order (the canonical vertex order, restricted), so the
-    // two values are identical.  One chunk unless a pass would exceed HV_INC_BUDGET incidences.
+    // the same sub-faces in the same order (by their smallest id and hash), so the two values are
+    // identical.  One chunk unless a pass would exceed HV_INC_BUDGET pairs.
     std::vector<int> hcell;
     {
         std::vector<int> hd((size_t)g0.nreal + 1);
@@ -1193,16 +1179,16 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
             for (int i : *mesh->cells)
                 if (!add(i)) return hv_fail(c, HV_ERR_STATE, "a listed cell of the mesh has no vertex");
         } else {
+            hcell.reserve((size_t)g0.nreal);
             for (int i = 0; i < g0.nreal; ++i)
                 if (!add(i)) return hv_fail(c, HV_ERR_STATE, "a cell of the mesh has no vertex");
         }
     }
     const int ncell = (int)hcell.size();
-    int64_t cmax = 1;
-    for (int m = 2; m <= D; ++m) cmax = std::max(cmax, binom(D + 1, m));
+    const double cmax = pairs_bound(D);
     int nchunk = 1;
-    if ((int64_t)nv * cmax > HV_INC_BUDGET)
-        nchunk = (int)std::min<int64_t>(std::max(ncell, 1), (int64_t)std::ceil(1.3 * (double)nv * (double)cmax / (double)HV_INC_BUDGET));
+    if ((double)nv * cmax > (double)HV_INC_BUDGET)
+        nchunk = (int)std::min<int64_t>(std::max(ncell, 1), (int64_t)std::ceil(1.3 * (double)nv * cmax / (double)HV_INC_BUDGET));
     if (nchunk > 1) {
         // chunks of nearby cells (Morton order of the generators), so that few vertices are in two
         std::vector<double> hx((size_t)std::max(1, ngen) * D);
@@ -1229,12 +1215,19 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
         std::sort(code.begin(), code.end());
         for (int q = 0; q < ncell; ++q) hcell[q] = code[q].second;
     }
-    uint8_t* cmask = iget<uint8_t>(c, "i_cmask", (size_t)std::max(1, nused));
-    int* dchunk = iget<int>(c, "i_chunk", (size_t)std::max(1, ncell));
-    if (!cmask || !dchunk) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
-    if (ncell) HVCK(hipMemcpyAsync(dchunk, hcell.data(), sizeof(int) * ncell, hipMemcpyHostToDevice, c->stream));
+    // no mask when every generator that occurs is a cell of the one chunk
     const bool whole = nchunk == 1 && !mesh->cells;   // every vertex takes part: no selection
+    const bool every = whole && ncell == ngen;
+    uint8_t* cmask = nullptr;
+    int* dchunk = nullptr;
+    if (!every) {
+        cmask = iget<uint8_t>(c, "i_cmask", (size_t)std::max(1, nused));
+        dchunk = iget<int>(c, "i_chunk", (size_t)std::max(1, ncell));
+        if (!cmask || !dchunk) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
+        if (ncell) HVCK(hipMemcpyAsync(dchunk, hcell.data(), sizeof(int) * ncell, hipMemcpyHostToDevice, c->stream));
+    }
     auto set_chunk = [&](int q, int nch) -> int {
+        if (every) return HV_OK;
         const int cb = (int)((int64_t)ncell * q / nch), ce = (int)((int64_t)ncell * (q + 1) / nch);
         HVCK(hipMemsetAsync(cmask, 0, (size_t)std::max(1, nused), c->stream));
         if (ce > cb) {
@@ -1246,7 +1239,7 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
     int64_t nvc_max = nv;   // vertices of the largest chunk
     if (!whole && nchunk > 1) {
         // a vertex of cells in several chunks is in each of them: more chunks until every
-        // chunk's passes fit (at most 2^31 - 1 incidences)
+        // chunk's passes fit (at most 2^31 - 1 pairs)
         unsigned long long* vcnt = iget<unsigned long long>(c, "i_vcnt", 1);
         if (!vcnt) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
         for (;;) {
@@ -1262,7 +1255,7 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
                 HVCK(hipStreamSynchronize(c->stream));
                 worst = std::max<int64_t>(worst, (int64_t)h);
             }
-            if (worst * cmax < (1ll << 31)) {
+            if ((double)worst * cmax < (double)(1ll << 31)) {
                 nvc_max = worst;
                 break;
             }
@@ -1271,58 +1264,62 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
         }
     }
     {
-        // the per-incidence buffers of the face passes at their largest size, once: growing them
+        // the per-pair buffers of the face passes at their largest size, once: growing them
         // between passes and chunks frees and maps tens of GB while the device idles
-        const int64_t tmax = nvc_max * cmax;
-        if (tmax >= (1ll << 31)) return hv_fail(c, HV_ERR_CAPACITY, "too many face incidences for one pass");
-        const size_t T = (size_t)std::max<int64_t>(tmax, 1);
+        if ((double)nvc_max * cmax >= (double)(1ll << 31)) return hv_fail(c, HV_ERR_CAPACITY, "too many face incidences for one pass");
+        const size_t T = (size_t)std::max<int64_t>((int64_t)((double)nvc_max * cmax), 1);
         bool ok = true;
-        ok = ok && c->pool->reserve("i_keys", 32 * T, c->stream);   // lo, hi, lo2, hi2 of a pass
-        for (const char* nmv : {"i_pa", "i_pb", "i_iota", "i_vida", "i_vidb", "i_foia", "i_foib"})
-            ok = ok && c->pool->reserve(nmv, 4 * T, c->stream);
-        ok = ok && c->pool->reserve("i_head", T, c->stream);
-        ok = ok && c->pool->reserve("i_fsta", 4 * (T + 1), c->stream) && c->pool->reserve("i_fstb", 4 * (T + 1), c->stream);
+        for (const char* nmv : {"i_key", "i_key2", "i_pay"}) ok = ok && c->pool->reserve(nmv, 4 * T, c->stream);
+        ok = ok && c->pool->reserve("i_head", T, c->stream) && c->pool->reserve("i_start", 4 * (T + 1), c->stream);
         if (!whole) {
             ok = ok && c->pool->reserve("i_vkc", sizeof(int) * (size_t)std::max<int64_t>(nvc_max, 1) * (D + 1), c->stream);
             ok = ok && c->pool->reserve("i_vcc", sizeof(double) * (size_t)std::max<int64_t>(nvc_max, 1) * D, c->stream);
         }
         if (!ok) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
-        size_t tb = 0, tb2 = 0;
-        uint64_t* k0 = (uint64_t*)c->pool->get("i_keys", 0);
-        HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k0, (int*)nullptr, (int*)nullptr, (int)tmax, 0, 64, c->stream));
-        HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb2, (int*)nullptr, (uint8_t*)nullptr, (int*)nullptr, cnt + 1, (int)tmax, c->stream));
-        if (!c->pool->reserve("i_tmp", tb, c->stream) || !c->pool->reserve("i_tmp2", tb2, c->stream))
-            return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
+        size_t tb = 0;
+        const rocprim::counting_iterator<uint32_t> it(0u);
+        HVCK(rocprim::radix_sort_pairs(nullptr, tb, (uint32_t*)nullptr, (uint32_t*)nullptr, it, (uint32_t*)nullptr, T, 0u, 32u,
+                                       c->stream));
+        if (!c->pool->reserve("i_tmp", tb, c->stream)) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
     }
-    int64_t ntot = 0;                                  // rows of the chunks so far
+    int64_t ntot = 0;   // row slots of the chunks so far
+    uint64_t* rk = nullptr;
+    double *ra = nullptr, *ri = nullptr;
     for (int q = 0; q < nchunk; ++q) {
         {
             int rc = set_chunk(q, nchunk);
             if (rc) return rc;
         }
-        const int* vkc = vk;
-        const double* vcc = vc;
-        const double* fvc = fv;
-        int nvc = nv;
+        FacePass P;
+        P.vk = vk;
+        P.vc = vc;
+        P.fv = fv;
+        P.nv = nv;
+        P.cmask = cmask;
+        P.hid = hid;
+        P.hb = std::min(HV_GROUP_HASH, 32 - zb);
+        P.zb = zb;
+        P.nf = nf;
+        P.bad = bad;
+        P.cnt = cnt;
         if (!whole) {
             // the vertices holding a cell of the chunk, in the canonical order
-            uint8_t* vflag = iget<uint8_t>(c, "i_vflag", (size_t)std::max(1, nv));
-            int* viota = iget<int>(c, "i_viota", (size_t)std::max(1, nv));
-            int* vsel = iget<int>(c, "i_vsel", (size_t)std::max(1, nv));
-            if (!vflag || !viota || !vsel) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
+            uint8_t* vflag = iget<uint8_t>(c, "i_vflag", nv1);
+            int* vsel = iget<int>(c, "i_vsel", nv1);
+            if (!vflag || !vsel) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integration)");
+            int nvc = 0;
             if (nv) {
-                k_vert_in_chunk<D><<<nblk(nv, 256), 256, 0, c->stream>>>(vk, nv, ngen, cmask, vflag, viota);
+                k_vert_in_chunk<D><<<nblk(nv, 256), 256, 0, c->stream>>>(vk, nv, ngen, cmask, vflag);
                 HVCK(hipGetLastError());
+                size_t tbf = 0;
+                const hipcub::CountingInputIterator<int> pos(0);
+                HVCK(hipcub::DeviceSelect::Flagged(nullptr, tbf, pos, vflag, vsel, cnt, nv, c->stream));
+                void* tmpf = c->pool->get("i_tmpf", tbf, false, c->stream);
+                if (!tmpf) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
+                HVCK(hipcub::DeviceSelect::Flagged(tmpf, tbf, pos, vflag, vsel, cnt, nv, c->stream));
+                HVCK(hipMemcpyAsync(&nvc, cnt, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+                HVCK(hipStreamSynchronize(c->stream));
             }
-            size_t tbf = 0;
-            HVCK(hipcub::DeviceSelect::Flagged(nullptr, tbf, viota, vflag, vsel, cnt + 1, nv, c->stream));
-            void* tmpf = c->pool->get("i_tmpf", tbf, false, c->stream);
-            if (!tmpf) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
-            HVCK(hipcub::DeviceSelect::Flagged(tmpf, tbf, viota, vflag, vsel, cnt + 1, nv, c->stream));
-            unsigned long long hsel = 0;
-            HVCK(hipMemcpyAsync(&hsel, cnt + 1, sizeof(hsel), hipMemcpyDeviceToHost, c->stream));
-            HVCK(hipStreamSynchronize(c->stream));
-            nvc = (int)hsel;
             int* vk2 = iget<int>(c, "i_vkc", (size_t)std::max(1, nvc) * (D + 1));
             double* vc2 = iget<double>(c, "i_vcc", (size_t)std::max(1, nvc) * D);
             double* fv2 = fi ? iget<double>(c, "i_fvc", (size_t)std::max(1, nvc) * nf) : nullptr;
@@ -1331,244 +1328,68 @@ static int facet_rows(hv_ctx* c, const hv_mesh* mesh, const IntGeo& g0, uint64_t
                 k_int_subset<D><<<nblk(nvc, 256), 256, 0, c->stream>>>(vsel, nvc, vk, vc, fv, nf, vk2, vc2, fv2);
                 HVCK(hipGetLastError());
             }
-            vkc = vk2;
-            vcc = vc2;
-            fvc = fv2;
+            P.vk = vk2;
+            P.vc = vc2;
+            P.fv = fv2;
+            P.nv = nvc;
         }
-        // per pass: sorted incidences (vid), face starts, keys, measures; "1" = pass m + 1
-        int nface1 = 0;
-        for (int m = D; m >= 2; --m) {
-            const int C = (int)binom(D + 1, m);
-            const int64_t tot = (int64_t)nvc * C;
-            if (tot >= (1ll << 31)) return hv_fail(c, HV_ERR_CAPACITY, "too many face incidences for one pass");
-            const char* sfx = (m & 1) ? "a" : "b";
-            auto nm = [&](const char* s) { return std::string(s) + sfx; };
-            // the pass's four key arrays in one allocation (their space holds the sub-face
-            // records once the face table is out)
-            uint64_t* keys = iget<uint64_t>(c, "i_keys", 4 * (size_t)tot);
-            uint64_t* lo = keys;
-            uint64_t* hi = keys ? keys + tot : nullptr;
-            uint64_t* lo2 = keys ? keys + 2 * tot : nullptr;
-            uint64_t* hi2 = keys ? keys + 3 * tot : nullptr;
-            int* pa = iget<int>(c, "i_pa", tot);
-            int* pb = iget<int>(c, "i_pb", tot);
-            uint8_t* head = iget<uint8_t>(c, "i_head", tot);
-            if (!lo || !hi || !lo2 || !hi2 || !pa || !pb || !head) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
-            // faces with a cell of the chunk (the others may be incomplete here)
-            k_face_emit<D><<<nblk(std::max<int64_t>(tot, 1), 256), 256, 0, c->stream>>>(vkc, nvc, m, g.N, cmask, C, lo, hi, pa);
-            HVCK(hipGetLastError());
-            // two stable radix passes: by lo, then by hi -> (hi, lo) order.  Only the id fields a
-            // pass uses: the empty ones are all ones in every real key, and a real key's last
-            // used field is below all ones, so the incidences sent past the end stay there
-            const int lo_bits = 21 * std::min(m, 3), hi_bits = 21 * std::max(m - 3, 0);
-            size_t tb = 0, tbh = 0;
-            HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, lo, lo2, pa, pb, (int)tot, 0, lo_bits, c->stream));
-            if (m > 3)
-                HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tbh, hi2, hi, pb, pa, (int)tot, 0, hi_bits, c->stream));
-            void* tmp = c->pool->get("i_tmp", std::max(tb, tbh), false, c->stream);
-            if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
-            HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, lo, lo2, pa, pb, (int)tot, 0, lo_bits, c->stream));
-            int* perm = pb;
-            if (m > 3) {
-                k_gather_u64<<<nblk(tot, 256), 256, 0, c->stream>>>(hi, pb, tot, hi2);
+        int rc = face_pass<D, D>(c, g, P);
+        if (rc) return rc;
+        const int nface = P.nface;   // facets
+        double* I = nullptr;
+        if (fi) {
+            double* fc = iget<double>(c, "i_fc", (size_t)std::max(nface, 1) * nf);
+            I = iget<double>(c, "i_If", (size_t)std::max(nface, 1) * nf);
+            if (!fc || !I) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integrand)");
+            rc = eval_integrand(c, fi, D, P.cen, nface, fc);
+            if (rc) return rc;
+            if (nface > 0) {
+                k_facet_int<D><<<nblk(nface, 256), 256, 0, c->stream>>>(nface, P.J, fc, P.F.f, nf, I);
                 HVCK(hipGetLastError());
-                HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tbh, hi2, hi, pb, pa, (int)tot, 0, hi_bits, c->stream));
-                perm = pa;
-                k_gather_u64<<<nblk(tot, 256), 256, 0, c->stream>>>(lo, perm, tot, lo2);
-                HVCK(hipGetLastError());
-            }
-            // (m <= 3: every key's hi word is all ones, no id past the third field, so hi needs
-            // no reordering)
-            // lo2 / hi: sorted keys; perm: sorted incidence numbers
-            k_first_sent<<<1, 64, 0, c->stream>>>(lo2, tot, cnt);
-            HVCK(hipGetLastError());
-            unsigned long long hsent = 0;
-            HVCK(hipMemcpyAsync(&hsent, cnt, sizeof(hsent), hipMemcpyDeviceToHost, c->stream));
-            HVCK(hipStreamSynchronize(c->stream));
-            const int64_t nvalid = tot - (int64_t)hsent;
-            int* vid = iget<int>(c, nm("i_vid").c_str(), nvalid);
-            int* fstart = iget<int>(c, nm("i_fst").c_str(), nvalid + 1);
-            int* iota = iget<int>(c, "i_iota", nvalid);
-            if (!vid || !fstart || !iota) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
-            k_face_heads<<<nblk(nvalid, 256), 256, 0, c->stream>>>(lo2, hi, perm, nvalid, C, vid, head);
-            HVCK(hipGetLastError());
-            k_iota64<<<nblk(nvalid, 256), 256, 0, c->stream>>>(iota, nvalid);
-            HVCK(hipGetLastError());
-            size_t tb2 = 0;
-            HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb2, iota, head, fstart, cnt + 1, (int)nvalid, c->stream));
-            void* tmp2 = c->pool->get("i_tmp2", tb2, false, c->stream);
-            if (!tmp2) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
-            HVCK(hipcub::DeviceSelect::Flagged(tmp2, tb2, iota, head, fstart, cnt + 1, (int)nvalid, c->stream));
-            unsigned long long hnf = 0;
-            HVCK(hipMemcpyAsync(&hnf, cnt + 1, sizeof(hnf), hipMemcpyDeviceToHost, c->stream));
-            HVCK(hipStreamSynchronize(c->stream));
-            const int nface = (int)hnf;
-            const int endv = (int)nvalid;
-            HVCK(hipMemcpyAsync(fstart + nface, &endv, sizeof(int), hipMemcpyHostToDevice, c->stream));
-            uint64_t* flo = iget<uint64_t>(c, nm("i_flo").c_str(), nface);
-            uint64_t* fhi = iget<uint64_t>(c, nm("i_fhi").c_str(), nface);
-            double* meas = iget<double>(c, nm("i_meas").c_str(), nface);
-            if (!flo || !fhi || !meas) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
-            k_face_table<<<nblk(nface, 256), 256, 0, c->stream>>>(fstart, nface, lo2, hi, flo, fhi);
-            HVCK(hipGetLastError());
-            if (m > 2) {   // the next pass finds its sub-faces here
-                int* foi = iget<int>(c, nm("i_foi").c_str(), tot);
-                if (!foi) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (faces)");
-                HVCK(hipMemsetAsync(foi, 0x80, sizeof(int) * tot, c->stream));   // no face: decodes past the end
-                k_face_inc<<<nblk(nface, 256), 256, 0, c->stream>>>(fstart, nface, perm, foi);
-                HVCK(hipGetLastError());
-            }
-            double* J = fi ? iget<double>(c, nm("i_J").c_str(), (size_t)nface * nf) : nullptr;
-            if (fi && !J) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integrand)");
-            if (m == D) {
-                k_edge_len<D><<<nblk(nface, 256), 256, 0, c->stream>>>(fstart, nface, vid, vcc, meas, bad);
-                if (fi) {
-                    HVCK(hipGetLastError());
-                    k_edge_int<<<nblk(nface, 256), 256, 0, c->stream>>>(fstart, nface, vid, meas, fvc, nf, J);
-                }
-            } else {
-                const char* s1 = (m & 1) ? "b" : "a";
-                auto n1 = [&](const char* s) { return std::string(s) + s1; };
-                const int C1 = (int)binom(D + 1, m + 1);
-                const int* foi1 = (const int*)c->pool->get(n1("i_foi"), 0);
-                const double* meas1 = (const double*)c->pool->get(n1("i_meas"), 0);
-                if (!foi1 || !meas1) return hv_fail(c, HV_ERR_DEVICE, "face tables of the previous pass missing");
-                const int L = hv_face_lanes(D, m);
-                // sub-face records in the key arrays' space, free once the face table is out
-                HvRec rec{nullptr, 0};
-                if (D - m <= 3) {   // facets in 6D (five entries) read the keys directly
-                    rec.p = keys;
-                    rec.ne = D + 1 - m;
-                    k_face_rec<D><<<nblk(std::max<int64_t>(tot, 1), 256), 256, 0, c->stream>>>(
-                        (const int*)vkc, tot, m, C, C1, foi1, rec);
-                    HVCK(hipGetLastError());
-                }
-#define HV_FM(LL) hv_face_launch<LL>(k_face_measure<D, LL>, nface, c->stream, g, m, nface, fstart, vid, flo, fhi, \
-                                     nface1, C1, foi1, meas1, (const int*)vkc, (const double*)vcc, (const int*)perm, \
-                                     rec, meas, bad)
-                if (L == 64) HV_FM(64);
-                else if (L == 16) HV_FM(16);
-                else HV_FM(1);
-#undef HV_FM
-                if (fi) {
-                    HVCK(hipGetLastError());
-                    double* cen = iget<double>(c, "i_cen", (size_t)nface * D);
-                    const double* J1 = (const double*)c->pool->get(n1("i_J"), 0);
-                    if (!cen || !J1) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integrand)");
-                    k_face_center<D><<<nblk(nface, 256), 256, 0, c->stream>>>(fstart, nface, vid, vcc, cen);
-                    HVCK(hipGetLastError());
-#define HV_FI(LL) hv_face_launch<LL>(k_face_int<D, LL>, nface, c->stream, g, m, nface, fstart, vid, flo, fhi, \
-                                     (const double*)cen, nface1, C1, foi1, J1, nf, (const int*)vkc, \
-                                     (const int*)perm, rec, J, bad)
-                    if (L == 64) HV_FI(64);
-                    else if (L == 16) HV_FI(16);
-                    else HV_FI(1);
-#undef HV_FI
-                }
-            }
-            HVCK(hipGetLastError());
-            double* Iface = nullptr;   // facet integrals (m == 2)
-            if (fi && m == 2) {
-                double* cen = iget<double>(c, "i_cen", (size_t)nface * D);
-                double* fc = iget<double>(c, "i_fc", (size_t)nface * nf);
-                Iface = iget<double>(c, "i_If", (size_t)nface * nf);
-                if (!cen || !fc || !Iface) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integrand)");
-                if (m == D) {   // d = 2: the facets are the edges, no centres yet
-                    k_face_center<D><<<nblk(nface, 256), 256, 0, c->stream>>>(fstart, nface, vid, vcc, cen);
-                    HVCK(hipGetLastError());
-                }
-                int rc = eval_integrand(c, fi, D, cen, nface, fc);
-                if (rc) return rc;
-                k_facet_int<D><<<nblk(nface, 256), 256, 0, c->stream>>>(nface, J, fc, meas, nf, Iface);
-                HVCK(hipGetLastError());
-            }
-            nface1 = nface;
-            if (m == 2) {
-                pkey = iget<uint64_t>(c, "i_pkey", (size_t)2 * nface);
-                uint64_t* pkey2 = iget<uint64_t>(c, "i_pkey2", (size_t)2 * nface);
-                parea = iget<double>(c, "i_parea", (size_t)2 * nface);
-                double* parea2 = iget<double>(c, "i_parea2", (size_t)2 * nface);
-                int* pface2 = iget<int>(c, "i_pface2", (size_t)2 * nface);
-                if (!pkey || !pkey2 || !parea || !parea2 || !pface2)
-                    return hv_fail(c, HV_ERR_DEVICE, "out of device memory (facets)");
-                HVCK(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), c->stream));
-                k_facet_pairs<<<nblk(nface, 256), 256, 0, c->stream>>>(nface, flo, meas, g.N, cmask, pkey2, parea2, pface2, cnt);
-                HVCK(hipGetLastError());
-                unsigned long long hp = 0;
-                HVCK(hipMemcpyAsync(&hp, cnt, sizeof(hp), hipMemcpyDeviceToHost, c->stream));
-                HVCK(hipStreamSynchronize(c->stream));
-                npair = (int64_t)hp;
-                size_t tb3 = 0;
-                HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb3, pkey2, pkey, parea2, parea, (int)npair, 0, 64, c->stream));
-                void* tmp3 = c->pool->get("i_tmp3", tb3, false, c->stream);
-                if (!tmp3) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
-                HVCK(hipcub::DeviceRadixSort::SortPairs(tmp3, tb3, pkey2, pkey, parea2, parea, (int)npair, 0, 64, c->stream));
-                if (fi) {
-                    // the same stable sort carrying the facet numbers, then the rows' integrals
-                    uint64_t* pkey3 = iget<uint64_t>(c, "i_pkey3", (size_t)2 * nface);
-                    int* pface = iget<int>(c, "i_pface", (size_t)2 * nface);
-                    *rint = iget<double>(c, "i_rint", (size_t)std::max<int64_t>(npair, 1) * nf);
-                    if (!pkey3 || !pface || !*rint) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (integrand)");
-                    size_t tb4 = 0;
-                    HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb4, pkey2, pkey3, pface2, pface, (int)npair, 0, 64, c->stream));
-                    void* tmp4 = c->pool->get("i_tmp4", tb4, false, c->stream);
-                    if (!tmp4) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
-                    HVCK(hipcub::DeviceRadixSort::SortPairs(tmp4, tb4, pkey2, pkey3, pface2, pface, (int)npair, 0, 64, c->stream));
-                    if (npair > 0) {
-                        k_row_int<<<nblk(npair, 256), 256, 0, c->stream>>>(npair, pface, Iface, nf, *rint);
-                        HVCK(hipGetLastError());
-                    }
-                }
             }
         }
-        if (!whole || nchunk > 1) {
-            // this chunk's rows after the rows of the chunks before
-            uint64_t* rk = (uint64_t*)c->pool->get("i_rk", sizeof(uint64_t) * (size_t)std::max<int64_t>(ntot + npair, 1), true, c->stream);
-            double* ra = (double*)c->pool->get("i_ra", sizeof(double) * (size_t)std::max<int64_t>(ntot + npair, 1), true, c->stream);
-            double* ri = fi ? (double*)c->pool->get("i_ri", sizeof(double) * (size_t)std::max<int64_t>(ntot + npair, 1) * nf, true, c->stream)
-                            : nullptr;
-            if (!rk || !ra || (fi && !ri)) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rows)");
-            if (npair) {
-                HVCK(hipMemcpyAsync(rk + ntot, pkey, sizeof(uint64_t) * npair, hipMemcpyDeviceToDevice, c->stream));
-                HVCK(hipMemcpyAsync(ra + ntot, parea, sizeof(double) * npair, hipMemcpyDeviceToDevice, c->stream));
-                if (fi) HVCK(hipMemcpyAsync(ri + ntot * nf, *rint, sizeof(double) * npair * nf, hipMemcpyDeviceToDevice, c->stream));
-            }
-            ntot += npair;
+        // this chunk's rows after the rows of the chunks before
+        const size_t slots = (size_t)std::max<int64_t>(ntot + 2 * (int64_t)nface, 1);
+        rk = (uint64_t*)c->pool->get("i_rk", sizeof(uint64_t) * slots, ntot > 0, c->stream);
+        ra = (double*)c->pool->get("i_ra", sizeof(double) * slots, ntot > 0, c->stream);
+        ri = fi ? (double*)c->pool->get("i_ri", sizeof(double) * slots * nf, ntot > 0, c->stream) : nullptr;
+        if (!rk || !ra || (fi && !ri)) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rows)");
+        if (nface > 0) {
+            k_facet_rows<<<nblk(nface, 256), 256, 0, c->stream>>>(nface, P.F, ngen, cmask, zb, rk + ntot, ra + ntot, I, nf,
+                                                                  fi ? ri + ntot * nf : nullptr);
+            HVCK(hipGetLastError());
         }
+        ntot += 2 * (int64_t)nface;
     }
-    if (!whole || nchunk > 1) {
-        // rows of all chunks, sorted by (cell, neighbour)
-        uint64_t* rk = (uint64_t*)c->pool->get("i_rk", 0);
-        double* ra = (double*)c->pool->get("i_ra", 0);
-        double* ri = fi ? (double*)c->pool->get("i_ri", 0) : nullptr;
-        npair = ntot;
-        pkey = iget<uint64_t>(c, "i_pkey", (size_t)npair);
-        parea = iget<double>(c, "i_parea", (size_t)npair);
-        int* ia = iget<int>(c, "i_rpa", (size_t)npair);
-        int* ib = iget<int>(c, "i_rpb", (size_t)npair);
-        if (fi) *rint = iget<double>(c, "i_rint", (size_t)std::max<int64_t>(npair, 1) * nf);
-        if (!rk || !ra || !pkey || !parea || !ia || !ib || (fi && (!ri || !*rint)))
-            return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rows)");
-        if (npair > 0) {
-            k_iota64<<<nblk(npair, 256), 256, 0, c->stream>>>(ia, npair);
-            HVCK(hipGetLastError());
-            size_t tbr = 0;
-            HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tbr, rk, pkey, ia, ib, (int)npair, 0, 64, c->stream));
-            void* tmpr = c->pool->get("i_tmpr", tbr, false, c->stream);
-            if (!tmpr) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
-            HVCK(hipcub::DeviceRadixSort::SortPairs(tmpr, tbr, rk, pkey, ia, ib, (int)npair, 0, 64, c->stream));
-            k_gather_rows<<<nblk(npair, 256), 256, 0, c->stream>>>(ib, npair, ra, parea, ri, fi ? *rint : nullptr, nf);
-            HVCK(hipGetLastError());
-        }
-    }
-    if (npair > 0) {
-        k_rows_to_ids<<<nblk(npair, 256), 256, 0, c->stream>>>(pkey, npair, gid);
+    // rows of all chunks, sorted by (cell, neighbour), in the caller's ids
+    if (ntot >= (1ll << 31)) return hv_fail(c, HV_ERR_CAPACITY, "too many rows");
+    const size_t nr = (size_t)std::max<int64_t>(ntot, 1);
+    uint64_t* rk2 = iget<uint64_t>(c, "i_rk2", nr);
+    int* rpb = iget<int>(c, "i_rpb", nr);
+    pkey = iget<uint64_t>(c, "i_pkey", nr);
+    parea = iget<double>(c, "i_parea", nr);
+    if (fi) *rint = iget<double>(c, "i_rint", nr * nf);
+    if (!rk2 || !rpb || !pkey || !parea || (fi && !*rint)) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rows)");
+    int hres[2] = {0, 0};   // flags, rows
+    HVCK(hipMemsetAsync(cnt, 0, sizeof(int), c->stream));
+    if (ntot > 0) {
+        // 2 zb bits and the one above them, set in the slots of no row only
+        size_t tbr = 0;
+        const rocprim::counting_iterator<int> it(0);
+        const unsigned nbits = (unsigned)std::min(2 * zb + 1, 64);
+        HVCK(rocprim::radix_sort_pairs(nullptr, tbr, rk, rk2, it, rpb, (size_t)ntot, 0u, nbits, c->stream));
+        void* tmpr = c->pool->get("i_tmpr", tbr, false, c->stream);
+        if (!tmpr) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
+        HVCK(rocprim::radix_sort_pairs(tmpr, tbr, rk, rk2, it, rpb, (size_t)ntot, 0u, nbits, c->stream));
+        k_rows_out<<<nblk(ntot, 256), 256, 0, c->stream>>>(rk2, rpb, ntot, zb, gid, ra, ri, nf, pkey, parea,
+                                                          fi ? *rint : nullptr, cnt);
         HVCK(hipGetLastError());
     }
-    int hbad = 0;
-    HVCK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HVCK(hipMemcpyAsync(&hres[0], bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HVCK(hipMemcpyAsync(&hres[1], cnt, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HVCK(hipStreamSynchronize(c->stream));
-    if (hbad) return hv_fail(c, HV_ERR_DEGENERATE, "a face is not in general position (integration)");
+    npair = hres[1];
+    if (hres[0]) return hv_fail(c, HV_ERR_DEGENERATE, "a face is not in general position (integration)");
     return HV_OK;
 }
 
