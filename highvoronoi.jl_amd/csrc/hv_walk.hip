@@ -1165,17 +1165,29 @@ __global__ __launch_bounds__(256) void k_ray_init(DevGeo g0, GeoSet F, DevRays R
 // (src/raycast.jl:877-916) is applied to them at the end.
 // One wavefront per workgroup: packets take very different times, and a workgroup of
 // several wavefronts holds its slots until its slowest packet is done.
-// The HV_KNN nearest generators of every generator, 64 Morton-consecutive queries per
-// wavefront: the packet's own 64 points first, then the 8-ary tree nearest-first, entering a
-// child when its box is within the current 16th distance of some query (FP32 test, widened);
-// each visited leaf is staged in LDS and scanned by every lane into a sorted top-16.
+// The HV_KNN nearest generators of every generator, one wavefront each: the 64 Morton neighbours of
+// the generator first (sorted across the lanes; the best 16 stay, one per lane, in each of the
+// four rows of 16 lanes), which leaves the 16th distance close to its final value, then the
+// 8-ary tree: eight waiting nodes are tested at once (a lane per child box), and reached leaves
+// are measured 64 points at a time; a point below the 16th distance is shifted into the list.
+// FP32 throughout, the box test widened: the lists only supply candidates that are measured in
+// FP64.  A wavefront that served 64 generators (every lane its own list) left the chip idle, 313
+// wavefronts at N=20k, and ran every insertion under divergence: 2D N=1000 146 -> 12 us, 4D N=20k
+// 1 140 -> 93 us, 5D N=100k mixture 3.6 -> 0.77 ms.
+constexpr int HV_KNN_WAVES = 4;     // wavefronts per workgroup
+constexpr int HV_KNN_STACK = 512;   // 8 popped and at most 64 pushed per level of at most 9
+
 template <int D, bool B>
-__global__ __launch_bounds__(64) void k_knn64(DevGeo g0, GeoSet F, const int* __restrict__ boff, int* __restrict__ knn0) {
-    __shared__ int stk[128], stkl[128];
-    __shared__ float cbx[16 * D];
-    __shared__ unsigned long long hms[8];
-    __shared__ float px[D][64];
-    const int lane = threadIdx.x;
+__global__ __launch_bounds__(64 * HV_KNN_WAVES) void k_knn(DevGeo g0, GeoSet F, const int* __restrict__ boff,
+                                                           int* __restrict__ knn0) {
+    static_assert(HV_KNN == 16, "one list entry per lane of a row of 16");
+    __shared__ int stk_[HV_KNN_WAVES][HV_KNN_STACK];
+    __shared__ float sd_[HV_KNN_WAVES][HV_KNN_STACK];
+    __shared__ int lq_[HV_KNN_WAVES][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int* stk = stk_[wv];
+    float* sd = sd_[wv];
+    int* lq = lq_[wv];
     int blk = hv_xcd_block(), mk = 0;
     if constexpr (B) {   // block of the whole grid -> (mesh, block of the mesh)
         mk = __builtin_amdgcn_readfirstlane(hv_mesh_of_item(boff, F.nmesh, blk));
@@ -1184,175 +1196,133 @@ __global__ __launch_bounds__(64) void k_knn64(DevGeo g0, GeoSet F, const int* __
     const DevGeo& g = hv_geo_mesh<B>(g0, F, mk);
     int* knn = B ? const_cast<int*>(g.knn) : knn0;
     const int N = g.n;   // sorted positions
-    const int base = blk * 64;
-    const int j = base + lane;
-    const bool act = j < N;
-    const int jj = act ? j : N - 1;
-    // FP32 distances: the lists only supply candidates that are always evaluated in FP64
+    const int j = __builtin_amdgcn_readfirstlane(blk * HV_KNN_WAVES + wv);
+    if (j >= N) return;   // no workgroup barrier below
+    const int base = j & ~63;
+    constexpr float FAR = 3.0e38f;
     float pf[D];
 #pragma unroll
-    for (int k = 0; k < D; ++k) pf[k] = (float)g.xs[(int64_t)jj * (D + 1) + k];
-    float bd[HV_KNN];
-    int bi[HV_KNN];
-#pragma unroll
-    for (int m = 0; m < HV_KNN; ++m) { bd[m] = 3.0e38f; bi[m] = jj; }
-    auto consider = [&](int q, float d2) {
-        if (!(d2 < bd[HV_KNN - 1]) || q == jj) return;
-        int pos = 0;
-#pragma unroll
-        for (int m = 0; m < HV_KNN; ++m) pos += (bd[m] <= d2) ? 1 : 0;
-#pragma unroll
-        for (int m = HV_KNN - 1; m > 0; --m) {
-            bd[m] = (m > pos) ? bd[m - 1] : ((m == pos) ? d2 : bd[m]);
-            bi[m] = (m > pos) ? bi[m - 1] : ((m == pos) ? q : bi[m]);
-        }
-        bd[0] = (pos == 0) ? d2 : bd[0];
-        bi[0] = (pos == 0) ? q : bi[0];
-    };
-    // scan the npts points staged in px (global ids q0 + s)
-    auto scan_staged = [&](int q0, int npts, bool skip_own) {
-        for (int s = 0; s < npts; ++s) {
-            const int q = q0 + s;
-            if (skip_own && q >= base && q < base + 64) continue;
-            float d2 = 0.f;
-#pragma unroll
-            for (int k = 0; k < D; ++k) {
-                const float a = px[k][s] - pf[k];
-                d2 = fmaf(a, a, d2);
-            }
-            consider(q, d2);
-        }
-    };
-    {
-        const int np = min(64, N - base);
-#pragma unroll
-        for (int k = 0; k < D; ++k) px[k][lane] = pf[k];
-        hv_wave_sync();
-        scan_staged(base, np, false);
-        hv_wave_sync();
-    }
-    // packet centre (uniform) orders the children
-    float pcf[D];
-    {
-        double c[D], cnt = act ? 1.0 : 0.0;
-#pragma unroll
-        for (int k = 0; k < D; ++k) c[k] = act ? (double)pf[k] : 0.0;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-            for (int k = 0; k < D; ++k) c[k] += __shfl_xor(c[k], off);
-            cnt += __shfl_xor(cnt, off);
-        }
-#pragma unroll
-        for (int k = 0; k < D; ++k)
-            pcf[k] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint((float)(c[k] / cnt))));
-    }
-    auto child_d2f = [&](int c, const float* q) {
+    for (int k = 0; k < D; ++k) pf[k] = g.xf[(int64_t)j * 8 + k];
+    auto dist = [&](int q) {
         float d2 = 0.f;
+        const float4 A = ((const float4*)g.xf)[(int64_t)q * 2];
+        float x[8] = {A.x, A.y, A.z, A.w, 0.f, 0.f, 0.f, 0.f};
+        if constexpr (D > 4) {
+            const float4 Bq = ((const float4*)g.xf)[(int64_t)q * 2 + 1];
+            x[4] = Bq.x; x[5] = Bq.y; x[6] = Bq.z; x[7] = Bq.w;
+        }
 #pragma unroll
         for (int k = 0; k < D; ++k) {
-            const float a = q[k] - __builtin_amdgcn_fmed3f(q[k], cbx[c * 2 * D + k], cbx[c * 2 * D + D + k]);
+            const float a = x[k] - pf[k];
             d2 = fmaf(a, a, d2);
         }
         return d2;
     };
+    // the generator's own block of 64, bitonic sort across the lanes by (distance, position)
+    float bd = FAR;
+    int bi = j;
+    if (base + lane < N && base + lane != j) {
+        bd = dist(base + lane);
+        bi = base + lane;
+    }
+#pragma unroll
+    for (int w = 2; w <= 64; w <<= 1)
+#pragma unroll
+        for (int s = w >> 1; s > 0; s >>= 1) {
+            const float od = __shfl_xor(bd, s);
+            const int oi = __shfl_xor(bi, s);
+            const bool up = (lane & w) == 0, low = (lane & s) == 0;
+            const bool less = od < bd || (od == bd && oi < bi);
+            const bool take = (low == up) ? less : (od > bd || (od == bd && oi > bi));
+            bd = take ? od : bd;
+            bi = take ? oi : bi;
+        }
+    bd = __shfl(bd, lane & 15);   // the best 16, ascending, in every row
+    bi = __shfl(bi, lane & 15);
+    float thr = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bd), 15));
     const float slack = 1e-6f * (float)(g.xmax + 1.0);
     auto reach = [&]() {   // widened radius^2 of the current 16th neighbour
-        const float r = sqrtf(bd[HV_KNN - 1]) + slack;
+        const float r = sqrtf(thr) + slack;
         return fminf(r * r * (1.0f + 1e-5f), 1e30f);
     };
-    // children ordered by distance to the packet centre (ties: lower index first): rank r
-    // holds child (ord >> 4r) & 7
-    uint32_t ord = 0u;
-    auto to_rank = [&](unsigned cm) {
-        unsigned rr = 0u;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) rr |= ((cm >> ((ord >> (4 * q)) & 7u)) & 1u) << q;
-        return rr;
-    };
+    float R2f = reach();
     int sp = 1;
-    stk[0] = 0;
-    stkl[0] = 0;
+    if (lane == 0) {
+        stk[0] = 0;
+        sd[0] = 0.f;
+    }
+    hv_wave_sync();
     while (sp > 0) {
-        --sp;
-        hv_wave_sync();
-        const int gid = __builtin_amdgcn_readfirstlane(stk[sp]);
-        const int l = __builtin_amdgcn_readfirstlane(stkl[sp]);
-        {
-            const float* src = g.cb + (int64_t)gid * (16 * D);
-            for (int q = lane; q < 16 * D; q += 64) cbx[q] = src[q];
-        }
-        hv_wave_sync();
-        const float R2f = reach();
-        unsigned rem = 0u;
+        const int nb = min(8, sp), grp = lane >> 3, c = lane & 7;
+        bool ok = false, leaf = false;
+        int child = 0;
+        float d2 = 0.f;
+        if (grp < nb && sd[sp - 1 - grp] <= R2f) {
+            const int e = stk[sp - 1 - grp];
+            const int l = e >> 27, gid = e & ((1 << 27) - 1);
+            const float* box = g.cb + ((int64_t)gid * 8 + c) * (2 * D);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const unsigned long long m = __ballot(act && (child_d2f(c, pf) <= R2f));
-            if (lane == 0) hms[c] = m;
-            rem |= (m != 0ull) ? (1u << c) : 0u;
-        }
-        {
-            const uint32_t kb = __float_as_uint(child_d2f(lane & 7, pcf));   // non-negative: orders as unsigned
-            const int me = lane & 7;
-            int rk = 0;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const uint32_t kc = __builtin_amdgcn_readlane(kb, c);
-                rk += (kc < kb || (kc == kb && c < me)) ? 1 : 0;
+            for (int k = 0; k < D; ++k) {
+                const float a = pf[k] - __builtin_amdgcn_fmed3f(pf[k], box[k], box[D + k]);
+                d2 = fmaf(a, a, d2);
             }
-            uint32_t o = 0u;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) o |= (uint32_t)c << (4 * __builtin_amdgcn_readlane(rk, c));
-            ord = o;
+            ok = d2 <= R2f;
+            leaf = l + 1 == g.h;
+            const int first = ((1 << (3 * l)) - 1) / 7;   // first node id of the level
+            child = leaf ? 8 * (gid - first) + c
+                         : (((l + 1) << 27) | (first + (1 << (3 * l)) + 8 * (gid - first) + c));
         }
-        rem = __builtin_amdgcn_readfirstlane(rem);
+        sp -= nb;
+        const unsigned long long mi = __ballot(ok && !leaf), ml = __ballot(ok && leaf);
+        const unsigned long long below = lane ? ((1ull << lane) - 1ull) : 0ull;
         hv_wave_sync();
-        if (rem == 0u) continue;
-        const int off = ((1 << (3 * l)) - 1) / 7;
-        const int i = gid - off;
-        if (l + 1 == g.h) {
-            unsigned rr = to_rank(rem);
-            while (rr) {
-                const int cc = (ord >> (4 * __builtin_ctz(rr))) & 7u;
-                rr &= rr - 1u;
-                const int leaf = 8 * i + cc;
-                const int j0 = leaf * g.L, npts = max(0, min(g.L, N - j0));
-                if (j0 >= base && j0 + npts <= base + 64) continue;   // the packet's own points
-                const bool hit = act && ((hms[cc] >> lane) & 1ull) && (child_d2f(cc, pf) <= reach());
-                if (__ballot(hit) == 0ull) continue;
-                for (int s0 = 0; s0 < npts; s0 += 64) {
-                    const int cnt = min(64, npts - s0);
-                    if (lane < cnt) {
-#pragma unroll
-                        for (int k = 0; k < D; ++k) px[k][lane] = (float)g.xs[(int64_t)(j0 + s0 + lane) * (D + 1) + k];
-                    }
-                    hv_wave_sync();
-                    if (hit) scan_staged(j0 + s0, cnt, true);
-                    hv_wave_sync();
+        if (ok && !leaf) {
+            const int at = sp + __popcll(mi & below);
+            stk[at] = child;
+            sd[at] = d2;
+        }
+        if (ok && leaf) lq[__popcll(ml & below)] = child;
+        sp += __popcll(mi);
+        hv_wave_sync();
+        const int nl = __popcll(ml);
+        // leaves of up to 32 points two at a time, larger ones in pieces of 64
+        const int per = g.L <= 32 ? 2 : 1;
+        for (int q0 = 0; q0 < nl; q0 += per) {
+            for (int s0 = 0; s0 < g.L; s0 += 64) {
+                const int in = per == 2 ? (lane & 31) : s0 + lane;
+                const int qq = q0 + (per == 2 ? (lane >> 5) : 0);
+                int q = N;
+                if (qq < nl && in < g.L) q = lq[qq] * g.L + in;
+                float dq = FAR;
+                if (q < N && (q < base || q >= base + 64)) dq = dist(q);
+                unsigned long long m = __ballot(dq < thr);
+                if (m == 0ull) continue;
+                while (m) {
+                    const int s = __ffsll((long long)m) - 1;
+                    const float dn = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(dq), s));
+                    const int qn = __builtin_amdgcn_readlane(q, s);
+                    // entries above dn move one lane up (row_shr:1; a row's first lane sees -1)
+                    const float ud = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(-1.0f), __float_as_int(bd),
+                                                                               0x111, 0xf, 0xf, false));
+                    const int ui = __builtin_amdgcn_update_dpp(0, bi, 0x111, 0xf, 0xf, false);
+                    const bool keep = bd <= dn, here = ud <= dn;
+                    bi = keep ? bi : (here ? qn : ui);
+                    bd = keep ? bd : (here ? dn : ud);
+                    thr = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bd), 15));
+                    m &= m - 1ull;
+                    m &= __ballot(dq < thr);
                 }
-            }
-        } else {
-            const int cbase = off + (1 << (3 * l)) + 8 * i;
-            unsigned rr = to_rank(rem);
-            while (rr) {
-                const int q = 31 - __builtin_clz(rr);
-                rr &= ~(1u << q);
-                const int c = (ord >> (4 * q)) & 7u;
-                stk[sp] = cbase + c;
-                stkl[sp] = l + 1;
-                ++sp;
+                R2f = reach();
             }
         }
+        hv_wave_sync();   // lq and the stack are read before the next step writes them
     }
-    if (act) {
-#pragma unroll
-        for (int m = 0; m < HV_KNN; ++m) knn[(int64_t)j * HV_KNN + m] = bi[m];
-    }
+    if (lane < HV_KNN) knn[(int64_t)j * HV_KNN + lane] = bi;
 }
 
 // Point-sample Monte Carlo: wavefront w holds samples 64w .. 64w+63, all in stratum
 // floor(64w / S) of a G^d grid over the domain box (S samples per stratum, a multiple of 64),
-// each uniform in its stratum from a counter-based stream.  A packet walk as in k_knn64 finds
+// each uniform in its stratum from a counter-based stream.  A packet walk as in k_raycast64 finds
 // each sample's nearest and second-nearest generators (FP64 distances to the staged leaves).
 // Accumulated: the samples of each nearest cell (one atomic per distinct cell of the
 // wavefront), and per (cell, neighbour) row the samples that lie within eps (counter 2 row)
@@ -2403,7 +2373,7 @@ static TreeDims tree_dims(int n, int L) {
 // the 16-NN lists of one tree
 template <int D>
 int build_knn(hv_ctx* c, const DevGeo& g, int* knn, hipStream_t st) {
-    k_knn64<D, false><<<nblk(g.n, 64), 64, 0, st>>>(g, GeoSet{}, nullptr, knn);
+    k_knn<D, false><<<nblk(g.n, HV_KNN_WAVES), 64 * HV_KNN_WAVES, 0, st>>>(g, GeoSet{}, nullptr, knn);
     HVCK(hipGetLastError());
     return HV_OK;
 }
@@ -3200,11 +3170,11 @@ static int build_forest(hv_ctx* c, int L, int tables, Forest& fo) {
     // 16-NN lists and scan tables of every mesh in one launch each (items numbered mesh after mesh)
     {
         std::vector<int> hoff(3 * (nm + 1), 0);
-        int* ob = hoff.data();             // blocks of 64 points (16-NN)
+        int* ob = hoff.data();             // blocks of HV_KNN_WAVES points (16-NN)
         int* og = ob + (nm + 1);           // groups of 8 leaves (origins)
         int* op = og + (nm + 1);           // padded points of whole leaves (K-vectors / FP32 rows)
         for (int k = 0; k < nm; ++k) {
-            ob[k + 1] = ob[k] + (fo.n[k] + 63) / 64;
+            ob[k + 1] = ob[k] + (fo.n[k] + HV_KNN_WAVES - 1) / HV_KNN_WAVES;
             og[k + 1] = og[k] + (fo.geo[k].nleaf + 7) / 8;
             op[k + 1] = op[k] + fo.geo[k].nleaf * 32;
         }
@@ -3212,7 +3182,7 @@ static int build_forest(hv_ctx* c, int L, int tables, Forest& fo) {
         if (!doff) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (batch trees)");
         HVCK(hipMemcpyAsync(doff, hoff.data(), sizeof(int) * hoff.size(), hipMemcpyHostToDevice, c->stream));
         GeoSet Ft{gs, mof, nm};
-        k_knn64<D, true><<<ob[nm], 64, 0, c->stream>>>(DevGeo{}, Ft, doff, nullptr);
+        k_knn<D, true><<<ob[nm], 64 * HV_KNN_WAVES, 0, c->stream>>>(DevGeo{}, Ft, doff, nullptr);
         HVCK(hipGetLastError());
         if (tables != HV_PREC_FP64) {
             k_leaf_origin<D, true><<<og[nm], 64, 0, c->stream>>>(DevGeo{}, Ft, doff + (nm + 1), nullptr);
