@@ -1743,12 +1743,13 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
         for (int z = 0; z < D; ++z) kid[lane][z] = G.e[z] < N ? g.rank[G.e[z]] : -1;
     }
     if constexpr (MODE == 1) rk4[lane][3] = hv_u32x4{0u, 0u, 0u, 0u};   // K-slots 24..31
-    auto leaf_known = [&](int leaf) -> uint32_t {
+    auto leaf_known = [&](int leaf) -> uint32_t {   // ids of the leaf differ from leaf * 32 in 5 bits
+        const uint32_t first = (uint32_t)leaf << 5;
         uint32_t km = 0u;
 #pragma unroll
         for (int z = 0; z < D + 2; ++z) {
-            const int id = z < D ? kid[lane][z] : (z == D ? T.i1 : T.i2);
-            km |= (id >= 0 && (id >> 5) == leaf) ? (1u << (id & 31)) : 0u;
+            const uint32_t x = (uint32_t)(z < D ? kid[lane][z] : (z == D ? T.i1 : T.i2)) ^ first;
+            km |= x < 32u ? (1u << x) : 0u;
         }
         return km;
     };
@@ -1761,18 +1762,6 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
             d2 = fmaf(a, a, d2);
         }
         return d2;
-    };
-    // children of the staged node ordered by distance to the packet centre (ties: lower
-    // index first): rank r holds child (ord >> 4r) & 7.  Distances are non-negative floats
-    // (or +inf), which order as unsigned integers.
-    uint32_t key[8];
-    uint32_t ord = 0u;
-    // child mask -> rank mask
-    auto to_rank = [&](unsigned cm) {
-        unsigned rr = 0u;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) rr |= ((cm >> ((ord >> (4 * q)) & 7u)) & 1u) << q;
-        return rr;
     };
     auto load_leaf = [&](int leaf, double* pf) {
         const int j0 = leaf * g.L, npts = max(0, min(g.L, g.n - j0));
@@ -1818,24 +1807,10 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
             prefetch(nx, nl);
         }
         hv_wave_sync();
-        // child distances to the packet centre (order, and the packet-sphere prefilter), then
-        // the children each lane's ball reaches (kept per lane) among those the sphere reaches
-        unsigned near = 0u;
-        {
-            const uint32_t kb = __float_as_uint(child_d2f(lane & 7, pcf));
-            const int me = lane & 7;
-            int rk = 0;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                key[c] = __builtin_amdgcn_readlane(kb, c);
-                near |= (key[c] <= __float_as_uint(rp2f)) ? (1u << c) : 0u;   // non-negative floats
-                rk += (key[c] < kb || (key[c] == kb && c < me)) ? 1 : 0;
-            }
-            uint32_t o = 0u;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) o |= (uint32_t)c << (4 * __builtin_amdgcn_readlane(rk, c));
-            ord = o;
-        }
+        // the children the packet sphere reaches (one per lane), then those each lane's ball reaches
+        // (kept per lane) among them
+        const float pd2 = child_d2f(lane & 7, pcf);
+        const unsigned near = (unsigned)(__ballot(pd2 <= rp2f) & 0xffull);
         unsigned rem = 0u, mine = 0u;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
@@ -1854,12 +1829,12 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
             if constexpr (MODE == 0) {
                 // children are leaves: nearest first, the next one loaded while this one is scanned
                 double pf[D + 1];
-                unsigned rr = to_rank(rem);
-                int cc = (ord >> (4 * __builtin_ctz(rr))) & 7u;
+                unsigned rr = rem;
+                int cc = __builtin_ctz(rr);
                 rr &= rr - 1u;
                 load_leaf(8 * i + cc, pf);
                 while (cc >= 0) {
-                    const int cn = rr ? (int)((ord >> (4 * __builtin_ctz(rr))) & 7u) : -1;
+                    const int cn = rr ? (int)__builtin_ctz(rr) : -1;
                     rr &= rr - 1u;
                     const int leaf = 8 * i + cc;
                     const int j0 = leaf * g.L, npts = max(0, min(g.L, g.n - j0));
@@ -1955,12 +1930,12 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
                         b = src[1];
                     }
                 };
-                unsigned rr = to_rank(rem);
-                int cc = (ord >> (4 * __builtin_ctz(rr))) & 7u;
+                unsigned rr = rem;
+                int cc = __builtin_ctz(rr);
                 rr &= rr - 1u;
                 load_leaf2(8 * i + cc, pa, pb);
                 while (cc >= 0) {
-                    const int cn = rr ? (int)((ord >> (4 * __builtin_ctz(rr))) & 7u) : -1;
+                    const int cn = rr ? (int)__builtin_ctz(rr) : -1;
                     rr &= rr - 1u;
                     const int leaf = 8 * i + cc;
                     const int j0 = leaf * 32, npts = max(0, min(32, g.n - j0));
@@ -2020,8 +1995,8 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
                     a0 = base[0];
                     a1 = base[16 * 4];
                 };
-                unsigned rr = to_rank(rem);
-                int cc = (ord >> (4 * __builtin_ctz(rr))) & 7u;
+                unsigned rr = rem;
+                int cc = __builtin_ctz(rr);
                 rr &= rr - 1u;
                 load_leaf1(8 * i + cc, pa0, pa1);
                 {
@@ -2035,7 +2010,7 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
                 }
                 hv_wave_sync();
                 while (cc >= 0) {
-                    const int cn = rr ? (int)((ord >> (4 * __builtin_ctz(rr))) & 7u) : -1;
+                    const int cn = rr ? (int)__builtin_ctz(rr) : -1;
                     rr &= rr - 1u;
                     const int leaf = 8 * i + cc;
                     const int j0 = leaf * 32, npts = max(0, min(32, g.n - j0));
@@ -2045,7 +2020,10 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
                     if (cn >= 0) load_leaf1(8 * i + cn, pa0, pa1);
                     if (m) {
                         leaves += 1;
-                        // survivors of this leaf for the lane's own ray (bit q = point j0 + q)
+                        // survivors of this leaf for the lane's own ray (bit q = point j0 + q).  The
+                        // rays are the rows of a tile and the points its columns, so a comparison of
+                        // result register e is the point mask of the rays 4 r + e in its four
+                        // 16-bit fields r: no lane exchange, only selects
                         uint32_t sv = 0u;
 #pragma unroll
                         for (int g4 = 0; g4 < 4; ++g4) {
@@ -2053,28 +2031,28 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
                             // both tiles issued before either result is read, so their latencies
                             // overlap (the second tile of a leaf with at most 16 points reads the
                             // padding records, whose form is positive for every ray)
-                            const hv_u32x4 bop = rk4[16 * g4 + (lane & 15)][lane >> 4];
-                            const hv_f32x4 acc0 = hv_mfma_bf16(ca0, bop);
-                            const hv_f32x4 acc1 = hv_mfma_bf16(ca1, bop);
+                            const hv_u32x4 aop = rk4[16 * g4 + (lane & 15)][lane >> 4];
+                            const hv_f32x4 acc0 = hv_mfma_bf16(aop, ca0);
+                            const hv_f32x4 acc1 = hv_mfma_bf16(aop, ca1);
+                            tiles += npts > 16 ? 2 : 1;
+                            uint32_t mine16[2];
 #pragma unroll
                             for (int t = 0; t < 2; ++t) {
-                                if (16 * t >= npts) continue;
-                                ++tiles;
                                 const hv_f32x4 acc = t == 0 ? acc0 : acc1;
-                                // lane holds points 16t + 4*(lane/16) + e of ray 16*g4 + lane%16
                                 const uint32_t ob = __float_as_uint(acc[0]) | __float_as_uint(acc[1]) |
                                                     __float_as_uint(acc[2]) | __float_as_uint(acc[3]);
+                                mine16[t] = 0u;
                                 if (__ballot((int)ob < 0) == 0ull) continue;
-                                uint32_t nib = 0u;
+                                uint32_t w[4];
 #pragma unroll
-                                for (int e = 0; e < 4; ++e) nib |= ((int)__float_as_uint(acc[e]) < 0) ? (1u << e) : 0u;
-                                // the ray's lane 16*g4 + c gathers the nibbles of lanes c, c+16, c+32, c+48
-                                uint32_t col = 0u;
-#pragma unroll
-                                for (int q = 0; q < 4; ++q)
-                                    col |= (uint32_t)__shfl((int)nib, (lane & 15) + 16 * q) << (4 * q);
-                                if ((lane >> 4) == g4) sv |= col << (16 * t);
+                                for (int e = 0; e < 4; ++e) {
+                                    const unsigned long long b = __ballot((int)__float_as_uint(acc[e]) < 0);
+                                    w[e] = (lane & 8) ? (uint32_t)(b >> 32) : (uint32_t)b;
+                                }
+                                const uint32_t w01 = (lane & 1) ? w[1] : w[0], w23 = (lane & 1) ? w[3] : w[2];
+                                mine16[t] = (((lane & 2) ? w23 : w01) >> (4 * (lane & 4))) & 0xffffu;
                             }
+                            if ((lane >> 4) == g4) sv = mine16[0] | (mine16[1] << 16);
                         }
                         // survivors the ray does not already hold go to FP64, every ray at once
                         if (sv) sv &= ~leaf_known(leaf) & (npts >= 32 ? 0xffffffffu : ((1u << npts) - 1u));
@@ -2100,19 +2078,27 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
                 }
             }
         } else {
-            // internal children: farthest pushed first so the nearest is walked next
+            // internal children, one per lane, pushed farthest from the packet centre first so that
+            // the nearest is walked next: a ray whose start ball is large (2D near the faces)
+            // finds its shrinking candidate early.  Leaves are taken as they come: the balls are
+            // tight by then, and ordering them cost more than it saved (5D N=100k mixture, scan
+            // per build: both ordered 21.4 ms, internal nodes only 18.8 ms; 2D N=1M 9.5, 9.9 and, nothing
+            // ordered, 14.3 ms per build)
             const int cbase = off + pw + 8 * i;
-            int last = -1;
-            unsigned rr = to_rank(rem);
-            while (rr) {
-                const int q = 31 - __builtin_clz(rr);
-                rr &= ~(1u << q);
-                const int c = (ord >> (4 * q)) & 7u;
-                stk[sp] = cbase + c;
-                stkl[sp] = l + 1;
-                ++sp;
-                last = cbase + c;
+            const uint32_t kb = __float_as_uint(pd2);   // non-negative floats order as unsigned
+            int behind = 0;                             // reached children farther than this lane's
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const uint32_t kc = __builtin_amdgcn_readlane(kb, c);
+                behind += ((rem >> c) & 1u) && (kc > kb || (kc == kb && c > (lane & 7))) ? 1 : 0;
             }
+            const int n = __builtin_popcount(rem);
+            if (lane < 8 && ((rem >> lane) & 1u)) {
+                stk[sp + behind] = cbase + lane;
+                stkl[sp + behind] = l + 1;
+            }
+            sp += n;
+            const int last = cbase + (int)__builtin_ctzll(__ballot(lane < 8 && ((rem >> lane) & 1u) && behind == n - 1));
             prefetch(last, l + 1);
         }
     }
