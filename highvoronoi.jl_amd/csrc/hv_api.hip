@@ -117,13 +117,14 @@ HvScratch::HvScratch(int device_ordinal, size_t bytes) : device(device_ordinal) 
     {
         std::lock_guard<std::mutex> lk(scratch_mu);
         auto& f = scratch_free[device];
-        for (size_t q = 0; q < f.size(); ++q)
-            if (f[q].n >= bytes) {
-                p = f[q].p;
-                n = f[q].n;
-                f.erase(f.begin() + q);
-                return;
-            }
+        size_t q = 0;
+        while (q < f.size() && f[q].n < bytes) ++q;
+        if (q < f.size() && f[q].n <= 2 * bytes + ((size_t)1 << 20)) {   // not a far larger one for a small owner
+            p = f[q].p;
+            n = f[q].n;
+            f.erase(f.begin() + q);
+            return;
+        }
     }
     if (hipMalloc(&p, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -172,6 +173,83 @@ void hv_scratch_release(int device_ordinal) {
             }
     }
     for (const DBuf& b : drop) (void)hipFree(b.p);
+}
+
+// Results leave the device through pinned staging buffers, one per worker thread with its own
+// stream: a worker's copy to the caller's memory (whose pages are mostly touched for the first
+// time there, the dearer part) runs beside the others' transfers.  256 MiB into fresh pages took
+// 25 ms with one copy by the runtime (10.6 GB/s, 57 GB/s into pinned memory).
+// A call takes the device's staging whole; one that finds it taken, or has little to copy, leaves
+// the copy to the runtime.
+constexpr int HV_STAGE_WORKERS = 8;
+constexpr size_t HV_STAGE_BYTES = (size_t)2 << 20;   // per worker: 16 MiB of pinned memory per device
+struct HvStaging {
+    std::mutex mu;
+    bool tried = false;
+    void* pin[HV_STAGE_WORKERS] = {};
+    hipStream_t st[HV_STAGE_WORKERS] = {};
+    int n = 0;   // workers with both
+};
+static HvStaging staging[64];   // per device ordinal, kept for the process
+
+hipError_t hv_copy_out(int device, void* dst, const void* src, size_t bytes) {
+    if (bytes == 0) return hipSuccess;
+    const size_t nchunk = (bytes + HV_STAGE_BYTES - 1) / HV_STAGE_BYTES;
+    std::unique_lock<std::mutex> lk;
+    int nw = 0;
+    if (device >= 0 && device < 64 && nchunk > 1) {
+        HvStaging& S = staging[device];
+        lk = std::unique_lock<std::mutex>(S.mu, std::try_to_lock);
+        if (lk.owns_lock()) {
+            if (!S.tried) {
+                S.tried = true;
+                for (int w = 0; w < HV_STAGE_WORKERS; ++w) {
+                    if (hipHostMalloc(&S.pin[w], HV_STAGE_BYTES, hipHostMallocDefault) != hipSuccess) break;
+                    if (hipStreamCreateWithFlags(&S.st[w], hipStreamNonBlocking) != hipSuccess) {
+                        (void)hipHostFree(S.pin[w]);
+                        break;
+                    }
+                    S.n = w + 1;
+                }
+                (void)hipGetLastError();
+            }
+            nw = (int)std::min<size_t>(S.n, nchunk);
+        }
+    }
+    if (nw == 0) {
+        const hipStream_t st = hipStreamPerThread;
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
+        return e != hipSuccess ? e : hipStreamSynchronize(st);
+    }
+    HvStaging& S = staging[device];
+    std::atomic<size_t> next{0};
+    std::atomic<int> err{hipSuccess};
+    auto work = [&](int w) {
+        (void)hipSetDevice(device);
+        for (;;) {
+            const size_t c = next.fetch_add(1);
+            if (c >= nchunk || err.load() != hipSuccess) break;
+            const size_t off = c * HV_STAGE_BYTES, len = std::min(HV_STAGE_BYTES, bytes - off);
+            hipError_t e = hipMemcpyAsync(S.pin[w], (const char*)src + off, len, hipMemcpyDeviceToHost, S.st[w]);
+            if (e == hipSuccess) e = hipStreamSynchronize(S.st[w]);
+            if (e != hipSuccess) {
+                err.store(e);
+                break;
+            }
+            std::memcpy((char*)dst + off, S.pin[w], len);
+        }
+    };
+    std::vector<std::thread> th;
+    for (int w = 1; w < nw; ++w) {
+        try {
+            th.emplace_back(work, w);
+        } catch (...) {
+            break;   // fewer workers: the ones running take every chunk
+        }
+    }
+    work(0);
+    for (auto& t : th) t.join();
+    return (hipError_t)err.load();
 }
 
 double* hv_points_for_write(hv_ctx* c, size_t bytes) {

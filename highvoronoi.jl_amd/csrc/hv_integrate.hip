@@ -38,6 +38,8 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <cstring>
+#include <memory>
 #include <numeric>
 
 #define HVCK(call)                                                                 \
@@ -913,15 +915,19 @@ __global__ void k_dense_geo(const int* __restrict__ gid, int nused, int ngen, in
 
 // ---- host driver -------------------------------------------------------------------------
 
+// Results stay on the device until hv_integral_export copies them into the caller's memory
+// (`host` holds them when the device has no room).
 struct hv_integral {
-    int64_t N = 0;
-    std::vector<double> vol, area;
-    std::vector<int64_t> ptr, nbr;
+    int64_t N = 0, rows = 0;
+    int device = 0;
+    std::unique_ptr<HvScratch> dev;
+    std::vector<char> host;
+    char* base = nullptr;              // dev or host memory: the parts below by offset
+    size_t vol = 0, ptr = 0, nbr = 0, area = 0, bulk = 0, iface = 0;
     double ms = 0.0;
     int64_t work = 0;                  // point samples: (sample, generator) distances evaluated
     double ms_kernel = 0.0;            // point samples: device time of the sampling kernel
     int nf = 0;                        // integrand components (0: none)
-    std::vector<double> bulk, iface;   // nf x N, nf x rows
 };
 
 static int64_t binom(int n, int k) {
@@ -1562,49 +1568,62 @@ static int make_geo(hv_ctx* c, const hv_mesh* mesh, IntGeo& g) {
     return HV_OK;
 }
 
+// neighbours of the rows (cell << 32 | neighbour), 1-based
+__global__ void k_row_nbr(const uint64_t* __restrict__ rows, int64_t n, int64_t* __restrict__ nbr) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) nbr[t] = (int64_t)(rows[t] & 0xffffffffull) + 1;
+}
+
 template <int D>
 static int finish(hv_ctx* c, int64_t ncell, const uint64_t* pkey, const double* area_d, const double* vol_d,
                   const int64_t* ptr_d, int64_t npair, float ms, hv_integral** out, int nf = 0,
                   const double* bulk_d = nullptr, const double* rint_d = nullptr) {
     // cells 0 .. ncell-1 (the originals) and their rows, which come first in the sorted order
-    hv_integral* I = new hv_integral();
-    I->N = ncell;
-    I->vol.resize(ncell);
-    I->ptr.resize(ncell + 1);
     if (ncell < c->N) {
-        if (hipMemcpyAsync(&npair, ptr_d + ncell, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-            hipStreamSynchronize(c->stream) != hipSuccess) {
-            delete I;
-            return hv_fail(c, HV_ERR_DEVICE, "integration copy-out failed");
-        }
+        HVCK(hipMemcpyAsync(&npair, ptr_d + ncell, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+        HVCK(hipStreamSynchronize(c->stream));
     }
-    I->area.resize(npair);
-    I->nbr.resize(npair);
-    std::vector<uint64_t> hk(npair);
-    hipError_t e = hipSuccess;
-    if (npair) {
-        e = hipMemcpyAsync(hk.data(), pkey, sizeof(uint64_t) * npair, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(I->area.data(), area_d, sizeof(double) * npair, hipMemcpyDeviceToHost, c->stream);
-    }
-    if (nf > 0) {
-        I->nf = nf;
-        I->bulk.resize((size_t)ncell * nf);
-        I->iface.resize((size_t)npair * nf);
-        if (e == hipSuccess && ncell)
-            e = hipMemcpyAsync(I->bulk.data(), bulk_d, sizeof(double) * I->bulk.size(), hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && npair)
-            e = hipMemcpyAsync(I->iface.data(), rint_d, sizeof(double) * I->iface.size(), hipMemcpyDeviceToHost, c->stream);
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(I->vol.data(), vol_d, sizeof(double) * ncell, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(I->ptr.data(), ptr_d, sizeof(int64_t) * (ncell + 1), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) {
-        delete I;
-        return hv_fail(c, HV_ERR_DEVICE, std::string("integration copy-out: ") + hipGetErrorString(e));
-    }
-    for (int64_t t = 0; t < npair; ++t) I->nbr[t] = (int64_t)(hk[t] & 0xffffffffull) + 1;
+    std::unique_ptr<hv_integral> I(new hv_integral());
+    I->N = ncell;
+    I->rows = npair;
+    I->device = c->device;
+    I->nf = nf;
     I->ms = ms;
-    *out = I;
+    size_t at = 0;
+    auto part = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) & ~(size_t)255; return o; };
+    I->vol = part(sizeof(double) * ncell);
+    I->ptr = part(sizeof(int64_t) * (ncell + 1));
+    I->nbr = part(sizeof(int64_t) * npair);
+    I->area = part(sizeof(double) * npair);
+    I->bulk = part(sizeof(double) * ncell * nf);
+    I->iface = part(sizeof(double) * npair * nf);
+    I->dev.reset(new HvScratch(c->device, at));
+    hipMemcpyKind kind = hipMemcpyDeviceToDevice;
+    if (I->dev->p) {
+        I->base = (char*)I->dev->p;
+    } else {
+        I->dev.reset();
+        I->host.resize(at);
+        I->base = I->host.data();
+        kind = hipMemcpyDeviceToHost;
+    }
+    auto put = [&](size_t off, const void* src, size_t bytes) {
+        return bytes ? hipMemcpyAsync(I->base + off, src, bytes, kind, c->stream) : hipSuccess;
+    };
+    if (npair) {
+        // in place for a host copy: the rows are this call's scratch
+        int64_t* nbr = I->dev ? (int64_t*)(I->base + I->nbr) : (int64_t*)pkey;
+        k_row_nbr<<<nblk(npair, 256), 256, 0, c->stream>>>(pkey, npair, nbr);
+        HVCK(hipGetLastError());
+        if (!I->dev) HVCK(put(I->nbr, nbr, sizeof(int64_t) * npair));
+    }
+    HVCK(put(I->area, area_d, sizeof(double) * npair));
+    HVCK(put(I->vol, vol_d, sizeof(double) * ncell));
+    HVCK(put(I->ptr, ptr_d, sizeof(int64_t) * (ncell + 1)));
+    HVCK(put(I->bulk, bulk_d, sizeof(double) * ncell * nf));
+    HVCK(put(I->iface, rint_d, sizeof(double) * npair * nf));
+    HVCK(hipStreamSynchronize(c->stream));
+    *out = I.release();
     return HV_OK;
 }
 
@@ -1767,27 +1786,37 @@ int hv_integral_work_impl(const hv_integral* I, int64_t* work, double* ms_kernel
 int hv_integral_counts_impl(const hv_integral* I, int64_t* ncells, int64_t* nnbr) {
     if (!I) return HV_ERR_ARG;
     if (ncells) *ncells = I->N;
-    if (nnbr) *nnbr = (int64_t)I->nbr.size();
+    if (nnbr) *nnbr = I->rows;
     return HV_OK;
+}
+
+// bytes of the results at offset `off` into the caller's memory
+static int integral_out(const hv_integral* I, void* dst, size_t off, size_t bytes) {
+    if (!dst || bytes == 0) return HV_OK;
+    if (!I->dev) {
+        std::memcpy(dst, I->base + off, bytes);
+        return HV_OK;
+    }
+    return hv_copy_out(I->device, dst, I->base + off, bytes) == hipSuccess ? HV_OK : HV_ERR_DEVICE;
 }
 
 int hv_integral_export_f_impl(const hv_integral* I, int32_t* nf, double* bulk, double* iface) {
     if (!I) return HV_ERR_ARG;
     if (nf) *nf = I->nf;
-    if (bulk) std::copy(I->bulk.begin(), I->bulk.end(), bulk);
-    if (iface) std::copy(I->iface.begin(), I->iface.end(), iface);
-    return HV_OK;
+    int rc = integral_out(I, bulk, I->bulk, sizeof(double) * I->N * I->nf);
+    if (!rc) rc = integral_out(I, iface, I->iface, sizeof(double) * I->rows * I->nf);
+    return rc;
 }
 
 int hv_integral_export_impl(const hv_integral* I, double* vol, int64_t* nbr_ptr, int64_t* nbr, double* area,
                             double* ms) {
     if (!I) return HV_ERR_ARG;
-    if (vol) std::copy(I->vol.begin(), I->vol.end(), vol);
-    if (nbr_ptr) std::copy(I->ptr.begin(), I->ptr.end(), nbr_ptr);
-    if (nbr) std::copy(I->nbr.begin(), I->nbr.end(), nbr);
-    if (area) std::copy(I->area.begin(), I->area.end(), area);
+    int rc = integral_out(I, vol, I->vol, sizeof(double) * I->N);
+    if (!rc) rc = integral_out(I, nbr_ptr, I->ptr, sizeof(int64_t) * (I->N + 1));
+    if (!rc) rc = integral_out(I, nbr, I->nbr, sizeof(int64_t) * I->rows);
+    if (!rc) rc = integral_out(I, area, I->area, sizeof(double) * I->rows);
     if (ms) *ms = I->ms;
-    return HV_OK;
+    return rc;
 }
 
 void hv_integral_free_impl(hv_integral* I) { delete I; }

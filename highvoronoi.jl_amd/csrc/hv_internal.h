@@ -44,12 +44,12 @@ struct DevArr {
     std::shared_ptr<DevArr> parent;
     ~DevArr();
 };
-// Device scratch of a call that owns no context (exports), for the lifetime of one object.  The
-// buffers come from a process-wide store of at most HV_SCRATCH_KEEP free buffers and
-// HV_SCRATCH_BYTES per device (each used by one call at a time; given back with
-// hv_batch_release); p is null when the device has no room.  The owner waits for its work
-// before the object goes.
-constexpr int HV_SCRATCH_KEEP = 4;
+// Device memory of an object that owns no context (an export's scratch, an integral's results), for
+// the lifetime of that object.  The buffers come from a process-wide store of at most
+// HV_SCRATCH_KEEP free buffers and HV_SCRATCH_BYTES per device (each used by one owner at a time;
+// given back with hv_batch_release); p is null when the device has no room.  The owner waits for
+// its work before the object goes.
+constexpr int HV_SCRATCH_KEEP = 8;
 constexpr size_t HV_SCRATCH_BYTES = (size_t)1 << 30;
 struct HvScratch {
     int device;
@@ -60,6 +60,9 @@ struct HvScratch {
     HvScratch(const HvScratch&) = delete;
     HvScratch& operator=(const HvScratch&) = delete;
 };
+// bytes of device memory into the caller's (pageable) memory; the data is complete (its stream has
+// been waited for).  Synchronous, callable from several threads at once.
+hipError_t hv_copy_out(int device, void* dst, const void* src, size_t bytes);
 void hv_scratch_release(int device_ordinal);   // frees the store's buffers (every device when negative)
 
 using ImgOrig = std::shared_ptr<const std::vector<int32_t>>;

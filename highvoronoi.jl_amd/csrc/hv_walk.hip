@@ -4335,10 +4335,9 @@ int hv_mesh_export_impl(const hv_mesh* m, int64_t* sig, double* coords) {
     for (int64_t r0 = 0; r0 < nv; r0 += chunk) {
         const int n = (int)std::min<int64_t>(chunk, nv - r0);
         k_export_rows<D><<<nblk((int64_t)n * (2 * D + 1), 256), 256, 0, st>>>(pb, (int)r0, n, ids, key, x, dsig, dx);
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(sig + r0 * (D + 1), dsig, sizeof(int64_t) * (D + 1) * n, hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipMemcpyAsync(coords + r0 * D, dx, sizeof(double) * D * n, hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess)
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess ||
+            hv_copy_out(m->device, sig + r0 * (D + 1), dsig, sizeof(int64_t) * (D + 1) * n) != hipSuccess ||
+            hv_copy_out(m->device, coords + r0 * D, dx, sizeof(double) * D * n) != hipSuccess)
             return HV_ERR_DEVICE;
     }
     return HV_OK;

@@ -219,7 +219,8 @@ int hv_build_mesh_batch(int device_ordinal, int32_t nmesh, const int32_t* d, con
 
 /* No counterpart in the reference: frees the contexts (streams and kept device tables) that
  * hv_build_mesh_batch's fused walks keep on the device between calls (device_ordinal < 0: on
- * every device) and the export scratch kept between calls (at most 1 GiB per device), for
+ * every device) and the exports' and integrals' buffers kept between calls (at most 1 GiB
+ * per device), for
  * callers that need the memory back.  Meshes already built stay valid; the
  * next batch call creates its contexts again.  Waits for a batch call running meanwhile. */
 int hv_batch_release(int device_ordinal);
@@ -308,7 +309,8 @@ int hv_integrate_mc_points(hv_ctx* ctx, const hv_mesh* mesh, int64_t nsamples, u
                            hv_integral** out);
 /* Voronoi_Integral's parity surface (src/integral.jl:11-21): volumes[ncells]; for cell i
  * its neighbours nbr[nbr_ptr[i] .. nbr_ptr[i+1]) sorted, 1-based (planes n+p), and the
- * interface areas aligned with them.  ms (optional) receives the device time. */
+ * interface areas aligned with them.  An integral holds its results in device memory (16 bytes
+ * per row and per cell, 8 nf more with an integrand) until hv_integral_free.  ms (optional) receives the device time. */
 int hv_integral_counts(const hv_integral* I, int64_t* ncells, int64_t* nnbr);
 /* No counterpart in the reference (a measurement): for hv_integrate_mc_points, the (sample,
  * generator) distances its sampling kernel evaluated and that kernel's device time in ms
