@@ -80,6 +80,7 @@ __device__ __forceinline__ const DevGeo& hv_geo_mesh(const DevGeo& g, const GeoS
 
 typedef unsigned int hv_u32x4 __attribute__((ext_vector_type(4)));
 typedef float hv_f32x4 __attribute__((ext_vector_type(4)));
+typedef float hv_f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 hv_bf16x8 __attribute__((ext_vector_type(8)));
 
 // BF16 round-to-nearest-even of a finite float, as the 16-bit pattern

@@ -1323,11 +1323,19 @@ __global__ __launch_bounds__(64 * HV_KNN_WAVES) void k_knn(DevGeo g0, GeoSet F, 
 // Point-sample Monte Carlo: wavefront w holds samples 64w .. 64w+63, all in stratum
 // floor(64w / S) of a G^d grid over the domain box (S samples per stratum, a multiple of 64),
 // each uniform in its stratum from a counter-based stream.  A packet walk as in k_raycast64 finds
-// each sample's nearest and second-nearest generators (FP64 distances to the staged leaves).
-// Accumulated: the samples of each nearest cell (one atomic per distinct cell of the
-// wavefront), and per (cell, neighbour) row the samples that lie within eps (counter 2 row)
-// and within 2 eps (counter 2 row + 1) of the bisector of their two nearest generators, or of
-// a boundary plane, on the cell's side.
+// each sample's nearest and second-nearest generators.
+//
+// What bounds it: vector instructions (93% busy).  In 6D a stratum is as wide as a cell and a packet
+// visits 530 leaves; measuring all their 64 x 32 distances took most of 118 ms (6D N=10k periodic,
+// 1e7 samples; 42 ms now), nearly all of them far from both neighbours.  One BF16 product of the matrix cores per 32 samples
+// bounds a leaf's distances from below instead (two 32x32x16 products, 64 cycles): with p' = p - c
+// and x' = x - c about the packet's centre c, x~ the point's BF16 rounding and m = -2 p' split in
+// two BF16 terms,
+//   slots 0..D-1: mh x~, 6: |x~|^2 high, 7: |x~|^2 low, 8..8+D-1: ml x~
+// sums to |p' - x~|^2 - |p'|^2 within 2^-14 (|p'| + r)^2 for |x'| <= |p'| + r (the split terms' own
+// rounding, 2^-16 each, and the FP32 sums), and |x' - x~| <= 2^-8 |x'|, so a generator within r of
+// the sample has a form of at most (r + 2^-8 |x'|)^2 - |p'|^2 and that margin.  What passes is
+// measured in FP32 from the point's own coordinates, in the points' order.
 __device__ __forceinline__ double hv_sample_unif(uint64_t seed, uint64_t idx) {
     return (double)(hv_mix64(seed ^ ((idx + 1ull) * 0x9E3779B97F4A7C15ull)) >> 11) * (1.0 / 9007199254740992.0);
 }
@@ -1353,7 +1361,7 @@ __device__ __forceinline__ void hv_row_add(const int64_t* __restrict__ ptr, cons
 constexpr int HV_MCP_SPREAD = 256;   // copies of the sample kernel's work counter
 
 template <int D>
-__global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, uint64_t seed, double eps,
+__global__ __launch_bounds__(64, 4) void k_mc_points(DevGeo g, int G, int64_t S, uint64_t seed, double eps,
                                                   const int64_t* __restrict__ ptr, const uint64_t* __restrict__ pkey,
                                                   unsigned long long* __restrict__ ccnt,
                                                   unsigned long long* __restrict__ pcnt, HvBox box, int pmask,
@@ -1370,14 +1378,10 @@ __global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, ui
     // (pkeys, pvals): key (original << 32) | shift code.
     __shared__ int stk[128], stkl[128];
     __shared__ float cbx[16 * D];
-    __shared__ unsigned long long hms[8];
-    __shared__ float px[D][64];
     const int lane = threadIdx.x;
     const int N = g.N;
     const int64_t smp = (int64_t)hv_xcd_block() * 64 + lane;
-    double p[D];
-    float pf[D];
-    {
+    auto draw = [&](double* p) {
         int64_t b = smp / S;
 #pragma unroll
         for (int k = 0; k < D; ++k) {
@@ -1385,24 +1389,19 @@ __global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, ui
             b /= G;
             const double wk = (box.hi[k] - box.lo[k]) / (double)G;
             p[k] = box.lo[k] + ((double)ck + hv_sample_unif(seed, (uint64_t)smp * D + k)) * wk;
-            pf[k] = (float)p[k];
         }
-    }
-    double bd0 = 1e300, bd1 = 1e300;
-    int bi0 = -1, bi1 = -1;
-    auto consider = [&](int q, double d2) {
-        const bool f = d2 < bd0, s2 = !f && d2 < bd1;
-        bd1 = f ? bd0 : (s2 ? d2 : bd1);
-        bi1 = f ? bi0 : (s2 ? q : bi1);
-        bd0 = f ? d2 : bd0;
-        bi0 = f ? q : bi0;
     };
-    // packet centre (uniform) orders the children
+    float pf[D];
+    // packet centre (uniform): orders the children, and the origin of the leaf forms
     float pcf[D];
     {
-        double cc[D];
+        double p[D], cc[D];
+        draw(p);
 #pragma unroll
-        for (int k = 0; k < D; ++k) cc[k] = p[k];
+        for (int k = 0; k < D; ++k) {
+            pf[k] = (float)p[k];
+            cc[k] = p[k];
+        }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
 #pragma unroll
@@ -1412,6 +1411,15 @@ __global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, ui
         for (int k = 0; k < D; ++k)
             pcf[k] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint((float)(cc[k] * (1.0 / 64.0)))));
     }
+    float bd0 = INFINITY, bd1 = INFINITY;
+    int bi0 = -1, bi1 = -1;
+    auto consider = [&](int q, float d2) {
+        const bool f = d2 < bd0, s2 = !f && d2 < bd1;
+        bd1 = f ? bd0 : (s2 ? d2 : bd1);
+        bi1 = f ? bi0 : (s2 ? q : bi1);
+        bd0 = f ? d2 : bd0;
+        bi0 = f ? q : bi0;
+    };
     auto child_d2f = [&](int c, const float* q) {
         float d2 = 0.f;
 #pragma unroll
@@ -1421,103 +1429,172 @@ __global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, ui
         }
         return d2;
     };
-    const double slack = 1e-6 * (g.xmax + 1.0);
-    auto reach = [&]() {   // widened FP32 radius^2 of the current second neighbour
-        const double r = sqrt(bd1) + slack;
-        return (float)fmin(r * r * (1.0 + 1e-5), 1e30);
-    };
-    uint32_t ord = 0u;   // children by distance to the packet centre: rank r holds (ord >> 4r) & 7
-    auto to_rank = [&](unsigned cm) {
-        unsigned rr = 0u;
+    // the samples' operands: column l % 32 of tile t is sample 32 t + l % 32, lanes 0..31 hold its
+    // slots 0..7 and lanes 32..63 its slots 8..15
+    hv_bf16x8 sb0, sb1;
+    float pp = 0.f;
+    {
+        hv_bf16x8 hi, lo;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) rr |= ((cm >> ((ord >> (4 * q)) & 7u)) & 1u) << q;
-        return rr;
+        for (int k = 0; k < 8; ++k) {
+            hi[k] = (__bf16)(k >= 6 ? 1.f : 0.f);
+            lo[k] = (__bf16)0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            const float pk = pf[k] - pcf[k], m = -2.f * pk;
+            pp = fmaf(pk, pk, pp);
+            hi[k] = (__bf16)m;
+            lo[k] = (__bf16)(m - (float)hi[k]);
+        }
+        const hv_u32x4 h4 = __builtin_bit_cast(hv_u32x4, hi), l4 = __builtin_bit_cast(hv_u32x4, lo);
+        hv_u32x4 a, b;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t lx = __shfl_xor(l4[q], 32), hx = __shfl_xor(h4[q], 32);
+            a[q] = lane < 32 ? h4[q] : lx;
+            b[q] = lane < 32 ? hx : l4[q];
+        }
+        sb0 = __builtin_bit_cast(hv_bf16x8, a);
+        sb1 = __builtin_bit_cast(hv_bf16x8, b);
+    }
+    const float slack = (float)(1e-6 * (g.xmax + 1.0)), pr = sqrtf(pp);
+    float R2f, thr0, thr1;   // of the current second neighbour: widened radius^2, the forms' limits of both tiles
+    auto set_reach = [&]() {
+        const float r = fminf(sqrtf(bd1) * (1.f + 2e-6f) + slack, 1e15f);
+        R2f = r * r * (1.f + 1e-5f);
+        const float m = pr + r, t = fmaf(m, 1.f / 250.f, r);
+        const float thr = fmaf(m * m, 1.f / 8192.f, t * t - pp), ox = __shfl_xor(thr, 32);
+        thr0 = lane < 32 ? thr : ox;
+        thr1 = lane < 32 ? ox : thr;
+    };
+    set_reach();
+    auto load_leaf = [&](int leaf, float4& a, float4& b) {   // point lane % 32 of the leaf (its last point beyond the end)
+        const float4* src = (const float4*)g.xf + (int64_t)min(leaf * 32 + (lane & 31), g.n - 1) * 2;
+        a = src[0];
+        if constexpr (D > 4) b = src[1];
+    };
+    // the child boxes of the node walked next, loaded while the current node is worked on
+    float cbr0 = 0.f, cbr1 = 0.f;
+    int pref = -1;
+    auto prefetch = [&](int node) {
+        const float* src = g.cb + (int64_t)node * (16 * D);
+        if (lane < 16 * D) cbr0 = src[lane];
+        if (lane < 16 * D - 64) cbr1 = src[lane + 64];
+        pref = node;
     };
     int sp = 1;
     stk[0] = 0;
     stkl[0] = 0;
-    unsigned work = 0u;   // (sample, generator) distances this lane evaluated
+    prefetch(0);
+    unsigned work = 0u;   // (sample, generator) distances of the leaves this lane's ball reached
     while (sp > 0) {
         --sp;
         hv_wave_sync();
         const int gid = __builtin_amdgcn_readfirstlane(stk[sp]);
         const int l = __builtin_amdgcn_readfirstlane(stkl[sp]);
-        {
-            const float* src = g.cb + (int64_t)gid * (16 * D);
-            for (int q = lane; q < 16 * D; q += 64) cbx[q] = src[q];
-        }
+        if (gid != pref) prefetch(gid);
+        if (lane < 16 * D) cbx[lane] = cbr0;
+        if (lane < 16 * D - 64) cbx[lane + 64] = cbr1;
+        if (l + 1 == g.h && sp > 0) prefetch(__builtin_amdgcn_readfirstlane(stk[sp - 1]));
         hv_wave_sync();
-        const float R2f = reach();
-        unsigned rem = 0u;
+        unsigned rem = 0u, mine = 0u;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            const unsigned long long m = __ballot(child_d2f(c, pf) <= R2f);
-            if (lane == 0) hms[c] = m;
-            rem |= (m != 0ull) ? (1u << c) : 0u;
-        }
-        {
-            const uint32_t kb = __float_as_uint(child_d2f(lane & 7, pcf));
-            const int me = lane & 7;
-            int rk = 0;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const uint32_t kc = __builtin_amdgcn_readlane(kb, c);
-                rk += (kc < kb || (kc == kb && c < me)) ? 1 : 0;
-            }
-            uint32_t o = 0u;
-#pragma unroll
-            for (int c = 0; c < 8; ++c) o |= (uint32_t)c << (4 * __builtin_amdgcn_readlane(rk, c));
-            ord = o;
+            const bool h = child_d2f(c, pf) <= R2f;
+            mine |= h ? (1u << c) : 0u;
+            rem |= (__ballot(h) != 0ull) ? (1u << c) : 0u;
         }
         rem = __builtin_amdgcn_readfirstlane(rem);
-        hv_wave_sync();
         if (rem == 0u) continue;
+        const float tnode = bd1;
+        // children by distance to the packet centre: lane c's rank among the reached ones
+        const uint32_t kb = __float_as_uint(child_d2f(lane & 7, pcf));
+        int before = 0;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const uint32_t kc = __builtin_amdgcn_readlane(kb, c);
+            before += ((rem >> c) & 1u) && (kc < kb || (kc == kb && c < (lane & 7))) ? 1 : 0;
+        }
+        const int nrem = __builtin_popcount(rem);
+        const bool reached = lane < 8 && ((rem >> lane) & 1u);
         const int off = ((1 << (3 * l)) - 1) / 7;
         const int i = gid - off;
         if (l + 1 == g.h) {
-            unsigned rr = to_rank(rem);
-            while (rr) {
-                const int cc = (ord >> (4 * __builtin_ctz(rr))) & 7u;
-                rr &= rr - 1u;
-                const int leaf = 8 * i + cc;
-                const int j0 = leaf * g.L, npts = max(0, min(g.L, N - j0));
-                const bool hit = ((hms[cc] >> lane) & 1ull) && (child_d2f(cc, pf) <= reach());
-                if (__ballot(hit) == 0ull) continue;
-                for (int s0 = 0; s0 < npts; s0 += 64) {
-                    const int cnt = min(64, npts - s0);
-                    if (lane < cnt) {   // FP32 rows; the two nearest are measured again in FP64
-#pragma unroll
-                        for (int k = 0; k < D; ++k) px[k][lane] = g.xf[(int64_t)(j0 + s0 + lane) * 8 + k];
-                    }
-                    hv_wave_sync();
-                    if (hit) {
-                        work += (unsigned)cnt;
-                        for (int q = 0; q < cnt; ++q) {
-                            float d2 = 0.f;
-#pragma unroll
-                            for (int k = 0; k < D; ++k) {
-                                const float a = px[k][q] - pf[k];
-                                d2 = fmaf(a, a, d2);
-                            }
-                            consider(j0 + s0 + q, (double)d2);
-                        }
-                    }
-                    hv_wave_sync();
+            auto child_at = [&](int rank) { return (int)__builtin_ctzll(__ballot(reached && before == rank)); };
+            float4 na{}, nb{};
+            int cn = child_at(0);
+            load_leaf(8 * i + cn, na, nb);
+            for (int q = 1; q <= nrem; ++q) {
+                const int cc = cn, leaf = 8 * i + cc, j0 = leaf * 32, npts = max(0, min(32, g.n - j0));
+                const float row[8] = {na.x, na.y, na.z, na.w, nb.x, nb.y, nb.z, nb.w};
+                if (q < nrem) {
+                    cn = child_at(q);
+                    load_leaf(8 * i + cn, na, nb);
                 }
+                const bool hit = ((mine >> cc) & 1u) && (bd1 == tnode || child_d2f(cc, pf) <= R2f);
+                if (__ballot(hit) == 0ull) continue;
+                work += hit ? (unsigned)npts : 0u;
+                hv_bf16x8 xa;
+                {
+                    float n2 = 0.f;
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) {
+                        xa[k] = (__bf16)(k < D ? row[k] - pcf[k < D ? k : 0] : 0.f);
+                        n2 = fmaf((float)xa[k], (float)xa[k], n2);
+                    }
+                    xa[6] = (__bf16)n2;
+                    xa[7] = (__bf16)(n2 - (float)xa[6]);
+                }
+                hv_f32x16 f0 = {}, f1 = {};
+                f0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, sb0, f0, 0, 0, 0);
+                f1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, sb1, f1, 0, 0, 0);
+                float m0 = f0[0], m1 = f1[0];
+#pragma unroll
+                for (int r = 1; r < 16; ++r) {
+                    m0 = fminf(m0, f0[r]);
+                    m1 = fminf(m1, f1[r]);
+                }
+                if (__ballot(m0 <= thr0 || m1 <= thr1) == 0ull) continue;
+                // result r of a lane is the form of point 8 (r / 4) + 4 (lane / 32) + r % 4
+                uint32_t s0 = 0u, s1 = 0u;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s0 |= f0[r] <= thr0 ? 1u << (8 * (r / 4) + r % 4) : 0u;
+                    s1 |= f1[r] <= thr1 ? 1u << (8 * (r / 4) + r % 4) : 0u;
+                }
+                s0 <<= 4 * (lane >> 5);
+                s1 <<= 4 * (lane >> 5);
+                uint32_t sv = (lane < 32 ? s0 : s1) | __shfl_xor(lane < 32 ? s1 : s0, 32);
+                sv = hit ? sv & (npts >= 32 ? 0xffffffffu : (1u << npts) - 1u) : 0u;
+                const float was = bd1;
+                while (__ballot(sv != 0u)) {   // every lane takes part: a point's row is in lane q
+                    const int q2 = sv ? (int)__builtin_ctz(sv) : 0;
+                    float d2 = 0.f;
+#pragma unroll
+                    for (int k = 0; k < D; ++k) {
+                        const float a = __shfl(row[k], q2) - pf[k];
+                        d2 = fmaf(a, a, d2);
+                    }
+                    if (sv) consider(j0 + q2, d2);
+                    sv &= sv - 1u;
+                }
+                if (__ballot(bd1 < was)) set_reach();
             }
         } else {
+            // the nearest is walked next
             const int cbase = off + (1 << (3 * l)) + 8 * i;
-            unsigned rr = to_rank(rem);
-            while (rr) {
-                const int q = 31 - __builtin_clz(rr);
-                rr &= ~(1u << q);
-                const int c = (ord >> (4 * q)) & 7u;
-                stk[sp] = cbase + c;
-                stkl[sp] = l + 1;
-                ++sp;
+            const int at = sp + nrem - 1 - before;
+            if (reached) {
+                stk[at] = cbase + lane;
+                stkl[at] = l + 1;
             }
+            sp += nrem;
+            prefetch(cbase + (int)__builtin_ctzll(__ballot(reached && before == 0)));
         }
     }
+    double p[D];
+    draw(p);
     {
         unsigned long long w = work;
 #pragma unroll
@@ -1526,6 +1603,7 @@ __global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, ui
         if (lane == 0) atomicAdd(&npairs[blockIdx.x % HV_MCP_SPREAD], w);
     }
     // the two nearest in FP64 (the FP32 scan may order a near tie either way)
+    double e0, e1 = 1e300;
     auto d2_64 = [&](int j) {
         double s2 = 0.0;
 #pragma unroll
@@ -1535,11 +1613,11 @@ __global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, ui
         }
         return s2;
     };
-    bd0 = d2_64(bi0);   // bi0 >= 0: the walk starts with an unbounded radius and N > d
+    e0 = d2_64(bi0);   // bi0 >= 0: the walk starts with an unbounded radius and N > d
     if (bi1 >= 0) {
-        bd1 = d2_64(bi1);
-        if (bd1 < bd0) {
-            const double td = bd0; bd0 = bd1; bd1 = td;
+        e1 = d2_64(bi1);
+        if (e1 < e0) {
+            const double td = e0; e0 = e1; e1 = td;
             const int ti = bi0; bi0 = bi1; bi1 = ti;
         }
     }
@@ -1590,7 +1668,7 @@ __global__ __launch_bounds__(64) void k_mc_points(DevGeo g, int G, int64_t S, ui
             const double a = g.xs[(int64_t)bi0 * (D + 1) + k] - g.xs[(int64_t)bi1 * (D + 1) + k];
             dd = fma(a, a, dd);
         }
-        const double gap = bd1 - bd0, w = 2.0 * eps * sqrt(dd);   // distance to the bisector = gap / (2|xi - xj|)
+        const double gap = e1 - e0, w = 2.0 * eps * sqrt(dd);   // distance to the bisector = gap / (2|xi - xj|)
         if (gap < 2.0 * w && nb1 >= 0) hv_row_add(ptr, pkey, pcnt, cell, nb1, gap < w);
     }
     for (int q = 0; q < g.P; ++q) {
@@ -5395,6 +5473,40 @@ int hv_inrange_impl(hv_ctx* c, int64_t nq, const double* q, const double* radius
     return HV_OK;
 }
 
+// The periodic working set's shift codes (4 bits per direction, shift + 8) and its open-addressing
+// table (original << 32) | code -> id, read by k_mc_points.  The keys are distinct, so the slot an
+// id takes does not matter to a look-up.  (On the host the table cost 40 ms a call at 6D N=10k,
+// a third of the sampling itself.)
+template <int D>
+__global__ __launch_bounds__(256) void k_mcp_images(int n, const int* __restrict__ orig, const int8_t* __restrict__ shift,
+                                                    uint32_t* __restrict__ code, unsigned long long* __restrict__ keys,
+                                                    int* __restrict__ vals, uint64_t mask, int* __restrict__ bad) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    uint32_t v = 0u;
+    bool far = false;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        const int sh = shift[(int64_t)i * D + k];
+        far = far || sh < -8 || sh > 7;
+        v |= (uint32_t)((sh + 8) & 15) << (4 * k);
+    }
+    if (far) {   // the caller refuses the set; its codes need not be distinct
+        *bad = 1;
+        return;
+    }
+    code[i] = v;
+    const unsigned long long key = ((unsigned long long)(unsigned)orig[i] << 32) | v;
+    uint64_t h = hv_mix64(key) & mask;
+    for (uint64_t probe = 0; probe <= mask; ++probe) {
+        if (atomicCAS(&keys[h], ~0ull, key) == ~0ull) {
+            vals[h] = i;
+            return;
+        }
+        h = (h + 1) & mask;
+    }
+}
+
 // Point-sample Monte Carlo counts (k_mc_points) for the rows (ptr, pkey) of the context's
 // mesh.  nsamples is rounded up to a whole number of strata of S samples (a multiple of 64);
 // the number used, the slab width and the box volume are returned.
@@ -5444,38 +5556,25 @@ int hv_mc_points_impl(hv_ctx* c, int64_t nsamples, uint64_t seed, double slab, c
         if (c->rmax + 4.0 * eps > c->delta)
             return hv_fail(c, HV_ERR_UNSUPPORTED, "slab too wide for the margin of the periodic images");
         const int64_t ne = c->N;
-        std::vector<uint32_t> code((size_t)ne);
-        for (int64_t i = 0; i < ne; ++i) {
-            uint32_t v = 0u;
-            for (int k = 0; k < D; ++k) {
-                const int sh = (*c->img_shift)[(size_t)i * D + k];
-                if (sh < -8 || sh > 7) return hv_fail(c, HV_ERR_CAPACITY, "periodic image shift beyond 7 box lengths");
-                v |= (uint32_t)(sh + 8) << (4 * k);
-            }
-            code[(size_t)i] = v;
-        }
-        // (original, shift code) -> id, open addressing at load <= 1/2
-        uint64_t hs = 1024;
+        uint64_t hs = 1024;   // (original, shift code) -> id at load <= 1/2
         while ((int64_t)hs < 2 * ne) hs <<= 1;
-        std::vector<unsigned long long> hk(hs, ~0ull);
-        std::vector<int> hv(hs, -1);
-        for (int64_t i = 0; i < ne; ++i) {
-            const unsigned long long key = ((unsigned long long)(unsigned)(*c->img_orig)[(size_t)i] << 32) | code[(size_t)i];
-            uint64_t h = hv_mix64(key) & (hs - 1);
-            while (hk[h] != ~0ull) h = (h + 1) & (hs - 1);
-            hk[h] = key;
-            hv[h] = (int)i;
-        }
         uint32_t* dcode = pget<uint32_t>(c, "pshift", (size_t)ne);
+        int8_t* dshift = pget<int8_t>(c, "pshift8", (size_t)ne * D);
         int* dorig = pget<int>(c, "porig", (size_t)ne);
         unsigned long long* dkeys = pget<unsigned long long>(c, "pkeys", hs);
         int* dvals = pget<int>(c, "pvals", hs);
-        if (!dcode || !dorig || !dkeys || !dvals) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
-        HVCK(hipMemcpyAsync(dcode, code.data(), sizeof(uint32_t) * ne, hipMemcpyHostToDevice, c->stream));
+        int* dbad = pget<int>(c, "pbad", 1);
+        if (!dcode || !dshift || !dorig || !dkeys || !dvals || !dbad) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
+        HVCK(hipMemcpyAsync(dshift, c->img_shift->data(), (size_t)ne * D, hipMemcpyHostToDevice, c->stream));
         HVCK(hipMemcpyAsync(dorig, c->img_orig->data(), sizeof(int) * ne, hipMemcpyHostToDevice, c->stream));
-        HVCK(hipMemcpyAsync(dkeys, hk.data(), sizeof(unsigned long long) * hs, hipMemcpyHostToDevice, c->stream));
-        HVCK(hipMemcpyAsync(dvals, hv.data(), sizeof(int) * hs, hipMemcpyHostToDevice, c->stream));
+        HVCK(hipMemsetAsync(dkeys, 0xff, sizeof(unsigned long long) * hs, c->stream));
+        HVCK(hipMemsetAsync(dbad, 0, sizeof(int), c->stream));
+        k_mcp_images<D><<<nblk(ne, 256), 256, 0, c->stream>>>((int)ne, dorig, dshift, dcode, dkeys, dvals, hs - 1, dbad);
+        HVCK(hipGetLastError());
+        int hbad = 0;
+        HVCK(hipMemcpyAsync(&hbad, dbad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         HVCK(hipStreamSynchronize(c->stream));
+        if (hbad) return hv_fail(c, HV_ERR_CAPACITY, "periodic image shift beyond 7 box lengths");
         pshift = dcode;
         porig = dorig;
         pkeys = dkeys;
