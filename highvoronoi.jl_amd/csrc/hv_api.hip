@@ -175,6 +175,36 @@ void hv_scratch_release(int device_ordinal) {
     for (const DBuf& b : drop) (void)hipFree(b.p);
 }
 
+static std::mutex pinned_mu;
+static std::vector<unsigned long long*> pinned_free;
+
+HvPinned::HvPinned() {
+    {
+        std::lock_guard<std::mutex> lk(pinned_mu);
+        if (!pinned_free.empty()) {
+            p = pinned_free.back();
+            pinned_free.pop_back();
+            return;
+        }
+    }
+    if (hipHostMalloc((void**)&p, 512, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+}
+
+HvPinned::~HvPinned() {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(pinned_mu);
+        if (pinned_free.size() < HV_PINNED_KEEP) {
+            pinned_free.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
 // Results leave the device through pinned staging buffers, one per worker thread with its own
 // stream: a worker's copy to the caller's memory (whose pages are mostly touched for the first
 // time there, the dearer part) runs beside the others' transfers.  256 MiB into fresh pages took

@@ -63,6 +63,17 @@ struct HvScratch {
 // bytes of device memory into the caller's (pageable) memory; the data is complete (its stream has
 // been waited for).  Synchronous, callable from several threads at once.
 hipError_t hv_copy_out(int device, void* dst, const void* src, size_t bytes);
+// Pinned host memory (512 bytes) that kernels write a call's counts into, for the lifetime of the
+// object: from a process-wide store of at most HV_PINNED_KEEP free blocks; p is null when there is
+// none to be had.
+constexpr size_t HV_PINNED_KEEP = 16;
+struct HvPinned {
+    unsigned long long* p = nullptr;
+    HvPinned();
+    ~HvPinned();
+    HvPinned(const HvPinned&) = delete;
+    HvPinned& operator=(const HvPinned&) = delete;
+};
 void hv_scratch_release(int device_ordinal);   // frees the store's buffers (every device when negative)
 
 using ImgOrig = std::shared_ptr<const std::vector<int32_t>>;

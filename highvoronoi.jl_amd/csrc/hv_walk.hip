@@ -477,22 +477,27 @@ __device__ __forceinline__ void hv_block_count4(unsigned long long* ctr, bool c0
                   (unsigned long long)part[threadIdx.x]);
 }
 
+// The winners' ids are appended at out[*nout ..]: one atomic per workgroup (a selection pass over
+// flags cost three launches).
 template <int D>
 __global__ __launch_bounds__(256) void k_insert(const int* __restrict__ status, int n, const int* __restrict__ n_dev,
                                                 const int* __restrict__ vkey, int64_t base, int* __restrict__ htab,
-                                                uint64_t hmask, uint8_t* __restrict__ win,
+                                                uint64_t hmask, int* __restrict__ out, int* __restrict__ nout,
                                                 unsigned long long* __restrict__ ctr, int cstride) {
-    // n_dev (when given): the candidate count in device memory; flags up to n are written
+    // n_dev (when given): the candidate count in device memory, n then only bounds the grid
+    __shared__ int wsum[4];
+    __shared__ int wbase;
+    if (n_dev) n = min(n, *n_dev);
+    if ((int64_t)blockIdx.x * blockDim.x >= n) return;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nv = n_dev ? min(n, *n_dev) : n;
-    bool dup = false, full = false, none = false, singular = false;
-    if (t >= nv && t < n) win[t] = 0;
-    if (t < nv) {
-        uint8_t won = 0;
-        none = status[t] == HV_ST_NONE;
-        singular = status[t] == HV_ST_SINGULAR;
-        if (status[t] > 0) {
-            const int id = (int)(base + t);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    bool won = false, dup = false, full = false, none = false, singular = false;
+    const int id = (int)(base + t);
+    if (t < n) {
+        const int st = status[t];
+        none = st == HV_ST_NONE;
+        singular = st == HV_ST_SINGULAR;
+        if (st > 0) {
             const int* key = vkey + (int64_t)id * (D + 1);
             uint64_t h = hv_hash_ints<D + 1>(key) & hmask;
             full = true;
@@ -500,14 +505,26 @@ __global__ __launch_bounds__(256) void k_insert(const int* __restrict__ status, 
                 int cur = htab[h];
                 if (cur < 0) {
                     const int old = atomicCAS(&htab[h], -1, id);
-                    if (old == -1) { won = 1; full = false; break; }
+                    if (old == -1) { won = true; full = false; break; }
                     cur = old;
                 }
                 if (keys_equal<D>(key, vkey + (int64_t)cur * (D + 1))) { dup = true; full = false; break; }
                 h = (h + 1) & hmask;
             }
         }
-        win[t] = won;
+    }
+    const unsigned long long m = __ballot(won);
+    if (lane == 0) wsum[wv] = __popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+        wbase = tot ? atomicAdd(nout, tot) : 0;
+    }
+    __syncthreads();
+    if (won) {
+        int at = wbase + __popcll(m & (lane ? (1ull << lane) - 1ull : 0ull));
+        for (int w = 0; w < wv; ++w) at += wsum[w];
+        out[at] = id;
     }
     hv_block_count4(ctr, dup, full, none, singular, cstride);
 }
@@ -539,41 +556,35 @@ __global__ void k_rehash_vertices(const int* __restrict__ ids, int64_t n, const 
 // that finds its other end point, so nothing older needs to be kept.  Slots: bits 0..34 the
 // value, bits 35..61 a fingerprint of the edge, bit 62 closed.
 template <int D>
-__global__ __launch_bounds__(256) void k_rt_build(DevRays R, int nr, const int* __restrict__ vkey,
-                                                  unsigned long long* __restrict__ rt, uint64_t rmask,
-                                                  unsigned long long* __restrict__ ctr) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    bool full = false;
-    if (t < nr) {
-        int e[D];
-        hv_edge_of<D>(vkey + (int64_t)R.v[t] * (D + 1), R.drop[t], e);
-        const uint64_t hfull = hv_hash_ints<D>(e);
-        const unsigned long long fp = HV_EDGE_FP(hfull);
-        const unsigned long long mine = fp | ((unsigned long long)t + 1ull);
-        uint64_t h = hfull & rmask;
-        int64_t out = -1;
-        for (uint64_t probe = 0; probe <= rmask; ++probe) {
-            unsigned long long cur = rt[h];
-            if (cur == 0ull) {
-                const unsigned long long old = atomicCAS(&rt[h], 0ull, mine);
-                if (old == 0ull) { out = (int64_t)h; break; }
-                cur = old;
-            }
-            if ((cur & HV_EDGE_FMASK) == fp) {
-                const int r2 = (int)((cur & HV_EDGE_VMASK) - 1ull);
-                int e2[D];
-                hv_edge_of<D>(vkey + (int64_t)R.v[r2] * (D + 1), R.drop[r2], e2);
-                bool eq = true;
-#pragma unroll
-                for (int j = 0; j < D; ++j) eq = eq && (e[j] == e2[j]);
-                if (eq) { out = (int64_t)h; break; }
-            }
-            h = (h + 1) & rmask;
+__device__ __forceinline__ bool hv_rt_insert(const DevRays& R, int t, const int* __restrict__ vkey,
+                                             unsigned long long* __restrict__ rt, uint64_t rmask) {
+    int e[D];
+    hv_edge_of<D>(vkey + (int64_t)R.v[t] * (D + 1), R.drop[t], e);
+    const uint64_t hfull = hv_hash_ints<D>(e);
+    const unsigned long long fp = HV_EDGE_FP(hfull);
+    const unsigned long long mine = fp | ((unsigned long long)t + 1ull);
+    uint64_t h = hfull & rmask;
+    int64_t out = -1;
+    for (uint64_t probe = 0; probe <= rmask; ++probe) {
+        unsigned long long cur = rt[h];
+        if (cur == 0ull) {
+            const unsigned long long old = atomicCAS(&rt[h], 0ull, mine);
+            if (old == 0ull) { out = (int64_t)h; break; }
+            cur = old;
         }
-        full = out < 0;
-        R.slot[t] = out < 0 ? 0 : out;
+        if ((cur & HV_EDGE_FMASK) == fp) {
+            const int r2 = (int)((cur & HV_EDGE_VMASK) - 1ull);
+            int e2[D];
+            hv_edge_of<D>(vkey + (int64_t)R.v[r2] * (D + 1), R.drop[r2], e2);
+            bool eq = true;
+#pragma unroll
+            for (int j = 0; j < D; ++j) eq = eq && (e[j] == e2[j]);
+            if (eq) { out = (int64_t)h; break; }
+        }
+        h = (h + 1) & rmask;
     }
-    hv_wave_count(&ctr[1], full);
+    R.slot[t] = out < 0 ? 0 : out;
+    return out >= 0;
 }
 
 // Walked edges: those with a generator below nwalk (all edges when nwalk is the generator
@@ -610,7 +621,7 @@ __global__ __launch_bounds__(256) void k_register(const int* __restrict__ fronti
             const unsigned long long fp = HV_EDGE_FP(hfull);
             // the edge of a ray of this level: its other end point is the ray's source
             bool ray_edge = false;
-            {
+            if (rt) {   // (the seeds' level has no rays)
                 uint64_t h = hfull & rmask;
                 for (uint64_t probe = 0; probe <= rmask; ++probe) {
                     const unsigned long long cur = rt[h];
@@ -778,11 +789,12 @@ __device__ __forceinline__ void hv_ray_setup(const DevGeo& g, const int* key, in
 constexpr int HV_EMIT_PER = 4;
 
 template <int D>
-__global__ __launch_bounds__(256) void k_emit(const int* __restrict__ frontier, int nf, const int* __restrict__ vkey,
-                                              const double* __restrict__ vx, DevGeo g,
+__global__ __launch_bounds__(256) void k_emit(const int* __restrict__ frontier, int nf, const int* __restrict__ nf_dev,
                                               const unsigned long long* __restrict__ nt,
-                                              const int64_t* __restrict__ reg, DevRays R, int* __restrict__ nrays,
-                                              double plane_tol) {
+                                              const int64_t* __restrict__ reg, DevRays R, int* __restrict__ nrays) {
+    // nf_dev (when given): the vertex count in device memory, nf then only bounds the grid
+    if (nf_dev) nf = min(nf, *nf_dev);
+    if ((int64_t)blockIdx.x * (256 * HV_EMIT_PER) >= (int64_t)nf * (D + 1)) return;
     __shared__ int wsum[4];
     __shared__ int wbase[4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -833,13 +845,18 @@ __global__ __launch_bounds__(256) void k_emit(const int* __restrict__ frontier, 
     }
 }
 
-// Direction, half-space threshold and orthogonality defect of rays [0, n) (dense: one
-// thread per emitted ray).
+// The edges of a level's nr rays into the ray-edge table (counter ctr: table overflow), and the
+// direction, half-space threshold and orthogonality defect of the nfresh new ones (those carried
+// from the level before follow them and hold theirs).
 template <int D, bool B>
-__global__ __launch_bounds__(256) void k_ray_dir(DevGeo g0, GeoSet F, DevRays R, int n, const int* __restrict__ vkey,
-                                                 const double* __restrict__ vx, double plane_tol) {
+__global__ __launch_bounds__(256) void k_ray_dir(DevGeo g0, GeoSet F, DevRays R, int nr, int nfresh,
+                                                 const int* __restrict__ vkey, const double* __restrict__ vx,
+                                                 double plane_tol, unsigned long long* __restrict__ rt, uint64_t rmask,
+                                                 unsigned long long* __restrict__ ctr) {
     const int t = hv_xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= n) return;
+    const bool full = t < nr && !hv_rt_insert<D>(R, t, vkey, rt, rmask);
+    hv_wave_count(ctr, full);
+    if (t >= nfresh) return;
     const int v = R.v[t], pos = R.drop[t];
     // key read straight from global memory: a private copy indexed by `pos` would live in scratch
     const int* key = vkey + (int64_t)v * (D + 1);
@@ -1148,6 +1165,7 @@ __global__ __launch_bounds__(256) void k_ray_init(DevGeo g0, GeoSet F, DevRays R
 #pragma unroll
     for (int k = 0; k < D; ++k) bc[k] = G.r[k] + (T.t1 + HV_W) * G.u[k];
     // over a forest: rays of one mesh together (mesh above the top Morton bits the sort uses)
+    if (!R.code) return;
     if constexpr (B) R.code[ray] = ((uint64_t)F.mof[gen0] << 32) | (hv_morton<D>(g, bc) >> HV_RAY_SORT_LO);
     else R.code[ray] = hv_morton<D>(g, bc);
 }
@@ -2950,40 +2968,161 @@ __device__ __forceinline__ bool hv_tent_key(const DevGeo& g, const DevRays& R, c
     return true;
 }
 
+// The primaries are put in order for the scan by a counting sort: at[t] = bucket << 32 | rank
+// within it (~0: not a primary), counted here, scanned (k_bucket_scan) and placed
+// (k_bucket_place).  Buckets follow the generators' Morton order, so they are finer where the
+// generators are dense: a bucket is a run of HV_BUCKET_SUB-ths of the gaps between the generators'
+// codes (mcode, sorted), found for the code of the ray's ball centre.  (A radix sort of every ray's
+// code and the selection of the primaries took 6 to 16 launches instead of 2; buckets by the
+// position of the ray's candidate cost the scan of a 5D N=100k mixture 19.0 -> 22.9 ms.)  Over a
+// forest, whose meshes are small, that position >> shift it is, the buckets of mesh m starting at
+// (goff[m] >> shift) + m so that none holds rays of two meshes.
+constexpr int HV_BUCKET_SUB = 4;
 template <int D, bool B>
 __global__ __launch_bounds__(256) void k_tent_group(DevGeo g0, GeoSet F, DevRays R, int nr, int nfresh,
                                                     const int* __restrict__ vkey, int* __restrict__ ttab, uint64_t tmask,
-                                                    int* __restrict__ prim_of, uint8_t* __restrict__ primary) {
+                                                    uint64_t* __restrict__ at, int* __restrict__ bcnt, int shift,
+                                                    const int* __restrict__ goff, const uint64_t* __restrict__ mcode) {
+    // at holds the rays' codes on entry (one tree)
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nr) return;
-    const DevGeo& g = hv_geo<B>(g0, F, vkey[(int64_t)R.v[t] * (D + 1)]);
+    const int gen0 = vkey[(int64_t)R.v[t] * (D + 1)];   // a generator: planes sort last
+    const DevGeo& g = hv_geo<B>(g0, F, gen0);
     int tk[D + 1];
+    bool primary = true;
     // carried rays (t >= nfresh) already waited once: scanned, and they claim no key
-    if (t >= nfresh || !hv_tent_key<D>(g, R, vkey, t, tk)) { prim_of[t] = t; primary[t] = 1; return; }
-    uint64_t h = hv_hash_ints<D + 1>(tk) & tmask;
-    for (uint64_t probe = 0; probe <= tmask; ++probe) {
-        int cur = ttab[h];
-        if (cur < 0) {
-            const int old = atomicCAS(&ttab[h], -1, t);
-            if (old == -1) { prim_of[t] = t; primary[t] = 1; return; }
-            cur = old;
+    if (t < nfresh && hv_tent_key<D>(g, R, vkey, t, tk)) {
+        uint64_t h = hv_hash_ints<D + 1>(tk) & tmask;
+        for (uint64_t probe = 0; probe <= tmask; ++probe) {
+            int cur = ttab[h];
+            if (cur < 0) {
+                const int old = atomicCAS(&ttab[h], -1, t);
+                if (old == -1) break;
+                cur = old;
+            }
+            // a claimer is a fresh ray with a key; over a forest it may belong to another mesh,
+            // whose tree maps its start candidate (a sorted position or a plane id of that mesh)
+            int ok[D + 1];
+            const DevGeo& gc = hv_geo<B>(g0, F, vkey[(int64_t)R.v[cur] * (D + 1)]);
+            hv_tent_key<D>(gc, R, vkey, cur, ok);
+            if (keys_equal<D>(tk, ok)) { primary = false; break; }
+            h = (h + 1) & tmask;
         }
-        // a claimer is a fresh ray with a key; over a forest it may belong to another mesh,
-        // whose tree maps its start candidate (a sorted position or a plane id of that mesh)
-        int ok[D + 1];
-        const DevGeo& gc = hv_geo<B>(g0, F, vkey[(int64_t)R.v[cur] * (D + 1)]);
-        hv_tent_key<D>(gc, R, vkey, cur, ok);
-        if (keys_equal<D>(tk, ok)) { prim_of[t] = cur; primary[t] = 0; return; }
-        h = (h + 1) & tmask;
     }
-    prim_of[t] = t;
-    primary[t] = 1;
+    if (!primary) {
+        at[t] = ~0ull;
+        return;
+    }
+    int b;
+    if constexpr (B) {
+        const int i1 = R.i1[t], m = F.mof[gen0];
+        b = ((i1 >= 0 && i1 < g.N ? i1 : g.rank[gen0]) >> shift) + (goff[m] >> shift) + m;
+    } else {
+        const uint64_t code = at[t];
+        int lo = 0, hi = g.n;   // generators with a smaller code
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (mcode[mid] < code) lo = mid + 1;
+            else hi = mid;
+        }
+        int q = 0;
+        if (lo > 0 && lo < g.n) {   // mcode[lo - 1] < code <= mcode[lo]
+            const float f = (float)(code - mcode[lo - 1]) / (float)(mcode[lo] - mcode[lo - 1]);
+            q = min(HV_BUCKET_SUB - 1, (int)(f * HV_BUCKET_SUB));
+        }
+        b = (int)(((int64_t)lo * HV_BUCKET_SUB + q) >> shift);
+    }
+    at[t] = ((uint64_t)b << 32) | (uint32_t)atomicAdd(&bcnt[b], 1);
 }
 
-__global__ void k_gather_flags(const int* __restrict__ ord, int nr, const uint8_t* __restrict__ by_ray,
-                               uint8_t* __restrict__ keep) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nr) keep[i] = by_ray[ord[i]];
+// off[b] = counts before bucket b, off[nb] = their sum; one workgroup (nb <= HV_BUCKETS_ONE: 64 KiB
+// of counts by one CU, below the launches of a scan over many)
+constexpr int HV_BUCKETS_ONE = 1 << 14;
+__global__ __launch_bounds__(1024) void k_bucket_scan(const int* __restrict__ cnt, int nb, int* __restrict__ off) {
+    __shared__ int wsum[16];
+    const int per = (nb + 1023) / 1024, b0 = min(nb, (int)threadIdx.x * per), b1 = min(nb, b0 + per);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int s = 0;
+    for (int b = b0; b < b1; ++b) s += cnt[b];
+    int inc = s;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(inc, o);
+        if (lane >= o) inc += v;
+    }
+    if (lane == 63) wsum[wv] = inc;
+    __syncthreads();
+    int base = inc - s;
+    for (int w = 0; w < wv; ++w) base += wsum[w];
+    for (int b = b0; b < b1; ++b) {
+        off[b] = base;
+        base += cnt[b];
+    }
+    if (threadIdx.x == 1023) off[nb] = base;
+}
+
+__global__ __launch_bounds__(256) void k_bucket_place(int nr, const uint64_t* __restrict__ at, const int* __restrict__ off,
+                                                      int* __restrict__ list) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nr) return;
+    const uint64_t a = at[t];
+    if (a != ~0ull) list[off[a >> 32] + (int)(uint32_t)a] = t;
+}
+
+// First launch of a level: its tables cleared, the rays carried from the level before appended at
+// `base`, the level's counts cleared.
+struct HvFill {
+    uint4* p;
+    int64_t n;    // 16-byte units
+    uint32_t v;
+};
+struct HvCarry {
+    int* v;
+    int* drop;
+    double* u;
+    double* c;
+    double* du;
+};
+template <int D>
+__global__ __launch_bounds__(256) void k_level_begin(HvFill f0, HvFill f1, HvFill f2, HvFill f3, int* __restrict__ dcount,
+                                                     HvCarry C, int ncar, DevRays R, int base) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    const HvFill f[4] = {f0, f1, f2, f3};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        for (int64_t i = t; i < f[q].n; i += step) f[q].p[i] = make_uint4(f[q].v, f[q].v, f[q].v, f[q].v);
+    if (t < 4) dcount[t] = 0;
+    for (int64_t i = t; i < ncar; i += step) {
+        const int64_t o = base + i;
+        R.v[o] = C.v[i];
+        R.drop[o] = C.drop[i];
+#pragma unroll
+        for (int k = 0; k < D; ++k) R.u[o * D + k] = C.u[i * D + k];
+        R.c[o] = C.c[i];
+        R.du[o] = C.du[i];
+    }
+}
+
+// The level's counters, and the scanned rays (nscan), into pinned host memory: one small launch
+// where each copy to pageable memory was a launch and a host wait of its own.
+constexpr int HV_CTL = 18;   // 64-bit words: 16 counters, 4 counts
+__global__ __launch_bounds__(64) void k_report(const unsigned long long* __restrict__ ctl, const int* __restrict__ nscan,
+                                               unsigned long long* __restrict__ host) {
+    if (threadIdx.x < HV_CTL) host[threadIdx.x] = ctl[threadIdx.x];
+    if (threadIdx.x == HV_CTL) host[HV_CTL] = nscan ? (unsigned long long)*nscan : 0ull;
+}
+
+// host[k] = the sum of counter k's `copies`
+__global__ __launch_bounds__(256) void k_report_spread(const unsigned long long* __restrict__ ctr, int copies,
+                                                       unsigned long long* __restrict__ host) {
+    __shared__ unsigned long long s;
+    if (threadIdx.x == 0) s = 0ull;
+    __syncthreads();
+    unsigned long long v = 0ull;
+    for (int q = threadIdx.x; q < copies; q += blockDim.x) v += ctr[(int64_t)blockIdx.x * copies + q];
+    if (v) atomicAdd(&s, v);
+    __syncthreads();
+    if (threadIdx.x == 0) host[blockIdx.x] = s;
 }
 
 // Rays that share a tentative end point with an earlier ray of the level wait: after the
@@ -2991,37 +3130,19 @@ __global__ void k_gather_flags(const int* __restrict__ ord, int nr, const uint8_
 // (the sequential walk would not walk that edge either); the others are carried into the
 // next level's rays, where they are scanned.
 template <int D>
-__global__ void k_carry_out(DevRays R, int nr, const uint8_t* __restrict__ primary,
-                            const unsigned long long* __restrict__ rt, int64_t* __restrict__ cs, int* __restrict__ cv,
-                            int* __restrict__ cd, double* __restrict__ cu, double* __restrict__ cc,
-                            double* __restrict__ cdu, int* __restrict__ count) {
+__global__ __launch_bounds__(256) void k_carry_out(DevRays R, int nr, const uint64_t* __restrict__ at,
+                                                   const unsigned long long* __restrict__ rt, HvCarry C,
+                                                   int* __restrict__ count) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool carry = t < nr && !primary[t] && !(rt[R.slot[t]] & HV_EDGE_DONE);
+    const bool carry = t < nr && at[t] == ~0ull && !(rt[R.slot[t]] & HV_EDGE_DONE);
     const int o = hv_wave_alloc(count, carry);
     if (!carry) return;
-    cs[o] = R.slot[t];
-    cv[o] = R.v[t];
-    cd[o] = R.drop[t];
+    C.v[o] = R.v[t];
+    C.drop[o] = R.drop[t];
 #pragma unroll
-    for (int k = 0; k < D; ++k) cu[(int64_t)o * D + k] = R.u[(int64_t)t * D + k];
-    cc[o] = R.c[t];
-    cdu[o] = R.du[t];
-}
-
-template <int D>
-__global__ void k_carry_in(const int64_t* __restrict__ cs, const int* __restrict__ cv, const int* __restrict__ cd,
-                           const double* __restrict__ cu, const double* __restrict__ cc, const double* __restrict__ cdu,
-                           int n, DevRays R, int base) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int o = base + t;
-    R.slot[o] = cs[t];
-    R.v[o] = cv[t];
-    R.drop[o] = cd[t];
-#pragma unroll
-    for (int k = 0; k < D; ++k) R.u[(int64_t)o * D + k] = cu[(int64_t)t * D + k];
-    R.c[o] = cc[t];
-    R.du[o] = cdu[t];
+    for (int k = 0; k < D; ++k) C.u[(int64_t)o * D + k] = R.u[(int64_t)t * D + k];
+    C.c[o] = R.c[t];
+    C.du[o] = R.du[t];
 }
 
 // Chunk selection (64-ray blocks interleaved over K chunks); a ray of a later chunk is
@@ -3060,6 +3181,13 @@ __global__ void k_pkt_count(const int* __restrict__ list, int n, const int* __re
         return lo;
     };
     cnt[m] = first_of(m + 1) - first_of(m);
+}
+
+// The same from the buckets' offsets (k_tent_group).
+__global__ void k_pkt_count_off(const int* __restrict__ off, const int* __restrict__ goff, int shift, int nmesh,
+                                int* __restrict__ cnt) {
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m < nmesh) cnt[m] = off[(goff[m + 1] >> shift) + m + 1] - off[(goff[m] >> shift) + m];
 }
 
 // Prefix sums over the meshes (a wavefront, 64 meshes per step): seg = first list position of
@@ -3364,6 +3492,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         if (!c->extended) record_tree(c, T.g, prec, L);
     }
     DevGeo& g = T.g;   // over a forest: unused (every kernel takes its mesh's tree from F)
+    const uint64_t* mcode = B ? nullptr : pget<uint64_t>(c, "code2", 0);   // the generators' codes, as the tree's build left them
     const int nmesh = B ? fo->nmesh : 1;
     // box corners, or the simple vertices of a general polytope (single meshes only)
     const bool poly = !B && c->dom_general;
@@ -3403,7 +3532,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
     double* vx = pget<double>(c, "vx", (size_t)vcap * D);
     int* ids = pget<int>(c, "ids", (size_t)vcap);
     int* htab = pget<int>(c, "htab", hsize);
-    unsigned long long* ctr = pget<unsigned long long>(c, "ctr", 16);
+    unsigned long long* ctr = pget<unsigned long long>(c, "ctr", HV_CTL);
     // the scan's statistics (0 pairs, 1 leaves, 2 ties, 6 FP64 rechecks, 7 rays rechecked), each
     // in HV_SCAN_SPREAD copies that the packets share out
     constexpr int HV_SCAN_SPREAD = 256;
@@ -3411,21 +3540,30 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
     // k_insert's counters (8 duplicates, 9 vertex-hash overflow, 10 rays without a vertex,
     // 11 singular vertices) likewise, after the scan's
     unsigned long long* ictr = sctr + 8 * HV_SCAN_SPREAD;
-    int* dcount = pget<int>(c, "dcount", 4);
-    if (!vkey || !vx || !ids || !htab || !ctr || !sctr || !dcount)
-        return hv_fail(c, HV_ERR_DEVICE, "out of device memory (tables)");
+    if (!vkey || !vx || !ids || !htab || !ctr || !sctr) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (tables)");
+    // counts: 0 carried rays, 1 new vertices, 3 new rays
+    int* dcount = (int*)(ctr + 16);
+    HvPinned pin;
+    if (!pin.p) return hv_fail(c, HV_ERR_DEVICE, "out of pinned memory");
     HVCK(hipMemsetAsync(htab, 0xff, hsize * sizeof(int), c->stream));
-    HVCK(hipMemsetAsync(ctr, 0, 16 * sizeof(unsigned long long), c->stream));
+    HVCK(hipMemsetAsync(ctr, 0, HV_CTL * sizeof(unsigned long long), c->stream));
     HVCK(hipMemsetAsync(sctr, 0, 12 * HV_SCAN_SPREAD * sizeof(unsigned long long), c->stream));
     hv_stats_t st{};
     unsigned long long hctr[16];
+    int hcount[4];     // the counts at the last wait
+    int64_t nscan = 0;
     int64_t vnext = 0;   // next provisional vertex id
     int64_t nlive = 0;   // live vertices: ids[0 .. nlive)
 
     // counters in ctr[]: 0 pairs, 1 leaves, 2 ties, 4 unique edges, 5 edge overflow, 8 dup, 9 vertex overflow
-    auto read_ctr = [&]() -> int {
-        HVCK(hipMemcpyAsync(hctr, ctr, sizeof hctr, hipMemcpyDeviceToHost, c->stream));
+    // scanned: the scan's ray count in device memory, read along
+    auto read_ctr = [&](const int* scanned = nullptr) -> int {
+        k_report<<<1, 64, 0, c->stream>>>(ctr, scanned, pin.p);
+        HVCK(hipGetLastError());
         HVCK(hipStreamSynchronize(c->stream));
+        std::memcpy(hctr, pin.p, sizeof hctr);
+        std::memcpy(hcount, pin.p + 16, sizeof hcount);
+        nscan = (int64_t)pin.p[HV_CTL];
         return HV_OK;
     };
     // per-level edge tables (see k_register): the ray-edge table of the current level and the
@@ -3436,17 +3574,6 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
     unsigned long long* ntab = nullptr;
     uint64_t nsize = 0;
     bool nt_fresh = true;   // the next registration starts a new level's table
-    auto build_rt = [&](const DevRays& R, int nr) -> int {
-        rsize = hpow(2 * (int64_t)nr + 64);
-        rtab = pget<unsigned long long>(c, "rtab", rsize);
-        if (!rtab) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (ray-edge table)");
-        HVCK(hipMemsetAsync(rtab, 0, rsize * sizeof(unsigned long long), c->stream));
-        if (nr > 0) {
-            k_rt_build<D><<<nblk(nr, 256), 256, 0, c->stream>>>(R, nr, vkey, rtab, rsize - 1, ctr + 4);
-            HVCK(hipGetLastError());
-        }
-        return HV_OK;
-    };
     // vertex table and vertex hash room for `incoming` more candidates
     auto ensure_vertices = [&](int64_t incoming) -> int {
         if (vnext + incoming > (int64_t)INT32_MAX) return hv_fail(c, HV_ERR_CAPACITY, "more than 2^31 vertex slots");
@@ -3473,26 +3600,23 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         }
         return HV_OK;
     };
-    // candidates at provisional ids base .. base+n with status > 0 -> hash -> new ids appended at ids[nlive]
-    // cnt_dev: leave the count in device memory (no host wait) instead of returning it in nsel
+    // candidates at provisional ids base .. base+n with status > 0 -> hash -> new ids appended at ids[nlive],
+    // their count in dcount[1] (clear before)
     // n_dev: the candidate count in device memory (n then bounds it)
-    auto insert_and_select = [&](const int* status, int n, int64_t base, int& nsel, int* cnt_dev = nullptr,
-                                 const int* n_dev = nullptr) -> int {
-        uint8_t* win = pget<uint8_t>(c, "win", n);
-        if (!win) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (win)");
-        k_insert<D><<<nblk(n, 256), 256, 0, c->stream>>>(status, n, n_dev, vkey, base, htab, hsize - 1, win, ictr,
-                                                         HV_SCAN_SPREAD);
+    auto insert_new = [&](const int* status, int n, int64_t base, const int* n_dev = nullptr) -> int {
+        k_insert<D><<<nblk(n, 256), 256, 0, c->stream>>>(status, n, n_dev, vkey, base, htab, hsize - 1, ids + nlive,
+                                                         dcount + 1, ictr, HV_SCAN_SPREAD);
         HVCK(hipGetLastError());
-        size_t tb = 0;
-        hipcub::CountingInputIterator<int> it((int)base);
-        int* cnt = cnt_dev ? cnt_dev : dcount;
-        HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb, it, win, ids + nlive, cnt, n, c->stream));
-        void* tmp = c->pool->get("cubtmp2", tb, false, c->stream);
-        if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
-        HVCK(hipcub::DeviceSelect::Flagged(tmp, tb, it, win, ids + nlive, cnt, n, c->stream));
-        if (cnt_dev) return HV_OK;
-        HVCK(hipMemcpyAsync(&nsel, dcount, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HVCK(hipStreamSynchronize(c->stream));
+        return HV_OK;
+    };
+    // the same, the count returned in nsel
+    auto insert_and_select = [&](const int* status, int n, int64_t base, int& nsel) -> int {
+        HVCK(hipMemsetAsync(dcount + 1, 0, sizeof(int), c->stream));
+        int r_ = insert_new(status, n, base);
+        if (r_) return r_;
+        r_ = read_ctr();
+        if (r_) return r_;
+        nsel = hcount[1];
         return HV_OK;
     };
     // edges of new vertices ids[first .. first+count); `bound` caps the new vertices the
@@ -3509,7 +3633,8 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         }
         if (count == 0) return HV_OK;
         k_register<D><<<nblk((int64_t)count * (D + 1), 256), 256, 0, c->stream>>>(
-            ids + first, count, count_dev, vkey, nwalk, cmask, N, R, rtab, rsize - 1, ntab, nsize - 1, reg, ctr + 4);
+            ids + first, count, count_dev, vkey, nwalk, cmask, N, R, R.v ? rtab : nullptr, rsize - 1, ntab, nsize - 1,
+            reg, ctr + 4);
         HVCK(hipGetLastError());
         return HV_OK;
     };
@@ -3548,9 +3673,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         int nsel = 0;
         rc = insert_and_select(status, nstart, vnext, nsel);
         if (rc) return rc;
-        DevRays none{};
-        rc = build_rt(none, 0);
-        if (rc) return rc;
+        const DevRays none{};
         rc = register_new(none, nlive, nsel, nsel, reg_cur);
         if (rc) return rc;
         vnext += nstart;
@@ -3561,7 +3684,27 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
     double ms_ray = 0.0;
     int64_t levels = 0, skipped = 0;
     int ncar = 0;   // rays carried from the previous level (waiting rays whose edge stayed open)
+    const int* bgoff = nullptr;   // first generator of each mesh (forest)
+    if constexpr (B) {
+        std::vector<int> hg(fo->goff.begin(), fo->goff.end());
+        hg.push_back((int)fo->ntot);
+        int* d = pget<int>(c, "w_goff", hg.size());
+        if (!d) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (batch)");
+        HVCK(hipMemcpyAsync(d, hg.data(), sizeof(int) * hg.size(), hipMemcpyHostToDevice, c->stream));
+        HVCK(hipStreamSynchronize(c->stream));   // hg is a local
+        bgoff = d;
+    }
+    // new rays of the frontier (its count on the device when fdev is given, n then bounds it) to R.v / R.drop
+    auto emit = [&](const DevRays& R, const int* frontier, int n, const int* fdev, const int64_t* reg) -> int {
+        k_emit<D><<<nblk((int64_t)n * (D + 1), 256 * HV_EMIT_PER), 256, 0, c->stream>>>(frontier, n, fdev, ntab, reg, R,
+                                                                                       dcount + 3);
+        HVCK(hipGetLastError());
+        return HV_OK;
+    };
+    bool emitted = false;   // the level's rays came out with the last wait
+    const bool chunks = opt.reserved0 > 0;
     for (int phase = 0;; ++phase) {
+    emitted = false;
     while (fcount > 0 || ncar > 0) {
         if (++levels > 1000000) return hv_fail(c, HV_ERR_CAPACITY, "walk did not terminate");
         const int64_t nslots = fcount * (D + 1) + ncar;
@@ -3593,39 +3736,59 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
             !R.t1 || !R.t2 || !R.i1 || !R.i2 ||
             !ordc || !keep || !status || !rwin || !rt || !reg_next)
             return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rays)");
-        HVCK(hipMemsetAsync(dcount, 0, sizeof(int), c->stream));
-        if (fcount > 0) {
-            k_emit<D><<<nblk(fcount * (D + 1), 256 * HV_EMIT_PER), 256, 0, c->stream>>>(
-                ids + fbeg, (int)fcount, vkey, vx, g, ntab, reg_cur, R, dcount, plane_tol);
-            HVCK(hipGetLastError());
+        if (!emitted) {
+            HVCK(hipMemsetAsync(dcount + 3, 0, sizeof(int), c->stream));
+            if (fcount > 0) {
+                rc = emit(R, ids + fbeg, (int)fcount, nullptr, reg_cur);
+                if (rc) return rc;
+            }
+            rc = read_ctr();
+            if (rc) return rc;
         }
-        int nr = 0;
-        HVCK(hipMemcpyAsync(&nr, dcount, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        rc = read_ctr();
-        if (rc) return rc;
+        emitted = false;
         if (hctr[5]) return hv_fail(c, HV_ERR_CAPACITY, "edge hash overflow");
-        const int nfresh = nr;
-        if (nfresh > 0) {
-            k_ray_dir<D, B><<<nblk(nfresh, 256), 256, 0, c->stream>>>(g, F, R, nfresh, vkey, vx, plane_tol);
-            HVCK(hipGetLastError());
-        }
-        if (ncar > 0) {
-            k_carry_in<D><<<nblk(ncar, 256), 256, 0, c->stream>>>(
-                (const int64_t*)c->pool->get("car_slot", 0), (const int*)c->pool->get("car_v", 0),
-                (const int*)c->pool->get("car_drop", 0), (const double*)c->pool->get("car_u", 0),
-                (const double*)c->pool->get("car_c", 0), (const double*)c->pool->get("car_du", 0), ncar, R, nr);
-            HVCK(hipGetLastError());
-            nr += ncar;
-            ncar = 0;
-        }
+        const int nfresh = hcount[3], nr = nfresh + ncar;
         if (nr == 0) break;
-        rc = build_rt(R, nr);
-        if (rc) return rc;
-        nt_fresh = true;
-        // start phase, then sort rays by the Morton code of their certificate-ball centre
-        k_ray_init<D, B><<<nblk(nr, 256), 256, 0, c->stream>>>(g, F, R, nr, vkey, vx, plane_tol);
-        HVCK(hipGetLastError());
+        // tables of the level: ray edges, new edges (their slots were read by k_emit), tentative keys, buckets
+        rsize = hpow(2 * (int64_t)nr + 64);
+        rtab = pget<unsigned long long>(c, "rtab", rsize);
+        nsize = hpow(2 * (D + 1) * (int64_t)nr + 64);
+        ntab = pget<unsigned long long>(c, "ntab", nsize);
+        const uint64_t tsz = hpow(2 * (int64_t)nr);
+        int* ttab = pget<int>(c, "ttab", tsz);
+        // at most two buckets a ray, and 2^19 (2 MiB of counts)
+        const int64_t bpos = B ? (int64_t)N : ((int64_t)N + 1) * HV_BUCKET_SUB;
+        int shift = 0;
+        while ((bpos >> shift) + nmesh > std::max<int64_t>(2048, std::min<int64_t>(2 * (int64_t)nr, 1 << 19))) ++shift;
+        const int nb = (int)(bpos >> shift) + nmesh + 1, nbc = (nb + 4) / 4 * 4;   // one empty bucket at least: its offset is the total
+        int* bcnt = pget<int>(c, "bk_cnt", (size_t)nbc);
+        int* boff = pget<int>(c, "bk_off", (size_t)nb + 1);
+        HvCarry car;
+        car.v = pget<int>(c, "car_v", nr, true);
+        car.drop = pget<int>(c, "car_drop", nr, true);
+        car.u = pget<double>(c, "car_u", (size_t)nr * D, true);   // the carried rays are read below
+        car.c = pget<double>(c, "car_c", nr, true);
+        car.du = pget<double>(c, "car_du", nr, true);
+        if (!rtab || !ntab || !ttab || !bcnt || !boff || !car.v || !car.drop || !car.u || !car.c || !car.du)
+            return hv_fail(c, HV_ERR_DEVICE, "out of device memory (level tables)");
         {
+            const HvFill f0{(uint4*)rtab, (int64_t)rsize / 2, 0u}, f1{(uint4*)ntab, (int64_t)nsize / 2, 0u};
+            const HvFill f2{(uint4*)ttab, chunks ? 0 : (int64_t)tsz / 4, ~0u}, f3{(uint4*)bcnt, chunks ? 0 : nbc / 4, 0u};
+            const int64_t most = std::max<int64_t>(std::max(f0.n, f1.n), ncar);
+            k_level_begin<D><<<(unsigned)std::min<int64_t>(2048, (most + 255) / 256), 256, 0, c->stream>>>(f0, f1, f2, f3, dcount, car, ncar, R, nfresh);
+            HVCK(hipGetLastError());
+        }
+        ncar = 0;
+        nt_fresh = false;
+        k_ray_dir<D, B><<<nblk(nr, 256), 256, 0, c->stream>>>(g, F, R, nr, nfresh, vkey, vx, plane_tol, rtab, rsize - 1, ctr + 5);
+        HVCK(hipGetLastError());
+        // start phase; R.code: the Morton code of the rays' certificate-ball centres (over a forest unused
+        // but with chunks)
+        DevRays Ri = R;
+        if (B && !chunks) Ri.code = nullptr;
+        k_ray_init<D, B><<<nblk(nr, 256), 256, 0, c->stream>>>(g, F, Ri, nr, vkey, vx, plane_tol);
+        HVCK(hipGetLastError());
+        if (chunks) {
             // over a forest the code holds the mesh above 32 Morton bits
             const int sb0 = B ? 0 : HV_RAY_SORT_LO, sb1 = B ? 32 + (B ? fo->mbits : 0) : 60;
             size_t tb = 0;
@@ -3637,11 +3800,9 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
             HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, R.code, code2, ord0, ord, nr, sb0, sb1, c->stream));
         }
         const int64_t level_begin = nlive;
-        // scan a list of rays, then new vertices -> hash -> registered edges
-        // defer: the new-vertex count stays in dcount[1] (the caller reads it with its next
-        // wait and then advances nlive and the scan time)
-        // n_dev (defer only): the ray count is in device memory and n bounds it
-        auto process = [&](const int* list, int n, bool defer, const int* n_dev = nullptr) -> int {
+        // scan a list of rays, their end points -> provisional vertices
+        // n_dev: the ray count is in device memory and n bounds it
+        auto scan = [&](const int* list, int n, const int* n_dev) -> int {
             int r_ = ensure_vertices(n);
             if (r_) return r_;
             if constexpr (B) {
@@ -3651,7 +3812,8 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
                 int* seg = pget<int>(c, "pk_seg", (size_t)nmesh + 1);
                 int* pko = pget<int>(c, "pk_off", (size_t)nmesh + 1);
                 if (!pcnt || !seg || !pko) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (packets)");
-                k_pkt_count<<<nblk(nmesh, 64), 64, 0, c->stream>>>(list, n, n_dev, R.code, nmesh, pcnt);
+                if (chunks) k_pkt_count<<<nblk(nmesh, 64), 64, 0, c->stream>>>(list, n, n_dev, R.code, nmesh, pcnt);
+                else k_pkt_count_off<<<nblk(nmesh, 64), 64, 0, c->stream>>>(boff, bgoff, shift, nmesh, pcnt);
                 HVCK(hipGetLastError());
                 k_pkt_plan<<<1, 64, 0, c->stream>>>(pcnt, nmesh, ppw, seg, pko);
                 HVCK(hipGetLastError());
@@ -3667,90 +3829,76 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
             HVCK(hipEventRecord(r1, c->stream));
             k_finalize<D, B><<<nblk(n, 256), 256, 0, c->stream>>>(g, F, R, list, n, n_dev, vkey, vx, vnext, status, rwin);
             HVCK(hipGetLastError());
-            int nsel = 0;
-            if (defer) {
-                r_ = insert_and_select(status, n, vnext, nsel, dcount + 1, n_dev);
-                if (r_) return r_;
-                r_ = register_new(R, nlive, n, n, reg_next + (nlive - level_begin) * (D + 1), dcount + 1);
-                if (r_) return r_;
-                vnext += n;   // provisional slots of all n; st.rays and nlive follow the caller's wait
-                return HV_OK;
-            }
-            r_ = insert_and_select(status, n, vnext, nsel);
-            if (r_) return r_;
+            return HV_OK;
+        };
+        auto scan_ms = [&]() -> int {
             float ms = 0.f;
             HVCK(hipEventElapsedTime(&ms, r0, r1));
             ms_ray += ms;
-            if (nsel || nt_fresh) {
-                r_ = register_new(R, nlive, nsel, KCH > 1 ? (int64_t)nr : nsel,
-                                  reg_next + (nlive - level_begin) * (D + 1));
-                if (r_) return r_;
-            }
-            st.rays += n;
-            nlive += nsel;
-            vnext += n;
             return HV_OK;
         };
-        auto select = [&](const int* in, const uint8_t* flags, int n, int* outl, int& nout) -> int {
-            size_t tb = 0;
-            HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb, in, flags, outl, dcount, n, c->stream));
-            void* tmp = c->pool->get("cubtmp2", tb, false, c->stream);
-            if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
-            HVCK(hipcub::DeviceSelect::Flagged(tmp, tb, in, flags, outl, dcount, n, c->stream));
-            HVCK(hipMemcpyAsync(&nout, dcount, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-            HVCK(hipStreamSynchronize(c->stream));
-            return HV_OK;
-        };
-        if (opt.reserved0 <= 0) {
+        if (!chunks) {
             // one scan per tentative end point (the ray start's best candidate); the other
             // rays of that end point wait and are carried to the next level if still open
-            uint64_t tsz = 1024;
-            while ((int64_t)tsz < 2 * (int64_t)nr) tsz <<= 1;
-            int* ttab = pget<int>(c, "ttab", tsz);
-            int* prim_of = pget<int>(c, "prim_of", nr);
-            uint8_t* pflag = pget<uint8_t>(c, "pflag", nr);
-            int64_t* cs = pget<int64_t>(c, "car_slot", nr);
-            int* cv = pget<int>(c, "car_v", nr);
-            int* cd = pget<int>(c, "car_drop", nr);
-            double* cu = pget<double>(c, "car_u", (size_t)nr * D);
-            double* cc = pget<double>(c, "car_c", nr);
-            double* cdu = pget<double>(c, "car_du", nr);
-            if (!ttab || !prim_of || !pflag || !cs || !cv || !cd || !cu || !cc || !cdu)
-                return hv_fail(c, HV_ERR_DEVICE, "out of device memory (groups)");
-            HVCK(hipMemsetAsync(ttab, 0xff, tsz * sizeof(int), c->stream));
-            k_tent_group<D, B><<<nblk(nr, 256), 256, 0, c->stream>>>(g, F, R, nr, nfresh, vkey, ttab, tsz - 1, prim_of, pflag);
+            k_tent_group<D, B><<<nblk(nr, 256), 256, 0, c->stream>>>(g, F, R, nr, nfresh, vkey, ttab, tsz - 1, R.code, bcnt, shift,
+                                                                     bgoff, mcode);
             HVCK(hipGetLastError());
-            k_gather_flags<<<nblk(nr, 256), 256, 0, c->stream>>>(ord, nr, pflag, keep);
-            HVCK(hipGetLastError());
-            // the primary rays (count in dcount[2]) are scanned without a host wait: the kernels
-            // read the count and nr bounds their grids
-            {
+            if (nb <= HV_BUCKETS_ONE) {
+                k_bucket_scan<<<1, 1024, 0, c->stream>>>(bcnt, nb, boff);
+                HVCK(hipGetLastError());
+            } else {
                 size_t tb = 0;
-                HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb, ord, keep, ordc, dcount + 2, nr, c->stream));
+                HVCK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, bcnt, boff, nb, c->stream));
+                void* tmp = c->pool->get("cubtmp2", tb, false, c->stream);
+                if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (scan)");
+                HVCK(hipcub::DeviceScan::ExclusiveSum(tmp, tb, bcnt, boff, nb, c->stream));
+            }
+            k_bucket_place<<<nblk(nr, 256), 256, 0, c->stream>>>(nr, R.code, boff, ordc);
+            HVCK(hipGetLastError());
+            // the primary rays (their count: the offset of the last bucket, which is empty) are scanned
+            // without a host wait: the kernels read the count and nr bounds their grids
+            const int* np_dev = boff + nb - 1;
+            rc = scan(ordc, nr, np_dev);
+            if (rc) return rc;
+            rc = insert_new(status, nr, vnext, np_dev);
+            if (rc) return rc;
+            rc = register_new(R, nlive, nr, nr, reg_next, dcount + 1);
+            if (rc) return rc;
+            vnext += nr;   // provisional slots of all nr
+            k_carry_out<D><<<nblk(nr, 256), 256, 0, c->stream>>>(R, nr, R.code, rtab, car, dcount);
+            HVCK(hipGetLastError());
+            // the next level's rays already, where the room for the most there can be is small (512 MiB): one
+            // wait a level
+            if ((int64_t)nr * (D + 1) <= (1ll << 26)) {
+                const size_t most = (size_t)nr * (D + 1) + nr;
+                DevRays Rn = R;
+                Rn.slot = pget<int64_t>(c, "ray_slot", most);
+                Rn.v = pget<int>(c, "ray_v", most);
+                Rn.drop = pget<int>(c, "ray_drop", most);
+                if (!Rn.slot || !Rn.v || !Rn.drop) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rays)");
+                rc = emit(Rn, ids + nlive, nr, dcount + 1, reg_next);
+                if (rc) return rc;
+                emitted = true;
+            }
+            rc = read_ctr(np_dev);
+            if (rc) return rc;
+            ncar = hcount[0];
+            nlive += hcount[1];
+            st.rays += nscan;
+            rc = scan_ms();
+            if (rc) return rc;
+            skipped += (int64_t)nr - nscan - ncar;
+        } else {
+            auto select = [&](const int* in, const uint8_t* flags, int n, int* outl, int& nout) -> int {
+                size_t tb = 0;
+                HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb, in, flags, outl, dcount, n, c->stream));
                 void* tmp = c->pool->get("cubtmp2", tb, false, c->stream);
                 if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
-                HVCK(hipcub::DeviceSelect::Flagged(tmp, tb, ord, keep, ordc, dcount + 2, nr, c->stream));
-            }
-            rc = process(ordc, nr, true, dcount + 2);
-            if (rc) return rc;
-            HVCK(hipMemsetAsync(dcount, 0, sizeof(int), c->stream));
-            k_carry_out<D><<<nblk(nr, 256), 256, 0, c->stream>>>(R, nr, pflag, rtab, cs, cv, cd, cu, cc, cdu, dcount);
-            HVCK(hipGetLastError());
-            // one wait: carried rays (dcount[0]), new vertices (dcount[1]), scanned rays (dcount[2])
-            int hc[3] = {0, 0, 0};
-            HVCK(hipMemcpyAsync(hc, dcount, 3 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-            HVCK(hipStreamSynchronize(c->stream));
-            ncar = hc[0];
-            const int np = hc[2];
-            nlive += hc[1];
-            st.rays += np;
-            {
-                float ms = 0.f;
-                HVCK(hipEventElapsedTime(&ms, r0, r1));
-                ms_ray += ms;
-            }
-            skipped += (int64_t)(nr - np) - ncar;
-        } else {
+                HVCK(hipcub::DeviceSelect::Flagged(tmp, tb, in, flags, outl, dcount, n, c->stream));
+                const int r_ = read_ctr();
+                nout = hcount[0];
+                return r_;
+            };
             // interleaved chunks: 64-ray blocks over K chunks, edge registration after each
             const int K = std::min(KCH, nr);
             const int nfull = nr >> 6, rem = nr & 63;
@@ -3769,8 +3917,18 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
                     skipped += nc - n;
                 }
                 if (n == 0) continue;
-                rc = process(rays_c, n, false);
+                rc = scan(rays_c, n, nullptr);
                 if (rc) return rc;
+                int nsel = 0;
+                rc = insert_and_select(status, n, vnext, nsel);
+                if (rc) return rc;
+                rc = scan_ms();
+                if (rc) return rc;
+                rc = register_new(R, nlive, nsel, nr, reg_next + (nlive - level_begin) * (D + 1));
+                if (rc) return rc;
+                st.rays += n;
+                nlive += nsel;
+                vnext += n;
             }
         }
         reg_cur = reg_next;
@@ -3810,9 +3968,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         int nsel = 0;
         rc = insert_and_select(status, nm, vnext, nsel);
         if (rc) return rc;
-        DevRays none{};
-        rc = build_rt(none, 0);
-        if (rc) return rc;
+        const DevRays none{};
         nt_fresh = true;
         reg_cur = pget<int64_t>(c, reg_is_a ? "regA" : "regB", (size_t)std::max(1, nsel) * (D + 1));
         if (!reg_cur) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
@@ -3825,17 +3981,11 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
     }
     }
     HVCK(hipEventRecord(e1, c->stream));
+    k_report_spread<<<12, 256, 0, c->stream>>>(sctr, HV_SCAN_SPREAD, pin.p + 32);
+    HVCK(hipGetLastError());
     rc = read_ctr();
     if (rc) return rc;
-    {
-        std::vector<unsigned long long> hs(12 * HV_SCAN_SPREAD);
-        HVCK(hipMemcpyAsync(hs.data(), sctr, sizeof(unsigned long long) * hs.size(), hipMemcpyDeviceToHost, c->stream));
-        HVCK(hipStreamSynchronize(c->stream));
-        for (int k : {0, 1, 2, 6, 7, 8, 9, 10, 11}) {
-            hctr[k] = 0;
-            for (int q = 0; q < HV_SCAN_SPREAD; ++q) hctr[k] += hs[(size_t)k * HV_SCAN_SPREAD + q];
-        }
-    }
+    for (int k : {0, 1, 2, 6, 7, 8, 9, 10, 11}) hctr[k] = pin.p[32 + k];
     float ms_all = 0.f;
     HVCK(hipEventElapsedTime(&ms_all, e0, e1));
     if (hctr[9]) return hv_fail(c, HV_ERR_CAPACITY, "vertex hash overflow");
