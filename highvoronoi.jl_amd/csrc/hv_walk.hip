@@ -1170,6 +1170,215 @@ __global__ __launch_bounds__(256) void k_ray_init(DevGeo g0, GeoSet F, DevRays R
     else R.code[ray] = hv_morton<D>(g, bc);
 }
 
+// The start phase of a small level, 16 lanes a ray: lane m looks at neighbour m of each of the
+// edge's lists, and the three best come out of three rounds of a 16-lane minimum.  A thread per ray
+// walks up to 96 dependent gathers alone, and a small level has too few wavefronts to hide them.
+template <int D, bool B>
+__global__ __launch_bounds__(256) void k_ray_init16(DevGeo g0, GeoSet F, DevRays R, int nrays, const int* __restrict__ vkey,
+                                                    const double* __restrict__ vx, double plane_tol) {
+    static_assert(HV_KNN == 16, "a lane per neighbour");
+    const int lane = threadIdx.x & 63, m = lane & 15;
+    const int slot = (blockIdx.x * 256 + threadIdx.x) >> 4;
+    if ((slot & ~3) >= nrays) return;   // the whole wavefront
+    const int ray = min(slot, nrays - 1);
+    const int gen0 = vkey[(int64_t)R.v[ray] * (D + 1)];   // a generator: planes sort last
+    const DevGeo& g = hv_geo<B>(g0, F, gen0);
+    const int N = g.N;
+    RayGeo<D> G;
+    hv_load_ray<D>(g, R, ray, vkey, vx, G);
+    int er[D];
+#pragma unroll
+    for (int a = 0; a < D; ++a) er[a] = G.e[a] < N ? g.rank[G.e[a]] : -1;
+    float tt[D];
+    int jj[D];
+    {
+        float uf[D], wf[D], x0f[D];
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            uf[k] = (float)G.u[k];
+            wf[k] = (float)(G.x0[k] - G.r[k]);
+            x0f[k] = (float)G.x0[k];
+        }
+        const float cf = (float)(G.cth - G.ux0);
+        const float4* xf4 = (const float4*)g.xf;
+#pragma unroll
+        for (int a = 0; a < D; ++a) jj[a] = er[a] >= 0 ? g.knn[(int64_t)er[a] * HV_KNN + m] : -1;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            const int j = jj[a];
+            bool edge = j < 0;
+#pragma unroll
+            for (int a2 = 0; a2 < D; ++a2) edge = edge || (j == er[a2]);
+            const float4 A = xf4[(int64_t)max(j, 0) * 2];
+            float x[8] = {A.x, A.y, A.z, A.w, 0.f, 0.f, 0.f, 0.f};
+            if constexpr (D > 4) {
+                const float4 Bq = xf4[(int64_t)max(j, 0) * 2 + 1];
+                x[4] = Bq.x; x[5] = Bq.y; x[6] = Bq.z; x[7] = Bq.w;
+            }
+            float vu = 0.f, vv = 0.f, vw = 0.f;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const float v = x[k] - x0f[k];
+                vu = fmaf(uf[k], v, vu);
+                vv = fmaf(v, v, vv);
+                vw = fmaf(v, wf[k], vw);
+            }
+            tt[a] = (!edge && vu > cf) ? __fdividef(fmaf(2.f, vw, vv), 2.f * vu) : INFINITY;
+        }
+    }
+    Top2 T;
+    for (int p = 0; p < g.P; ++p) {
+        const int id = N + p;
+        bool member = (id == G.s);
+#pragma unroll
+        for (int j = 0; j < D; ++j) member = member || (G.e[j] == id);
+        if (member) continue;
+        double nu = 0.0, dist = g.ph[p], nr = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            const double nk = g.pn[p * D + k];
+            nu = fma(nk, G.u[k], nu);
+            dist = fma(-nk, G.x0[k], dist);
+            nr = fma(nk, G.r[k], nr);
+        }
+        if (!(G.ux0 + 2.0 * dist * nu > G.cth)) continue;
+        T.offer((g.ph[p] - nr) / nu, id);   // one closer than plane_tol ends the ray (hv_consider)
+    }
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+        float bt = INFINITY;
+        int bj = -1;
+#pragma unroll
+        for (int a = 0; a < D; ++a)
+            if (tt[a] < bt) { bt = tt[a]; bj = jj[a]; }
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) {
+            const float t2 = __shfl_xor(bt, off);
+            const int j2 = __shfl_xor(bj, off);
+            if (t2 < bt || (t2 == bt && j2 > bj)) { bt = t2; bj = j2; }
+        }
+#pragma unroll
+        for (int a = 0; a < D; ++a)
+            if (jj[a] == bj) tt[a] = INFINITY;
+        if (bj >= 0) {
+            double xk[D];
+#pragma unroll
+            for (int k = 0; k < D; ++k) xk[k] = g.xs[(int64_t)bj * (D + 1) + k];
+            hv_consider<D>(G, T, xk, g.xs[(int64_t)bj * (D + 1) + D], bj, plane_tol);
+        }
+    }
+    if (m != 0 || slot >= nrays) return;
+    if (g.unbounded && T.i1 < 0) hv_probe<D>(g, G, T, plane_tol);
+    R.t1[ray] = T.t1;
+    R.t2[ray] = T.t2;
+    R.i1[ray] = T.i1;
+    R.i2[ray] = T.i2;
+    if (!R.code) return;
+    double bc[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) bc[k] = G.r[k] + (T.t1 + HV_W) * G.u[k];
+    if constexpr (B) R.code[ray] = ((uint64_t)F.mof[gen0] << 32) | (hv_morton<D>(g, bc) >> HV_RAY_SORT_LO);
+    else R.code[ray] = hv_morton<D>(g, bc);
+}
+
+// A level of at most this many rays is small: started 16 lanes a ray, scanned a wavefront a ray
+// (k_raycast1).  Both take longer than a thread a ray and packets once the chip is full, the earlier
+// the more a ray reaches.  Start and scan of one level, against packets: 3D, 8 to 32 thousand rays
+// 26 against 148 us, larger 301 against 185 us; 4D and 5D, 8 to 32 thousand rays 111 against 96 and 102
+// against 86 us; 3D levels of a few hundred rays (a refinement's) 20 against 127 us.
+constexpr int hv_small_level(int D) { return D <= 3 ? 1 << 15 : 1 << 13; }
+template <int D, bool B>
+static void launch_ray_init(const DevGeo& g, const GeoSet& F, const DevRays& R, int n, const int* vkey, const double* vx,
+                            double plane_tol, hipStream_t st) {
+    if (n <= hv_small_level(D)) k_ray_init16<D, B><<<nblk((int64_t)n * 16, 256), 256, 0, st>>>(g, F, R, n, vkey, vx, plane_tol);
+    else k_ray_init<D, B><<<nblk(n, 256), 256, 0, st>>>(g, F, R, n, vkey, vx, plane_tol);
+}
+
+// The end of ray rid from its two best candidates: status, winner (original id) and t by the
+// reference's near-tie rule; returns whether that rule was needed.
+template <int D>
+__device__ __forceinline__ bool hv_ray_result(const DevGeo& g, const RayGeo<D>& G, const Top2& T, double du, double plane_tol,
+                                              int rid, int* __restrict__ status, int* __restrict__ win,
+                                              double* __restrict__ tout) {
+    const int N = g.N;
+    bool tie = false;
+    if (T.i1 < 0) {
+        status[rid] = HV_ST_NONE;
+    } else {
+        // original indices and the reference's form of t (src/raycast.jl:424-431)
+        double x0t[D];
+#pragma unroll
+        for (int k = 0; k < D; ++k) x0t[k] = g.xo[(int64_t)G.e[0] * D + k];
+        auto orig = [&](int i) { return i < N ? g.sidx[i] : i; };
+        auto t_ref = [&](int w, double tscan, double& score, double& cosang) -> double {
+            if (w >= N) {
+                const int p = w - N;
+                double nu = 0.0, dist = g.ph[p];
+#pragma unroll
+                for (int k = 0; k < D; ++k) {
+                    nu = fma(g.pn[p * D + k], G.u[k], nu);
+                    dist = fma(-g.pn[p * D + k], x0t[k], dist);
+                }
+                score = 2.0 * dist * nu;
+                cosang = nu;
+                return tscan;
+            }
+            double num = 0.0, den = 0.0, dd = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const double xk = g.xo[(int64_t)(w) * D + k];
+                const double dx = xk - x0t[k];
+                num = fma(dx, x0t[k] + xk - 2.0 * G.r[k], num);
+                den = fma(G.u[k], dx, den);
+                dd = fma(dx, dx, dd);
+            }
+            score = den;
+            cosang = den / sqrt(dd);
+            return num / (2.0 * den);
+        };
+        int w1 = orig(T.i1);
+        double s1, c1;
+        double tw = t_ref(w1, T.t1, s1, c1);
+        int st = HV_ST_FOUND;
+        // the nearest candidate closer than plane_tol: the reference's window is empty, no
+        // vertex (src/raycast.jl:883-894 drops it and upper_t excludes every other)
+        if (!(tw >= plane_tol)) st = HV_ST_NONE;
+        else if (T.i2 >= 0) {
+            const int w2 = orig(T.i2);
+            double s2, c2;
+            const double tw2 = t_ref(w2, T.t2, s2, c2);
+            double rn = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) rn = fma(G.r[k], G.r[k], rn);
+            const double full_error = (tw * du + sqrt(rn) * 1e-15) / c1;
+            const double window = fmin(1e-7, (10.0 + D) * full_error);
+            double to = tw2, so = s2;   // the candidate that does not win
+            if (tw2 < tw || tw2 <= tw + window) {
+                // near tie: the larger <u, x - x0> wins (src/raycast.jl:903-916)
+                st = HV_ST_TIE;
+                tie = true;
+                if (s2 > s1) { to = tw; so = s1; w1 = w2; tw = tw2; }
+            }
+            // The reference's key takes every candidate whose distance from the new vertex is
+            // within rounding of the key's own (src/raycast.jl:926-950): the other candidate
+            // inside the chosen sphere (to < tw), or on it -- |x_o - r|^2 - R^2 = 2 (to - tw)
+            // <u, x_o - x0> within a few ulps of R^2 -- makes a key longer than d + 1, a
+            // vertex out of general position, which the device walk reports instead.
+            double R2 = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const double a = x0t[k] - fma(tw, G.u[k], G.r[k]);
+                R2 = fma(a, a, R2);
+            }
+            if (to < tw || (to - tw) * so <= 16.0 * 2.220446049250313e-16 * R2) st = HV_ST_SINGULAR;
+        }
+        win[rid] = w1;
+        status[rid] = st;
+        tout[rid] = tw;
+    }
+    return tie;
+}
+
 // One wavefront serves 64 rays at once (a packet).  Every generator x with t(x) < tau
 // lies strictly inside the certificate ball B(tau) = {x : |x - p|^2 < |x0 - p|^2},
 // p = r + tau u: for x ahead of the edge, |x-p|^2 - |x0-p|^2 = 2<u,x-x0>(t(x) - tau), and
@@ -2210,83 +2419,7 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
         if (lane == 0 && rechecks) atomicAdd(&ctr[6 * cstride], rechecks);
         hv_wave_count(&ctr[7 * cstride], flagged && act);
     }
-    bool tie = false;
-    if (act) {
-        if (T.i1 < 0) {
-            status[rid] = HV_ST_NONE;
-        } else {
-            // original indices and the reference's form of t (src/raycast.jl:424-431)
-            double x0t[D];
-#pragma unroll
-            for (int k = 0; k < D; ++k) x0t[k] = g.xo[(int64_t)e0 * D + k];
-            auto orig = [&](int i) { return i < N ? g.sidx[i] : i; };
-            auto t_ref = [&](int w, double tscan, double& score, double& cosang) -> double {
-                if (w >= N) {
-                    const int p = w - N;
-                    double nu = 0.0, dist = g.ph[p];
-#pragma unroll
-                    for (int k = 0; k < D; ++k) {
-                        nu = fma(g.pn[p * D + k], G.u[k], nu);
-                        dist = fma(-g.pn[p * D + k], x0t[k], dist);
-                    }
-                    score = 2.0 * dist * nu;
-                    cosang = nu;
-                    return tscan;
-                }
-                double num = 0.0, den = 0.0, dd = 0.0;
-#pragma unroll
-                for (int k = 0; k < D; ++k) {
-                    const double xk = g.xo[(int64_t)(w) * D + k];
-                    const double dx = xk - x0t[k];
-                    num = fma(dx, x0t[k] + xk - 2.0 * G.r[k], num);
-                    den = fma(G.u[k], dx, den);
-                    dd = fma(dx, dx, dd);
-                }
-                score = den;
-                cosang = den / sqrt(dd);
-                return num / (2.0 * den);
-            };
-            int w1 = orig(T.i1);
-            double s1, c1;
-            double tw = t_ref(w1, T.t1, s1, c1);
-            int st = HV_ST_FOUND;
-            // the nearest candidate closer than plane_tol: the reference's window is empty, no
-            // vertex (src/raycast.jl:883-894 drops it and upper_t excludes every other)
-            if (!(tw >= plane_tol)) st = HV_ST_NONE;
-            else if (T.i2 >= 0) {
-                const int w2 = orig(T.i2);
-                double s2, c2;
-                const double tw2 = t_ref(w2, T.t2, s2, c2);
-                double rn = 0.0;
-#pragma unroll
-                for (int k = 0; k < D; ++k) rn = fma(G.r[k], G.r[k], rn);
-                const double full_error = (tw * R.du[ray] + sqrt(rn) * 1e-15) / c1;
-                const double window = fmin(1e-7, (10.0 + D) * full_error);
-                double to = tw2, so = s2;   // the candidate that does not win
-                if (tw2 < tw || tw2 <= tw + window) {
-                    // near tie: the larger <u, x - x0> wins (src/raycast.jl:903-916)
-                    st = HV_ST_TIE;
-                    tie = true;
-                    if (s2 > s1) { to = tw; so = s1; w1 = w2; tw = tw2; }
-                }
-                // The reference's key takes every candidate whose distance from the new vertex is
-                // within rounding of the key's own (src/raycast.jl:926-950): the other candidate
-                // inside the chosen sphere (to < tw), or on it -- |x_o - r|^2 - R^2 = 2 (to - tw)
-                // <u, x_o - x0> within a few ulps of R^2 -- makes a key longer than d + 1, a
-                // vertex out of general position, which the device walk reports instead.
-                double R2 = 0.0;
-#pragma unroll
-                for (int k = 0; k < D; ++k) {
-                    const double a = x0t[k] - fma(tw, G.u[k], G.r[k]);
-                    R2 = fma(a, a, R2);
-                }
-                if (to < tw || (to - tw) * so <= 16.0 * 2.220446049250313e-16 * R2) st = HV_ST_SINGULAR;
-            }
-            win[rid] = w1;
-            status[rid] = st;
-            tout[rid] = tw;
-        }
-    }
+    const bool tie = act && hv_ray_result<D>(g, G, T, R.du[ray], plane_tol, rid, status, win, tout);
     hv_wave_count(&ctr[2 * cstride], tie);
 }
 
@@ -2301,6 +2434,174 @@ static inline int hv_packet_rays(int64_t n, const HvTiles& t = HvTiles{}) {
     int p = t.ppw_max;
     while (p > t.ppw_min && n < (int64_t)p * t.min_packets) p >>= 1;
     return p;
+}
+
+// The scan of a small level: a wavefront per ray.  A packet's walk is a serial chain of some forty
+// nodes and leaves whatever the level's size, and a level of a few thousand rays does not fill the
+// chip with packets; one ray reaches few nodes, and the lanes test eight nodes' children, or two
+// leaves' points (FP64, as MODE 0), at a time.  The rules are k_raycast64's: boxes the certificate
+// ball reaches, exact t of the points ahead below the best so far, the ball shrinking with it.
+constexpr int HV_R1_WAVES = 4;     // wavefronts per workgroup, a ray each
+constexpr int HV_R1_STACK = 576;   // one level at a time on top: at most 64 waiting nodes per level, 9 levels
+template <int D, bool B>
+__global__ __launch_bounds__(64 * HV_R1_WAVES) void k_raycast1(DevGeo g0, GeoSet F, DevRays R, const int* __restrict__ order,
+                                                               int nrays, const int* __restrict__ nrays_dev,
+                                                               const int* __restrict__ vkey, const double* __restrict__ vx,
+                                                               int* __restrict__ status, int* __restrict__ win,
+                                                               double* __restrict__ tout, double plane_tol,
+                                                               unsigned long long* __restrict__ ctr0, int cstride, int mixed) {
+    // mixed: a scan of a mixed precision is replaced, whose counts of candidates formed exactly, and of
+    // rays with any, are kept up
+    __shared__ int stk[HV_R1_WAVES][HV_R1_STACK];   // level << 27 | node id
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (nrays_dev) nrays = min(nrays, *nrays_dev);
+    const int rid = blockIdx.x * HV_R1_WAVES + wv;
+    if (rid >= nrays) return;   // no workgroup barrier below
+    unsigned long long* __restrict__ ctr = ctr0 + (cstride > 1 ? blockIdx.x % (unsigned)cstride : 0u);
+    int* S = stk[wv];
+    const int ray = order[rid];
+    const DevGeo& g = hv_geo<B>(g0, F, vkey[(int64_t)R.v[ray] * (D + 1)]);
+    RayGeo<D> G;
+    hv_load_ray<D>(g, R, ray, vkey, vx, G);
+    Top2 T;
+    T.t1 = R.t1[ray];
+    T.t2 = R.t2[ray];
+    T.i1 = R.i1[ray];
+    T.i2 = R.i2[ray];
+    const double slackf = 1e-6 * (g.xmax + 1.0);
+    float bcf[D], R2f;
+    auto set_ball = [&](double tau) {   // as k_raycast64's: widened so that FP32 box tests keep what FP64 would
+        double R2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            const double b = fma(tau, G.u[k], G.r[k]), t = b - G.x0[k];
+            R2 = fma(t, t, R2);
+            bcf[k] = (float)b;
+        }
+        R2 = R2 * (1.0 + 1e-9) + 1e-300;
+        const double rr = sqrt(R2) + slackf;
+        R2f = (float)(rr * rr * (1.0 + 1e-5));
+    };
+    set_ball(T.t1 < 1e299 ? T.t1 + HV_W : 0.0);
+    unsigned leaves = 0, exact = 0;
+    int sp = 1;
+    if (lane == 0) S[0] = 0;
+    hv_wave_sync();
+    while (sp > 0) {
+        // the topmost nodes of one level, at most eight
+        const int l = __builtin_amdgcn_readfirstlane(S[sp - 1]) >> 27;
+        const int mine = sp - 1 - (lane >> 3);
+        const int e = mine >= 0 ? S[mine] : -1;
+        const bool have = mine >= 0 && (e >> 27) == l;   // a level's nodes are adjacent
+        const int gid = e & ((1 << 27) - 1);
+        float lo[D], hi[D];
+#pragma unroll
+        for (int k = 0; k < D; ++k) { lo[k] = 1e30f; hi[k] = 1e30f; }
+        if (have) {
+            const float* box = g.cb + ((int64_t)gid * 8 + (lane & 7)) * (2 * D);
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                lo[k] = box[k];
+                hi[k] = box[D + k];
+            }
+        }
+        auto box_d2 = [&]() {   // an empty child's point box at 1e30 is out of every ball's reach
+            float d2 = 0.f;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const float a = bcf[k] - __builtin_amdgcn_fmed3f(bcf[k], lo[k], hi[k]);
+                d2 = fmaf(a, a, d2);
+            }
+            return d2;
+        };
+        sp -= __popcll(__ballot(have)) >> 3;
+        const float d2 = box_d2();
+        unsigned long long hit = __ballot(have && d2 <= R2f);
+        hv_wave_sync();   // the popped entries are read before they are written over
+        const int first = l == 0 ? 0 : ((1 << (3 * l)) - 1) / 7;   // first node id of the level
+        const int child = 8 * (gid - first) + (lane & 7);          // index in its level
+        if (l + 1 < g.h) {
+            // the children near the ball's centre on top, so that a ball that starts large shrinks early
+            const bool h = (hit >> lane) & 1ull;
+            const unsigned long long near = __ballot(h && d2 <= 0.0625f * R2f), far = hit & ~near;
+            const unsigned long long below = lane ? (1ull << lane) - 1ull : 0ull;
+            if (h) {
+                const int at = (near >> lane) & 1ull ? __popcll(far) + __popcll(near & below) : __popcll(far & below);
+                S[sp + at] = ((l + 1) << 27) | (first + (1 << (3 * l)) + child);
+            }
+            sp += __popcll(hit);
+            hv_wave_sync();
+            continue;
+        }
+        // leaves, two at a time, a point per lane; the next pair is loaded while this one is tested
+        double x[D + 1];
+        int j = -1;
+        auto load = [&]() {   // the next two leaves of `hit`
+            const int c0 = __builtin_ctzll(hit);
+            hit &= hit - 1ull;
+            const int c1 = hit ? (int)__builtin_ctzll(hit) : -1;
+            hit &= hit - 1ull;   // 0 stays 0: 0 & ~0
+            const int l0 = __builtin_amdgcn_readlane(child, c0), l1 = c1 < 0 ? -1 : __builtin_amdgcn_readlane(child, c1);
+            const int leaf = lane < 32 ? l0 : l1;
+            j = leaf < 0 || leaf >= g.nleaf ? -1 : leaf * 32 + (lane & 31);
+            if (j >= g.n) j = -1;
+            leaves += c1 < 0 ? 1u : 2u;
+            if (j >= 0) {
+#pragma unroll
+                for (int k = 0; k <= D; ++k) x[k] = g.xs[(int64_t)j * (D + 1) + k];
+            }
+        };
+        if (hit) {
+            load();
+            for (;;) {
+                double xc[D + 1];
+                const int jc = j;
+#pragma unroll
+                for (int k = 0; k <= D; ++k) xc[k] = x[k];
+                const bool more = hit != 0ull;
+                if (more) load();
+                double num = 0.0, den2 = 1.0;
+                bool pass = false;
+                if (jc >= 0) {   // hv_consider's test
+                    double ux = 0.0, rxj = 0.0;
+#pragma unroll
+                    for (int k = 0; k < D; ++k) {
+                        ux = fma(G.u[k], xc[k], ux);
+                        rxj = fma(G.r[k], xc[k], rxj);
+                    }
+                    den2 = 2.0 * (ux - G.ux0);
+                    num = fma(-2.0, rxj, xc[D] + G.K);
+                    pass = ux > G.cth && num < den2 * (T.t1 + HV_W);
+                }
+                unsigned long long pm = __ballot(pass);
+                if (pm) {
+                    const double t = num / den2, before = T.t1;
+                    exact += (unsigned)__popcll(pm);
+                    while (pm) {
+                        const int q = __builtin_ctzll(pm);
+                        pm &= pm - 1ull;
+                        T.offer(__shfl(t, q), __shfl(jc, q));
+                    }
+                    if (T.t1 < before) {
+                        set_ball(T.t1 + HV_W);
+                        hit &= __ballot(box_d2() <= R2f);   // a pair already loaded is tested all the same
+                    }
+                }
+                if (!more) break;
+            }
+        }
+        hv_wave_sync();
+    }
+    if (lane == 0) {
+        atomicAdd(&ctr[0], 32ull * leaves);
+        atomicAdd(&ctr[cstride], (unsigned long long)leaves);
+        if (mixed && exact) {
+            atomicAdd(&ctr[6 * cstride], (unsigned long long)exact);
+            atomicAdd(&ctr[7 * cstride], 1ull);
+        }
+    }
+    const bool tie = lane == 0 && hv_ray_result<D>(g, G, T, R.du[ray], plane_tol, rid, status, win, tout);
+    hv_wave_count(&ctr[2 * cstride], tie);
 }
 
 // ppw rays per packet in nblocks workgroups (over a forest: the packet plan pk_off / seg)
@@ -2324,6 +2625,13 @@ template <int D>
 static void launch_scan1(int precision, const DevGeo& g, const DevRays& R, const int* list, int n, const int* n_dev,
                          const int* vkey, const double* vx, int* status, int* win, double* tout, double plane_tol,
                          unsigned long long* ctr, hipStream_t st, const HvTiles& tiles = HvTiles{}, int cstride = 1) {
+    // a walk's n bounds its rays from above by a factor of two or three
+    if ((n_dev ? n : 2 * (int64_t)n) <= hv_small_level(D) && g.L == 32) {
+        k_raycast1<D, false><<<nblk(n, HV_R1_WAVES), 64 * HV_R1_WAVES, 0, st>>>(g, GeoSet{}, R, list, n, n_dev, vkey, vx, status,
+                                                                               win, tout, plane_tol, ctr, cstride,
+                                                                               precision != HV_PREC_FP64);
+        return;
+    }
     const int ppw = hv_packet_rays(n, tiles);
     launch_scan<D, false>(precision, g, GeoSet{}, nullptr, nullptr, ppw, nblk(n, ppw), R, list, n, n_dev, vkey, vx, status,
                           win, tout, plane_tol, ctr, st, cstride);
@@ -3786,7 +4094,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         // but with chunks)
         DevRays Ri = R;
         if (B && !chunks) Ri.code = nullptr;
-        k_ray_init<D, B><<<nblk(nr, 256), 256, 0, c->stream>>>(g, F, Ri, nr, vkey, vx, plane_tol);
+        launch_ray_init<D, B>(g, F, Ri, nr, vkey, vx, plane_tol, c->stream);
         HVCK(hipGetLastError());
         if (chunks) {
             // over a forest the code holds the mesh above 32 Morton bits
@@ -3805,7 +4113,12 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         auto scan = [&](const int* list, int n, const int* n_dev) -> int {
             int r_ = ensure_vertices(n);
             if (r_) return r_;
-            if constexpr (B) {
+            if (B && n <= hv_small_level(D) && L == 32) {
+                HVCK(hipEventRecord(r0, c->stream));
+                k_raycast1<D, B><<<nblk(n, HV_R1_WAVES), 64 * HV_R1_WAVES, 0, c->stream>>>(
+                    g, F, R, list, n, n_dev, vkey, vx, status, rwin, rt, plane_tol, sctr, HV_SCAN_SPREAD,
+                    prec != HV_PREC_FP64);
+            } else if constexpr (B) {
                 // packets of one mesh each: rays and packets per mesh of the (mesh-ordered) list
                 const int ppw = hv_packet_rays(n, tiles);
                 int* pcnt = pget<int>(c, "pk_cnt", (size_t)nmesh);
@@ -5337,7 +5650,7 @@ int hv_raycast_batch_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t
     const double plane_tol = 1e-12;
     k_setup_rays<D><<<nblk(nrays, 256), 256, 0, c->stream>>>((int)nrays, vkey, vx, dd, g, R, plane_tol);
     HVCK(hipGetLastError());
-    k_ray_init<D, false><<<nblk(nrays, 256), 256, 0, c->stream>>>(g, GeoSet{}, R, (int)nrays, vkey, vx, plane_tol);
+    launch_ray_init<D, false>(g, GeoSet{}, R, (int)nrays, vkey, vx, plane_tol, c->stream);
     HVCK(hipGetLastError());
     size_t tb = 0;
     HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, R.code, code2, ord0, ord, (int)nrays, HV_RAY_SORT_LO, 60, c->stream));
@@ -5548,7 +5861,7 @@ int hv_raycast_noalloc_impl(hv_ctx* c, int precision, int64_t nrays, const int64
     const double plane_tol = 1e-12;
     k_setup_rays<D><<<nblk(n, 256), 256, 0, c->stream>>>(n, vkey, vx, dd, g, R, plane_tol);
     HVCK(hipGetLastError());
-    k_ray_init<D, false><<<nblk(n, 256), 256, 0, c->stream>>>(g, GeoSet{}, R, n, vkey, vx, plane_tol);
+    launch_ray_init<D, false>(g, GeoSet{}, R, n, vkey, vx, plane_tol, c->stream);
     HVCK(hipGetLastError());
     k_iota<<<nblk(n, 256), 256, 0, c->stream>>>(ord0, n);
     HVCK(hipGetLastError());
