@@ -205,51 +205,68 @@ HvPinned::~HvPinned() {
     (void)hipHostFree(p);
 }
 
-// Results leave the device through pinned staging buffers, one per worker thread with its own
-// stream: a worker's copy to the caller's memory (whose pages are mostly touched for the first
-// time there, the dearer part) runs beside the others' transfers.  256 MiB into fresh pages took
-// 25 ms with one copy by the runtime (10.6 GB/s, 57 GB/s into pinned memory).
-// A call takes the device's staging whole; one that finds it taken, or has little to copy, leaves
-// the copy to the runtime.
+// Arrays larger than HV_STAGE_MIN leave and reach the device through pinned staging buffers, one per
+// worker thread with its own stream: a worker's copy to or from the caller's memory (whose pages are
+// mostly touched for the first time there, the dearer part) runs beside the others' transfers.
+// 256 MiB into fresh pages took 25 ms with one copy by the runtime (10.6 GB/s, 57 GB/s into pinned
+// memory).  A call takes the device's staging whole; one that finds it taken, or has little to copy,
+// leaves the copies to the runtime.
 constexpr int HV_STAGE_WORKERS = 8;
-constexpr size_t HV_STAGE_BYTES = (size_t)2 << 20;   // per worker: 16 MiB of pinned memory per device
+constexpr size_t HV_STAGE_MIN = (size_t)1 << 20;
 struct HvStaging {
     std::mutex mu;
-    bool tried = false;
-    void* pin[HV_STAGE_WORKERS] = {};
+    void* pin[HV_STAGE_WORKERS] = {};   // HV_STAGE_BYTES each: at most 16 MiB of pinned memory per device
     hipStream_t st[HV_STAGE_WORKERS] = {};
-    int n = 0;   // workers with both
+    bool block(int w) {   // worker w's buffer; the caller holds mu
+        if (!pin[w] && hipHostMalloc(&pin[w], HV_STAGE_BYTES, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            pin[w] = nullptr;
+        }
+        return pin[w] != nullptr;
+    }
+    bool ready(int w) {
+        if (!block(w)) return false;
+        if (!st[w] && hipStreamCreateWithFlags(&st[w], hipStreamNonBlocking) != hipSuccess) {
+            (void)hipGetLastError();
+            st[w] = nullptr;
+        }
+        return st[w] != nullptr;
+    }
 };
 static HvStaging staging[64];   // per device ordinal, kept for the process
 
-hipError_t hv_copy_out(int device, void* dst, const void* src, size_t bytes) {
-    if (bytes == 0) return hipSuccess;
-    const size_t nchunk = (bytes + HV_STAGE_BYTES - 1) / HV_STAGE_BYTES;
+hipError_t hv_copies(int device, bool out, const HvCopy* copies, int ncopies) {
+    size_t total = 0;
+    for (int k = 0; k < ncopies; ++k) total += copies[k].bytes;
+    if (total == 0) return hipSuccess;
+    // pieces of equal size within each array, about two per worker
+    const size_t chunk = std::min(HV_STAGE_BYTES, std::max<size_t>((total / (2 * HV_STAGE_WORKERS) + 65535) & ~(size_t)65535,
+                                                                   (size_t)256 << 10));
+    std::vector<HvCopy> piece;
     std::unique_lock<std::mutex> lk;
     int nw = 0;
-    if (device >= 0 && device < 64 && nchunk > 1) {
+    if (device >= 0 && device < 64 && total > HV_STAGE_MIN) {
         HvStaging& S = staging[device];
         lk = std::unique_lock<std::mutex>(S.mu, std::try_to_lock);
         if (lk.owns_lock()) {
-            if (!S.tried) {
-                S.tried = true;
-                for (int w = 0; w < HV_STAGE_WORKERS; ++w) {
-                    if (hipHostMalloc(&S.pin[w], HV_STAGE_BYTES, hipHostMallocDefault) != hipSuccess) break;
-                    if (hipStreamCreateWithFlags(&S.st[w], hipStreamNonBlocking) != hipSuccess) {
-                        (void)hipHostFree(S.pin[w]);
-                        break;
-                    }
-                    S.n = w + 1;
-                }
-                (void)hipGetLastError();
-            }
-            nw = (int)std::min<size_t>(S.n, nchunk);
+            for (int k = 0; k < ncopies; ++k)
+                for (size_t o = 0; o < copies[k].bytes; o += chunk)
+                    piece.push_back({(char*)copies[k].dst + o, (const char*)copies[k].src + o, std::min(chunk, copies[k].bytes - o)});
+            while (nw < HV_STAGE_WORKERS && nw < (int)piece.size() && S.ready(nw)) ++nw;
         }
     }
     if (nw == 0) {
         const hipStream_t st = hipStreamPerThread;
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-        return e != hipSuccess ? e : hipStreamSynchronize(st);
+        for (int k = 0; k < ncopies; ++k) {
+            if (!copies[k].bytes) continue;
+            const hipError_t e = hipMemcpyAsync(copies[k].dst, copies[k].src, copies[k].bytes,
+                                                out ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, st);
+            if (e != hipSuccess) {
+                (void)hipStreamSynchronize(st);
+                return e;
+            }
+        }
+        return hipStreamSynchronize(st);
     }
     HvStaging& S = staging[device];
     std::atomic<size_t> next{0};
@@ -258,15 +275,17 @@ hipError_t hv_copy_out(int device, void* dst, const void* src, size_t bytes) {
         (void)hipSetDevice(device);
         for (;;) {
             const size_t c = next.fetch_add(1);
-            if (c >= nchunk || err.load() != hipSuccess) break;
-            const size_t off = c * HV_STAGE_BYTES, len = std::min(HV_STAGE_BYTES, bytes - off);
-            hipError_t e = hipMemcpyAsync(S.pin[w], (const char*)src + off, len, hipMemcpyDeviceToHost, S.st[w]);
+            if (c >= piece.size() || err.load() != hipSuccess) break;
+            const HvCopy& p = piece[c];
+            if (!out) std::memcpy(S.pin[w], p.src, p.bytes);
+            hipError_t e = out ? hipMemcpyAsync(S.pin[w], p.src, p.bytes, hipMemcpyDeviceToHost, S.st[w])
+                               : hipMemcpyAsync(p.dst, S.pin[w], p.bytes, hipMemcpyHostToDevice, S.st[w]);
             if (e == hipSuccess) e = hipStreamSynchronize(S.st[w]);
             if (e != hipSuccess) {
                 err.store(e);
                 break;
             }
-            std::memcpy((char*)dst + off, S.pin[w], len);
+            if (out) std::memcpy(p.dst, S.pin[w], p.bytes);
         }
     };
     std::vector<std::thread> th;
@@ -274,12 +293,20 @@ hipError_t hv_copy_out(int device, void* dst, const void* src, size_t bytes) {
         try {
             th.emplace_back(work, w);
         } catch (...) {
-            break;   // fewer workers: the ones running take every chunk
+            break;   // fewer workers: the ones running take every piece
         }
     }
     work(0);
     for (auto& t : th) t.join();
     return (hipError_t)err.load();
+}
+
+HvLease::HvLease(int device) {
+    if (device < 0 || device >= 64) return;
+    HvStaging& S = staging[device];
+    lk = std::unique_lock<std::mutex>(S.mu, std::try_to_lock);
+    if (lk.owns_lock() && S.block(0)) base = (char*)S.pin[0];
+    else if (lk.owns_lock()) lk.unlock();
 }
 
 double* hv_points_for_write(hv_ctx* c, size_t bytes) {

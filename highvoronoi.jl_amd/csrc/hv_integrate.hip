@@ -1790,33 +1790,58 @@ int hv_integral_counts_impl(const hv_integral* I, int64_t* ncells, int64_t* nnbr
     return HV_OK;
 }
 
-// bytes of the results at offset `off` into the caller's memory
-static int integral_out(const hv_integral* I, void* dst, size_t off, size_t bytes) {
-    if (!dst || bytes == 0) return HV_OK;
+// Parts of the results, at offsets from their base, into the caller's memory (null: not wanted).  On
+// the device they are adjacent: a small set comes in one copy through a pinned block.
+struct IntegralPart {
+    void* dst;
+    size_t off, bytes;
+};
+static int integral_out(const hv_integral* I, const IntegralPart* part, int n) {
+    HvCopy list[4];
+    int m = 0;
+    size_t lo = ~(size_t)0, hi = 0;
+    for (int k = 0; k < n; ++k) {
+        if (!part[k].dst || part[k].bytes == 0) continue;
+        list[m++] = {part[k].dst, I->base + part[k].off, part[k].bytes};
+        lo = std::min(lo, part[k].off);
+        hi = std::max(hi, part[k].off + part[k].bytes);
+    }
+    if (m == 0) return HV_OK;
     if (!I->dev) {
-        std::memcpy(dst, I->base + off, bytes);
+        for (int k = 0; k < m; ++k) std::memcpy(list[k].dst, list[k].src, list[k].bytes);
         return HV_OK;
     }
-    return hv_copy_out(I->device, dst, I->base + off, bytes) == hipSuccess ? HV_OK : HV_ERR_DEVICE;
+    if (hi - lo <= HV_STAGE_BYTES) {
+        HvLease pin(I->device);
+        if (pin.base) {
+            const hipStream_t st = hipStreamPerThread;
+            if (hipMemcpyAsync(pin.base, I->base + lo, hi - lo, hipMemcpyDeviceToHost, st) != hipSuccess ||
+                hipStreamSynchronize(st) != hipSuccess)
+                return HV_ERR_DEVICE;
+            for (int k = 0; k < m; ++k)
+                std::memcpy(list[k].dst, pin.base + ((const char*)list[k].src - (I->base + lo)), list[k].bytes);
+            return HV_OK;
+        }
+    }
+    return hv_copies(I->device, true, list, m) == hipSuccess ? HV_OK : HV_ERR_DEVICE;
 }
 
 int hv_integral_export_f_impl(const hv_integral* I, int32_t* nf, double* bulk, double* iface) {
     if (!I) return HV_ERR_ARG;
     if (nf) *nf = I->nf;
-    int rc = integral_out(I, bulk, I->bulk, sizeof(double) * I->N * I->nf);
-    if (!rc) rc = integral_out(I, iface, I->iface, sizeof(double) * I->rows * I->nf);
-    return rc;
+    const IntegralPart part[2] = {{bulk, I->bulk, sizeof(double) * I->N * I->nf}, {iface, I->iface, sizeof(double) * I->rows * I->nf}};
+    return integral_out(I, part, 2);
 }
 
 int hv_integral_export_impl(const hv_integral* I, double* vol, int64_t* nbr_ptr, int64_t* nbr, double* area,
                             double* ms) {
     if (!I) return HV_ERR_ARG;
-    int rc = integral_out(I, vol, I->vol, sizeof(double) * I->N);
-    if (!rc) rc = integral_out(I, nbr_ptr, I->ptr, sizeof(int64_t) * (I->N + 1));
-    if (!rc) rc = integral_out(I, nbr, I->nbr, sizeof(int64_t) * I->rows);
-    if (!rc) rc = integral_out(I, area, I->area, sizeof(double) * I->rows);
+    const IntegralPart part[4] = {{vol, I->vol, sizeof(double) * I->N},
+                                  {nbr_ptr, I->ptr, sizeof(int64_t) * (I->N + 1)},
+                                  {nbr, I->nbr, sizeof(int64_t) * I->rows},
+                                  {area, I->area, sizeof(double) * I->rows}};
     if (ms) *ms = I->ms;
-    return rc;
+    return integral_out(I, part, 4);
 }
 
 void hv_integral_free_impl(hv_integral* I) { delete I; }

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <map>
+#include <cstring>
 #include <mutex>
 #include <memory>
 #include <string>
@@ -60,9 +61,37 @@ struct HvScratch {
     HvScratch(const HvScratch&) = delete;
     HvScratch& operator=(const HvScratch&) = delete;
 };
-// bytes of device memory into the caller's (pageable) memory; the data is complete (its stream has
-// been waited for).  Synchronous, callable from several threads at once.
-hipError_t hv_copy_out(int device, void* dst, const void* src, size_t bytes);
+// Copies between device memory and the caller's (pageable) memory, out of the device or into it; the
+// data is complete (its stream has been waited for) and so are the copies on return.  Callable from
+// several threads at once.
+struct HvCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+hipError_t hv_copies(int device, bool out, const HvCopy* copies, int ncopies);
+// A pinned block that kernels read a small call's inputs from and write its results to, for the
+// lifetime of the object (two copies each way cost more than the kernel's own accesses over the bus):
+// base is null when another call holds it.
+constexpr size_t HV_STAGE_BYTES = (size_t)2 << 20;
+struct HvLease {
+    std::unique_lock<std::mutex> lk;
+    char* base = nullptr;
+    size_t at = 0;
+    explicit HvLease(int device);
+    template <typename T>
+    T* take(size_t count) {
+        T* p = (T*)(base + at);
+        at += (count * sizeof(T) + 255) & ~(size_t)255;
+        return p;
+    }
+    template <typename T>
+    T* put(const T* src, size_t count) {
+        T* p = take<T>(count);
+        std::memcpy(p, src, count * sizeof(T));
+        return p;
+    }
+};
 // Pinned host memory (512 bytes) that kernels write a call's counts into, for the lifetime of the
 // object: from a process-wide store of at most HV_PINNED_KEEP free blocks; p is null when there is
 // none to be had.

@@ -2621,12 +2621,16 @@ static void launch_scan(int precision, const DevGeo& g, const GeoSet& F, const i
                                                     plane_tol, ctr, cstride);
 }
 
+// a walk's n bounds its rays from above by a factor of two or three
+static inline bool hv_scan_by_wave(int D, int n, bool bound, int L) {
+    return (bound ? (int64_t)n : 2 * (int64_t)n) <= hv_small_level(D) && L == 32;
+}
+
 template <int D>
 static void launch_scan1(int precision, const DevGeo& g, const DevRays& R, const int* list, int n, const int* n_dev,
                          const int* vkey, const double* vx, int* status, int* win, double* tout, double plane_tol,
                          unsigned long long* ctr, hipStream_t st, const HvTiles& tiles = HvTiles{}, int cstride = 1) {
-    // a walk's n bounds its rays from above by a factor of two or three
-    if ((n_dev ? n : 2 * (int64_t)n) <= hv_small_level(D) && g.L == 32) {
+    if (hv_scan_by_wave(D, n, n_dev != nullptr, g.L)) {
         k_raycast1<D, false><<<nblk(n, HV_R1_WAVES), 64 * HV_R1_WAVES, 0, st>>>(g, GeoSet{}, R, list, n, n_dev, vkey, vx, status,
                                                                                win, tout, plane_tol, ctr, cstride,
                                                                                precision != HV_PREC_FP64);
@@ -2637,15 +2641,11 @@ static void launch_scan1(int precision, const DevGeo& g, const DevRays& R, const
                           win, tout, plane_tol, ctr, st, cstride);
 }
 
+// (of the ray at position rid of the scanned list)
 template <int D, bool B>
-__global__ __launch_bounds__(256) void k_finalize(DevGeo g0, GeoSet F, DevRays R, const int* __restrict__ order, int nrays,
-                           const int* __restrict__ nrays_dev, int* __restrict__ vkey, double* __restrict__ vx,
-                           int64_t base, int* __restrict__ status, const int* __restrict__ win) {
-    if (nrays_dev) nrays = min(nrays, *nrays_dev);
-    const int blk = hv_xcd_block_first((nrays + (int)blockDim.x - 1) / (int)blockDim.x);
-    if (blk < 0) return;
-    const int rid = blk * blockDim.x + threadIdx.x;
-    if (rid >= nrays) return;
+__device__ __forceinline__ void hv_finalize(const DevGeo& g0, const GeoSet& F, const DevRays& R, const int* __restrict__ order,
+                                            int rid, int* __restrict__ vkey, double* __restrict__ vx, int64_t base,
+                                            int* __restrict__ status, const int* __restrict__ win) {
     if (status[rid] <= 0) return;
     const int ray = order[rid];
     const int v = R.v[ray], pos = R.drop[ray];
@@ -2668,6 +2668,17 @@ __global__ __launch_bounds__(256) void k_finalize(DevGeo g0, GeoSet F, DevRays R
     for (int j = 0; j <= D; ++j) vkey[id * (D + 1) + j] = nk[j];
 #pragma unroll
     for (int k = 0; k < D; ++k) vx[id * D + k] = xn[k];
+}
+
+template <int D, bool B>
+__global__ __launch_bounds__(256) void k_finalize(DevGeo g0, GeoSet F, DevRays R, const int* __restrict__ order, int nrays,
+                           const int* __restrict__ nrays_dev, int* __restrict__ vkey, double* __restrict__ vx,
+                           int64_t base, int* __restrict__ status, const int* __restrict__ win) {
+    if (nrays_dev) nrays = min(nrays, *nrays_dev);
+    const int blk = hv_xcd_block_first((nrays + (int)blockDim.x - 1) / (int)blockDim.x);
+    if (blk < 0) return;
+    const int rid = blk * blockDim.x + threadIdx.x;
+    if (rid < nrays) hv_finalize<D, B>(g0, F, R, order, rid, vkey, vx, base, status, win);
 }
 
 __global__ void k_iota(int* __restrict__ a, int n) {
@@ -4113,7 +4124,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         auto scan = [&](const int* list, int n, const int* n_dev) -> int {
             int r_ = ensure_vertices(n);
             if (r_) return r_;
-            if (B && n <= hv_small_level(D) && L == 32) {
+            if (B && hv_scan_by_wave(D, n, true, L)) {
                 HVCK(hipEventRecord(r0, c->stream));
                 k_raycast1<D, B><<<nblk(n, HV_R1_WAVES), 64 * HV_R1_WAVES, 0, c->stream>>>(
                     g, F, R, list, n, n_dev, vkey, vx, status, rwin, rt, plane_tol, sctr, HV_SCAN_SPREAD,
@@ -4873,13 +4884,24 @@ int hv_mesh_export_impl(const hv_mesh* m, int64_t* sig, double* coords) {
         first = false;
         e = b;
     }
+    if (row * nv + 512 <= HV_STAGE_BYTES) {   // a small table is written straight into pinned memory
+        HvLease pin(m->device);
+        if (pin.base) {
+            int64_t* psig = pin.take<int64_t>((size_t)nv * (D + 1));
+            double* px = pin.take<double>((size_t)nv * D);
+            k_export_rows<D><<<nblk(nv * (2 * D + 1), 256), 256, 0, st>>>(pb, 0, (int)nv, ids, key, x, psig, px);
+            if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return HV_ERR_DEVICE;
+            std::memcpy(sig, psig, sizeof(int64_t) * (D + 1) * nv);
+            std::memcpy(coords, px, sizeof(double) * D * nv);
+            return HV_OK;
+        }
+    }
     for (int64_t r0 = 0; r0 < nv; r0 += chunk) {
         const int n = (int)std::min<int64_t>(chunk, nv - r0);
         k_export_rows<D><<<nblk((int64_t)n * (2 * D + 1), 256), 256, 0, st>>>(pb, (int)r0, n, ids, key, x, dsig, dx);
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess ||
-            hv_copy_out(m->device, sig + r0 * (D + 1), dsig, sizeof(int64_t) * (D + 1) * n) != hipSuccess ||
-            hv_copy_out(m->device, coords + r0 * D, dx, sizeof(double) * D * n) != hipSuccess)
-            return HV_ERR_DEVICE;
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return HV_ERR_DEVICE;
+        const HvCopy list[2] = {{sig + r0 * (D + 1), dsig, sizeof(int64_t) * (D + 1) * n}, {coords + r0 * D, dx, sizeof(double) * D * n}};
+        if (hv_copies(m->device, true, list, 2) != hipSuccess) return HV_ERR_DEVICE;
     }
     return HV_OK;
 }
@@ -4887,30 +4909,56 @@ int hv_mesh_export_impl(const hv_mesh* m, int64_t* sig, double* coords) {
 // ---------------------------------------------------------------------------------
 // ray-level and query entry points (hv_raycast_batch, hv_nn_halfspace_batch, hv_inrange_batch)
 
+// The caller's rays (1-based int64 keys, drop positions, vertices; on the device or pinned) -> the
+// walk's records, directions included; rays in order of arrival.  A ray that is refused (the key
+// unsorted or out of range, the position out of range, no generator on the edge) sets *bad, in pinned
+// memory, and is replaced by one of the first d + 1 generators, so that what follows stays in bounds.
 template <int D>
-__global__ __launch_bounds__(256) void k_setup_rays(int n, const int* __restrict__ vkey, const double* __restrict__ vx,
-                             const int* __restrict__ drop, DevGeo g, DevRays R, double plane_tol) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_rays_in(int n, const int64_t* __restrict__ sig, const int32_t* __restrict__ drop,
+                                                 const double* __restrict__ r0, DevGeo g, int* __restrict__ vkey,
+                                                 double* __restrict__ vx, DevRays R, int* __restrict__ ord,
+                                                 int* __restrict__ status, unsigned long long* __restrict__ bad,
+                                                 double plane_tol) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    // key read straight from global memory: a private copy indexed by `pos` would live in scratch
-    const int* key = vkey + (int64_t)t * (D + 1);
+    bool ok = true;
+    int64_t prev = 0;
+#pragma unroll
+    for (int j = 0; j <= D; ++j) {
+        const int64_t e = sig[(int64_t)t * (D + 1) + j];
+        ok = ok && e >= 1 && e <= (int64_t)g.N + g.P && e > prev;
+        prev = e;
+    }
+    int p = drop[t];
+    ok = ok && p >= 0 && p <= D;
+    // the walked edge holds a generator: its smallest element
+    if (ok) ok = (p == 0 ? sig[(int64_t)t * (D + 1) + 1] : sig[(int64_t)t * (D + 1)]) <= g.N;
+    if (!ok) {
+        *bad = 1ull;
+        p = 0;
+    }
     double r[D];
 #pragma unroll
-    for (int k = 0; k < D; ++k) r[k] = vx[(int64_t)t * D + k];
+    for (int j = 0; j <= D; ++j) vkey[(int64_t)t * (D + 1) + j] = ok ? (int)(sig[(int64_t)t * (D + 1) + j] - 1) : j;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        r[k] = r0[(int64_t)t * D + k];
+        vx[(int64_t)t * D + k] = r[k];
+    }
+    // key read straight from global memory: a private copy indexed by `p` would live in scratch
+    const int* key = vkey + (int64_t)t * (D + 1);
     double u[D], c, du, rho;
-    hv_ray_setup<D>(g, key, drop[t], r, plane_tol, u, c, du, rho);
+    hv_ray_setup<D>(g, key, p, r, plane_tol, u, c, du, rho);
     R.v[t] = t;
-    R.drop[t] = drop[t];
+    R.drop[t] = p;
 #pragma unroll
     for (int k = 0; k < D; ++k) R.u[(int64_t)t * D + k] = u[k];
     R.c[t] = c;
     R.du[t] = du;
-    double pe[D];
-#pragma unroll
-    for (int k = 0; k < D; ++k) pe[k] = r[k] + rho * u[k];
-    R.code[t] = hv_morton<D>(g, pe);
+    ord[t] = t;
+    status[t] = 0;
+    (void)rho;
 }
-
 
 // Queries: one wavefront per query walks the 8-ary tree depth-first, nearest children first.  Eight
 // lanes test a node's child boxes, two leaves of 32 points are measured at once, a point per lane.
@@ -5585,6 +5633,68 @@ __global__ __launch_bounds__(128) void k_full_key(DevGeo g, DevRays R, const int
     olen[rid] = over ? -1 : n;
 }
 
+// The end points of the scanned rays, and the results in the caller's ray order (ord: position -> ray;
+// on the device or pinned); nothing is written when a ray was refused.
+template <int D>
+__global__ __launch_bounds__(256) void k_rays_out(int n, DevGeo g, DevRays R, const int* __restrict__ ord,
+                                                  int* __restrict__ status, const int* __restrict__ win, int* __restrict__ vkey,
+                                                  double* __restrict__ vx, const double* __restrict__ tout,
+                                                  const volatile unsigned long long* bad, int64_t* __restrict__ out_sig,
+                                                  double* __restrict__ out_r, double* __restrict__ out_t,
+                                                  int32_t* __restrict__ out_status) {
+    const int rid = blockIdx.x * blockDim.x + threadIdx.x;
+    if (rid >= n || *bad) return;
+    hv_finalize<D, false>(g, GeoSet{}, R, ord, rid, vkey, vx, n, status, win);
+    const int k = ord[rid];
+    const int s = status[rid];
+    out_status[k] = s == HV_ST_FOUND ? 0 : (s == HV_ST_TIE ? 2 : (s == HV_ST_NONE ? 1 : -1));
+#pragma unroll
+    for (int j = 0; j <= D; ++j)
+        out_sig[(int64_t)k * (D + 1) + j] = s > 0 ? (int64_t)vkey[((int64_t)n + rid) * (D + 1) + j] + 1 : 0;
+#pragma unroll
+    for (int q = 0; q < D; ++q) out_r[(int64_t)k * D + q] = s > 0 ? vx[((int64_t)n + rid) * D + q] : (double)NAN;
+    out_t[k] = s > 0 ? tout[rid] : (double)INFINITY;
+}
+
+// Device buffers of one batch of rays, and the batch's launches: no host wait.
+struct RayBatch {
+    int* vkey;      // 2 n keys: the rays' vertices, their end points
+    double* vx;
+    DevRays R;
+    uint64_t* code2;
+    int *ord0, *ord, *status, *win;
+    double* t;
+    unsigned long long* ctr;   // the scan's statistics, not read
+    void* tmp;      // the sort's
+    size_t tb;
+    // the order the results are in
+    const int* order = nullptr;
+};
+template <int D>
+static int run_rays(hv_ctx* c, const DevGeo& g, int precision, int n, RayBatch& b, const int64_t* sig, const int32_t* drop,
+                    const double* r, unsigned long long* bad, int64_t* out_sig, double* out_r, double* out_t,
+                    int32_t* out_status) {
+    const double plane_tol = 1e-12;
+    k_rays_in<D><<<nblk(n, 256), 256, 0, c->stream>>>(n, sig, drop, r, g, b.vkey, b.vx, b.R, b.ord0, b.status, bad, plane_tol);
+    HVCK(hipGetLastError());
+    const bool wave = hv_scan_by_wave(D, n, false, g.L);   // a wavefront a ray: in any order
+    DevRays Ri = b.R;
+    if (wave) Ri.code = nullptr;
+    launch_ray_init<D, false>(g, GeoSet{}, Ri, n, b.vkey, b.vx, plane_tol, c->stream);
+    HVCK(hipGetLastError());
+    b.order = b.ord0;
+    if (!wave) {
+        HVCK(hipcub::DeviceRadixSort::SortPairs(b.tmp, b.tb, b.R.code, b.code2, b.ord0, b.ord, n, HV_RAY_SORT_LO, 60, c->stream));
+        b.order = b.ord;
+    }
+    launch_scan1<D>(precision, g, b.R, b.order, n, nullptr, b.vkey, b.vx, b.status, b.win, b.t, plane_tol, b.ctr, c->stream);
+    HVCK(hipGetLastError());
+    k_rays_out<D><<<nblk(n, 256), 256, 0, c->stream>>>(n, g, b.R, b.order, b.status, b.win, b.vkey, b.vx, b.t, bad, out_sig,
+                                                       out_r, out_t, out_status);
+    HVCK(hipGetLastError());
+    return HV_OK;
+}
+
 template <int D>
 int hv_raycast_batch_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t* sig, const int32_t* drop,
                           const double* r, int64_t* out_sig, double* out_r, double* out_t, int32_t* out_status,
@@ -5597,119 +5707,135 @@ int hv_raycast_batch_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t
     const int P = c->P;
     int rc = check_box(c, D);
     if (rc) return rc;
-    // host validation: sorted keys, an edge with a real generator
-    std::vector<int> hkey((size_t)nrays * (D + 1));
-    std::vector<int> hdrop(nrays);
-    for (int64_t k = 0; k < nrays; ++k) {
-        for (int j = 0; j <= D; ++j) {
-            const int64_t e = sig[k * (D + 1) + j];
-            if (e < 1 || e > (int64_t)N + P) return hv_fail(c, HV_ERR_ARG, "key element out of range");
-            if (j && e <= sig[k * (D + 1) + j - 1]) return hv_fail(c, HV_ERR_ARG, "keys must be sorted and distinct");
-            hkey[k * (D + 1) + j] = (int)(e - 1);
+    // what the kernels refuse (k_rays_in), named: sorted keys, an edge with a real generator
+    auto refused = [&]() -> int {
+        for (int64_t k = 0; k < nrays; ++k) {
+            const int64_t* e = sig + k * (D + 1);
+            for (int j = 0; j <= D; ++j) {
+                if (e[j] < 1 || e[j] > (int64_t)N + P) return hv_fail(c, HV_ERR_ARG, "key element out of range");
+                if (j && e[j] <= e[j - 1]) return hv_fail(c, HV_ERR_ARG, "keys must be sorted and distinct");
+            }
+            if (drop[k] < 0 || drop[k] > D) return hv_fail(c, HV_ERR_ARG, "drop position out of range");
+            if (e[drop[k] == 0 ? 1 : 0] > N) return hv_fail(c, HV_ERR_ARG, "the walked edge must contain a generator");
         }
-        if (drop[k] < 0 || drop[k] > D) return hv_fail(c, HV_ERR_ARG, "drop position out of range");
-        hdrop[k] = drop[k];
-        const int first = (drop[k] == 0) ? hkey[k * (D + 1) + 1] : hkey[k * (D + 1)];
-        if (first >= N) return hv_fail(c, HV_ERR_ARG, "the walked edge must contain a generator");
-    }
+        return hv_fail(c, HV_ERR_ARG, "a ray was refused");
+    };
+    if (N <= D) return refused();
     Tree T;
     rc = build_tree<D>(c, 32, T, precision, TREE_RAYS);
     if (rc) return rc;
     record_tree(c, T.g, precision, 32);
     DevGeo& g = T.g;
-    int* vkey = pget<int>(c, "b_vkey", (size_t)2 * nrays * (D + 1));
-    double* vx = pget<double>(c, "b_vx", (size_t)2 * nrays * D);
-    int* dd = pget<int>(c, "b_drop", nrays);
-    DevRays R;
-    R.v = pget<int>(c, "b_rv", nrays);
-    R.drop = pget<int>(c, "b_rd", nrays);
-    R.u = pget<double>(c, "b_ru", (size_t)nrays * D);
-    R.c = pget<double>(c, "b_rc", nrays);
-    R.du = pget<double>(c, "b_rdu", nrays);
-    R.tinit = nullptr;
-    R.code = pget<uint64_t>(c, "b_code", nrays);
-    R.t1 = pget<double>(c, "b_t1", nrays);
-    R.t2 = pget<double>(c, "b_t2", nrays);
-    R.i1 = pget<int>(c, "b_i1", nrays);
-    R.i2 = pget<int>(c, "b_i2", nrays);
-    uint64_t* code2 = pget<uint64_t>(c, "b_code2", nrays);
-    int* ord0 = pget<int>(c, "b_ord0", nrays);
-    int* ord = pget<int>(c, "b_ord", nrays);
-    int* status = pget<int>(c, "b_status", nrays);
-    double* tout = pget<double>(c, "b_t", nrays);
-    int* rwin = pget<int>(c, "b_win", nrays);
-    unsigned long long* ctr = pget<unsigned long long>(c, "b_ctr", 16);
-    if (!vkey || !vx || !dd || !R.v || !R.drop || !R.u || !R.c || !R.du || !R.code || !code2 || !ord0 || !ord ||
-        !status || !tout || !ctr || !rwin || !R.t1 || !R.t2 || !R.i1 || !R.i2)
+    const int n = (int)nrays;
+    RayBatch b;
+    b.vkey = pget<int>(c, "b_vkey", (size_t)2 * nrays * (D + 1));
+    b.vx = pget<double>(c, "b_vx", (size_t)2 * nrays * D);
+    b.R = DevRays{};
+    b.R.v = pget<int>(c, "b_rv", nrays);
+    b.R.drop = pget<int>(c, "b_rd", nrays);
+    b.R.u = pget<double>(c, "b_ru", (size_t)nrays * D);
+    b.R.c = pget<double>(c, "b_rc", nrays);
+    b.R.du = pget<double>(c, "b_rdu", nrays);
+    b.R.code = pget<uint64_t>(c, "b_code", nrays);
+    b.R.t1 = pget<double>(c, "b_t1", nrays);
+    b.R.t2 = pget<double>(c, "b_t2", nrays);
+    b.R.i1 = pget<int>(c, "b_i1", nrays);
+    b.R.i2 = pget<int>(c, "b_i2", nrays);
+    b.code2 = pget<uint64_t>(c, "b_code2", nrays);
+    b.ord0 = pget<int>(c, "b_ord0", nrays);
+    b.ord = pget<int>(c, "b_ord", nrays);
+    b.status = pget<int>(c, "b_status", nrays);
+    b.t = pget<double>(c, "b_t", nrays);
+    b.win = pget<int>(c, "b_win", nrays);
+    b.ctr = pget<unsigned long long>(c, "b_ctr", 16);
+    if (!b.vkey || !b.vx || !b.R.v || !b.R.drop || !b.R.u || !b.R.c || !b.R.du || !b.R.code || !b.code2 || !b.ord0 || !b.ord ||
+        !b.status || !b.t || !b.ctr || !b.win || !b.R.t1 || !b.R.t2 || !b.R.i1 || !b.R.i2)
         return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
-    HVCK(hipMemcpyAsync(vkey, hkey.data(), sizeof(int) * hkey.size(), hipMemcpyHostToDevice, c->stream));
-    HVCK(hipMemcpyAsync(vx, r, sizeof(double) * nrays * D, hipMemcpyHostToDevice, c->stream));
-    HVCK(hipMemcpyAsync(dd, hdrop.data(), sizeof(int) * nrays, hipMemcpyHostToDevice, c->stream));
-    HVCK(hipMemsetAsync(ctr, 0, 16 * sizeof(unsigned long long), c->stream));
-    HVCK(hipMemsetAsync(status, 0, sizeof(int) * nrays, c->stream));
-    const double plane_tol = 1e-12;
-    k_setup_rays<D><<<nblk(nrays, 256), 256, 0, c->stream>>>((int)nrays, vkey, vx, dd, g, R, plane_tol);
-    HVCK(hipGetLastError());
-    launch_ray_init<D, false>(g, GeoSet{}, R, (int)nrays, vkey, vx, plane_tol, c->stream);
-    HVCK(hipGetLastError());
-    size_t tb = 0;
-    HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, R.code, code2, ord0, ord, (int)nrays, HV_RAY_SORT_LO, 60, c->stream));
-    void* tmp = c->pool->get("cubtmp", tb, false, c->stream);
-    if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
-    k_iota<<<nblk(nrays, 256), 256, 0, c->stream>>>(ord0, (int)nrays);
-    HVCK(hipGetLastError());
-    HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, R.code, code2, ord0, ord, (int)nrays, HV_RAY_SORT_LO, 60, c->stream));
-    launch_scan1<D>(precision, g, R, ord, (int)nrays, nullptr, vkey, vx, status, rwin, tout, plane_tol, ctr, c->stream);
-    HVCK(hipGetLastError());
-    k_finalize<D, false><<<nblk(nrays, 256), 256, 0, c->stream>>>(g, GeoSet{}, R, ord, (int)nrays, nullptr, vkey, vx, nrays,
-                                                                  status, rwin);
-    HVCK(hipGetLastError());
-    // full keys of the rays out of general position (hv_raycast_batch_keys)
-    std::vector<int> hfk, hfl;
-    std::vector<double> hfx;
-    if (full_sig) {
-        int* fk = pget<int>(c, "b_fkey", (size_t)nrays * max_sig);
-        int* fl = pget<int>(c, "b_flen", nrays);
-        double* fx = pget<double>(c, "b_fx", (size_t)nrays * D);
-        if (!fk || !fl || !fx) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (full keys)");
-        k_full_key<D><<<nblk(nrays, 128), 128, 0, c->stream>>>(g, R, ord, (int)nrays, vkey, vx, status, tout, max_sig,
-                                                               fk, fl, fx);
-        HVCK(hipGetLastError());
-        hfk.resize((size_t)nrays * max_sig);
-        hfl.resize(nrays);
-        hfx.resize((size_t)nrays * D);
-        HVCK(hipMemcpyAsync(hfk.data(), fk, sizeof(int) * hfk.size(), hipMemcpyDeviceToHost, c->stream));
-        HVCK(hipMemcpyAsync(hfl.data(), fl, sizeof(int) * nrays, hipMemcpyDeviceToHost, c->stream));
-        HVCK(hipMemcpyAsync(hfx.data(), fx, sizeof(double) * hfx.size(), hipMemcpyDeviceToHost, c->stream));
+    b.tb = 0;
+    HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, b.tb, b.R.code, b.code2, b.ord0, b.ord, n, HV_RAY_SORT_LO, 60, c->stream));
+    b.tmp = c->pool->get("cubtmp", b.tb, false, c->stream);
+    if (!b.tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
+    HvPinned pin;
+    if (!pin.p) return hv_fail(c, HV_ERR_DEVICE, "out of pinned memory");
+    *pin.p = 0ull;
+    // the caller's arrays: a small batch's through a pinned block the kernels work on, a large one's copied
+    const size_t nk = (size_t)nrays * (D + 1), nx = (size_t)nrays * D;
+    if (16 * nk + 16 * nx + 16 * (size_t)nrays + 7 * 256 <= HV_STAGE_BYTES && !full_sig) {
+        HvLease L(c->device);
+        if (L.base) {
+            const int64_t* psig = L.put(sig, nk);
+            const double* pr = L.put(r, nx);
+            const int32_t* pdrop = L.put(drop, (size_t)nrays);
+            int64_t* osig = L.take<int64_t>(nk);
+            double* orr = L.take<double>(nx);
+            double* ot = L.take<double>((size_t)nrays);
+            int32_t* ost = L.take<int32_t>((size_t)nrays);
+            rc = run_rays<D>(c, g, precision, n, b, psig, pdrop, pr, pin.p, osig, orr, ot, ost);
+            if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = hv_fail(c, HV_ERR_DEVICE, "device error");
+            if (rc) return rc;
+            if (*pin.p) return refused();
+            std::memcpy(out_sig, osig, sizeof(int64_t) * nk);
+            std::memcpy(out_r, orr, sizeof(double) * nx);
+            std::memcpy(out_t, ot, sizeof(double) * nrays);
+            std::memcpy(out_status, ost, sizeof(int32_t) * nrays);
+            return HV_OK;
+        }
     }
-    std::vector<int> hord(nrays), hst(nrays), hk((size_t)nrays * (D + 1));
-    std::vector<double> hx((size_t)nrays * D), ht(nrays);
-    HVCK(hipMemcpyAsync(hord.data(), ord, sizeof(int) * nrays, hipMemcpyDeviceToHost, c->stream));
-    HVCK(hipMemcpyAsync(hst.data(), status, sizeof(int) * nrays, hipMemcpyDeviceToHost, c->stream));
-    HVCK(hipMemcpyAsync(hk.data(), vkey + (size_t)nrays * (D + 1), sizeof(int) * hk.size(), hipMemcpyDeviceToHost, c->stream));
-    HVCK(hipMemcpyAsync(hx.data(), vx + (size_t)nrays * D, sizeof(double) * hx.size(), hipMemcpyDeviceToHost, c->stream));
-    HVCK(hipMemcpyAsync(ht.data(), tout, sizeof(double) * nrays, hipMemcpyDeviceToHost, c->stream));
-    HVCK(hipStreamSynchronize(c->stream));
+    int64_t* dsig = pget<int64_t>(c, "b_sig", nk);
+    double* dr = pget<double>(c, "b_r", nx);
+    int32_t* ddrop = pget<int32_t>(c, "b_drop", nrays);
+    int64_t* dosig = pget<int64_t>(c, "b_osig", nk);
+    double* dor = pget<double>(c, "b_or", nx);
+    double* dot = pget<double>(c, "b_ot", nrays);
+    int32_t* dost = pget<int32_t>(c, "b_ost", nrays);
+    if (!dsig || !dr || !ddrop || !dosig || !dor || !dot || !dost) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
+    const HvCopy in[3] = {{dsig, sig, sizeof(int64_t) * nk}, {dr, r, sizeof(double) * nx}, {ddrop, drop, sizeof(int32_t) * nrays}};
+    HVCK(hv_copies(c->device, false, in, 3));
+    rc = run_rays<D>(c, g, precision, n, b, dsig, ddrop, dr, pin.p, dosig, dor, dot, dost);
+    // full keys of the rays out of general position (hv_raycast_batch_keys)
+    int* fk = nullptr;
+    int* fl = nullptr;
+    double* fx = nullptr;
+    if (!rc && full_sig) {
+        fk = pget<int>(c, "b_fkey", (size_t)nrays * max_sig);
+        fl = pget<int>(c, "b_flen", nrays);
+        fx = pget<double>(c, "b_fx", nx);
+        if (fk && fl && fx) {
+            k_full_key<D><<<nblk(nrays, 128), 128, 0, c->stream>>>(g, b.R, b.order, n, b.vkey, b.vx, b.status, b.t, max_sig, fk, fl, fx);
+            if (hipGetLastError() != hipSuccess) rc = hv_fail(c, HV_ERR_DEVICE, "device error");
+        } else {
+            rc = hv_fail(c, HV_ERR_DEVICE, "out of device memory (full keys)");
+        }
+    }
+    if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = hv_fail(c, HV_ERR_DEVICE, "device error");
+    if (rc) return rc;
+    if (*pin.p) return refused();
+    const HvCopy res[4] = {{out_sig, dosig, sizeof(int64_t) * nk},
+                           {out_r, dor, sizeof(double) * nx},
+                           {out_t, dot, sizeof(double) * nrays},
+                           {out_status, dost, sizeof(int32_t) * nrays}};
+    HVCK(hv_copies(c->device, true, res, 4));
+    if (!full_sig) return HV_OK;
+    std::vector<int> hord(nrays), hst(nrays), hfk((size_t)nrays * max_sig), hfl(nrays);
+    std::vector<double> hfx(nx), ht(nrays);
+    const HvCopy more[6] = {{hord.data(), b.order, sizeof(int) * nrays}, {hst.data(), b.status, sizeof(int) * nrays},
+                            {hfk.data(), fk, sizeof(int) * hfk.size()},  {hfl.data(), fl, sizeof(int) * nrays},
+                            {hfx.data(), fx, sizeof(double) * nx},       {ht.data(), b.t, sizeof(double) * nrays}};
+    HVCK(hv_copies(c->device, true, more, 6));
     for (int64_t rid = 0; rid < nrays; ++rid) {
         const int k = hord[rid];
         const int s = hst[rid];
-        out_status[k] = s == HV_ST_FOUND ? 0 : (s == HV_ST_TIE ? 2 : (s == HV_ST_NONE ? 1 : -1));
-        for (int j = 0; j <= D; ++j) out_sig[(int64_t)k * (D + 1) + j] = s > 0 ? (int64_t)hk[rid * (D + 1) + j] + 1 : 0;
-        for (int q = 0; q < D; ++q) out_r[(int64_t)k * D + q] = s > 0 ? hx[rid * D + q] : NAN;
-        out_t[k] = s > 0 ? ht[rid] : INFINITY;
-        if (full_sig) {
-            int64_t* fs = full_sig + (int64_t)k * max_sig;
-            const int fl = hfl[rid];
-            full_len[k] = s > 0 ? D + 1 : (s == HV_ST_SINGULAR ? fl : 0);
-            for (int j = 0; j < max_sig; ++j) fs[j] = 0;
-            if (s > 0) {
-                for (int j = 0; j <= D && j < max_sig; ++j) fs[j] = out_sig[(int64_t)k * (D + 1) + j];
-            } else if (s == HV_ST_SINGULAR && fl > 0) {
-                for (int j = 0; j < fl; ++j) fs[j] = (int64_t)hfk[(size_t)rid * max_sig + j] + 1;
-                for (int q = 0; q < D; ++q) out_r[(int64_t)k * D + q] = hfx[(size_t)rid * D + q];
-                out_t[k] = ht[rid];
-                out_status[k] = 3;
-            }
+        int64_t* fs = full_sig + (int64_t)k * max_sig;
+        const int len = hfl[rid];
+        full_len[k] = s > 0 ? D + 1 : (s == HV_ST_SINGULAR ? len : 0);
+        for (int j = 0; j < max_sig; ++j) fs[j] = 0;
+        if (s > 0) {
+            for (int j = 0; j <= D && j < max_sig; ++j) fs[j] = out_sig[(int64_t)k * (D + 1) + j];
+        } else if (s == HV_ST_SINGULAR && len > 0) {
+            for (int j = 0; j < len; ++j) fs[j] = (int64_t)hfk[(size_t)rid * max_sig + j] + 1;
+            for (int q = 0; q < D; ++q) out_r[(int64_t)k * D + q] = hfx[(size_t)rid * D + q];
+            out_t[k] = ht[rid];
+            out_status[k] = 3;
         }
     }
     return HV_OK;
@@ -5727,6 +5853,7 @@ static __device__ __align__(256) unsigned char scratch[HV_NA_BYTES];
 
 static std::mutex hv_na_mu;
 static void* hv_na_ptr[64] = {};   // per device ordinal: the address of `scratch`
+static unsigned long long* hv_na_pin[64] = {};   // and a pinned word that tells of a refused ray
 
 int hv_scratch_init(int device) {
     if (device < 0 || device >= 64) return HV_ERR_ARG;
@@ -5740,6 +5867,11 @@ int hv_scratch_init(int device) {
     (void)hipSetDevice(cur);
     if (e != hipSuccess || !p) {
         (void)hipGetLastError();
+        return HV_ERR_DEVICE;
+    }
+    if (hipHostMalloc((void**)&hv_na_pin[device], 64, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        hv_na_pin[device] = nullptr;
         return HV_ERR_DEVICE;
     }
     hv_na_ptr[device] = p;
@@ -5760,50 +5892,6 @@ struct NaCarve {
     bool ok() const { return off <= cap; }
 };
 
-// caller's rays (1-based int64 keys, drop positions, vertices) -> the walk's records, checked
-template <int D>
-__global__ void k_na_rays_in(int n, const int64_t* __restrict__ sig, const int32_t* __restrict__ drop,
-                             const double* __restrict__ r, int N, int P, int* __restrict__ vkey, double* __restrict__ vx,
-                             int* __restrict__ dd, int* __restrict__ bad) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    bool ok = true;
-    int64_t prev = 0;
-#pragma unroll
-    for (int j = 0; j <= D; ++j) {
-        const int64_t e = sig[(int64_t)t * (D + 1) + j];
-        ok = ok && e >= 1 && e <= (int64_t)N + P && e > prev;
-        prev = e;
-        vkey[(int64_t)t * (D + 1) + j] = ok ? (int)(e - 1) : 0;
-    }
-    const int p = drop[t];
-    ok = ok && p >= 0 && p <= D;
-    // the walked edge holds a generator: its smallest element
-    if (ok) ok = (p == 0 ? sig[(int64_t)t * (D + 1) + 1] : sig[(int64_t)t * (D + 1)]) <= N;
-    dd[t] = ok ? p : 0;
-#pragma unroll
-    for (int k = 0; k < D; ++k) vx[(int64_t)t * D + k] = r[(int64_t)t * D + k];
-    if (!ok) atomicOr(bad, 1);
-}
-
-// results in the caller's ray order (ord: sorted position -> ray), as hv_raycast_batch returns them
-template <int D>
-__global__ void k_na_out(int n, const int* __restrict__ ord, const int* __restrict__ status, const int* __restrict__ vkey,
-                         const double* __restrict__ vx, const double* __restrict__ tout, int64_t* __restrict__ out_sig,
-                         double* __restrict__ out_r, double* __restrict__ out_t, int32_t* __restrict__ out_status) {
-    const int rid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (rid >= n) return;
-    const int k = ord[rid];
-    const int s = status[rid];
-    out_status[k] = s == HV_ST_FOUND ? 0 : (s == HV_ST_TIE ? 2 : (s == HV_ST_NONE ? 1 : -1));
-#pragma unroll
-    for (int j = 0; j <= D; ++j)
-        out_sig[(int64_t)k * (D + 1) + j] = s > 0 ? (int64_t)vkey[((int64_t)n + rid) * (D + 1) + j] + 1 : 0;
-#pragma unroll
-    for (int q = 0; q < D; ++q) out_r[(int64_t)k * D + q] = s > 0 ? vx[((int64_t)n + rid) * D + q] : (double)NAN;
-    out_t[k] = s > 0 ? tout[rid] : (double)INFINITY;
-}
-
 template <int D>
 int hv_raycast_noalloc_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t* sig, const int32_t* drop,
                             const double* r, int64_t* out_sig, double* out_r, double* out_t, int32_t* out_status) {
@@ -5822,59 +5910,43 @@ int hv_raycast_noalloc_impl(hv_ctx* c, int precision, int64_t nrays, const int64
     const int n = (int)nrays;
     const DevGeo& g = c->tree_g;
     NaCarve cv{(unsigned char*)sp, 0, HV_NA_BYTES};
-    int* vkey = cv.take<int>((size_t)2 * n * (D + 1));
-    double* vx = cv.take<double>((size_t)2 * n * D);
-    int* dd = cv.take<int>(n);
-    DevRays R{};
-    R.v = cv.take<int>(n);
-    R.drop = cv.take<int>(n);
-    R.u = cv.take<double>((size_t)n * D);
-    R.c = cv.take<double>(n);
-    R.du = cv.take<double>(n);
-    R.code = cv.take<uint64_t>(n);
-    R.t1 = cv.take<double>(n);
-    R.t2 = cv.take<double>(n);
-    R.i1 = cv.take<int>(n);
-    R.i2 = cv.take<int>(n);
-    uint64_t* code2 = cv.take<uint64_t>(n);
-    int* ord0 = cv.take<int>(n);
-    int* ord = cv.take<int>(n);
-    int* status = cv.take<int>(n);
-    double* tout = cv.take<double>(n);
-    int* rwin = cv.take<int>(n);
-    unsigned long long* ctr = cv.take<unsigned long long>(16);
-    int* bad = cv.take<int>(1);
-    size_t tb = 0;
-    HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, R.code, code2, ord0, ord, n, HV_RAY_SORT_LO, 60, c->stream));
-    void* tmp = cv.take<unsigned char>(tb);
+    RayBatch b;
+    b.vkey = cv.take<int>((size_t)2 * n * (D + 1));
+    b.vx = cv.take<double>((size_t)2 * n * D);
+    b.R = DevRays{};
+    b.R.v = cv.take<int>(n);
+    b.R.drop = cv.take<int>(n);
+    b.R.u = cv.take<double>((size_t)n * D);
+    b.R.c = cv.take<double>(n);
+    b.R.du = cv.take<double>(n);
+    b.R.code = cv.take<uint64_t>(n);
+    b.R.t1 = cv.take<double>(n);
+    b.R.t2 = cv.take<double>(n);
+    b.R.i1 = cv.take<int>(n);
+    b.R.i2 = cv.take<int>(n);
+    b.code2 = cv.take<uint64_t>(n);
+    b.ord0 = cv.take<int>(n);
+    b.ord = cv.take<int>(n);
+    b.status = cv.take<int>(n);
+    b.t = cv.take<double>(n);
+    b.win = cv.take<int>(n);
+    b.ctr = cv.take<unsigned long long>(16);
+    b.tb = 0;
+    HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, b.tb, b.R.code, b.code2, b.ord0, b.ord, n, HV_RAY_SORT_LO, 60, c->stream));
+    b.tmp = cv.take<unsigned char>(b.tb);
     if (!cv.ok()) return hv_fail(c, HV_ERR_CAPACITY, "the rays do not fit the scratch array");
-    HVCK(hipMemsetAsync(ctr, 0, 16 * sizeof(unsigned long long), c->stream));
-    HVCK(hipMemsetAsync(status, 0, sizeof(int) * n, c->stream));
-    HVCK(hipMemsetAsync(bad, 0, sizeof(int), c->stream));
-    k_na_rays_in<D><<<nblk(n, 256), 256, 0, c->stream>>>(n, sig, drop, r, g.N, g.P, vkey, vx, dd, bad);
-    HVCK(hipGetLastError());
-    int hbad = 0;
-    HVCK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HVCK(hipStreamSynchronize(c->stream));
-    if (hbad) return hv_fail(c, HV_ERR_ARG, "a key is unsorted or out of range, a drop position is out of range, or "
-                                           "a walked edge holds no generator");
-    const double plane_tol = 1e-12;
-    k_setup_rays<D><<<nblk(n, 256), 256, 0, c->stream>>>(n, vkey, vx, dd, g, R, plane_tol);
-    HVCK(hipGetLastError());
-    launch_ray_init<D, false>(g, GeoSet{}, R, n, vkey, vx, plane_tol, c->stream);
-    HVCK(hipGetLastError());
-    k_iota<<<nblk(n, 256), 256, 0, c->stream>>>(ord0, n);
-    HVCK(hipGetLastError());
-    HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, R.code, code2, ord0, ord, n, HV_RAY_SORT_LO, 60, c->stream));
-    launch_scan1<D>(precision, g, R, ord, n, nullptr, vkey, vx, status, rwin, tout, plane_tol, ctr, c->stream);
-    HVCK(hipGetLastError());
-    k_finalize<D, false><<<nblk(n, 256), 256, 0, c->stream>>>(g, GeoSet{}, R, ord, n, nullptr, vkey, vx, nrays, status, rwin);
-    HVCK(hipGetLastError());
-    k_na_out<D><<<nblk(n, 256), 256, 0, c->stream>>>(n, ord, status, vkey, vx, tout, out_sig, out_r, out_t, out_status);
-    HVCK(hipGetLastError());
-    HVCK(hipStreamSynchronize(c->stream));
+    unsigned long long* bad = hv_na_pin[c->device];
+    *bad = 0ull;
+    rc = run_rays<D>(c, g, precision, n, b, sig, drop, r, bad, out_sig, out_r, out_t, out_status);
+    if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = hv_fail(c, HV_ERR_DEVICE, "device error");
+    if (rc) return rc;
+    if (*bad) return hv_fail(c, HV_ERR_ARG, "a key is unsorted or out of range, a drop position is out of range, or "
+                                            "a walked edge holds no generator");
     return HV_OK;
 }
+
+// queries of at most this many bytes, results included, are worked on in pinned memory
+constexpr size_t HV_QUERY_PINNED = HV_STAGE_BYTES;
 
 template <int D>
 int hv_nn_halfspace_impl(hv_ctx* c, int64_t nq, const double* q, const double* u, const double* cc,
@@ -5883,20 +5955,36 @@ int hv_nn_halfspace_impl(hv_ctx* c, int64_t nq, const double* q, const double* u
     Tree T;
     int rc = build_tree<D>(c, 32, T, HV_PREC_FP64, TREE_SEARCH);
     if (rc) return rc;
-    double* dq = pget<double>(c, "q_q", (size_t)nq * D);
-    double* du_ = pget<double>(c, "q_u", (size_t)nq * D);
+    const size_t nx = (size_t)nq * D;
+    if (16 * nx + 24 * (size_t)nq + 5 * 256 <= HV_QUERY_PINNED) {
+        HvLease L(c->device);
+        if (L.base) {   // the kernel reads the queries and writes the results over the bus
+            const double* pq = L.put(q, nx);
+            const double* pu = L.put(u, nx);
+            const double* pc = L.put(cc, (size_t)nq);
+            int64_t* pi = L.take<int64_t>((size_t)nq);
+            double* pd = L.take<double>((size_t)nq);
+            k_nn_halfspace<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, pq, pu, pc, pi, pd);
+            HVCK(hipGetLastError());
+            HVCK(hipStreamSynchronize(c->stream));
+            std::memcpy(idx, pi, sizeof(int64_t) * nq);
+            std::memcpy(dist, pd, sizeof(double) * nq);
+            return HV_OK;
+        }
+    }
+    double* dq = pget<double>(c, "q_q", nx);
+    double* du_ = pget<double>(c, "q_u", nx);
     double* dc = pget<double>(c, "q_c", nq);
     int64_t* di = pget<int64_t>(c, "q_i", nq);
     double* dd = pget<double>(c, "q_d", nq);
     if (!dq || !du_ || !dc || !di || !dd) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
-    HVCK(hipMemcpyAsync(dq, q, sizeof(double) * nq * D, hipMemcpyHostToDevice, c->stream));
-    HVCK(hipMemcpyAsync(du_, u, sizeof(double) * nq * D, hipMemcpyHostToDevice, c->stream));
-    HVCK(hipMemcpyAsync(dc, cc, sizeof(double) * nq, hipMemcpyHostToDevice, c->stream));
+    const HvCopy in[3] = {{dq, q, sizeof(double) * nx}, {du_, u, sizeof(double) * nx}, {dc, cc, sizeof(double) * nq}};
+    HVCK(hv_copies(c->device, false, in, 3));
     k_nn_halfspace<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, dq, du_, dc, di, dd);
     HVCK(hipGetLastError());
-    HVCK(hipMemcpyAsync(idx, di, sizeof(int64_t) * nq, hipMemcpyDeviceToHost, c->stream));
-    HVCK(hipMemcpyAsync(dist, dd, sizeof(double) * nq, hipMemcpyDeviceToHost, c->stream));
     HVCK(hipStreamSynchronize(c->stream));
+    const HvCopy res[2] = {{idx, di, sizeof(int64_t) * nq}, {dist, dd, sizeof(double) * nq}};
+    HVCK(hv_copies(c->device, true, res, 2));
     return HV_OK;
 }
 
@@ -5907,32 +5995,58 @@ int hv_inrange_impl(hv_ctx* c, int64_t nq, const double* q, const double* radius
     Tree T;
     int rc = build_tree<D>(c, 32, T, HV_PREC_FP64, TREE_SEARCH);
     if (rc) return rc;
-    double* dq = pget<double>(c, "q_q", (size_t)nq * D);
+    const size_t nx = (size_t)nq * D;
+    const int64_t total = idx ? ptr[nq] : 0;
+    auto ordered = [&]() {   // the lists the kernel does not sort
+        for (int64_t k = 0; k < nq; ++k)
+            if (ptr[k + 1] - ptr[k] > HV_Q_LIST) std::sort(idx + ptr[k], idx + ptr[k + 1]);
+    };
+    if (8 * nx + 16 * (size_t)nq + 8 * (size_t)total + 5 * 256 <= HV_QUERY_PINNED) {
+        HvLease L(c->device);
+        if (L.base) {   // as hv_nn_halfspace_impl
+            const double* pq = L.put(q, nx);
+            const double* pr = L.put(radius, (size_t)nq);
+            const int64_t* pp = idx ? L.put(ptr, (size_t)nq + 1) : nullptr;
+            int64_t* po = L.take<int64_t>(idx ? (size_t)total : (size_t)nq);
+            k_inrange<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, pq, pr, pp, idx ? po : nullptr,
+                                                                                 idx ? nullptr : po);
+            HVCK(hipGetLastError());
+            HVCK(hipStreamSynchronize(c->stream));
+            if (idx) {
+                std::memcpy(idx, po, sizeof(int64_t) * total);
+                ordered();
+            } else {
+                for (int64_t k = 0; k < nq; ++k) ptr[k + 1] = ptr[k] + po[k];
+            }
+            return HV_OK;
+        }
+    }
+    double* dq = pget<double>(c, "q_q", nx);
     double* dr = pget<double>(c, "q_r", nq);
     int64_t* dcnt = pget<int64_t>(c, "q_cnt", nq);
     int64_t* dptr = pget<int64_t>(c, "q_ptr", nq + 1);
     if (!dq || !dr || !dcnt || !dptr) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
-    HVCK(hipMemcpyAsync(dq, q, sizeof(double) * nq * D, hipMemcpyHostToDevice, c->stream));
-    HVCK(hipMemcpyAsync(dr, radius, sizeof(double) * nq, hipMemcpyHostToDevice, c->stream));
+    const HvCopy in[3] = {{dq, q, sizeof(double) * nx}, {dr, radius, sizeof(double) * nq},
+                          {dptr, ptr, idx ? sizeof(int64_t) * (nq + 1) : 0}};
+    HVCK(hv_copies(c->device, false, in, 3));
     if (!idx) {
         k_inrange<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, dq, dr, nullptr, nullptr, dcnt);
         HVCK(hipGetLastError());
-        std::vector<int64_t> cnt(nq);
-        HVCK(hipMemcpyAsync(cnt.data(), dcnt, sizeof(int64_t) * nq, hipMemcpyDeviceToHost, c->stream));
         HVCK(hipStreamSynchronize(c->stream));
+        std::vector<int64_t> cnt(nq);
+        const HvCopy res{cnt.data(), dcnt, sizeof(int64_t) * nq};
+        HVCK(hv_copies(c->device, true, &res, 1));
         for (int64_t k = 0; k < nq; ++k) ptr[k + 1] = ptr[k] + cnt[k];
         return HV_OK;
     }
-    const int64_t total = ptr[nq];
     int64_t* dout = pget<int64_t>(c, "q_out", std::max<int64_t>(total, 1));
     if (!dout) return hv_fail(c, HV_ERR_DEVICE, "out of device memory");
-    HVCK(hipMemcpyAsync(dptr, ptr, sizeof(int64_t) * (nq + 1), hipMemcpyHostToDevice, c->stream));
     k_inrange<D><<<nblk(nq, HV_Q_WAVES), 64 * HV_Q_WAVES, 0, c->stream>>>(T.g, (int)nq, dq, dr, dptr, dout, nullptr);
     HVCK(hipGetLastError());
-    if (total) HVCK(hipMemcpyAsync(idx, dout, sizeof(int64_t) * total, hipMemcpyDeviceToHost, c->stream));
     HVCK(hipStreamSynchronize(c->stream));
-    for (int64_t k = 0; k < nq; ++k)
-        if (ptr[k + 1] - ptr[k] > HV_Q_LIST) std::sort(idx + ptr[k], idx + ptr[k + 1]);
+    const HvCopy res{idx, dout, sizeof(int64_t) * total};
+    HVCK(hv_copies(c->device, true, &res, 1));
+    ordered();
     return HV_OK;
 }
 
