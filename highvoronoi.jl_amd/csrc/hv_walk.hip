@@ -4960,80 +4960,129 @@ __global__ __launch_bounds__(256) void k_rays_in(int n, const int64_t* __restric
     (void)rho;
 }
 
-// Queries: one wavefront per query walks the 8-ary tree depth-first, nearest children first.  Eight
-// lanes test a node's child boxes, two leaves of 32 points are measured at once, a point per lane.
-// The boxes are rounded outward and tested in FP64 with the points' own chain of operations, so a
-// box's distance (and its largest <u, x>) bounds those of its points as computed, not only in
-// exact arithmetic: what is skipped could not have changed the result.  Latency is what bounds a
-// query, and a wavefront per query gives small batches a chip's worth of them: 3D N=100k, 1 000
-// half-space queries 18.6 -> 0.09 ms against a thread per query in heap order.
-constexpr int HV_Q_WAVES = 4;    // wavefronts per workgroup, one query each
-constexpr int HV_Q_STACK = 96;   // at most 7 waiting nodes per level (at most 9 levels), 8 on top
-constexpr int HV_Q_LIST = 512;   // hits of one query sorted in LDS (k_inrange)
+// Queries: one wavefront per query walks the 8-ary tree depth-first, nearest children first.  The
+// lanes test the child boxes of up to eight waiting nodes of one level at once, then two leaves of 32
+// points, a point per lane, the next two loaded meanwhile.  The boxes are rounded outward and tested
+// in FP64 with the points' own chain of operations, so a box's distance (and its largest <u, x>)
+// bounds those of its points as computed, not only in exact arithmetic: what is skipped could not have
+// changed the result.  Latency is what bounds a query, and a wavefront per query gives small batches a
+// chip's worth of them: 3D N=100k, 1 000 half-space queries 18.6 -> 0.08 ms
+// against a thread per query in heap order, 0.055 ms with eight nodes at a time instead of one.
+constexpr int HV_Q_WAVES = 4;     // wavefronts per workgroup, one query each
+constexpr int HV_Q_STACK = 576;   // nodes of one level at a time on top: at most 64 per level, 9 levels
+constexpr int HV_Q_LIST = 512;    // hits of one query sorted in LDS (k_inrange)
 
 struct HvQueryStack {
     int node[HV_Q_STACK];      // level << 27 | node id
-    double d2[HV_Q_STACK];
-    int child[8];              // a last-level node's leaves, nearest first
-    double cd2[8];
+    float d2[HV_Q_STACK];      // rounded down
 };
 
 // reach(lo, hi, d2): whether the box may hold a wanted point, and its distance^2; limit(): the
-// current bound on the distance^2; leaf(j): every lane with its point (-1: none)
-template <int D, typename Reach, typename Limit, typename Leaf>
+// current bound on the distance^2; leaf(j, x): every lane with its point (j -1: none).  NEAR: the
+// bound shrinks, leaves are taken nearest first.
+template <int D, bool NEAR, typename Reach, typename Limit, typename Leaf>
 __device__ __forceinline__ void hv_query_walk(const DevGeo& g, HvQueryStack& S, Reach reach, Limit limit, Leaf leaf) {
-    const int lane = threadIdx.x & 63, c = lane & 7;
+    const int lane = threadIdx.x & 63, c = lane & 7, grp = lane >> 3;
     int sp = 1;
     if (lane == 0) {
         S.node[0] = 0;
-        S.d2[0] = 0.0;
+        S.d2[0] = 0.f;
     }
     hv_wave_sync();
     while (sp > 0) {
-        --sp;
-        const int e = __builtin_amdgcn_readfirstlane(S.node[sp]);
-        const double nd2 = S.d2[sp];
-        if (!(nd2 <= limit())) continue;
-        const int l = e >> 27, gid = e & ((1 << 27) - 1);
-        const float* box = g.cb + ((int64_t)gid * 8 + c) * (2 * D);
-        double lo[D], hi[D], d2 = 0.0;
+        // the topmost nodes of one level (a level's nodes are adjacent), eight lanes each
+        const int l = __builtin_amdgcn_readfirstlane(S.node[sp - 1]) >> 27;
+        const int mine = sp - 1 - grp;
+        const int e = mine >= 0 ? S.node[mine] : -1;
+        const bool have = mine >= 0 && (e >> 27) == l;
+        const int gid = e & ((1 << 27) - 1);
+        bool ok = have && (double)S.d2[max(mine, 0)] <= limit();
+        double d2 = 0.0;
+        if (ok) {
+            const float* box = g.cb + ((int64_t)gid * 8 + c) * (2 * D);
+            double lo[D], hi[D];
 #pragma unroll
-        for (int k = 0; k < D; ++k) {
-            lo[k] = (double)box[k];
-            hi[k] = (double)box[D + k];
+            for (int k = 0; k < D; ++k) {
+                lo[k] = (double)box[k];
+                hi[k] = (double)box[D + k];
+            }
+            const bool empty = box[0] == 1e30f && box[D] == 1e30f;
+            ok = !empty && reach(lo, hi, d2);
         }
-        const bool empty = box[0] == 1e30f && box[D] == 1e30f;
-        const bool ok = lane < 8 && !empty && reach(lo, hi, d2);
-        const unsigned m = (unsigned)(__ballot(ok) & 0xffull);
-        if (m == 0u) continue;
-        const int nv = __popc(m);
-        int rk = 0;   // rank among the reached children
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const double dq = __shfl(d2, q);
-            rk += (((m >> q) & 1u) && (dq < d2 || (dq == d2 && q < c))) ? 1 : 0;
-        }
+        sp -= __popcll(__ballot(have)) >> 3;
+        unsigned long long m = __ballot(ok);
+        hv_wave_sync();   // the popped entries are read before they are written over
+        if (m == 0ull) continue;
         const int first = l == 0 ? 0 : ((1 << (3 * l)) - 1) / 7;   // first node id of the level
-        hv_wave_sync();
-        if (l + 1 == g.h) {
+        const int child = 8 * (gid - first) + c;                   // index in its level
+        if (l + 1 < g.h) {
+            // the nearest child of the topmost node on top
+            const unsigned fam = (unsigned)(m >> (8 * grp)) & 0xffu;
+            int rk = 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const double dq = __shfl(d2, 8 * grp + q);
+                rk += (((fam >> q) & 1u) && (dq < d2 || (dq == d2 && q < c))) ? 1 : 0;
+            }
             if (ok) {
-                S.child[rk] = 8 * (gid - first) + c;
-                S.cd2[rk] = d2;
+                const unsigned long long under = grp < 7 ? m >> (8 * (grp + 1)) : 0ull;
+                const int at = sp + __popcll(under) + __popc(fam) - 1 - rk;
+                S.node[at] = ((l + 1) << 27) | (first + (1 << (3 * l)) + child);
+                S.d2[at] = __double2float_rd(d2);
             }
+            sp += __popcll(m);
             hv_wave_sync();
-            for (int q = 0; q < nv; q += 2) {
-                if (!(S.cd2[q] <= limit())) break;
-                const int half = lane >> 5;
-                const int j = (q + half < nv) ? S.child[q + half] * 32 + (lane & 31) : g.n;
-                leaf(j < g.n ? j : -1);
+            continue;
+        }
+        // the next two leaves: by distance (NEAR; the lane number in the low bits of the key), or as they come
+        auto next = [&]() -> int {   // a lane's point of them
+            int c0, c1;
+            if constexpr (NEAR) {
+                m &= __ballot(d2 <= limit());
+                if (m == 0ull) return -1;
+                uint32_t k0 = (m >> lane) & 1ull ? (__float_as_uint((float)d2) & ~63u) | (uint32_t)lane : 0xffffffffu, k1 = 0xffffffffu;
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) {
+                    const uint32_t a = __shfl_xor(k0, off), b = __shfl_xor(k1, off);
+                    k1 = min(max(k0, a), min(k1, b));
+                    k0 = min(k0, a);
+                }
+                c0 = (int)(__builtin_amdgcn_readfirstlane(k0) & 63u);
+                const uint32_t s1 = __builtin_amdgcn_readfirstlane(k1);
+                c1 = s1 == 0xffffffffu ? -1 : (int)(s1 & 63u);
+                m &= ~(1ull << c0);
+                if (c1 >= 0) m &= ~(1ull << c1);
+            } else {
+                c0 = __builtin_ctzll(m);
+                m &= m - 1ull;
+                c1 = m ? (int)__builtin_ctzll(m) : -1;
+                m &= m - 1ull;   // 0 stays 0
             }
-        } else {
-            if (ok) {   // the nearest on top
-                const int at = sp + nv - 1 - rk;
-                S.node[at] = ((l + 1) << 27) | (first + (1 << (3 * l)) + 8 * (gid - first) + c);
-                S.d2[at] = d2;
+            const int l0 = __builtin_amdgcn_readlane(child, c0), l1 = c1 < 0 ? -1 : __builtin_amdgcn_readlane(child, c1);
+            const int lf = lane < 32 ? l0 : l1;
+            const int j = lf < 0 || lf >= g.nleaf ? -1 : lf * 32 + (lane & 31);
+            return j < g.n ? j : -1;
+        };
+        double x[D];
+        auto load = [&](int j) {
+            if (j >= 0) {
+#pragma unroll
+                for (int k = 0; k < D; ++k) x[k] = g.xs[(int64_t)j * (D + 1) + k];
             }
-            sp += nv;
+        };
+        int j = next();
+        load(j);
+        while (__ballot(j >= 0)) {
+            const int jc = j;
+            double xc[D];
+#pragma unroll
+            for (int k = 0; k < D; ++k) xc[k] = x[k];
+            j = -1;
+            if (m) {
+                j = next();
+                load(j);
+            }
+            leaf(jc, xc);
         }
         hv_wave_sync();
     }
@@ -5055,7 +5104,7 @@ __global__ __launch_bounds__(64 * HV_Q_WAVES) void k_nn_halfspace(DevGeo g, int 
     double bound = INFINITY;   // of the whole wavefront
     double best = INFINITY;    // of this lane's points
     int bi = -1;
-    hv_query_walk<D>(
+    hv_query_walk<D, true>(
         g, stk[wv],
         [&](const double* lo, const double* hi, double& d2) {
             double um = 0.0;
@@ -5068,13 +5117,13 @@ __global__ __launch_bounds__(64 * HV_Q_WAVES) void k_nn_halfspace(DevGeo g, int 
             return d2 <= bound && um > c;
         },
         [&]() { return bound; },
-        [&](int j) {
+        [&](int j, const double* x) {
             bool better = false;
             if (j >= 0) {
                 double d2 = 0.0, ux = 0.0;
 #pragma unroll
                 for (int k = 0; k < D; ++k) {
-                    const double xk = g.xs[(int64_t)j * (D + 1) + k];
+                    const double xk = x[k];
                     const double a = xk - p[k];
                     d2 = fma(a, a, d2);
                     ux = fma(uu[k], xk, ux);
@@ -5124,7 +5173,7 @@ __global__ __launch_bounds__(64 * HV_Q_WAVES) void k_inrange(DevGeo g, int nq, c
     const int64_t room = out ? ptr[t + 1] - ptr[t] : 0;
     const bool in_lds = room <= HV_Q_LIST;
     int64_t cnt = 0;
-    hv_query_walk<D>(
+    hv_query_walk<D, false>(
         g, stk[wv],
         [&](const double* lo, const double* hi, double& d2) {
 #pragma unroll
@@ -5135,13 +5184,13 @@ __global__ __launch_bounds__(64 * HV_Q_WAVES) void k_inrange(DevGeo g, int nq, c
             return d2 <= r2;
         },
         [&]() { return r2; },
-        [&](int j) {
+        [&](int j, const double* x) {
             bool hit = false;
             if (j >= 0) {
                 double d2 = 0.0;
 #pragma unroll
                 for (int k = 0; k < D; ++k) {
-                    const double a = g.xs[(int64_t)j * (D + 1) + k] - p[k];
+                    const double a = x[k] - p[k];
                     d2 = fma(a, a, d2);
                 }
                 hit = d2 <= r2;
