@@ -6249,13 +6249,65 @@ int hv_mc_points_impl(hv_ctx* c, int64_t nsamples, uint64_t seed, double slab, c
 // vertex a neighbour of the new cell, so the tested set is the same).  Every other vertex of
 // the refined mesh holds a new point and comes from the walk of the new cells.
 
-// keep[t] = 1 when vertex ids[t] of the old mesh has no new point (sorted position j with
-// sidx[j] >= nold) strictly inside its circumsphere shrunk by 1 + 1e-7
+// The new points in tree order (list: their sorted positions), boxes of each 32 of them and of each
+// 1 024: a vertex tests only boxes of new points.  In the tree of the union nearly every leaf that a
+// circumsphere reaches holds old points alone (3D N=50k with 500 new points: the refinement took 1.0 of
+// its 5.2 ms longer there).
+constexpr int HV_NEW_BOX = 32, HV_NEW_SUPER = 1024;
+struct HvNewSelect {   // positions of new points
+    const int* sidx;
+    int nold;
+    __device__ bool operator()(int j) const { return sidx[j] >= nold; }
+};
+// One workgroup per super box, a thread per point: rows of D coordinates, boxes lo then hi.
 template <int D>
-__global__ __launch_bounds__(128) void k_refine_keep(DevGeo g, int nv, const int* __restrict__ ids,
+__global__ __launch_bounds__(HV_NEW_SUPER) void k_new_boxes(DevGeo g, const int* __restrict__ list, int m, double* __restrict__ x,
+                                                            double* __restrict__ box, double* __restrict__ sup) {
+    __shared__ double slo[HV_NEW_SUPER / HV_NEW_BOX][D], shi[HV_NEW_SUPER / HV_NEW_BOX][D];
+    const int i = blockIdx.x * HV_NEW_SUPER + threadIdx.x, b = threadIdx.x / HV_NEW_BOX;
+    double lo[D], hi[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        double v = 0.0;
+        if (i < m) {
+            v = g.xs[(int64_t)list[i] * (D + 1) + k];
+            x[(int64_t)i * D + k] = v;
+        }
+        lo[k] = i < m ? v : 1e300;
+        hi[k] = i < m ? v : -1e300;
+#pragma unroll
+        for (int off = HV_NEW_BOX / 2; off > 0; off >>= 1) {
+            lo[k] = fmin(lo[k], __shfl_xor(lo[k], off));
+            hi[k] = fmax(hi[k], __shfl_xor(hi[k], off));
+        }
+        if (threadIdx.x % HV_NEW_BOX == 0) {
+            slo[b][k] = lo[k];
+            shi[b][k] = hi[k];
+            if (i < m) {
+                box[((int64_t)(i / HV_NEW_BOX) * 2) * D + k] = lo[k];
+                box[((int64_t)(i / HV_NEW_BOX) * 2 + 1) * D + k] = hi[k];
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < D) {
+        double a = 1e300, c = -1e300;
+        for (int q = 0; q < HV_NEW_SUPER / HV_NEW_BOX; ++q) {
+            a = fmin(a, slo[q][threadIdx.x]);
+            c = fmax(c, shi[q][threadIdx.x]);
+        }
+        sup[((int64_t)blockIdx.x * 2) * D + threadIdx.x] = a;
+        sup[((int64_t)blockIdx.x * 2 + 1) * D + threadIdx.x] = c;
+    }
+}
+
+// keep[t] = 1 when vertex ids[t] of the old mesh has none of the m new points strictly inside its
+// circumsphere shrunk by 1 + 1e-7
+template <int D>
+__global__ __launch_bounds__(256) void k_refine_keep(int m, const double* __restrict__ x, const double* __restrict__ box,
+                                                     const double* __restrict__ sup, int nv, const int* __restrict__ ids,
                                                      const int* __restrict__ vkey, const double* __restrict__ vx,
-                                                     const double* __restrict__ xo, int nold,
-                                                     uint8_t* __restrict__ keep) {
+                                                     const double* __restrict__ xo, uint8_t* __restrict__ keep) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nv) return;
     const int64_t v = ids[t];
@@ -6269,25 +6321,32 @@ __global__ __launch_bounds__(128) void k_refine_keep(DevGeo g, int nv, const int
     }
     const double f = 1.0 + 1e-7;
     const double lim = R2 / (f * f);
+    auto reached = [&](const double* b) {
+        double d2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            const double a = fmax(fmax(b[k] - r[k], r[k] - b[D + k]), 0.0);
+            d2 = fma(a, a, d2);
+        }
+        return d2 < lim;
+    };
     bool hit = false;
-    int node = 1;
-    while (node && !hit) {
-        if (hv_box_d2<D>(g, node, r) < lim) {
-            if (node < g.P2) { node = 2 * node; continue; }
-            const int leaf = node - g.P2;
-            const int j0 = leaf * g.L, j1 = min(j0 + g.L, g.n);
-            for (int j = j0; j < j1; ++j) {
-                if (g.sidx[j] < nold) continue;
+    for (int s = 0; s * HV_NEW_SUPER < m && !hit; ++s) {
+        if (!reached(sup + (int64_t)s * 2 * D)) continue;
+        const int b1 = min((s + 1) * (HV_NEW_SUPER / HV_NEW_BOX), (m + HV_NEW_BOX - 1) / HV_NEW_BOX);
+        for (int b = s * (HV_NEW_SUPER / HV_NEW_BOX); b < b1 && !hit; ++b) {
+            if (!reached(box + (int64_t)b * 2 * D)) continue;
+            const int i1 = min((b + 1) * HV_NEW_BOX, m);
+            for (int i = b * HV_NEW_BOX; i < i1; ++i) {
                 double d2 = 0.0;
 #pragma unroll
                 for (int k = 0; k < D; ++k) {
-                    const double a = g.xs[(int64_t)j * (D + 1) + k] - r[k];
+                    const double a = x[(int64_t)i * D + k] - r[k];
                     d2 = fma(a, a, d2);
                 }
                 if (d2 < lim) { hit = true; break; }
             }
         }
-        node = hv_next_node(node);
     }
     keep[t] = hit ? 0 : 1;
 }
@@ -6329,9 +6388,26 @@ int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** o
     if (!keep || !sel || !dcnt) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
     int nkeep = 0;
     if (nv0 > 0) {
-        k_refine_keep<D><<<nblk(nv0, 128), 128, 0, c->stream>>>(T.g, nv0, (const int*)old->ids.p, (const int*)old->key.p,
-                                                               (const double*)old->x.p, (const double*)c->xw->p, nold,
-                                                               keep);
+        const int m = shift, nsup = (m + HV_NEW_SUPER - 1) / HV_NEW_SUPER;
+        int* list = pget<int>(c, "rf_list", (size_t)std::max(m, 1));
+        double* nx = pget<double>(c, "rf_x", (size_t)std::max(m, 1) * D);
+        double* nbox = pget<double>(c, "rf_box", (size_t)std::max(nsup, 1) * (HV_NEW_SUPER / HV_NEW_BOX) * 2 * D);
+        double* nsupb = pget<double>(c, "rf_sup", (size_t)std::max(nsup, 1) * 2 * D);
+        if (!list || !nx || !nbox || !nsupb) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
+        if (m > 0) {
+            size_t ts = 0;
+            hipcub::CountingInputIterator<int> it(0);
+            const HvNewSelect isnew{T.g.sidx, nold};
+            HVCK(hipcub::DeviceSelect::If(nullptr, ts, it, list, dcnt, (int)c->N, isnew, c->stream));
+            void* tmp = c->pool->get("cubtmp2", ts, false, c->stream);
+            if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
+            HVCK(hipcub::DeviceSelect::If(tmp, ts, it, list, dcnt, (int)c->N, isnew, c->stream));
+            k_new_boxes<D><<<nsup, HV_NEW_SUPER, 0, c->stream>>>(T.g, list, m, nx, nbox, nsupb);
+            HVCK(hipGetLastError());
+        }
+        k_refine_keep<D><<<nblk(nv0, 256), 256, 0, c->stream>>>(m, nx, nbox, nsupb, nv0, (const int*)old->ids.p,
+                                                               (const int*)old->key.p, (const double*)old->x.p,
+                                                               (const double*)c->xw->p, keep);
         HVCK(hipGetLastError());
         size_t tb = 0;
         HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb, (const int*)old->ids.p, keep, sel, dcnt, nv0, c->stream));
