@@ -753,12 +753,86 @@ __device__ __forceinline__ double hv_unif(uint64_t seed, uint64_t s) {
 
 constexpr int HV_MC_MAXK = 512;
 
+// One workgroup per cell, its neighbours in LDS as w = e - x (e the neighbour or its mirror image) and
+// 1 / |w|^2.  A direction u ends at the neighbour of least t = |w|^2 / (2 <u, w>), that is of the largest
+// <u, w> / |w|^2: a product and a comparison per neighbour where the quotient took 45 FP64 instructions,
+// and t is formed once, for that neighbour.  A thread sweeps up to four directions together, so a
+// row is read once for them.  Bound by the FP64 sweep and the directions' logarithms and sines; 4D
+// N=20k, 1 000 directions a cell: 1.28 -> 0.61 ms.
+template <int D, int NQ>
+__device__ __forceinline__ double hv_mc_sweep(const double (*row)[D + 1], int K, double* acc, uint64_t first, int64_t q0, int64_t step,
+                                              int64_t ndir, uint64_t seed) {
+    constexpr int DP = (D + 1) & ~1;
+    double u[NQ][D], best[NQ];
+    int win[NQ];
+#pragma unroll
+    for (int z = 0; z < NQ; ++z) {
+        const uint64_t base = (first + (uint64_t)(q0 + z * step)) * (uint64_t)DP;
+        double uu = 0.0;
+#pragma unroll
+        for (int c = 0; c < D; c += 2) {
+            const uint64_t p = (base + c) >> 1;
+            const double u1 = fmax(hv_unif(seed, 2 * p), 1e-300), u2 = hv_unif(seed, 2 * p + 1);
+            const double rad = sqrt(-2.0 * log(u1));
+            double sn, cs;
+            sincos(2.0 * M_PI * u2, &sn, &cs);
+            u[z][c] = rad * cs;
+            if (c + 1 < D) u[z][c + 1] = rad * sn;
+        }
+#pragma unroll
+        for (int c = 0; c < D; ++c) uu = fma(u[z][c], u[z][c], uu);
+        uu = sqrt(uu);
+#pragma unroll
+        for (int c = 0; c < D; ++c) u[z][c] /= uu;
+        best[z] = 0.0;
+        win[z] = -1;
+    }
+    for (int t = 0; t < K; ++t) {
+        double w[D + 1];
+#pragma unroll
+        for (int c = 0; c <= D; ++c) w[c] = row[t][c];
+#pragma unroll
+        for (int z = 0; z < NQ; ++z) {
+            double den = 0.0;
+#pragma unroll
+            for (int c = 0; c < D; ++c) den = fma(u[z][c], w[c], den);
+            den *= w[D];
+            const bool up = den > best[z];
+            best[z] = up ? den : best[z];
+            win[z] = up ? t : win[z];
+        }
+    }
+    double V = 0.0;
+#pragma unroll
+    for (int z = 0; z < NQ; ++z) {
+        if (q0 + z * step >= ndir) continue;
+        double ts = INFINITY, cn = 0.0;
+        if (win[z] >= 0) {
+            double num = 0.0, den = 0.0;
+#pragma unroll
+            for (int c = 0; c < D; ++c) {
+                const double w = row[win[z]][c];
+                num = fma(w, w, num);
+                den = fma(u[z][c], w, den);
+            }
+            ts = num / (2.0 * den);
+            cn = den / sqrt(num);
+        }
+        double tp = 1.0;
+#pragma unroll
+        for (int c = 0; c < D - 1; ++c) tp *= ts;
+        V += tp * ts;
+        if (win[z] >= 0 && ts < INFINITY) atomicAdd(&acc[win[z]], tp / fabs(cn));
+    }
+    return V;
+}
+
 template <int D>
 __global__ __launch_bounds__(256) void k_mc_cell(IntGeo g, const int64_t* __restrict__ ptr,
                                                  const uint64_t* __restrict__ pkey, int64_t ndir, uint64_t seed,
                                                  double cvol, double carea, double* __restrict__ vol,
                                                  double* __restrict__ area) {
-    __shared__ double ext[HV_MC_MAXK][D], nrm[HV_MC_MAXK][D];
+    __shared__ double row[HV_MC_MAXK][D + 1];
     __shared__ double acc[HV_MC_MAXK];
     __shared__ double vred[256];
     const int i = blockIdx.x;
@@ -784,64 +858,28 @@ __global__ __launch_bounds__(256) void k_mc_cell(IntGeo g, const int64_t* __rest
         }
         double s = 0.0;
 #pragma unroll
-        for (int c = 0; c < D; ++c) s = fma(e[c] - x[c], e[c] - x[c], s);
-        s = sqrt(s);
-#pragma unroll
         for (int c = 0; c < D; ++c) {
-            ext[t][c] = e[c];
-            nrm[t][c] = (e[c] - x[c]) / s;
+            row[t][c] = e[c] - x[c];
+            s = fma(e[c] - x[c], e[c] - x[c], s);
         }
+        row[t][D] = 1.0 / s;
         acc[t] = 0.0;
     }
     __syncthreads();
-    constexpr int DP = (D + 1) & ~1;
     double V = 0.0;
-    for (int64_t q = threadIdx.x; q < ndir; q += blockDim.x) {
-        const uint64_t base = ((uint64_t)i * (uint64_t)ndir + (uint64_t)q) * (uint64_t)DP;
-        double u[D], uu = 0.0;
-#pragma unroll
-        for (int c = 0; c < D; c += 2) {
-            const uint64_t p = (base + c) >> 1;
-            const double u1 = fmax(hv_unif(seed, 2 * p), 1e-300), u2 = hv_unif(seed, 2 * p + 1);
-            const double rad = sqrt(-2.0 * log(u1));
-            double sn, cs;
-            sincos(2.0 * M_PI * u2, &sn, &cs);
-            u[c] = rad * cs;
-            if (c + 1 < D) u[c + 1] = rad * sn;
-        }
-#pragma unroll
-        for (int c = 0; c < D; ++c) uu = fma(u[c], u[c], uu);
-        uu = sqrt(uu);
-        double c0 = 0.0;
-#pragma unroll
-        for (int c = 0; c < D; ++c) {
-            u[c] /= uu;
-            c0 = fma(x[c], u[c], c0);
-        }
-        double ts = INFINITY;
-        int win = -1;
-        for (int t = 0; t < K; ++t) {
-            double eu = 0.0, num = 0.0, den = 0.0;
-#pragma unroll
-            for (int c = 0; c < D; ++c) {
-                const double e = ext[t][c];
-                eu = fma(e, u[c], eu);
-                num = fma(x[c] - e, x[c] - e, num);
-                den = fma(u[c], e - x[c], den);
-            }
-            if (eu <= c0) continue;
-            const double tt = num / (2.0 * den);
-            if (tt > 0.0 && tt < ts) { ts = tt; win = t; }
-        }
-        double tp = 1.0;
-#pragma unroll
-        for (int c = 0; c < D - 1; ++c) tp *= ts;
-        V += tp * ts;
-        if (win >= 0 && ts < INFINITY) {
-            double cn = 0.0;
-#pragma unroll
-            for (int c = 0; c < D; ++c) cn = fma(nrm[win][c], u[c], cn);
-            atomicAdd(&acc[win], tp / fabs(cn));
+    const uint64_t first = (uint64_t)i * (uint64_t)ndir;
+    const int64_t step = blockDim.x;
+    for (int64_t q = 0; q < ndir;) {   // uniform over the workgroup
+        const int64_t q0 = q + threadIdx.x, left = ndir - q;
+        if (left > 2 * step) {
+            V += hv_mc_sweep<D, 4>(row, K, acc, first, q0, step, ndir, seed);
+            q += 4 * step;
+        } else if (left > step) {
+            V += hv_mc_sweep<D, 2>(row, K, acc, first, q0, step, ndir, seed);
+            q += 2 * step;
+        } else {
+            if (q0 < ndir) V += hv_mc_sweep<D, 1>(row, K, acc, first, q0, step, ndir, seed);
+            q += step;
         }
     }
     vred[threadIdx.x] = V;
