@@ -135,50 +135,94 @@ __global__ void k_points_in(const double* __restrict__ xin, int N, DevGeo g, dou
 // xo and rank: this tree's rows (local index); sidx receives global ids (goff + local)
 template <int D>
 __global__ void k_points_sorted(const double* __restrict__ xo, const int* __restrict__ idx, int N, int goff,
-                                double* __restrict__ xs, int* __restrict__ sidx, int* __restrict__ rank) {
+                                double* __restrict__ xs, float* __restrict__ xf, int* __restrict__ sidx,
+                                int* __restrict__ rank) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= N) return;
     int gi = idx[j];
     sidx[j] = goff + gi;
     rank[gi] = j;
     double s = 0.0;
+    float row[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < D; ++k) {
         double v = xo[(int64_t)gi * D + k];
         xs[(int64_t)j * (D + 1) + k] = v;
+        row[k] = (float)v;
         s = fma(v, v, s);
     }
     xs[(int64_t)j * (D + 1) + D] = s;
+    float4* rows = (float4*)(xf + (int64_t)j * 8);
+    rows[0] = make_float4(row[0], row[1], row[2], row[3]);
+    rows[1] = make_float4(row[4], row[5], row[6], row[7]);
 }
 
+// Boxes of the complete binary tree over the leaves (node 1 the root, P2 .. 2 P2 - 1 the leaves):
+// a workgroup takes HV_BOX_ITEMS nodes of the level first .. 2 first - 1 (leaves: from their points,
+// four threads a leaf; else as an earlier launch left them) and forms the eight levels above them in
+// LDS.  A tree takes one to three launches, where a launch a level took five to twenty.
+constexpr int HV_BOX_ITEMS = 256;
 template <int D>
-__global__ void k_leaf_boxes(DevGeo g, double* __restrict__ blo, double* __restrict__ bhi) {
-    int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= g.P2) return;
-    int node = g.P2 + l;
-    int j0 = l * g.L, j1 = min(j0 + g.L, g.n);
+__global__ __launch_bounds__(4 * HV_BOX_ITEMS) void k_tree_boxes(DevGeo g, int first, bool leaves, double* __restrict__ blo,
+                                                                 double* __restrict__ bhi) {
+    __shared__ double slo[D][HV_BOX_ITEMS], shi[D][HV_BOX_ITEMS];
+    const int it = threadIdx.x >> 2, part = threadIdx.x & 3;
+    const int item = blockIdx.x * HV_BOX_ITEMS + it;
+    if (item < first) {
+        const int j0 = item * g.L, j1 = min(j0 + g.L, g.n);
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-        double lo = 1e300, hi = -1e300;
-        for (int j = j0; j < j1; ++j) {
-            double v = g.xs[(int64_t)(j) * (D + 1) + k];
-            lo = fmin(lo, v);
-            hi = fmax(hi, v);
+        for (int k = 0; k < D; ++k) {
+            double lo = 1e300, hi = -1e300;
+            if (leaves) {
+                for (int j = j0 + part; j < j1; j += 4) {
+                    const double v = g.xs[(int64_t)j * (D + 1) + k];
+                    lo = fmin(lo, v);
+                    hi = fmax(hi, v);
+                }
+#pragma unroll
+                for (int off = 1; off < 4; off <<= 1) {
+                    lo = fmin(lo, __shfl_xor(lo, off));
+                    hi = fmax(hi, __shfl_xor(hi, off));
+                }
+                if (part == 0) {
+                    blo[(int64_t)k * g.NN + first + item] = lo;
+                    bhi[(int64_t)k * g.NN + first + item] = hi;
+                }
+            } else if (part == 0) {
+                lo = blo[(int64_t)k * g.NN + first + item];
+                hi = bhi[(int64_t)k * g.NN + first + item];
+            }
+            if (part == 0) {
+                slo[k][it] = lo;
+                shi[k][it] = hi;
+            }
         }
-        blo[(int64_t)k * g.NN + node] = lo;
-        bhi[(int64_t)k * g.NN + node] = hi;
     }
-}
-
-template <int D>
-__global__ void k_node_boxes(int first, int count, int NN, double* __restrict__ blo, double* __restrict__ bhi) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    int node = first + t;
+    __syncthreads();
+    int count = min(HV_BOX_ITEMS, first);   // this workgroup's nodes of the level (powers of two)
+    for (int level = first / 2; count > 1; level /= 2) {
+        count /= 2;
+        double lo[D], hi[D];
+        const int t = threadIdx.x;
+        if (t < count) {
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-        blo[(int64_t)k * NN + node] = fmin(blo[(int64_t)k * NN + 2 * node], blo[(int64_t)k * NN + 2 * node + 1]);
-        bhi[(int64_t)k * NN + node] = fmax(bhi[(int64_t)k * NN + 2 * node], bhi[(int64_t)k * NN + 2 * node + 1]);
+            for (int k = 0; k < D; ++k) {
+                lo[k] = fmin(slo[k][2 * t], slo[k][2 * t + 1]);
+                hi[k] = fmax(shi[k][2 * t], shi[k][2 * t + 1]);
+            }
+        }
+        __syncthreads();
+        if (t < count) {
+            const int node = level + blockIdx.x * count + t;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                slo[k][t] = lo[k];
+                shi[k][t] = hi[k];
+                blo[(int64_t)k * g.NN + node] = lo[k];
+                bhi[(int64_t)k * g.NN + node] = hi[k];
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -187,46 +231,34 @@ __global__ void k_node_boxes(int first, int count, int NN, double* __restrict__ 
 // contiguously, in FP32 rounded outward, so one load per visited node tests 8 children.
 // An empty child is the point box lo = hi = 1e30: its distance^2 overflows to +inf for every
 // query, with the clamp form p - med3(p, lo, hi) as with max(lo - p, p - hi, 0).
+// Child c of node (l, i) covers 8^(h - l - 1) leaves, a node of the binary tree (or more than all of it),
+// so every level comes from the binary boxes in one launch.
 template <int D>
-__global__ void k_tree8_level(DevGeo g, int l, int nodes_at_l, float* __restrict__ cb) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nodes_at_l * 8) return;
-    const int i = t >> 3, c = t & 7;
-    int off = 0, pw = 1;
-    for (int q = 0; q < l; ++q) { off += pw; pw *= 8; }
-    const int gid = off + i;
-    float lo[D], hi[D];
-#pragma unroll
-    for (int k = 0; k < D; ++k) { lo[k] = 1e30f; hi[k] = -1e30f; }
-    const int child = 8 * i + c;
-    if (l + 1 == g.h) {
-        const int j0 = child * g.L, j1 = min(j0 + g.L, g.n);
-#pragma unroll
-        for (int k = 0; k < D; ++k) {
-            double mn = 1e300, mx = -1e300;
-            for (int j = j0; j < j1; ++j) {
-                const double v = g.xs[(int64_t)(j) * (D + 1) + k];
-                mn = fmin(mn, v);
-                mx = fmax(mx, v);
-            }
-            if (j1 > j0) { lo[k] = __double2float_rd(mn); hi[k] = __double2float_ru(mx); }
-        }
-    } else {
-        const int cg = off + pw + child;   // global id of the child node at level l+1
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const float* b = cb + ((int64_t)cg * 8 + q) * (2 * D);
-            if (b[0] == 1e30f && b[D] == 1e30f) continue;   // empty grandchild
-#pragma unroll
-            for (int k = 0; k < D; ++k) { lo[k] = fminf(lo[k], b[k]); hi[k] = fmaxf(hi[k], b[D + k]); }
-        }
+__global__ __launch_bounds__(256) void k_tree8(DevGeo g, int64_t ninternal, float* __restrict__ cb) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ninternal * 8) return;
+    const int gid = (int)(t >> 3), c = (int)(t & 7);
+    int off = 0, pw = 1, l = 0;
+    while (gid >= off + pw) {
+        off += pw;
+        pw *= 8;
+        ++l;
     }
-    const bool empty = !(lo[0] <= hi[0]);
-    float* o = cb + ((int64_t)gid * 8 + c) * (2 * D);
+    const int child = 8 * (gid - off) + c, sh = 3 * (g.h - l - 1);
+    const int nb = sh < 31 ? g.P2 >> sh : 0;   // binary nodes of that size
+    const int node = nb > 0 ? (child < nb ? nb + child : 0) : (child == 0 ? 1 : 0);
+    double lo[D], hi[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-        o[k] = empty ? 1e30f : lo[k];
-        o[D + k] = empty ? 1e30f : hi[k];
+        lo[k] = node ? g.blo[(int64_t)k * g.NN + node] : 1e300;
+        hi[k] = node ? g.bhi[(int64_t)k * g.NN + node] : -1e300;
+    }
+    const bool empty = !(lo[0] <= hi[0]);
+    float* o = cb + t * (2 * D);
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        o[k] = empty ? 1e30f : __double2float_rd(lo[k]);
+        o[D + k] = empty ? 1e30f : __double2float_ru(hi[k]);
     }
 }
 
@@ -333,14 +365,6 @@ __global__ void k_point_kvec(DevGeo g0, GeoSet F, const int* __restrict__ off, c
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) pkv[(int64_t)j * 4 + q] = hv_pack_slots<D>(sl, q);
-}
-
-template <int D>
-__global__ void k_point_rows32(DevGeo g, float* __restrict__ xf) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= g.n) return;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) xf[(int64_t)j * 8 + k] = k < D ? (float)g.xs[(int64_t)j * (D + 1) + k] : 0.f;
 }
 
 template <int D, bool B>
@@ -2861,33 +2885,26 @@ int build_tree_core(hv_ctx* c, int L, int tables, const TreeOut& o, Tree& T, hip
     void* tmp = c->pool->get("cubtmp" + sfx, tmpb, false, st);
     if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
     HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tmpb, code, code2, idx, idx2, N, 0, 64, st));
-    k_points_sorted<D><<<nblk(N, 256), 256, 0, st>>>(xo, idx2, N, o.goff, o.xs, o.sidx, o.rank_base + o.goff);
+    k_points_sorted<D><<<nblk(N, 256), 256, 0, st>>>(xo, idx2, N, o.goff, o.xs, o.xf, o.sidx, o.rank_base + o.goff);
     HVCK(hipGetLastError());
     g.xo = o.xo_base;
     g.xs = o.xs;
     g.sidx = o.sidx;
     g.rank = o.rank_base;
     g.knn = o.knn;
-    k_point_rows32<D><<<nblk(N, 256), 256, 0, st>>>(g, o.xf);
-    HVCK(hipGetLastError());
     g.xf = o.xf;
     g.blo = o.blo;
     g.bhi = o.bhi;
-    k_leaf_boxes<D><<<nblk(g.P2, 256), 256, 0, st>>>(g, o.blo, o.bhi);
-    HVCK(hipGetLastError());
-    for (int first = g.P2 / 2; first >= 1; first /= 2) {
-        k_node_boxes<D><<<nblk(first, 256), 256, 0, st>>>(first, first, g.NN, o.blo, o.bhi);
+    for (int first = g.P2;; first /= HV_BOX_ITEMS) {
+        k_tree_boxes<D><<<nblk(first, HV_BOX_ITEMS), 4 * HV_BOX_ITEMS, 0, st>>>(g, first, first == g.P2, o.blo, o.bhi);
         HVCK(hipGetLastError());
+        if (first <= HV_BOX_ITEMS) break;
     }
-    // 8-ary tree of child boxes (levels bottom-up)
+    // 8-ary tree of child boxes
     g.h = td.h;
     g.cb = o.cb;
-    for (int l = g.h - 1; l >= 0; --l) {
-        int nodes = 1;
-        for (int q = 0; q < l; ++q) nodes *= 8;
-        k_tree8_level<D><<<nblk((int64_t)nodes * 8, 256), 256, 0, st>>>(g, l, nodes, o.cb);
-        HVCK(hipGetLastError());
-    }
+    k_tree8<D><<<nblk(td.ninternal * 8, 256), 256, 0, st>>>(g, td.ninternal, o.cb);
+    HVCK(hipGetLastError());
     if (tables != HV_PREC_FP64 && L != 32) return hv_fail(c, HV_ERR_UNSUPPORTED, "the mixed-precision scans use leaves of 32 points");
     if (tables != HV_PREC_FP64) g.lorg = o.lorg;
     if (tables == HV_PREC_BF16) g.pkv = (const uint32_t*)o.pkv;
@@ -3293,10 +3310,11 @@ __device__ __forceinline__ bool hv_tent_key(const DevGeo& g, const DevRays& R, c
 // generators are dense: a bucket is a run of HV_BUCKET_SUB-ths of the gaps between the generators'
 // codes (mcode, sorted), found for the code of the ray's ball centre.  (A radix sort of every ray's
 // code and the selection of the primaries took 6 to 16 launches instead of 2; buckets by the
-// position of the ray's candidate cost the scan of a 5D N=100k mixture 19.0 -> 22.9 ms.)  Over a
+// position of the ray's candidate cost the scan of a 5D N=100k mixture 19.0 -> 22.9 ms, quarters of
+// the gaps 20.0, sixteenths 18.9.)  Over a
 // forest, whose meshes are small, that position >> shift it is, the buckets of mesh m starting at
 // (goff[m] >> shift) + m so that none holds rays of two meshes.
-constexpr int HV_BUCKET_SUB = 4;
+constexpr int HV_BUCKET_SUB = 16;
 template <int D, bool B>
 __global__ __launch_bounds__(256) void k_tent_group(DevGeo g0, GeoSet F, DevRays R, int nr, int nfresh,
                                                     const int* __restrict__ vkey, int* __restrict__ ttab, uint64_t tmask,
@@ -4075,10 +4093,10 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         ntab = pget<unsigned long long>(c, "ntab", nsize);
         const uint64_t tsz = hpow(2 * (int64_t)nr);
         int* ttab = pget<int>(c, "ttab", tsz);
-        // at most two buckets a ray, and 2^19 (2 MiB of counts)
+        // at most two buckets a ray, and 2^21 (8 MiB of counts)
         const int64_t bpos = B ? (int64_t)N : ((int64_t)N + 1) * HV_BUCKET_SUB;
         int shift = 0;
-        while ((bpos >> shift) + nmesh > std::max<int64_t>(2048, std::min<int64_t>(2 * (int64_t)nr, 1 << 19))) ++shift;
+        while ((bpos >> shift) + nmesh > std::max<int64_t>(2048, std::min<int64_t>(2 * (int64_t)nr, 1 << 21))) ++shift;
         const int nb = (int)(bpos >> shift) + nmesh + 1, nbc = (nb + 4) / 4 * 4;   // one empty bucket at least: its offset is the total
         int* bcnt = pget<int>(c, "bk_cnt", (size_t)nbc);
         int* boff = pget<int>(c, "bk_off", (size_t)nb + 1);
