@@ -778,18 +778,16 @@ static int refine_periodic(hv_ctx* c, const hv_opts* o, const hv_mesh* old, int6
     const int D = old->D;
     const int64_t n = old->nreal, nu = n + m;
     if (nu >= (1ll << 30)) return hv_fail(c, HV_ERR_UNSUPPORTED, "too many generators for 32-bit keys");
-    double* u = nullptr;
-    if (hipMalloc(&u, sizeof(double) * D * nu) != hipSuccess) {
-        (void)hipGetLastError();
-        return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
-    }
+    HvScratch buf(c->device, sizeof(double) * D * nu);
+    double* u = (double*)buf.p;
+    if (!u) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
     int rc = HV_OK;
     // the originals lead the mesh's working set
     if (hipMemcpyAsync(u, old->xw->p, sizeof(double) * D * n, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
         hipMemcpyAsync(u + D * n, xs_new, sizeof(double) * D * m, hipMemcpyHostToDevice, c->stream) != hipSuccess)
         rc = hv_fail(c, HV_ERR_DEVICE, "copy of the points failed");
     if (!rc) rc = set_points_common(c, D, nu, u, hipMemcpyDeviceToDevice);
-    (void)hipFree(u);
+    (void)hipStreamSynchronize(c->stream);   // before the buffer is another's
     if (rc) return rc;
     rc = hv_set_boundary(c, old->P, old->P ? old->pbase.data() : nullptr, old->P ? old->pnormal.data() : nullptr,
                          old->pbc.empty() ? nullptr : old->pbc.data());
@@ -832,17 +830,15 @@ int hv_refine_mesh(hv_ctx* c, const hv_opts* o, const hv_mesh* old, int64_t m, c
     if (nu >= (1ll << 30)) return hv_fail(c, HV_ERR_UNSUPPORTED, "too many generators for 32-bit keys");
     (void)hipSetDevice(c->device);
     // the union in device memory: the mesh's generators, then the new points
-    double* u = nullptr;
-    if (hipMalloc(&u, sizeof(double) * D * nu) != hipSuccess) {
-        (void)hipGetLastError();
-        return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
-    }
+    HvScratch buf(c->device, sizeof(double) * D * nu);
+    double* u = (double*)buf.p;
+    if (!u) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
     int rc = HV_OK;
     if (hipMemcpyAsync(u, old->xw->p, sizeof(double) * D * n, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
         hipMemcpyAsync(u + D * n, xs_new, sizeof(double) * D * m, hipMemcpyHostToDevice, c->stream) != hipSuccess)
         rc = hv_fail(c, HV_ERR_DEVICE, "copy of the points failed");
     if (!rc) rc = set_points_common(c, D, nu, u, hipMemcpyDeviceToDevice);
-    (void)hipFree(u);
+    (void)hipStreamSynchronize(c->stream);   // before the buffer is another's
     if (rc) return rc;
     rc = hv_set_boundary(c, old->P, old->P ? old->pbase.data() : nullptr, old->P ? old->pnormal.data() : nullptr,
                          old->pbc.empty() ? nullptr : old->pbc.data());

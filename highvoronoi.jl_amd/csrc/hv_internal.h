@@ -194,7 +194,7 @@ struct hv_mesh {
     std::shared_ptr<const std::vector<int>> cells;
     // meshes of one batched walk share one allocation for their vertex tables (key, x, ids
     // point into it); null when the mesh owns its tables
-    std::shared_ptr<DevArr> store;
+    std::shared_ptr<HvScratch> store;
 };
 
 // Meshes of one dimension walked together (hv_build_mesh_batch): inputs, the forest of their

@@ -4383,14 +4383,8 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         }
         const size_t kb = ((size_t)nlive * (D + 1) * sizeof(int) + 255) / 256 * 256;
         const size_t xb = ((size_t)nlive * D * sizeof(double) + 255) / 256 * 256;
-        auto store = std::make_shared<DevArr>();
-        store->device = c->device;
-        if (hipMalloc(&store->p, kb + xb + sizeof(int) * (size_t)maxc) != hipSuccess) {
-            (void)hipGetLastError();
-            store->p = nullptr;
-            return hv_fail(c, HV_ERR_DEVICE, "out of device memory (batch meshes)");
-        }
-        store->n = kb + xb + sizeof(int) * (size_t)maxc;
+        auto store = std::make_shared<HvScratch>(c->device, kb + xb + sizeof(int) * (size_t)maxc);
+        if (!store->p) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (batch meshes)");
         int* okey = (int*)store->p;
         double* ox = (double*)((char*)store->p + kb);
         int* oid = (int*)((char*)store->p + kb + xb);
@@ -6446,14 +6440,15 @@ int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** o
     M->key.n = nk * (D + 1) * sizeof(int);
     M->x.n = nk * D * sizeof(double);
     M->ids.n = nk * sizeof(int);
-    if (hipMalloc(&M->key.p, M->key.n) != hipSuccess || hipMalloc(&M->x.p, M->x.n) != hipSuccess ||
-        hipMalloc(&M->ids.p, M->ids.n) != hipSuccess) {
-        for (DBuf* b : {&M->key, &M->x, &M->ids})
-            if (b->p) (void)hipFree(b->p);
+    const size_t ob = (M->x.n + 255) / 256 * 256, kb = (M->key.n + 255) / 256 * 256;
+    M->store = std::make_shared<HvScratch>(c->device, ob + kb + M->ids.n);
+    if (!M->store->p) {
         delete M;
-        (void)hipGetLastError();
         return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refined mesh)");
     }
+    M->x.p = M->store->p;
+    M->key.p = (char*)M->store->p + ob;
+    M->ids.p = (char*)M->store->p + ob + kb;
     if (nkeep > 0)
         k_refine_copy<D><<<nblk(nkeep, 256), 256, 0, c->stream>>>(nkeep, sel, (const int*)old->key.p,
                                                                   (const double*)old->x.p, nold, shift, 0,

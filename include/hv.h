@@ -219,9 +219,9 @@ int hv_build_mesh_batch(int device_ordinal, int32_t nmesh, const int32_t* d, con
 
 /* No counterpart in the reference: frees the contexts (streams and kept device tables) that
  * hv_build_mesh_batch's fused walks keep on the device between calls (device_ordinal < 0: on
- * every device) and the exports' and integrals' buffers kept between calls (at most 1 GiB
- * per device), for
- * callers that need the memory back.  Meshes already built stay valid; the
+ * every device), the buffers of exports, integrals, batches' and refined meshes kept after
+ * their owners (at most 1 GiB per device) and the streams and tables kept of destroyed contexts
+ * (at most four, of at most 256 MiB each, per device), for callers that need the memory back.  Meshes already built stay valid; the
  * next batch call creates its contexts again.  Waits for a batch call running meanwhile. */
 int hv_batch_release(int device_ordinal);
 
