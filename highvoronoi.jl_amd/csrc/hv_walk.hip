@@ -136,12 +136,13 @@ __global__ void k_points_in(const double* __restrict__ xin, int N, DevGeo g, dou
 template <int D>
 __global__ void k_points_sorted(const double* __restrict__ xo, const int* __restrict__ idx, int N, int goff,
                                 double* __restrict__ xs, float* __restrict__ xf, int* __restrict__ sidx,
-                                int* __restrict__ rank) {
+                                int* __restrict__ rank, const uint64_t* __restrict__ code, uint64_t* __restrict__ mcode) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= N) return;
     int gi = idx[j];
     sidx[j] = goff + gi;
     rank[gi] = j;
+    if (mcode) mcode[j] = code[j];
     double s = 0.0;
     float row[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -2799,6 +2800,7 @@ struct TreeOut {
     hv_u32x4* pkv = nullptr;
     float* pxf = nullptr;
     int* bad = nullptr;            // points outside the planes are counted here
+    uint64_t* mcode = nullptr;     // (forest) this tree's sorted Morton codes are kept here
     bool planes_ready = false;     // pn / ph already hold the planes
     const double* dom_lo = nullptr;    // a general polytope's bounding box (null: axis planes)
     const double* dom_hi = nullptr;
@@ -2916,7 +2918,7 @@ int build_tree_core(hv_ctx* c, int L, int tables, const TreeOut& o, Tree& T, hip
     void* tmp = c->pool->get("cubtmp" + sfx, tmpb, false, st);
     if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
     HVCK(hipcub::DeviceRadixSort::SortPairs(tmp, tmpb, code, code2, idx, idx2, N, 0, 64, st));
-    k_points_sorted<D><<<nblk(N, 256), 256, 0, st>>>(xo, idx2, N, o.goff, o.xs, o.xf, o.sidx, o.rank_base + o.goff);
+    k_points_sorted<D><<<nblk(N, 256), 256, 0, st>>>(xo, idx2, N, o.goff, o.xs, o.xf, o.sidx, o.rank_base + o.goff, code2, o.mcode);
     HVCK(hipGetLastError());
     g.xo = o.xo_base;
     g.xs = o.xs;
@@ -3343,15 +3345,15 @@ __device__ __forceinline__ bool hv_tent_key(const DevGeo& g, const DevRays& R, c
 // code and the selection of the primaries took 6 to 16 launches instead of 2; buckets by the
 // position of the ray's candidate cost the scan of a 5D N=100k mixture 19.0 -> 22.9 ms, quarters of
 // the gaps 20.0, sixteenths 18.9.)  Over a
-// forest, whose meshes are small, that position >> shift it is, the buckets of mesh m starting at
-// (goff[m] >> shift) + m so that none holds rays of two meshes.
+// forest the gaps of mesh m start at (goff[m] + m) HV_BUCKET_SUB and its buckets at that >> shift, plus
+// m, so that no bucket holds rays of two meshes.
 constexpr int HV_BUCKET_SUB = 16;
 template <int D, bool B>
 __global__ __launch_bounds__(256) void k_tent_group(DevGeo g0, GeoSet F, DevRays R, int nr, int nfresh,
                                                     const int* __restrict__ vkey, int* __restrict__ ttab, uint64_t tmask,
                                                     uint64_t* __restrict__ at, int* __restrict__ bcnt, int shift,
                                                     const int* __restrict__ goff, const uint64_t* __restrict__ mcode) {
-    // at holds the rays' codes on entry (one tree)
+    // at holds the rays' codes on entry
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nr) return;
     const int gen0 = vkey[(int64_t)R.v[t] * (D + 1)];   // a generator: planes sort last
@@ -3381,25 +3383,25 @@ __global__ __launch_bounds__(256) void k_tent_group(DevGeo g0, GeoSet F, DevRays
         at[t] = ~0ull;
         return;
     }
-    int b;
-    if constexpr (B) {
-        const int i1 = R.i1[t], m = F.mof[gen0];
-        b = ((i1 >= 0 && i1 < g.N ? i1 : g.rank[gen0]) >> shift) + (goff[m] >> shift) + m;
-    } else {
-        const uint64_t code = at[t];
-        int lo = 0, hi = g.n;   // generators with a smaller code
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (mcode[mid] < code) lo = mid + 1;
-            else hi = mid;
-        }
-        int q = 0;
-        if (lo > 0 && lo < g.n) {   // mcode[lo - 1] < code <= mcode[lo]
-            const float f = (float)(code - mcode[lo - 1]) / (float)(mcode[lo] - mcode[lo - 1]);
-            q = min(HV_BUCKET_SUB - 1, (int)(f * HV_BUCKET_SUB));
-        }
-        b = (int)(((int64_t)lo * HV_BUCKET_SUB + q) >> shift);
+    // over a forest a ray's code holds the mesh above the top 32 of its 60 bits
+    constexpr int DOWN = B ? HV_RAY_SORT_LO : 0;
+    const uint64_t code = B ? (at[t] & 0xffffffffull) : at[t];
+    const int m = B ? F.mof[gen0] : 0;
+    const uint64_t* mc = B ? mcode + goff[m] : mcode;
+    int lo = 0, hi = g.n;   // generators with a smaller code
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if ((mc[mid] >> DOWN) < code) lo = mid + 1;
+        else hi = mid;
     }
+    int q = 0;
+    if (lo > 0 && lo < g.n) {   // code of lo - 1 < code <= code of lo
+        const uint64_t c0 = mc[lo - 1] >> DOWN;
+        const float f = (float)(code - c0) / (float)((mc[lo] >> DOWN) - c0);
+        q = min(HV_BUCKET_SUB - 1, (int)(f * HV_BUCKET_SUB));
+    }
+    const int64_t first = B ? (int64_t)goff[m] + m : 0;
+    const int b = (int)(((first + lo) * HV_BUCKET_SUB + q) >> shift) + m;
     at[t] = ((uint64_t)b << 32) | (uint32_t)atomicAdd(&bcnt[b], 1);
 }
 
@@ -3555,7 +3557,8 @@ __global__ void k_pkt_count(const int* __restrict__ list, int n, const int* __re
 __global__ void k_pkt_count_off(const int* __restrict__ off, const int* __restrict__ goff, int shift, int nmesh,
                                 int* __restrict__ cnt) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < nmesh) cnt[m] = off[(goff[m + 1] >> shift) + m + 1] - off[(goff[m] >> shift) + m];
+    auto start = [&](int k) { return off[(int)(((int64_t)goff[k] + k) * HV_BUCKET_SUB >> shift) + k]; };
+    if (m < nmesh) cnt[m] = start(m + 1) - start(m);
 }
 
 // Prefix sums over the meshes (a wavefront, 64 meshes per step): seg = first list position of
@@ -3690,6 +3693,8 @@ static int build_forest(hv_ctx* c, int L, int tables, Forest& fo) {
         }
         HVCK(hipStreamSynchronize(c->stream));
     }
+    uint64_t* mcode = pget<uint64_t>(c, "f_mcode", (size_t)ntot);
+    if (!mcode) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (batch trees)");
     for (int k = 0; k < nm; ++k) {
         TreeOut o;
         o.xin = dxo + (int64_t)fo.goff[k] * D;
@@ -3702,6 +3707,7 @@ static int build_forest(hv_ctx* c, int L, int tables, Forest& fo) {
         o.pn = pn + (size_t)k * P * D;
         o.ph = ph + (size_t)k * P;
         o.planes_ready = true;
+        o.mcode = mcode + fo.goff[k];
         o.xo_base = dxo;
         o.xs = xs + soff[k] * (D + 1);
         o.sidx = sidx + soff[k];
@@ -3860,7 +3866,8 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         if (!c->extended) record_tree(c, T.g, prec, L);
     }
     DevGeo& g = T.g;   // over a forest: unused (every kernel takes its mesh's tree from F)
-    const uint64_t* mcode = B ? nullptr : pget<uint64_t>(c, "code2", 0);   // the generators' codes, as the tree's build left them
+    // the generators' codes, as the trees' builds left them
+    const uint64_t* mcode = pget<uint64_t>(c, B ? "f_mcode" : "code2", 0);
     const int nmesh = B ? fo->nmesh : 1;
     // box corners, or the simple vertices of a general polytope (single meshes only)
     const bool poly = !B && c->dom_general;
@@ -4125,7 +4132,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         const uint64_t tsz = hpow(2 * (int64_t)nr);
         int* ttab = pget<int>(c, "ttab", tsz);
         // at most two buckets a ray, and 2^21 (8 MiB of counts)
-        const int64_t bpos = B ? (int64_t)N : ((int64_t)N + 1) * HV_BUCKET_SUB;
+        const int64_t bpos = ((int64_t)N + nmesh) * HV_BUCKET_SUB;
         int shift = 0;
         while ((bpos >> shift) + nmesh > std::max<int64_t>(2048, std::min<int64_t>(2 * (int64_t)nr, 1 << 21))) ++shift;
         const int nb = (int)(bpos >> shift) + nmesh + 1, nbc = (nb + 4) / 4 * 4;   // one empty bucket at least: its offset is the total
@@ -4150,11 +4157,8 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         nt_fresh = false;
         k_ray_dir<D, B><<<nblk(nr, 256), 256, 0, c->stream>>>(g, F, R, nr, nfresh, vkey, vx, plane_tol, rtab, rsize - 1, ctr + 5);
         HVCK(hipGetLastError());
-        // start phase; R.code: the Morton code of the rays' certificate-ball centres (over a forest unused
-        // but with chunks)
-        DevRays Ri = R;
-        if (B && !chunks) Ri.code = nullptr;
-        launch_ray_init<D, B>(g, F, Ri, nr, vkey, vx, plane_tol, c->stream);
+        // start phase; R.code: the Morton code of the rays' certificate-ball centres
+        launch_ray_init<D, B>(g, F, R, nr, vkey, vx, plane_tol, c->stream);
         HVCK(hipGetLastError());
         if (chunks) {
             // over a forest the code holds the mesh above 32 Morton bits
