@@ -1646,8 +1646,12 @@ __global__ __launch_bounds__(64, 4) void k_mc_points(DevGeo g, int G, int64_t S,
     float pf[D];
     // packet centre (uniform): orders the children, and the origin of the leaf forms
     float pcf[D];
+    // up to 3D the samples stay in registers and the packet's bounds are left out: a packet's walk is
+    // short there (2D N=1000, 1e8 samples: both cost 0.4 of 12.5 ms)
+    constexpr bool WIDE = D > 3;
+    double p[D];
     {
-        double p[D], cc[D];
+        double cc[D];
         draw(p);
 #pragma unroll
         for (int k = 0; k < D; ++k) {
@@ -1714,7 +1718,7 @@ __global__ __launch_bounds__(64, 4) void k_mc_points(DevGeo g, int G, int64_t S,
     // of every sample, one test by eight lanes instead of eight by all (the same run 42 -> 37 ms)
     float plo[D], phi[D];
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
+    for (int k = 0; WIDE && k < D; ++k) {
         float lo = pf[k], hi = pf[k];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
@@ -1734,10 +1738,12 @@ __global__ __launch_bounds__(64, 4) void k_mc_points(DevGeo g, int G, int64_t S,
         const float thr = fmaf(m * m, 1.f / 8192.f, t * t - pp), ox = __shfl_xor(thr, 32);
         thr0 = lane < 32 ? thr : ox;
         thr1 = lane < 32 ? ox : thr;
-        float w = R2f;
+        if constexpr (WIDE) {
+            float w = R2f;
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) w = fmaxf(w, __shfl_xor(w, off));
-        R2max = w * (1.f + 1e-5f);
+            for (int off = 32; off > 0; off >>= 1) w = fmaxf(w, __shfl_xor(w, off));
+            R2max = w * (1.f + 1e-5f);
+        }
     };
     set_reach();
     auto load_leaf = [&](int leaf, float4& a, float4& b) {   // point lane % 32 of the leaf (its last point beyond the end)
@@ -1769,8 +1775,8 @@ __global__ __launch_bounds__(64, 4) void k_mc_points(DevGeo g, int G, int64_t S,
         if (lane < 16 * D - 64) cbx[lane + 64] = cbr1;
         if (l + 1 == g.h && sp > 0) prefetch(__builtin_amdgcn_readfirstlane(stk[sp - 1]));
         hv_wave_sync();
-        unsigned near;
-        {
+        unsigned near = 0xffu;
+        if constexpr (WIDE) {
             float d2 = 0.f;
             const int c = lane & 7;
 #pragma unroll
@@ -1783,7 +1789,7 @@ __global__ __launch_bounds__(64, 4) void k_mc_points(DevGeo g, int G, int64_t S,
         unsigned rem = 0u, mine = 0u;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            if (!((near >> c) & 1u)) continue;
+            if (WIDE && !((near >> c) & 1u)) continue;
             const bool h = child_d2f(c, pf) <= R2f;
             mine |= h ? (1u << c) : 0u;
             rem |= (__ballot(h) != 0ull) ? (1u << c) : 0u;
@@ -1876,8 +1882,7 @@ __global__ __launch_bounds__(64, 4) void k_mc_points(DevGeo g, int G, int64_t S,
             prefetch(cbase + (int)__builtin_ctzll(__ballot(reached && before == 0)));
         }
     }
-    double p[D];
-    draw(p);
+    if constexpr (WIDE) draw(p);   // again: their registers served the walk
     {
         unsigned long long w = work;
 #pragma unroll
