@@ -4102,19 +4102,19 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         R.t2 = pget<double>(c, "ray_t2", nslots);
         R.i1 = pget<int>(c, "ray_i1", nslots);
         R.i2 = pget<int>(c, "ray_i2", nslots);
-        uint64_t* code2 = pget<uint64_t>(c, "ray_code2", nslots);
-        int* ord0 = pget<int>(c, "ray_ord0", nslots);
-        int* ord = pget<int>(c, "ray_ord", nslots);
-        int* cand = pget<int>(c, "ray_cand", nslots);
         int* ordc = pget<int>(c, "ray_ordc", nslots);
-        uint8_t* keep = pget<uint8_t>(c, "ray_keep", nslots);
+        // the sorted order of a walk in chunks
+        uint64_t* code2 = chunks ? pget<uint64_t>(c, "ray_code2", nslots) : nullptr;
+        int* ord0 = chunks ? pget<int>(c, "ray_ord0", nslots) : nullptr;
+        int* ord = chunks ? pget<int>(c, "ray_ord", nslots) : nullptr;
+        int* cand = chunks ? pget<int>(c, "ray_cand", nslots) : nullptr;
+        uint8_t* keep = chunks ? pget<uint8_t>(c, "ray_keep", nslots) : nullptr;
         int* status = pget<int>(c, "status", nslots);
         int* rwin = pget<int>(c, "ray_win", nslots);
         double* rt = pget<double>(c, "ray_t", nslots);
         int64_t* reg_next = pget<int64_t>(c, reg_is_a ? "regB" : "regA", nslots * (D + 1));
-        if (!R.slot || !R.v || !R.drop || !R.u || !R.c || !R.du || !R.code || !code2 || !ord0 || !ord || !cand ||
-            !R.t1 || !R.t2 || !R.i1 || !R.i2 ||
-            !ordc || !keep || !status || !rwin || !rt || !reg_next)
+        if (!R.slot || !R.v || !R.drop || !R.u || !R.c || !R.du || !R.code || !R.t1 || !R.t2 || !R.i1 || !R.i2 ||
+            (chunks && (!code2 || !ord0 || !ord || !cand || !keep)) || !ordc || !status || !rwin || !rt || !reg_next)
             return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rays)");
         if (!emitted) {
             HVCK(hipMemsetAsync(dcount + 3, 0, sizeof(int), c->stream));
