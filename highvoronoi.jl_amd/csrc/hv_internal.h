@@ -11,6 +11,7 @@
 #include <vector>
 #include "../../include/hv.h"
 #include "hv_device.h"
+#include "hv_plan.h"
 
 // Device buffer pool: tables survive between builds so a steady-state build does no
 // hipMalloc; a finished mesh takes ownership of its vertex tables and returns them.

@@ -3351,8 +3351,7 @@ __device__ __forceinline__ bool hv_tent_key(const DevGeo& g, const DevRays& R, c
 // position of the ray's candidate cost the scan of a 5D N=100k mixture 19.0 -> 22.9 ms, quarters of
 // the gaps 20.0, sixteenths 18.9.)  Over a
 // forest the gaps of mesh m start at (goff[m] + m) HV_BUCKET_SUB and its buckets at that >> shift, plus
-// m, so that no bucket holds rays of two meshes.
-constexpr int HV_BUCKET_SUB = 16;
+// m, so that no bucket holds rays of two meshes (hv_buckets).
 template <int D, bool B>
 __global__ __launch_bounds__(256) void k_tent_group(DevGeo g0, GeoSet F, DevRays R, int nr, int nfresh,
                                                     const int* __restrict__ vkey, int* __restrict__ ttab, uint64_t tmask,
@@ -4136,11 +4135,8 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         ntab = pget<unsigned long long>(c, "ntab", nsize);
         const uint64_t tsz = hpow(2 * (int64_t)nr);
         int* ttab = pget<int>(c, "ttab", tsz);
-        // at most two buckets a ray, and 2^21 (8 MiB of counts)
-        const int64_t bpos = ((int64_t)N + nmesh) * HV_BUCKET_SUB;
-        int shift = 0;
-        while ((bpos >> shift) + nmesh > std::max<int64_t>(2048, std::min<int64_t>(2 * (int64_t)nr, 1 << 21))) ++shift;
-        const int nb = (int)(bpos >> shift) + nmesh + 1, nbc = (nb + 4) / 4 * 4;   // one empty bucket at least: its offset is the total
+        const HvBuckets bk = hv_buckets(N, nmesh, nr);
+        const int shift = bk.shift, nb = bk.count, nbc = (nb + 4) / 4 * 4;
         int* bcnt = pget<int>(c, "bk_cnt", (size_t)nbc);
         int* boff = pget<int>(c, "bk_off", (size_t)nb + 1);
         HvCarry car;
