@@ -20,3 +20,13 @@ inline HvBuckets hv_buckets(int64_t n, int64_t nmesh, int64_t nr) {
     while ((positions >> shift) > limit) ++shift;
     return {shift, (int)((positions >> shift) + nmesh + 1)};
 }
+
+// Levels of internal nodes of the 8-ary tree, and k_knn's waiting nodes.  A tree has at most 2^29
+// leaves (leaves of one point; node numbers of the binary tree are 32-bit), so at most ten levels.
+// A step takes the topmost eight nodes, of whatever levels, and puts their internal children, at
+// most 64, in their place.  A node of level l then never waits above position 63 l: the root waits at
+// 0, and a child of a taken node of level l lands at most 63 above the lowest taken position, which
+// is no higher than that node's own.
+constexpr int HV_TREE_LEVELS = 10;
+constexpr int HV_KNN_STACK = 576;
+static_assert(HV_KNN_STACK > 63 * (HV_TREE_LEVELS - 1), "room for the deepest node's highest position");

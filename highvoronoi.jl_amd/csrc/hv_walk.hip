@@ -1427,7 +1427,6 @@ __device__ __forceinline__ bool hv_ray_result(const DevGeo& g, const RayGeo<D>& 
 // wavefronts at N=20k, and ran every insertion under divergence: 2D N=1000 146 -> 12 us, 4D N=20k
 // 1 140 -> 93 us, 5D N=100k mixture 3.6 -> 0.77 ms.
 constexpr int HV_KNN_WAVES = 4;     // wavefronts per workgroup
-constexpr int HV_KNN_STACK = 512;   // 8 popped and at most 64 pushed per level of at most 9
 
 template <int D, bool B>
 __global__ __launch_bounds__(64 * HV_KNN_WAVES) void k_knn(DevGeo g0, GeoSet F, const int* __restrict__ boff,

@@ -1,5 +1,6 @@
 """The walk's launch plans (csrc/hv_plan.h, plain C++) on the host: the buckets a level's rays are
-counted into, for more meshes than the buckets' limit as well (the choice of the shift has to end)."""
+counted into, for more meshes than the buckets' limit as well (the choice of the shift has to end),
+and the room for the waiting nodes of the 16-NN lists' walk."""
 import os
 import subprocess
 
