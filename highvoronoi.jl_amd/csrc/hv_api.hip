@@ -112,7 +112,7 @@ DevArr::~DevArr() {
 static std::mutex scratch_mu;
 static std::map<int, std::vector<DBuf>> scratch_free;   // per device, smallest first
 
-HvScratch::HvScratch(int device_ordinal, size_t bytes) : device(device_ordinal) {
+HvScratch::HvScratch(int device_ordinal, size_t bytes, hipStream_t s) : device(device_ordinal), stream(s) {
     bytes = std::max<size_t>(bytes, 256);
     {
         std::lock_guard<std::mutex> lk(scratch_mu);
@@ -140,6 +140,7 @@ HvScratch::HvScratch(int device_ordinal, size_t bytes) : device(device_ordinal) 
 
 HvScratch::~HvScratch() {
     if (!p) return;
+    if (queued) (void)hipStreamSynchronize(stream);
     std::vector<DBuf> drop;
     {
         std::lock_guard<std::mutex> lk(scratch_mu);
@@ -178,7 +179,7 @@ void hv_scratch_release(int device_ordinal) {
 static std::mutex pinned_mu;
 static std::vector<unsigned long long*> pinned_free;
 
-HvPinned::HvPinned() {
+HvPinned::HvPinned(hipStream_t s) : stream(s) {
     {
         std::lock_guard<std::mutex> lk(pinned_mu);
         if (!pinned_free.empty()) {
@@ -195,6 +196,7 @@ HvPinned::HvPinned() {
 
 HvPinned::~HvPinned() {
     if (!p) return;
+    if (queued) (void)hipStreamSynchronize(stream);
     {
         std::lock_guard<std::mutex> lk(pinned_mu);
         if (pinned_free.size() < HV_PINNED_KEEP) {
@@ -778,7 +780,7 @@ static int refine_periodic(hv_ctx* c, const hv_opts* o, const hv_mesh* old, int6
     const int D = old->D;
     const int64_t n = old->nreal, nu = n + m;
     if (nu >= (1ll << 30)) return hv_fail(c, HV_ERR_UNSUPPORTED, "too many generators for 32-bit keys");
-    HvScratch buf(c->device, sizeof(double) * D * nu);
+    HvScratch buf(c->device, sizeof(double) * D * nu, c->stream);
     double* u = (double*)buf.p;
     if (!u) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
     int rc = HV_OK;
@@ -787,8 +789,8 @@ static int refine_periodic(hv_ctx* c, const hv_opts* o, const hv_mesh* old, int6
         hipMemcpyAsync(u + D * n, xs_new, sizeof(double) * D * m, hipMemcpyHostToDevice, c->stream) != hipSuccess)
         rc = hv_fail(c, HV_ERR_DEVICE, "copy of the points failed");
     if (!rc) rc = set_points_common(c, D, nu, u, hipMemcpyDeviceToDevice);
-    (void)hipStreamSynchronize(c->stream);   // before the buffer is another's
     if (rc) return rc;
+    buf.settled();   // set_points_common has waited
     rc = hv_set_boundary(c, old->P, old->P ? old->pbase.data() : nullptr, old->P ? old->pnormal.data() : nullptr,
                          old->pbc.empty() ? nullptr : old->pbc.data());
     if (rc) return rc;
@@ -830,7 +832,7 @@ int hv_refine_mesh(hv_ctx* c, const hv_opts* o, const hv_mesh* old, int64_t m, c
     if (nu >= (1ll << 30)) return hv_fail(c, HV_ERR_UNSUPPORTED, "too many generators for 32-bit keys");
     (void)hipSetDevice(c->device);
     // the union in device memory: the mesh's generators, then the new points
-    HvScratch buf(c->device, sizeof(double) * D * nu);
+    HvScratch buf(c->device, sizeof(double) * D * nu, c->stream);
     double* u = (double*)buf.p;
     if (!u) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
     int rc = HV_OK;
@@ -838,8 +840,8 @@ int hv_refine_mesh(hv_ctx* c, const hv_opts* o, const hv_mesh* old, int64_t m, c
         hipMemcpyAsync(u + D * n, xs_new, sizeof(double) * D * m, hipMemcpyHostToDevice, c->stream) != hipSuccess)
         rc = hv_fail(c, HV_ERR_DEVICE, "copy of the points failed");
     if (!rc) rc = set_points_common(c, D, nu, u, hipMemcpyDeviceToDevice);
-    (void)hipStreamSynchronize(c->stream);   // before the buffer is another's
     if (rc) return rc;
+    buf.settled();   // set_points_common has waited
     rc = hv_set_boundary(c, old->P, old->P ? old->pbase.data() : nullptr, old->P ? old->pnormal.data() : nullptr,
                          old->pbc.empty() ? nullptr : old->pbc.data());
     if (rc) return rc;

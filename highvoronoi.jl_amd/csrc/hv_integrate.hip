@@ -1571,7 +1571,7 @@ static int neighbor_rows(hv_ctx* c, const hv_mesh* mesh, uint64_t*& pkey, int64_
     int* res = iget<int>(c, "n_full", 3);           // set overflow, k_rows_most
     int* cnt = iget<int>(c, "n_cnt", (size_t)N + 1);
     ptr = iget<int64_t>(c, "i_ptr", (size_t)N + 1);
-    HvPinned pin;
+    HvPinned pin(c->stream);
     if (!res || !cnt || !ptr || !pin.p) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (neighbours)");
     size_t tb = 0;
     HVCK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, CountRows{cnt}.begin(), ptr, N + 1, c->stream));
@@ -1610,6 +1610,7 @@ static int neighbor_rows(hv_ctx* c, const hv_mesh* mesh, uint64_t*& pkey, int64_
         if (attempt >= 4 || tsize >= (1ull << 29)) return hv_fail(c, HV_ERR_CAPACITY, "neighbour set overflow");
         tsize <<= 2;
     }
+    pin.settled();
     if (npair > (int64_t)INT32_MAX) return hv_fail(c, HV_ERR_CAPACITY, "more than 2^31 neighbour rows");
     uint64_t* rows = iget<uint64_t>(c, "n_rows", (size_t)std::max<int64_t>(npair, 1));
     if (!rows) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (neighbours)");
@@ -1692,7 +1693,7 @@ static int finish(hv_ctx* c, int64_t ncell, const uint64_t* pkey, const double* 
     I->area = part(sizeof(double) * npair);
     I->bulk = part(sizeof(double) * ncell * nf);
     I->iface = part(sizeof(double) * npair * nf);
-    I->dev.reset(new HvScratch(c->device, at));
+    I->dev.reset(new HvScratch(c->device, at, c->stream));
     hipMemcpyKind kind = hipMemcpyDeviceToDevice;
     if (I->dev->p) {
         I->base = (char*)I->dev->p;
@@ -1718,6 +1719,7 @@ static int finish(hv_ctx* c, int64_t ncell, const uint64_t* pkey, const double* 
     HVCK(put(I->bulk, bulk_d, sizeof(double) * ncell * nf));
     HVCK(put(I->iface, rint_d, sizeof(double) * npair * nf));
     HVCK(hipStreamSynchronize(c->stream));
+    if (I->dev) I->dev->settled();   // it outlives the stream
     *out = I.release();
     return HV_OK;
 }

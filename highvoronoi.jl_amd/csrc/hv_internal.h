@@ -49,16 +49,20 @@ struct DevArr {
 // Device memory of an object that owns no context (an export's scratch, an integral's results), for
 // the lifetime of that object.  The buffers come from a process-wide store of at most
 // HV_SCRATCH_KEEP free buffers and HV_SCRATCH_BYTES per device (each used by one owner at a time;
-// given back with hv_batch_release); p is null when the device has no room.  The owner waits for
-// its work before the object goes.
+// given back with hv_batch_release); p is null when the device has no room.  The owner's work is
+// queued on `stream`: until it calls settled(), having waited for it, the destructor waits, so that
+// no exit leaves work queued on a buffer that is another's.
 constexpr int HV_SCRATCH_KEEP = 8;
 constexpr size_t HV_SCRATCH_BYTES = (size_t)1 << 30;
 struct HvScratch {
     int device;
     void* p = nullptr;
     size_t n = 0;
-    HvScratch(int device_ordinal, size_t bytes);
+    hipStream_t stream;
+    bool queued = true;
+    HvScratch(int device_ordinal, size_t bytes, hipStream_t stream);
     ~HvScratch();
+    void settled() { queued = false; }
     HvScratch(const HvScratch&) = delete;
     HvScratch& operator=(const HvScratch&) = delete;
 };
@@ -95,12 +99,16 @@ struct HvLease {
 };
 // Pinned host memory (512 bytes) that kernels write a call's counts into, for the lifetime of the
 // object: from a process-wide store of at most HV_PINNED_KEEP free blocks; p is null when there is
-// none to be had.
+// none to be had.  The destructor waits for the stream of those kernels unless settled() was called,
+// as HvScratch's does.
 constexpr size_t HV_PINNED_KEEP = 16;
 struct HvPinned {
     unsigned long long* p = nullptr;
-    HvPinned();
+    hipStream_t stream;
+    bool queued = true;
+    explicit HvPinned(hipStream_t stream);
     ~HvPinned();
+    void settled() { queued = false; }
     HvPinned(const HvPinned&) = delete;
     HvPinned& operator=(const HvPinned&) = delete;
 };

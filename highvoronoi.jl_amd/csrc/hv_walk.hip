@@ -3921,7 +3921,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
     if (!vkey || !vx || !ids || !htab || !ctr || !sctr) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (tables)");
     // counts: 0 carried rays, 1 new vertices, 3 new rays
     int* dcount = (int*)(ctr + 16);
-    HvPinned pin;
+    HvPinned pin(c->stream);
     if (!pin.p) return hv_fail(c, HV_ERR_DEVICE, "out of pinned memory");
     HVCK(hipMemsetAsync(htab, 0xff, hsize * sizeof(int), c->stream));
     HVCK(hipMemsetAsync(ctr, 0, HV_CTL * sizeof(unsigned long long), c->stream));
@@ -4362,6 +4362,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
     HVCK(hipGetLastError());
     rc = read_ctr();
     if (rc) return rc;
+    pin.settled();
     for (int k : {0, 1, 2, 6, 7, 8, 9, 10, 11}) hctr[k] = pin.p[32 + k];
     float ms_all = 0.f;
     HVCK(hipEventElapsedTime(&ms_all, e0, e1));
@@ -4418,7 +4419,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         }
         const size_t kb = ((size_t)nlive * (D + 1) * sizeof(int) + 255) / 256 * 256;
         const size_t xb = ((size_t)nlive * D * sizeof(double) + 255) / 256 * 256;
-        auto store = std::make_shared<HvScratch>(c->device, kb + xb + sizeof(int) * (size_t)maxc);
+        auto store = std::make_shared<HvScratch>(c->device, kb + xb + sizeof(int) * (size_t)maxc, c->stream);
         if (!store->p) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (batch meshes)");
         int* okey = (int*)store->p;
         double* ox = (double*)((char*)store->p + kb);
@@ -4433,6 +4434,7 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
         k_iota<<<nblk(maxc, 256), 256, 0, c->stream>>>(oid, maxc);
         HVCK(hipGetLastError());
         HVCK(hipStreamSynchronize(c->stream));
+        store->settled();   // it outlives the stream
         for (int k = 0; k < nm; ++k) {
             hv_mesh* mk = new hv_mesh();
             mk->pool = nullptr;
@@ -4900,7 +4902,7 @@ int hv_mesh_export_impl(const hv_mesh* m, int64_t* sig, double* coords) {
     const int chunk = (int)std::min<int64_t>(nv, (int64_t)(HV_EXPORT_CHUNK / row));
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t bw = up(sizeof(uint64_t) * nv), bp = up(sizeof(int) * nv), bt = up(tb);
-    HvScratch tmp(m->device, 2 * bw + 2 * bp + bt + up(sizeof(int64_t) * (D + 1) * chunk) + sizeof(double) * D * chunk);
+    HvScratch tmp(m->device, 2 * bw + 2 * bp + bt + up(sizeof(int64_t) * (D + 1) * chunk) + sizeof(double) * D * chunk, st);
     if (!tmp.p) return export_on_host<D>(m, sig, coords);
     char* at = (char*)tmp.p;
     auto take = [&](size_t b) { char* p = at; at += b; return p; };
@@ -4938,6 +4940,7 @@ int hv_mesh_export_impl(const hv_mesh* m, int64_t* sig, double* coords) {
             double* px = pin.take<double>((size_t)nv * D);
             k_export_rows<D><<<nblk(nv * (2 * D + 1), 256), 256, 0, st>>>(pb, 0, (int)nv, ids, key, x, psig, px);
             if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return HV_ERR_DEVICE;
+            tmp.settled();
             std::memcpy(sig, psig, sizeof(int64_t) * (D + 1) * nv);
             std::memcpy(coords, px, sizeof(double) * D * nv);
             return HV_OK;
@@ -4950,6 +4953,7 @@ int hv_mesh_export_impl(const hv_mesh* m, int64_t* sig, double* coords) {
         const HvCopy list[2] = {{sig + r0 * (D + 1), dsig, sizeof(int64_t) * (D + 1) * n}, {coords + r0 * D, dx, sizeof(double) * D * n}};
         if (hv_copies(m->device, true, list, 2) != hipSuccess) return HV_ERR_DEVICE;
     }
+    tmp.settled();
     return HV_OK;
 }
 
@@ -5851,7 +5855,7 @@ int hv_raycast_batch_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t
     HVCK(hipcub::DeviceRadixSort::SortPairs(nullptr, b.tb, b.R.code, b.code2, b.ord0, b.ord, n, HV_RAY_SORT_LO, 60, c->stream));
     b.tmp = c->pool->get("cubtmp", b.tb, false, c->stream);
     if (!b.tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (sort)");
-    HvPinned pin;
+    HvPinned pin(c->stream);
     if (!pin.p) return hv_fail(c, HV_ERR_DEVICE, "out of pinned memory");
     *pin.p = 0ull;
     // the caller's arrays: a small batch's through a pinned block the kernels work on, a large one's copied
@@ -5868,6 +5872,7 @@ int hv_raycast_batch_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t
             int32_t* ost = L.take<int32_t>((size_t)nrays);
             rc = run_rays<D>(c, g, precision, n, b, psig, pdrop, pr, pin.p, osig, orr, ot, ost);
             if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = hv_fail(c, HV_ERR_DEVICE, "device error");
+            pin.settled();
             if (rc) return rc;
             if (*pin.p) return refused();
             std::memcpy(out_sig, osig, sizeof(int64_t) * nk);
@@ -5904,6 +5909,7 @@ int hv_raycast_batch_impl(hv_ctx* c, int precision, int64_t nrays, const int64_t
         }
     }
     if (hipStreamSynchronize(c->stream) != hipSuccess && !rc) rc = hv_fail(c, HV_ERR_DEVICE, "device error");
+    pin.settled();
     if (rc) return rc;
     if (*pin.p) return refused();
     const HvCopy res[4] = {{out_sig, dosig, sizeof(int64_t) * nk},
@@ -6476,7 +6482,7 @@ int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** o
     M->x.n = nk * D * sizeof(double);
     M->ids.n = nk * sizeof(int);
     const size_t ob = (M->x.n + 255) / 256 * 256, kb = (M->key.n + 255) / 256 * 256;
-    M->store = std::make_shared<HvScratch>(c->device, ob + kb + M->ids.n);
+    M->store = std::make_shared<HvScratch>(c->device, ob + kb + M->ids.n, c->stream);
     if (!M->store->p) {
         delete M;
         return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refined mesh)");
@@ -6496,6 +6502,7 @@ int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** o
         hv_mesh_free(M);
         return hv_fail(c, HV_ERR_DEVICE, "refine copy failed");
     }
+    M->store->settled();   // it outlives the stream
     M->stats = S->stats;
     M->stats.vertices = tot;
     hv_mesh_snapshot(c, M);

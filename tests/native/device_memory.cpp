@@ -1,0 +1,78 @@
+// Checks of the library's device and pinned memory on a HIP runtime of host memory (fake_hip.h): the
+// name of a check is the argument; exit status 0 when it holds.
+#include "fake_hip.h"
+#include "hv_internal.h"
+#include <memory>
+#include <string>
+
+#define CHECK(c)                                                            \
+    do {                                                                    \
+        if (!(c)) {                                                         \
+            std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);             \
+            return 1;                                                       \
+        }                                                                   \
+    } while (0)
+
+constexpr size_t MiB = (size_t)1 << 20;
+
+// Work queued for an export that fails part way is waited for before its buffer is another's.
+static int failed_export() {
+    const int nv = 1000, D = 3;
+    hv_mesh m;
+    m.D = D;
+    m.N = 200;
+    m.nreal = 200;
+    m.nv = nv;
+    std::vector<int> ids(nv), key(nv * (D + 1));
+    std::vector<double> x(nv * D);
+    for (int v = 0; v < nv; ++v) ids[v] = v;
+    m.ids.p = ids.data();
+    m.key.p = key.data();
+    m.x.p = x.data();
+    std::vector<int64_t> sig(nv * (D + 1));
+    std::vector<double> coords(nv * D);
+    CHECK(hv_mesh_export(&m, sig.data(), coords.data()) == HV_OK);
+    const int all = fake::S().launches;
+    CHECK(all > 2);
+    for (int k = 0; k < all; ++k) {
+        fake::S().launches = 0;
+        fake::S().fail_at = k;
+        CHECK(hv_mesh_export(&m, sig.data(), coords.data()) == HV_ERR_DEVICE);
+        CHECK(fake::waiting() == 0);
+    }
+    return 0;
+}
+
+// The same of the objects themselves, when their owner leaves before it has waited; one that was
+// settled does not touch its stream again.
+static int queued_work() {
+    hipStream_t st = nullptr;
+    CHECK(hipStreamCreateWithFlags(&st, 0) == hipSuccess);
+    {
+        HvScratch b(0, 1000, st);
+        fake::queue(st);
+    }
+    CHECK(fake::waiting() == 0);
+    {
+        HvPinned b(st);
+        fake::queue(st);
+    }
+    CHECK(fake::waiting() == 0);
+    {
+        HvScratch b(0, 1000, st);
+        HvPinned q(st);
+        b.settled();
+        q.settled();
+        fake::queue(st);
+    }
+    CHECK(fake::waiting() == 1);
+    return 0;
+}
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "failed_export") return failed_export();
+    if (what == "queued_work") return queued_work();
+    std::printf("no check of that name\n");
+    return 2;
+}
