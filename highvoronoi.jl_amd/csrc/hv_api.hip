@@ -110,7 +110,9 @@ DevArr::~DevArr() {
 }
 
 static std::mutex scratch_mu;
-static std::map<int, std::vector<DBuf>> scratch_free;   // per device, smallest first
+// Per device, smallest first.  Never destroyed, as the other stores here: an object may be released by
+// a handler that runs after this library's own at the end of the process.
+static auto& scratch_free = *new std::map<int, std::vector<DBuf>>();
 
 HvScratch::HvScratch(int device_ordinal, size_t bytes, hipStream_t s) : device(device_ordinal), stream(s) {
     bytes = std::max<size_t>(bytes, 256);
@@ -177,7 +179,7 @@ void hv_scratch_release(int device_ordinal) {
 }
 
 static std::mutex pinned_mu;
-static std::vector<unsigned long long*> pinned_free;
+static auto& pinned_free = *new std::vector<unsigned long long*>();   // never destroyed
 
 HvPinned::HvPinned(hipStream_t s) : stream(s) {
     {

@@ -2,6 +2,7 @@
 // name of a check is the argument; exit status 0 when it holds.
 #include "fake_hip.h"
 #include "hv_internal.h"
+#include <unistd.h>
 #include <memory>
 #include <string>
 
@@ -69,9 +70,35 @@ static int queued_work() {
     return 0;
 }
 
+// An object released at the end of the process, after the library's own statics are gone: the handler
+// is registered before any library is initialised, so it runs last.
+static HvScratch* late_scratch = nullptr;
+static HvPinned* late_pinned = nullptr;
+extern "C" int __cxa_atexit(void (*)(void*), void*, void*) noexcept;
+static void late(void*) {
+    delete late_scratch;
+    delete late_pinned;
+    if (late_scratch) {
+        HvScratch again(0, 3000, nullptr);
+        HvPinned word(nullptr);
+        if (!again.p || !word.p || fake::S().device.size() != 2) _exit(1);   // both taken from the stores again
+    }
+}
+static void before_all() { __cxa_atexit(late, nullptr, nullptr); }
+__attribute__((section(".preinit_array"), used)) static void (*preinit)() = before_all;
+static int released_at_exit() {
+    HvScratch* a = new HvScratch(0, 1000000, nullptr);
+    { HvScratch b(0, 1000, nullptr); }
+    late_pinned = new HvPinned(nullptr);
+    { HvPinned b(nullptr); }
+    late_scratch = a;
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "failed_export") return failed_export();
+    if (what == "released_at_exit") return released_at_exit();
     if (what == "queued_work") return queued_work();
     std::printf("no check of that name\n");
     return 2;
