@@ -243,6 +243,7 @@ hipError_t hv_copies(int device, bool out, const HvCopy* copies, int ncopies) {
     size_t total = 0;
     for (int k = 0; k < ncopies; ++k) total += copies[k].bytes;
     if (total == 0) return hipSuccess;
+    (void)hipSetDevice(device);
     // pieces of equal size within each array, about two per worker
     const size_t chunk = std::min(HV_STAGE_BYTES, std::max<size_t>((total / (2 * HV_STAGE_WORKERS) + 65535) & ~(size_t)65535,
                                                                    (size_t)256 << 10));
@@ -307,6 +308,7 @@ hipError_t hv_copies(int device, bool out, const HvCopy* copies, int ncopies) {
 
 HvLease::HvLease(int device) {
     if (device < 0 || device >= 64) return;
+    (void)hipSetDevice(device);
     HvStaging& S = staging[device];
     lk = std::unique_lock<std::mutex>(S.mu, std::try_to_lock);
     if (lk.owns_lock() && S.block(0)) base = (char*)S.pin[0];

@@ -953,21 +953,6 @@ __global__ void k_dense_geo(const int* __restrict__ gid, int nused, int ngen, in
 
 // ---- host driver -------------------------------------------------------------------------
 
-// Results stay on the device until hv_integral_export copies them into the caller's memory
-// (`host` holds them when the device has no room).
-struct hv_integral {
-    int64_t N = 0, rows = 0;
-    int device = 0;
-    std::unique_ptr<HvScratch> dev;
-    std::vector<char> host;
-    char* base = nullptr;              // dev or host memory: the parts below by offset
-    size_t vol = 0, ptr = 0, nbr = 0, area = 0, bulk = 0, iface = 0;
-    double ms = 0.0;
-    int64_t work = 0;                  // point samples: (sample, generator) distances evaluated
-    double ms_kernel = 0.0;            // point samples: device time of the sampling kernel
-    int nf = 0;                        // integrand components (0: none)
-};
-
 static int64_t binom(int n, int k) {
     int64_t r = 1;
     for (int i = 1; i <= k; ++i) r = r * (n - k + i) / i;
@@ -1902,6 +1887,7 @@ static int integral_out(const hv_integral* I, const IntegralPart* part, int n) {
         hi = std::max(hi, part[k].off + part[k].bytes);
     }
     if (m == 0) return HV_OK;
+    (void)hipSetDevice(I->device);
     if (!I->dev) {
         for (int k = 0; k < m; ++k) std::memcpy(list[k].dst, list[k].src, list[k].bytes);
         return HV_OK;

@@ -68,7 +68,8 @@ struct HvScratch {
 };
 // Copies between device memory and the caller's (pageable) memory, out of the device or into it; the
 // data is complete (its stream has been waited for) and so are the copies on return.  Callable from
-// several threads at once.
+// several threads at once; selects the device for the calling thread, as HvLease does (the streams
+// and pinned blocks made on the way are kept for that device).
 struct HvCopy {
     void* dst;
     const void* src;
@@ -206,6 +207,21 @@ struct hv_mesh {
     std::shared_ptr<HvScratch> store;
 };
 
+// Results stay on the device until hv_integral_export copies them into the caller's memory
+// (`host` holds them when the device has no room).
+struct hv_integral {
+    int64_t N = 0, rows = 0;
+    int device = 0;
+    std::unique_ptr<HvScratch> dev;
+    std::vector<char> host;
+    char* base = nullptr;              // dev or host memory: the parts below by offset
+    size_t vol = 0, ptr = 0, nbr = 0, area = 0, bulk = 0, iface = 0;
+    double ms = 0.0;
+    int64_t work = 0;                  // point samples: (sample, generator) distances evaluated
+    double ms_kernel = 0.0;            // point samples: device time of the sampling kernel
+    int nf = 0;                        // integrand components (0: none)
+};
+
 // Meshes of one dimension walked together (hv_build_mesh_batch): inputs, the forest of their
 // trees and the resulting meshes.  Generator ids are global over the meshes (mesh k holds ids
 // goff[k] .. goff[k] + n[k] - 1) and mesh k's boundary plane p has id ntot + 2 D k + p.
@@ -310,7 +326,6 @@ template <int D>
 int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** out, int64_t* removed);
 
 // cell volumes and interface areas (hv_integrate.hip)
-struct hv_integral;
 template <int D>
 int hv_integrate_polytope_impl(hv_ctx* c, const hv_mesh* mesh, hv_integral** out);
 template <int D>

@@ -95,8 +95,47 @@ static int released_at_exit() {
     return 0;
 }
 
+// Copies, the pinned block and an integral's export work on their own device, whichever the thread used last.
+static int devices() {
+    std::vector<char> a(4 * MiB, 1), b(4 * MiB, 0);
+    const HvCopy one{b.data(), a.data(), a.size()};
+    CHECK(hipSetDevice(0) == hipSuccess);
+    CHECK(hv_copies(1, true, &one, 1) == hipSuccess && a == b);
+    CHECK(fake::S().stream_device.size() > 1 && !fake::S().host.empty());
+    for (auto& kv : fake::S().stream_device) CHECK(kv.second == 1);
+    for (auto& kv : fake::S().host) CHECK(kv.second.device == 1);
+    for (int d : fake::S().copy_device) CHECK(d == 1);
+    CHECK(hipSetDevice(1) == hipSuccess);
+    {
+        HvLease L(0);
+        CHECK(L.base && fake::S().host[L.base].device == 0);
+    }
+    CHECK(hipSetDevice(1) == hipSuccess);
+    hv_integral I;
+    const int64_t n = 5, rows = 20;
+    I.N = n;
+    I.rows = rows;
+    I.device = 1;
+    I.ptr = 256;
+    I.nbr = 512;
+    I.area = 1024;
+    I.dev.reset(new HvScratch(1, 2048, nullptr));
+    I.dev->settled();
+    I.base = (char*)I.dev->p;
+    for (int64_t k = 0; k < n; ++k) ((double*)(I.base + I.vol))[k] = 0.5 + k;
+    CHECK(hipSetDevice(0) == hipSuccess);
+    fake::S().copy_device.clear();
+    std::vector<double> vol(n), area(rows);
+    std::vector<int64_t> ptr(n + 1), nbr(rows);
+    CHECK(hv_integral_export(&I, vol.data(), ptr.data(), nbr.data(), area.data(), nullptr) == HV_OK);
+    CHECK(vol[3] == 3.5 && !fake::S().copy_device.empty());
+    for (int d : fake::S().copy_device) CHECK(d == 1);
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "devices") return devices();
     if (what == "failed_export") return failed_export();
     if (what == "released_at_exit") return released_at_exit();
     if (what == "queued_work") return queued_work();
