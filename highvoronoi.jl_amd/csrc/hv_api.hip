@@ -15,6 +15,54 @@
 #include <string>
 
 // ---------------------------------------------------------------- device pool
+// Parts of destroyed contexts, for the next ones: a program that makes a context per point set (the
+// geometry class does) paid 100 allocations, as many frees and a stream for each, 0.3 of the 1.4 ms
+// of a 2D N=1000 geometry.  At most HV_PARK contexts' parts per device and HV_PARK_BYTES of device
+// memory in each; idle (hv_destroy waits for the stream), used by one context at a time, given back
+// with hv_batch_release.
+constexpr size_t HV_PARK = 4, HV_PARK_BYTES = (size_t)256 << 20;
+struct HvParked {
+    hipStream_t stream = nullptr;
+    hipEvent_t ev[4] = {};
+    std::shared_ptr<DevPool> pool;
+};
+static std::mutex park_mu;
+static auto& parked = *new std::map<int, std::vector<HvParked>>();   // never destroyed: the runtime may go first at exit
+
+static void park_free(HvParked& k) {
+    for (auto e : k.ev)
+        if (e) (void)hipEventDestroy(e);
+    if (k.stream) (void)hipStreamDestroy(k.stream);
+    k.pool.reset();
+}
+
+static void park_release(int device) {   // every device when negative
+    std::vector<HvParked> drop;
+    {
+        std::lock_guard<std::mutex> lk(park_mu);
+        for (auto& kv : parked)
+            if (kv.first == device || device < 0) {
+                drop.insert(drop.end(), kv.second.begin(), kv.second.end());
+                kv.second.clear();
+            }
+    }
+    for (auto& k : drop) park_free(k);
+}
+
+hipError_t hv_device_malloc(int device, void** p, size_t bytes) {
+    *p = nullptr;
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    hv_scratch_release(device);
+    park_release(device);
+    e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return e;
+}
+
 DevPool::~DevPool() {
     (void)hipSetDevice(device);
     for (auto& kv : bufs)
@@ -28,10 +76,7 @@ void* DevPool::get(const std::string& name, size_t bytes, bool keep_contents, hi
     if (bytes == 0) return b.p;
     size_t want = bytes + bytes / 4 + 256;
     void* p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    if (hv_device_malloc(device, &p, want) != hipSuccess) return nullptr;
     if (keep_contents && b.p && b.n) {
         if (hipMemcpyAsync(p, b.p, b.n, hipMemcpyDeviceToDevice, s) != hipSuccess) {
             (void)hipFree(p);
@@ -59,10 +104,7 @@ void* DevPool::reserve(const std::string& name, size_t bytes, hipStream_t s) {
         b.n = 0;
     }
     void* p = nullptr;
-    if (hipMalloc(&p, std::max<size_t>(bytes, 256)) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    if (hv_device_malloc(device, &p, std::max<size_t>(bytes, 256)) != hipSuccess) return nullptr;
     b.p = p;
     b.n = std::max<size_t>(bytes, 256);
     return p;
@@ -128,16 +170,7 @@ HvScratch::HvScratch(int device_ordinal, size_t bytes, hipStream_t s) : device(d
             return;
         }
     }
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        hv_scratch_release(device);   // room held by smaller buffers
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            p = nullptr;
-            return;
-        }
-    }
-    n = bytes;
+    if (hv_device_malloc(device, &p, bytes) == hipSuccess) n = bytes;
 }
 
 HvScratch::~HvScratch() {
@@ -319,11 +352,7 @@ double* hv_points_for_write(hv_ctx* c, size_t bytes) {
     if (c->xw && c->xw.use_count() == 1 && c->xw->n >= bytes) return (double*)c->xw->p;
     auto a = std::make_shared<DevArr>();
     a->device = c->device;
-    if (hipMalloc(&a->p, bytes ? bytes : 8) != hipSuccess) {
-        (void)hipGetLastError();
-        a->p = nullptr;
-        return nullptr;
-    }
+    if (hv_device_malloc(c->device, &a->p, bytes ? bytes : 8) != hipSuccess) return nullptr;
     a->n = bytes;
     c->xw = std::move(a);
     return (double*)c->xw->p;
@@ -507,40 +536,6 @@ static std::vector<std::vector<uint64_t>> mesh_labels(const hv_mesh* m, int* rc)
 }
 
 extern "C" {
-
-// Parts of destroyed contexts, for the next ones: a program that makes a context per point set (the
-// geometry class does) paid 100 allocations, as many frees and a stream for each, 0.3 of the 1.4 ms
-// of a 2D N=1000 geometry.  At most HV_PARK contexts' parts per device and HV_PARK_BYTES of device
-// memory in each; idle (hv_destroy waits for the stream), used by one context at a time, given back
-// with hv_batch_release.
-constexpr size_t HV_PARK = 4, HV_PARK_BYTES = (size_t)256 << 20;
-struct HvParked {
-    hipStream_t stream = nullptr;
-    hipEvent_t ev[4] = {};
-    std::shared_ptr<DevPool> pool;
-};
-static std::mutex park_mu;
-static auto& parked = *new std::map<int, std::vector<HvParked>>();   // never destroyed: the runtime may go first at exit
-
-static void park_free(HvParked& k) {
-    for (auto e : k.ev)
-        if (e) (void)hipEventDestroy(e);
-    if (k.stream) (void)hipStreamDestroy(k.stream);
-    k.pool.reset();
-}
-
-static void park_release(int device) {   // every device when negative
-    std::vector<HvParked> drop;
-    {
-        std::lock_guard<std::mutex> lk(park_mu);
-        for (auto& kv : parked)
-            if (kv.first == device || device < 0) {
-                drop.insert(drop.end(), kv.second.begin(), kv.second.end());
-                kv.second.clear();
-            }
-    }
-    for (auto& k : drop) park_free(k);
-}
 
 int hv_create(hv_ctx** out, int device_ordinal) {
     if (!out) return HV_ERR_ARG;

@@ -36,6 +36,10 @@ struct DevPool {
     size_t total();   // bytes held
 };
 
+// hipMalloc on the device in use (`device`): when it has no room, what the process keeps idle there
+// (HvScratch's store, the parts of destroyed contexts) is given back first.
+hipError_t hv_device_malloc(int device, void** p, size_t bytes);
+
 // A device allocation shared by a context and the meshes built from it (the generator
 // set a mesh refers to stays alive as long as the mesh does).
 struct DevArr {

@@ -3612,11 +3612,8 @@ static int build_forest(hv_ctx* c, int L, int tables, Forest& fo) {
     // points: packed on the host, one copy, kept by the meshes (their generator sets)
     auto xo = std::make_shared<DevArr>();
     xo->device = c->device;
-    if (hipMalloc(&xo->p, sizeof(double) * (size_t)std::max<int64_t>(ntot, 1) * D) != hipSuccess) {
-        (void)hipGetLastError();
-        xo->p = nullptr;
+    if (hv_device_malloc(c->device, &xo->p, sizeof(double) * (size_t)std::max<int64_t>(ntot, 1) * D) != hipSuccess)
         return hv_fail(c, HV_ERR_DEVICE, "out of device memory (batch points)");
-    }
     xo->n = sizeof(double) * (size_t)ntot * D;
     fo.xo = xo;
     double* dxo = (double*)xo->p;
@@ -4244,18 +4241,19 @@ int hv_walk_impl(hv_ctx* c, const hv_opts* o, hv_mesh** out, int nwalk, const st
             vnext += nr;   // provisional slots of all nr
             k_carry_out<D><<<nblk(nr, 256), 256, 0, c->stream>>>(R, nr, R.code, rtab, car, dcount);
             HVCK(hipGetLastError());
-            // the next level's rays already, where the room for the most there can be is small (512 MiB): one
-            // wait a level
+            // the next level's rays already, where the room for the most there can be is small (512 MiB) and
+            // there: one wait a level
             if ((int64_t)nr * (D + 1) <= (1ll << 26)) {
                 const size_t most = (size_t)nr * (D + 1) + nr;
                 DevRays Rn = R;
                 Rn.slot = pget<int64_t>(c, "ray_slot", most);
                 Rn.v = pget<int>(c, "ray_v", most);
                 Rn.drop = pget<int>(c, "ray_drop", most);
-                if (!Rn.slot || !Rn.v || !Rn.drop) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (rays)");
-                rc = emit(Rn, ids + nlive, nr, dcount + 1, reg_next);
-                if (rc) return rc;
-                emitted = true;
+                if (Rn.slot && Rn.v && Rn.drop) {
+                    rc = emit(Rn, ids + nlive, nr, dcount + 1, reg_next);
+                    if (rc) return rc;
+                    emitted = true;
+                }
             }
             rc = read_ctr(np_dev);
             if (rc) return rc;

@@ -221,8 +221,10 @@ int hv_build_mesh_batch(int device_ordinal, int32_t nmesh, const int32_t* d, con
  * hv_build_mesh_batch's fused walks keep on the device between calls (device_ordinal < 0: on
  * every device), the buffers of exports, integrals, batches' and refined meshes kept after
  * their owners (at most 1 GiB per device) and the streams and tables kept of destroyed contexts
- * (at most four, of at most 256 MiB each, per device), for callers that need the memory back.  Meshes already built stay valid; the
- * next batch call creates its contexts again.  Waits for a batch call running meanwhile. */
+ * (at most four, of at most 256 MiB each, per device), for callers that need the memory back.  What is
+ * kept after its owner is also given back by itself when an allocation of this library finds no room.
+ * Meshes already built stay valid; the next batch call creates its contexts again.  Waits for a batch
+ * call running meanwhile. */
 int hv_batch_release(int device_ordinal);
 
 /* Ray-level entry point: one walkray per input (src/raycast.jl:125-164 via

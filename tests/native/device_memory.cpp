@@ -133,10 +133,45 @@ static int devices() {
     return 0;
 }
 
+// What is kept of destroyed objects is given back when an allocation finds no room: a pool's (grown and
+// reserved), a context's points, a buffer of the store.
+static int idle_given_back() {
+    auto& used = fake::S().used[0];
+    auto keep = []() -> int {   // 12 MiB in the store and 10 of a context, all of it idle
+        { HvScratch a(0, 12 * MiB, nullptr); }
+        hv_ctx* c = nullptr;
+        CHECK(hv_create(&c, 0) == HV_OK);
+        CHECK(c->pool->get("x", 8 * MiB));
+        CHECK(hv_destroy(c) == HV_OK);
+        return 0;
+    };
+    fake::S().limit[0] = 30 * MiB;
+    for (int way = 0; way < 4; ++way) {
+        hv_ctx *c = nullptr, *d = nullptr;
+        CHECK(hv_create(&c, 0) == HV_OK);
+        CHECK(hv_create(&d, 0) == HV_OK);
+        CHECK(keep() == 0 && used >= 22 * MiB);
+        std::vector<double> x(2 * 20 * MiB / 16, 0.5);
+        if (way == 0) CHECK(c->pool->get("y", 20 * MiB));
+        if (way == 1) CHECK(c->pool->reserve("y", 20 * MiB, c->stream));
+        if (way == 2) CHECK(hv_set_points(c, 2, (int64_t)x.size() / 2, x.data()) == HV_OK);
+        if (way == 3) {
+            HvScratch s(0, 20 * MiB, nullptr);
+            CHECK(s.p);
+        }
+        CHECK(!c->pool->get("z", 64 * MiB));   // more than there is: refused, and nothing lost
+        hv_destroy(c);
+        hv_destroy(d);
+        CHECK(hv_batch_release(0) == HV_OK && used == 0);
+    }
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "devices") return devices();
     if (what == "failed_export") return failed_export();
+    if (what == "idle_given_back") return idle_given_back();
     if (what == "released_at_exit") return released_at_exit();
     if (what == "queued_work") return queued_work();
     std::printf("no check of that name\n");
