@@ -59,6 +59,11 @@ hipError_t hv_device_malloc(int device, void** p, size_t bytes) {
     e = hipMalloc(p, bytes);
     if (e == hipSuccess) return e;
     (void)hipGetLastError();
+    hv_integrals_to_host(device);
+    hv_scratch_release(device);   // what they held
+    e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
     *p = nullptr;
     return e;
 }

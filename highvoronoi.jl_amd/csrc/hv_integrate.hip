@@ -41,6 +41,7 @@
 #include <cstring>
 #include <memory>
 #include <numeric>
+#include <set>
 
 #define HVCK(call)                                                                 \
     do {                                                                           \
@@ -1678,6 +1679,7 @@ static int finish(hv_ctx* c, int64_t ncell, const uint64_t* pkey, const double* 
     I->area = part(sizeof(double) * npair);
     I->bulk = part(sizeof(double) * ncell * nf);
     I->iface = part(sizeof(double) * npair * nf);
+    I->bytes = at;
     I->dev.reset(new HvScratch(c->device, at, c->stream));
     hipMemcpyKind kind = hipMemcpyDeviceToDevice;
     if (I->dev->p) {
@@ -1705,6 +1707,7 @@ static int finish(hv_ctx* c, int64_t ncell, const uint64_t* pkey, const double* 
     HVCK(put(I->iface, rint_d, sizeof(double) * npair * nf));
     HVCK(hipStreamSynchronize(c->stream));
     if (I->dev) I->dev->settled();   // it outlives the stream
+    hv_integral_keep(I.get());
     *out = I.release();
     return HV_OK;
 }
@@ -1877,6 +1880,7 @@ struct IntegralPart {
     size_t off, bytes;
 };
 static int integral_out(const hv_integral* I, const IntegralPart* part, int n) {
+    std::lock_guard<std::mutex> own(I->mu);
     HvCopy list[4];
     int m = 0;
     size_t lo = ~(size_t)0, hi = 0;
@@ -1925,7 +1929,44 @@ int hv_integral_export_impl(const hv_integral* I, double* vol, int64_t* nbr_ptr,
     return integral_out(I, part, 4);
 }
 
-void hv_integral_free_impl(hv_integral* I) { delete I; }
+// The integrals that may give their device memory back (never destroyed: one may be freed after this
+// library's statics).  Whoever holds live_mu takes an integral's own lock by trying only.
+static std::mutex live_mu;
+static auto& live = *new std::set<hv_integral*>();
+
+void hv_integral_keep(hv_integral* I) {
+    std::lock_guard<std::mutex> lk(live_mu);
+    live.insert(I);
+}
+
+void hv_integrals_to_host(int device) {
+    std::lock_guard<std::mutex> lk(live_mu);
+    for (hv_integral* I : live) {
+        if (I->device != device) continue;
+        std::unique_lock<std::mutex> own(I->mu, std::try_to_lock);
+        if (!own.owns_lock() || !I->dev) continue;
+        try {
+            I->host.resize(I->bytes);
+        } catch (...) {
+            continue;   // no room there either
+        }
+        const HvCopy all{I->host.data(), I->base, I->bytes};
+        if (hv_copies(device, true, &all, 1) != hipSuccess) {
+            std::vector<char>().swap(I->host);
+            continue;
+        }
+        I->base = I->host.data();
+        I->dev.reset();
+    }
+}
+
+void hv_integral_free_impl(hv_integral* I) {
+    {
+        std::lock_guard<std::mutex> lk(live_mu);
+        live.erase(I);
+    }
+    delete I;
+}
 
 #define HV_IINST(D)                                                                                 \
     template int hv_integrate_polytope_impl<D>(hv_ctx*, const hv_mesh*, hv_integral**);          \

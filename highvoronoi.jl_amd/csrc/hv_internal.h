@@ -37,7 +37,8 @@ struct DevPool {
 };
 
 // hipMalloc on the device in use (`device`): when it has no room, what the process keeps idle there
-// (HvScratch's store, the parts of destroyed contexts) is given back first.
+// (HvScratch's store, the parts of destroyed contexts) is given back first, then the integrals' results
+// move to host memory.
 hipError_t hv_device_malloc(int device, void** p, size_t bytes);
 
 // A device allocation shared by a context and the meshes built from it (the generator
@@ -212,14 +213,16 @@ struct hv_mesh {
 };
 
 // Results stay on the device until hv_integral_export copies them into the caller's memory
-// (`host` holds them when the device has no room).
+// (`host` holds them when the device has no room, or another allocation found none: mu is held
+// while they move and while they are copied out).
 struct hv_integral {
+    mutable std::mutex mu;
     int64_t N = 0, rows = 0;
     int device = 0;
     std::unique_ptr<HvScratch> dev;
     std::vector<char> host;
     char* base = nullptr;              // dev or host memory: the parts below by offset
-    size_t vol = 0, ptr = 0, nbr = 0, area = 0, bulk = 0, iface = 0;
+    size_t vol = 0, ptr = 0, nbr = 0, area = 0, bulk = 0, iface = 0, bytes = 0;
     double ms = 0.0;
     int64_t work = 0;                  // point samples: (sample, generator) distances evaluated
     double ms_kernel = 0.0;            // point samples: device time of the sampling kernel
@@ -346,3 +349,7 @@ int hv_integral_work_impl(const hv_integral* I, int64_t* work, double* ms_kernel
 int hv_integral_export_impl(const hv_integral* I, double* vol, int64_t* nbr_ptr, int64_t* nbr, double* area,
                             double* ms);
 void hv_integral_free_impl(hv_integral* I);
+// A finished integral, until it is freed: its results may move to host memory from here on.
+void hv_integral_keep(hv_integral* I);
+// The results of the device's integrals to host memory, except of one that is being copied out.
+void hv_integrals_to_host(int device);

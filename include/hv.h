@@ -312,7 +312,8 @@ int hv_integrate_mc_points(hv_ctx* ctx, const hv_mesh* mesh, int64_t nsamples, u
 /* Voronoi_Integral's parity surface (src/integral.jl:11-21): volumes[ncells]; for cell i
  * its neighbours nbr[nbr_ptr[i] .. nbr_ptr[i+1]) sorted, 1-based (planes n+p), and the
  * interface areas aligned with them.  An integral holds its results in device memory (16 bytes
- * per row and per cell, 8 nf more with an integrand) until hv_integral_free.  ms (optional) receives the device time. */
+ * per row and per cell, 8 nf more with an integrand) until hv_integral_free, or in host memory once an
+ * allocation of this library has found no room beside them.  ms (optional) receives the device time. */
 int hv_integral_counts(const hv_integral* I, int64_t* ncells, int64_t* nnbr);
 /* No counterpart in the reference (a measurement): for hv_integrate_mc_points, the (sample,
  * generator) distances its sampling kernel evaluated and that kernel's device time in ms

@@ -95,6 +95,34 @@ static int released_at_exit() {
     return 0;
 }
 
+// an integral of n cells and `rows` rows, each value told by its place, and whether its export is that
+static hv_integral* integral(int device, int64_t n, int64_t rows) {
+    (void)hipSetDevice(device);
+    hv_integral* I = new hv_integral();
+    I->N = n;
+    I->rows = rows;
+    I->device = device;
+    I->ptr = 8 * n;
+    I->nbr = I->ptr + 8 * (n + 1);
+    I->area = I->nbr + 8 * rows;
+    I->bytes = I->area + 8 * rows;
+    I->dev.reset(new HvScratch(device, I->bytes, nullptr));
+    I->dev->settled();
+    I->base = (char*)I->dev->p;
+    for (size_t k = 0; k < I->bytes / 8; ++k) ((int64_t*)I->base)[k] = 1000 + (int64_t)k;
+    return I;
+}
+static bool integral_intact(const hv_integral* I) {
+    const int64_t n = I->N, rows = I->rows;
+    std::vector<int64_t> v(2 * n + 1 + 2 * rows);   // the four arrays one after another
+    if (hv_integral_export(I, (double*)v.data(), v.data() + n, v.data() + 2 * n + 1, (double*)(v.data() + 2 * n + 1 + rows),
+                           nullptr) != HV_OK)
+        return false;
+    for (size_t k = 0; k < v.size(); ++k)
+        if (v[k] != 1000 + (int64_t)k) return false;
+    return true;
+}
+
 // Copies, the pinned block and an integral's export work on their own device, whichever the thread used last.
 static int devices() {
     std::vector<char> a(4 * MiB, 1), b(4 * MiB, 0);
@@ -111,25 +139,13 @@ static int devices() {
         CHECK(L.base && fake::S().host[L.base].device == 0);
     }
     CHECK(hipSetDevice(1) == hipSuccess);
-    hv_integral I;
-    const int64_t n = 5, rows = 20;
-    I.N = n;
-    I.rows = rows;
-    I.device = 1;
-    I.ptr = 256;
-    I.nbr = 512;
-    I.area = 1024;
-    I.dev.reset(new HvScratch(1, 2048, nullptr));
-    I.dev->settled();
-    I.base = (char*)I.dev->p;
-    for (int64_t k = 0; k < n; ++k) ((double*)(I.base + I.vol))[k] = 0.5 + k;
+    hv_integral* I = integral(1, 5, 20);
     CHECK(hipSetDevice(0) == hipSuccess);
     fake::S().copy_device.clear();
-    std::vector<double> vol(n), area(rows);
-    std::vector<int64_t> ptr(n + 1), nbr(rows);
-    CHECK(hv_integral_export(&I, vol.data(), ptr.data(), nbr.data(), area.data(), nullptr) == HV_OK);
-    CHECK(vol[3] == 3.5 && !fake::S().copy_device.empty());
+    CHECK(integral_intact(I));
+    CHECK(!fake::S().copy_device.empty());
     for (int d : fake::S().copy_device) CHECK(d == 1);
+    CHECK(hv_integral_free(I) == HV_OK);
     return 0;
 }
 
@@ -167,10 +183,29 @@ static int idle_given_back() {
     return 0;
 }
 
+// Finished integrals make room for an allocation that finds none, and keep their results; one of another
+// device stays where it is.
+static int integrals_make_room() {
+    fake::S().limit[0] = 30 * MiB;
+    hv_integral *a = integral(0, 1000, 600000), *b = integral(0, 1000, 600000), *other = integral(1, 10, 600000);   // 9.6 MB each
+    for (hv_integral* I : {a, b, other}) hv_integral_keep(I);
+    CHECK(hipSetDevice(0) == hipSuccess);
+    DevPool pool;
+    CHECK(pool.get("y", 20 * MiB));
+    CHECK(!a->dev && !b->dev && other->dev);
+    CHECK(integral_intact(a) && integral_intact(b) && integral_intact(other));
+    CHECK(hipSetDevice(0) == hipSuccess);
+    CHECK(!pool.get("z", 64 * MiB));
+    for (hv_integral* I : {a, b, other}) CHECK(hv_integral_free(I) == HV_OK);
+    hv_integrals_to_host(0);   // none is left
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "devices") return devices();
     if (what == "failed_export") return failed_export();
+    if (what == "integrals_make_room") return integrals_make_room();
     if (what == "idle_given_back") return idle_given_back();
     if (what == "released_at_exit") return released_at_exit();
     if (what == "queued_work") return queued_work();
