@@ -6300,17 +6300,29 @@ int hv_mc_points_impl(hv_ctx* c, int64_t nsamples, uint64_t seed, double slab, c
 // vertex a neighbour of the new cell, so the tested set is the same).  Every other vertex of
 // the refined mesh holds a new point and comes from the walk of the new cells.
 
-// The new points in tree order (list: their sorted positions), boxes of each 32 of them and of each
-// 1 024: a vertex tests only boxes of new points.  In the tree of the union nearly every leaf that a
-// circumsphere reaches holds old points alone (3D N=50k with 500 new points: the refinement took 1.0 of
-// its 5.2 ms longer there).
+// Which old vertices a new point takes.  Two ways, by how many of the points are new:
+// - the new points in tree order (list: their sorted positions) and boxes over them, of 32 points, of 32
+//   boxes and so on, every box of the highest level tested (at most 32 of them up to 2^25 new points):
+//   in the tree of the union nearly every leaf that a circumsphere reaches holds old points alone;
+// - the tree of the union, where it holds hardly any others.
+// Time over all old vertices in us, union's tree / boxes: 3D N=50k with 500 new points 920 / 57, 200 000
+// 1 330 / 750; 3D N=20k with 20 000 790 / 290, 320 000 (16 times N) 970 / 940, 10^6 1 120 / 1 380; 2D N=100k
+// with as many 410 / 390, twice as many 420 / 470, 10 times 540 / 720; 3D N=500k with as many 9 850 / 3 500
+// (4 200 with boxes of 1 024 points as the highest); 4D N=100 with 30 000 980 / 830, 5D N=100 with 8 000
+// 1 030 / 470, 6D N=30 with 3 000 710 / 300.
 constexpr int HV_NEW_BOX = 32, HV_NEW_SUPER = 1024;
+constexpr int HV_NEW_TOP = 3;   // highest level: boxes of 2^20 points
+struct HvNewBoxes {
+    const double* x;                     // the points' rows
+    const double* box[HV_NEW_TOP + 1];   // each level's, lo then hi
+    int n[HV_NEW_TOP + 2];               // points, then boxes of each level
+};
 struct HvNewSelect {   // positions of new points
     const int* sidx;
     int nold;
     __device__ bool operator()(int j) const { return sidx[j] >= nold; }
 };
-// One workgroup per super box, a thread per point: rows of D coordinates, boxes lo then hi.
+// Levels 0 and 1: one workgroup per box of 1024, a thread per point; also rows of D coordinates.
 template <int D>
 __global__ __launch_bounds__(HV_NEW_SUPER) void k_new_boxes(DevGeo g, const int* __restrict__ list, int m, double* __restrict__ x,
                                                             double* __restrict__ box, double* __restrict__ sup) {
@@ -6351,12 +6363,56 @@ __global__ __launch_bounds__(HV_NEW_SUPER) void k_new_boxes(DevGeo g, const int*
         sup[((int64_t)blockIdx.x * 2 + 1) * D + threadIdx.x] = c;
     }
 }
-
-// keep[t] = 1 when vertex ids[t] of the old mesh has none of the m new points strictly inside its
-// circumsphere shrunk by 1 + 1e-7
+// A further level from the one below (count boxes of it), a thread per coordinate of a box.
 template <int D>
-__global__ __launch_bounds__(256) void k_refine_keep(int m, const double* __restrict__ x, const double* __restrict__ box,
-                                                     const double* __restrict__ sup, int nv, const int* __restrict__ ids,
+__global__ __launch_bounds__(256) void k_new_level(const double* __restrict__ below, int count, double* __restrict__ level,
+                                                   int n) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / D, k = t - i * D;
+    if (i >= n) return;
+    double a = 1e300, c = -1e300;
+    for (int q = 32 * i; q < min(32 * i + 32, count); ++q) {
+        a = fmin(a, below[((int64_t)q * 2) * D + k]);
+        c = fmax(c, below[((int64_t)q * 2 + 1) * D + k]);
+    }
+    level[((int64_t)i * 2) * D + k] = a;
+    level[((int64_t)i * 2 + 1) * D + k] = c;
+}
+
+// whether a point of the boxes i0 .. i1 - 1 of level L lies within sqrt(lim) of r
+template <int D, int L>
+__device__ __forceinline__ bool hv_new_within(const HvNewBoxes& B, int i0, int i1, const double* r, double lim) {
+    if constexpr (L < 0) {
+        for (int i = i0; i < i1; ++i) {
+            double d2 = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const double a = B.x[(int64_t)i * D + k] - r[k];
+                d2 = fma(a, a, d2);
+            }
+            if (d2 < lim) return true;
+        }
+    } else {
+        bool hit = false;
+        for (int i = i0; i < i1 && !hit; ++i) {
+            const double* b = B.box[L] + (int64_t)i * 2 * D;
+            double d2 = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const double a = fmax(fmax(b[k] - r[k], r[k] - b[D + k]), 0.0);
+                d2 = fma(a, a, d2);
+            }
+            if (!(d2 < lim)) continue;
+            hit = hv_new_within<D, L - 1>(B, i * HV_NEW_BOX, min((i + 1) * HV_NEW_BOX, B.n[L]), r, lim);
+        }
+        return hit;
+    }
+    return false;
+}
+
+// keep[t] = 1 when vertex ids[t] of the old mesh has none of the new points strictly inside its
+// circumsphere shrunk by 1 + 1e-7; every box of level TOP is tested
+template <int D, int TOP>
+__global__ __launch_bounds__(256) void k_refine_keep(HvNewBoxes B, int nv, const int* __restrict__ ids,
                                                      const int* __restrict__ vkey, const double* __restrict__ vx,
                                                      const double* __restrict__ xo, uint8_t* __restrict__ keep) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -6371,33 +6427,47 @@ __global__ __launch_bounds__(256) void k_refine_keep(int m, const double* __rest
         R2 = fma(a, a, R2);
     }
     const double f = 1.0 + 1e-7;
-    const double lim = R2 / (f * f);
-    auto reached = [&](const double* b) {
-        double d2 = 0.0;
+    keep[t] = hv_new_within<D, TOP>(B, 0, B.n[TOP + 1], r, R2 / (f * f)) ? 0 : 1;
+}
+
+// the same on the tree of the union (new: original id at or above nold)
+template <int D>
+__global__ __launch_bounds__(128) void k_refine_keep_tree(DevGeo g, int nv, const int* __restrict__ ids,
+                                                          const int* __restrict__ vkey, const double* __restrict__ vx,
+                                                          const double* __restrict__ xo, int nold,
+                                                          uint8_t* __restrict__ keep) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nv) return;
+    const int64_t v = ids[t];
+    const int64_t g0 = vkey[v * (D + 1)];   // the smallest id of a key is a generator
+    double r[D], R2 = 0.0;
 #pragma unroll
-        for (int k = 0; k < D; ++k) {
-            const double a = fmax(fmax(b[k] - r[k], r[k] - b[D + k]), 0.0);
-            d2 = fma(a, a, d2);
-        }
-        return d2 < lim;
-    };
+    for (int k = 0; k < D; ++k) {
+        r[k] = vx[v * D + k];
+        const double a = xo[g0 * D + k] - r[k];
+        R2 = fma(a, a, R2);
+    }
+    const double f = 1.0 + 1e-7;
+    const double lim = R2 / (f * f);
     bool hit = false;
-    for (int s = 0; s * HV_NEW_SUPER < m && !hit; ++s) {
-        if (!reached(sup + (int64_t)s * 2 * D)) continue;
-        const int b1 = min((s + 1) * (HV_NEW_SUPER / HV_NEW_BOX), (m + HV_NEW_BOX - 1) / HV_NEW_BOX);
-        for (int b = s * (HV_NEW_SUPER / HV_NEW_BOX); b < b1 && !hit; ++b) {
-            if (!reached(box + (int64_t)b * 2 * D)) continue;
-            const int i1 = min((b + 1) * HV_NEW_BOX, m);
-            for (int i = b * HV_NEW_BOX; i < i1; ++i) {
+    int node = 1;
+    while (node && !hit) {
+        if (hv_box_d2<D>(g, node, r) < lim) {
+            if (node < g.P2) { node = 2 * node; continue; }
+            const int leaf = node - g.P2;
+            const int j0 = leaf * g.L, j1 = min(j0 + g.L, g.n);
+            for (int j = j0; j < j1; ++j) {
+                if (g.sidx[j] < nold) continue;
                 double d2 = 0.0;
 #pragma unroll
                 for (int k = 0; k < D; ++k) {
-                    const double a = x[(int64_t)i * D + k] - r[k];
+                    const double a = g.xs[(int64_t)j * (D + 1) + k] - r[k];
                     d2 = fma(a, a, d2);
                 }
                 if (d2 < lim) { hit = true; break; }
             }
         }
+        node = hv_next_node(node);
     }
     keep[t] = hit ? 0 : 1;
 }
@@ -6439,13 +6509,31 @@ int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** o
     if (!keep || !sel || !dcnt) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
     int nkeep = 0;
     if (nv0 > 0) {
-        const int m = shift, nsup = (m + HV_NEW_SUPER - 1) / HV_NEW_SUPER;
-        int* list = pget<int>(c, "rf_list", (size_t)std::max(m, 1));
-        double* nx = pget<double>(c, "rf_x", (size_t)std::max(m, 1) * D);
-        double* nbox = pget<double>(c, "rf_box", (size_t)std::max(nsup, 1) * (HV_NEW_SUPER / HV_NEW_BOX) * 2 * D);
-        double* nsupb = pget<double>(c, "rf_sup", (size_t)std::max(nsup, 1) * 2 * D);
-        if (!list || !nx || !nbox || !nsupb) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
-        if (m > 0) {
+        const int m = shift;
+        // (the line where the tree of the union takes less: see above)
+        const bool by_tree = D <= 3 && m > (D == 2 ? 2 : 16) * old->N;
+        if (by_tree) {
+            k_refine_keep_tree<D><<<nblk(nv0, 128), 128, 0, c->stream>>>(T.g, nv0, (const int*)old->ids.p, (const int*)old->key.p,
+                                                                        (const double*)old->x.p, (const double*)c->xw->p, nold,
+                                                                        keep);
+        } else {
+            HvNewBoxes B{};
+            size_t first[HV_NEW_TOP + 2] = {};   // of each level's boxes
+            B.n[0] = m;
+            for (int l = 0; l <= HV_NEW_TOP; ++l) {
+                B.n[l + 1] = (B.n[l] + HV_NEW_BOX - 1) / HV_NEW_BOX;
+                first[l + 1] = first[l] + B.n[l + 1];
+            }
+            int* list = pget<int>(c, "rf_list", (size_t)std::max(m, 1));
+            double* nx = pget<double>(c, "rf_x", (size_t)std::max(m, 1) * D);
+            double* box = pget<double>(c, "rf_box", std::max<size_t>(first[HV_NEW_TOP + 1], 1) * 2 * D);
+            if (!list || !nx || !box) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (refine)");
+            B.x = nx;
+            double* level[HV_NEW_TOP + 1];
+            for (int l = 0; l <= HV_NEW_TOP; ++l) B.box[l] = level[l] = box + first[l] * 2 * D;
+            // up to 32 boxes of the highest level that is tested
+            int top = 1;
+            while (top < HV_NEW_TOP && B.n[top + 1] > HV_NEW_BOX) ++top;
             size_t ts = 0;
             hipcub::CountingInputIterator<int> it(0);
             const HvNewSelect isnew{T.g.sidx, nold};
@@ -6453,12 +6541,20 @@ int hv_refine_merge(hv_ctx* c, const hv_mesh* old, const hv_mesh* S, hv_mesh** o
             void* tmp = c->pool->get("cubtmp2", ts, false, c->stream);
             if (!tmp) return hv_fail(c, HV_ERR_DEVICE, "out of device memory (select)");
             HVCK(hipcub::DeviceSelect::If(tmp, ts, it, list, dcnt, (int)c->N, isnew, c->stream));
-            k_new_boxes<D><<<nsup, HV_NEW_SUPER, 0, c->stream>>>(T.g, list, m, nx, nbox, nsupb);
+            k_new_boxes<D><<<B.n[2], HV_NEW_SUPER, 0, c->stream>>>(T.g, list, m, nx, level[0], level[1]);
             HVCK(hipGetLastError());
+            for (int l = 2; l <= top; ++l) {
+                k_new_level<D><<<nblk((int64_t)B.n[l + 1] * D, 256), 256, 0, c->stream>>>(level[l - 1], B.n[l], level[l], B.n[l + 1]);
+                HVCK(hipGetLastError());
+            }
+            auto test = [&](auto kernel) {
+                kernel<<<nblk(nv0, 256), 256, 0, c->stream>>>(B, nv0, (const int*)old->ids.p, (const int*)old->key.p,
+                                                              (const double*)old->x.p, (const double*)c->xw->p, keep);
+            };
+            if (top == 1) test(k_refine_keep<D, 1>);
+            else if (top == 2) test(k_refine_keep<D, 2>);
+            else test(k_refine_keep<D, 3>);
         }
-        k_refine_keep<D><<<nblk(nv0, 256), 256, 0, c->stream>>>(m, nx, nbox, nsupb, nv0, (const int*)old->ids.p,
-                                                               (const int*)old->key.p, (const double*)old->x.p,
-                                                               (const double*)c->xw->p, keep);
         HVCK(hipGetLastError());
         size_t tb = 0;
         HVCK(hipcub::DeviceSelect::Flagged(nullptr, tb, (const int*)old->ids.p, keep, sel, dcnt, nv0, c->stream));
