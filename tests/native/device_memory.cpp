@@ -5,6 +5,7 @@
 #include <unistd.h>
 #include <memory>
 #include <string>
+#include <thread>
 
 #define CHECK(c)                                                            \
     do {                                                                    \
@@ -201,10 +202,27 @@ static int integrals_make_room() {
     return 0;
 }
 
+// A thread that finds the staging taken copies all the same, and gets no lease.
+static int staging_taken() {
+    HvLease held(0);
+    CHECK(held.base);
+    int bad = 0;
+    std::thread other([&]() {
+        HvLease second(0);
+        std::vector<char> a(4 * MiB, 3), b(4 * MiB, 0);
+        const HvCopy one{b.data(), a.data(), a.size()};
+        bad = second.base != nullptr || hv_copies(0, false, &one, 1) != hipSuccess || a != b;
+    });
+    other.join();
+    CHECK(bad == 0 && fake::waiting() == 0);
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "devices") return devices();
     if (what == "failed_export") return failed_export();
+    if (what == "staging_taken") return staging_taken();
     if (what == "integrals_make_room") return integrals_make_room();
     if (what == "idle_given_back") return idle_given_back();
     if (what == "released_at_exit") return released_at_exit();

@@ -21,7 +21,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["failed_export", "queued_work", "released_at_exit", "devices", "idle_given_back",
-                                   "integrals_make_room"])
+                                   "integrals_make_room", "staging_taken"])
 def test_device_memory(program, check):
     r = subprocess.run([program, check], timeout=120, capture_output=True, text=True,
                        env=dict(os.environ, MALLOC_PERTURB_="90"))   # freed memory is filled
