@@ -923,8 +923,9 @@ __device__ __forceinline__ void hv_wave_sync() {
 }
 
 constexpr double HV_W = 1e-7;
-// Rays are ordered by the top 32 of the 60 Morton bits of their ball centre (2^(32/d) cells
-// per axis: far finer than a level's rays are spread), half the radix passes of all 60.
+// Where rays are sorted (large ray batches, walks in chunks) it is by the top 32 of the 60 Morton bits of
+// their ball centre (2^(32/d) cells per axis: far finer than a level's rays are spread), half the
+// radix passes of all 60.
 constexpr int HV_RAY_SORT_LO = 28;
 
 
@@ -1308,9 +1309,10 @@ __global__ __launch_bounds__(256) void k_ray_init16(DevGeo g0, GeoSet F, DevRays
 
 // A level of at most this many rays is small: started 16 lanes a ray, scanned a wavefront a ray
 // (k_raycast1).  Both take longer than a thread a ray and packets once the chip is full, the earlier
-// the more a ray reaches.  Start and scan of one level, against packets: 3D, 8 to 32 thousand rays
-// 26 against 148 us, larger 301 against 185 us; 4D and 5D, 8 to 32 thousand rays 111 against 96 and 102
-// against 86 us; 3D levels of a few hundred rays (a refinement's) 20 against 127 us.
+// the more a ray reaches.  Start and scan of one level, against packets (us, rays of the level in
+// thousands): 2D 32-64 60 / 111, 128-256 300 / 219; 3D 8-16 27 / 123, 32-64 90 / 114, 64-128 269 / 120; 4D 8-16
+// 52 / 77, 16-32 87 / 84; 5D 8-16 40 / 64, 16-32 92 / 72; 6D 4-8 36 / 93, 8-16 55 / 87, 32-64 141 / 94; 3D levels of
+// a few hundred rays (a refinement's) 20 / 127.
 constexpr int hv_small_level(int D) { return D <= 3 ? 1 << 15 : 1 << 13; }
 template <int D, bool B>
 static void launch_ray_init(const DevGeo& g, const GeoSet& F, const DevRays& R, int n, const int* vkey, const double* vx,
@@ -1988,7 +1990,7 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
     // workgroups spread over cstride copies (same-address atomics from every packet, one per
     // wavefront, cost about 1 ms per build at 5D N=100k)
     unsigned long long* __restrict__ ctr = ctr0 + (cstride > 1 ? blockIdx.x % (unsigned)cstride : 0u);
-    // MODE 0: the staged leaf (FP64).  MODE 1: ray K-vectors of the current node (MFMA B
+    // MODE 0: the staged leaf (FP64).  MODE 1: ray K-vectors of the current node (MFMA A
     // operand source, 80-byte rows).  MODE 2: the staged leaf (FP32 rows relative to the
     // group origin).  MODE 1 and 2: the sorted ids of each ray's edge generators (the
     // candidates it already holds) and the group origin.
@@ -2192,7 +2194,7 @@ __global__ __launch_bounds__(64, MODE == 1 ? 4 : 1) void k_raycast64(DevGeo g0, 
         const int i = gid - off;
         if (l + 1 == g.h) {
             if constexpr (MODE == 0) {
-                // children are leaves: nearest first, the next one loaded while this one is scanned
+                // children are leaves: as they come, the next one loaded while this one is scanned
                 double pf[D + 1];
                 unsigned rr = rem;
                 int cc = __builtin_ctz(rr);
